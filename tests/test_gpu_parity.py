@@ -1078,6 +1078,47 @@ def test_random_shapes_every_operator_against_fp32_products():
         _close("dW_gate alone", ops_bwd.dw_bwd(dg, x), f(dg).T @ f(x))
 
 
+@pytest.mark.parametrize(
+    "M,K,N",
+    [
+        (32, 32, 32),        # one partial reduction tile in every GEMM
+        (1, 8, 8),           # a single chunk of it
+        (257, 120, 136),     # one whole tile and all but one chunk of the next; one chunk of a third
+        (130, 1096, 2056),   # split reductions (several workgroups per tile), rotated start
+        (4500, 3272, 3400),  # large tiles, thin last round: stream-K or two launches
+    ],
+)
+def test_reduction_tails_every_operator_against_fp32_products(M, K, N):
+    """Reduction lengths that end inside a 64-wide reduction tile.  What the tail of a row would alias
+    if it were not cut off is the start of the next row, so every row of the left operand starts with
+    8 elements 64 times the usual size: one aliased chunk is far outside the tolerance, whatever the
+    other operand holds there."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    print(f"reduction tails: M={M} K={K} N={N}", flush=True)
+    g = torch.Generator().manual_seed(5)
+    rnd = lambda *shape, s=1.0: s * torch.randn(*shape, generator=g)
+
+    def heavy(t):
+        t[:, :8] *= 64.0
+        return t.half().to(dev)
+
+    f = lambda t: t.float().cpu()
+    x, dy, h = heavy(rnd(M, K, s=0.1)), heavy(rnd(M, K, s=0.1)), heavy(rnd(M, N, s=0.1))
+    dg, du = heavy(rnd(M, N, s=0.1)), heavy(rnd(M, N, s=0.1))
+    wg, wu, wd = (rnd(*s, s=0.03).half().to(dev) for s in ((N, K), (N, K), (K, N)))
+    hs = ops_fwd.gateup_fwd(x, wg, None, wu, None, save_activations=True)
+    _close("G", hs.gate, f(x) @ f(wg).T)
+    _close("U", hs.up, f(x) @ f(wu).T)
+    _close("Y", ops_fwd.linear_fwd(h, wd), f(h) @ f(wd).T)
+    ones = torch.ones_like(hs.up)
+    du_got = ops_bwd.dh_bwd(dy, wd, ones, ones, act_fn="no_act")[1]  # dU = dH
+    _close("dH", du_got, f(dy) @ f(wd))
+    _close("dX", ops_bwd.dx_bwd(dg, du, wg, wu), f(dg) @ f(wg) + f(du) @ f(wu))
+
+
 def test_random_modules_through_the_one_call_entries_no_worse_than_torch_16bit():
     """Four dozen seeded random modules (token counts 1 to 6144, widths that are multiples of 8, 64
     or 256, both 16-bit dtypes, biases, dropout, five activations) through FusedGatedMLP, i.e. through

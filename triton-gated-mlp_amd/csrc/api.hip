@@ -132,19 +132,18 @@ int group_tile_class(int64_t large_tiles, int64_t medium_tiles) {
 // Tile class for an output of rows x cols with reduction length red (all in elements).
 // The pipelined kernels (LARGE: 256 x bn_large tiles, one workgroup per CU; MEDIUM_FULL: tiles of
 // half that in each direction, two per CU) take any rows and cols; they need 32-bit byte offsets
-// into the operands, padded to whole tiles, and a reduction that is a multiple of 64 unless both
-// operands are reduction-strided (`both_ks`).  Everything else runs on the predicated MEDIUM class.
+// into the operands, padded to whole tiles.  Everything else runs on the predicated MEDIUM class.
 // Between the two pipelined classes the choice is estimated time in rounds of workgroups: a round
 // of small tiles (two per CU) takes 2/3 of a round of large ones (a quarter of the work at 75 % of
 // the throughput, two at a time), and a last round filled to the fraction f costs 0.6 + 0.4 f of
 // a full one (the busy CUs clock higher, but not in proportion; fitted to measurements).
-int pick_tile(int dtype, int64_t rows, int64_t cols, int64_t red, int bn_large, bool both_ks = false) {
+int pick_tile(int dtype, int64_t rows, int64_t cols, int64_t red, int bn_large) {
   if (dtype == GMLP_F32) return gmlp::TILE_MEDIUM;  // the float32 kernel has one tile shape
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
   // the buffer base sits up to 4 KB below the operand (shared-M0 loads)
   const int64_t limit = ((int64_t)1 << 31) - 4096;
   bool offsets_fit = up(rows, 256) * up(red, 64) * 2 < limit && up(cols, 256) * up(red, 64) * 2 < limit;
-  if (!offsets_fit || (red % 64 != 0 && !both_ks)) return gmlp::TILE_MEDIUM;
+  if (!offsets_fit) return gmlp::TILE_MEDIUM;
   const int64_t large_tiles = (up(rows, 256) / 256) * (up(cols, bn_large) / bn_large);
   const int64_t medium_tiles = (up(rows, 128) / 128) * (up(cols, bn_large / 2) / (bn_large / 2));
   return group_tile_class(large_tiles, medium_tiles);
@@ -282,26 +281,26 @@ size_t gmlp_workspace_bytes(int op, int64_t M, int64_t K, int64_t N, int dtype) 
   // Each operation asks for the larger of what its split-reduction form (short batches) and its
   // stream-K form (large tiles whose grid ends in a thinly filled round) would use.
   auto larger = [](size_t a, size_t b) { return a > b ? a : b; };
-  auto sk = [&](int64_t rows, int64_t cols, int64_t red_tiles, int bn, bool both_ks = false) -> size_t {
-    if (pick_tile(dtype, rows, cols, red_tiles * 64, bn, both_ks) != gmlp::TILE_LARGE) return 0;
+  auto sk = [&](int64_t rows, int64_t cols, int64_t red_tiles, int bn) -> size_t {
+    if (pick_tile(dtype, rows, cols, red_tiles * 64, bn) != gmlp::TILE_LARGE) return 0;
     return plan_streamk(dtype, cdiv(rows, 256) * cdiv(cols, bn), red_tiles).ws_bytes;
   };
   // gmlp_gateup_fwd(M, K, N): two accumulator sets [M,N], reduction K
   if (op == GMLP_OP_GATEUP_FWD)
     return larger(split_workspace_bytes(pick_splits(dtype, M, N, K, (K + 63) / 64, 128), M, N, 2),
-                  K % 64 == 0 ? sk(M, N, K / 64, 128) : 0);
+                  sk(M, N, cdiv(K, 64), 128));
   // gmlp_linear_fwd(M, R = K, C = N): out [M,N], reduction K
   if (op == GMLP_OP_LINEAR_FWD)
     return larger(split_workspace_bytes(pick_splits(dtype, M, N, K, (K + 63) / 64), M, N),
-                  K % 64 == 0 ? sk(M, N, K / 64, 256) : 0);
+                  sk(M, N, cdiv(K, 64), 256));
   // gmlp_dx_bwd(M, K, N): out [M,K], reduction over two segments of N
   if (op == GMLP_OP_DX_BWD)
     return larger(split_workspace_bytes(pick_splits(dtype, M, K, N, 2 * ((N + 63) / 64)), M, K),
-                  N % 64 == 0 ? sk(M, K, 2 * (N / 64), 256) : 0);
+                  sk(M, K, 2 * cdiv(N, 64), 256));
   // gmlp_dh_bwd(M, K, N): out [M,N], reduction K
-  if (op == GMLP_OP_DH_BWD) return K % 64 == 0 ? sk(M, N, K / 64, 256) : 0;
+  if (op == GMLP_OP_DH_BWD) return sk(M, N, cdiv(K, 64), 256);
   // gmlp_dw_bwd(Mred = M, R = K, C = N): out [K,N], reduction over the M token rows
-  if (op == GMLP_OP_DW_BWD) return sk(K, N, (M + 63) / 64, 256, true);
+  if (op == GMLP_OP_DW_BWD) return sk(K, N, (M + 63) / 64, 256);
   return 0;
 }
 
@@ -360,7 +359,7 @@ int gmlp_gateup_fwd(const void* x, const void* w_gate, const void* w_up, const v
     if (dtype != GMLP_F32 && pick_tile(dtype, M, N, K, 128) == TILE_LARGE) {
       const int64_t tiles_m = (M + 255) / 256, tiles_n = (N + 127) / 128, cus = num_cu();
       // a long reduction: the tiles of the last round are shared out by reduction range instead
-      const StreamK sk = plan_streamk(dtype, tiles_m * tiles_n, K / 64);
+      const StreamK sk = plan_streamk(dtype, tiles_m * tiles_n, cdiv(K, 64));
       if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, N, false, TILE_LARGE, &sk);
       const int64_t rounds = tiles_m * tiles_n / cus, tail = tiles_m * tiles_n % cus;
       const int64_t whole_cols = rounds * cus / tiles_m;  // tile columns of the whole rounds
@@ -413,7 +412,7 @@ int gmlp_linear_fwd(const void* a, const void* w, const void* bias, void* out, i
     // gmlp_gateup_fwd)
     if (dtype != GMLP_F32 && pick_tile(dtype, M, C, R, 256) == TILE_LARGE) {
       const int64_t tiles_m = (M + 255) / 256, tiles_n = (C + 255) / 256, cus = num_cu();
-      const StreamK sk = plan_streamk(dtype, tiles_m * tiles_n, R / 64);
+      const StreamK sk = plan_streamk(dtype, tiles_m * tiles_n, cdiv(R, 64));
       if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, C, false, TILE_LARGE, &sk);
       const int64_t rounds = tiles_m * tiles_n / cus, tail = tiles_m * tiles_n % cus;
       const int64_t whole_cols = rounds * cus / tiles_m;
@@ -461,7 +460,7 @@ int gmlp_dh_bwd(const void* dy, const void* w_down, const void* g, const void* u
       return launch_dh<T>(force_class >= 0 ? force_class : pick_tile(dtype, rows, N, K, 256), ga, ea, s);
     };
     if (dtype != GMLP_F32 && pick_tile(dtype, M, N, K, 256) == TILE_LARGE) {
-      const StreamK sk = plan_streamk(dtype, cdiv(M, 256) * cdiv(N, 256), K / 64);
+      const StreamK sk = plan_streamk(dtype, cdiv(M, 256) * cdiv(N, 256), cdiv(K, 64));
       if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, M, TILE_LARGE, &sk);
     }
     int64_t whole = whole_round_tile_rows(dtype, M, N, K);
@@ -536,7 +535,7 @@ int gmlp_dx_bwd(const void* dg, const void* du, const void* w_gate, const void* 
       return launch_dx<T>(force_class >= 0 ? force_class : pick_tile(dtype, rows, K, N, 256), ga, ea, s);
     };
     if (dtype != GMLP_F32 && pick_tile(dtype, M, K, N, 256) == TILE_LARGE) {
-      const StreamK sk = plan_streamk(dtype, cdiv(M, 256) * cdiv(K, 256), 2 * (N / 64));
+      const StreamK sk = plan_streamk(dtype, cdiv(M, 256) * cdiv(K, 256), 2 * cdiv(N, 64));
       if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, M, false, TILE_LARGE, &sk);
     }
     int64_t whole = whole_round_tile_rows(dtype, M, K, N);
@@ -566,7 +565,7 @@ int gmlp_dw_bwd(const void* lhs, const void* rhs, void* dw, int64_t Mred, int64_
   ga.A[0] = lhs; ga.A[1] = lhs; ga.B[0] = rhs; ga.B[1] = rhs;
   ga.M = (int)R; ga.N = (int)C; ga.K = (int)Mred; ga.lda = (int)R; ga.ldb = (int)C;
   ga.nseg = 1; ga.group_m = pick_group(R, C);
-  int tc = pick_tile(dtype, R, C, Mred, 256, true);
+  int tc = pick_tile(dtype, R, C, Mred, 256);
   if (tc == TILE_LARGE) use_streamk(plan_streamk(dtype, cdiv(R, 256) * cdiv(C, 256), cdiv(Mred, 64)), ga, workspace, workspace_bytes);
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = by_dtype(dtype, [&](auto tag) {
@@ -582,7 +581,7 @@ size_t gmlp_dw_bwd_grouped_workspace_bytes(int count, int64_t Mred, const int64_
   if (count < 1 || count > GEMM_GROUP_MAX || R == nullptr || C == nullptr || Mred < 1 || dtype == GMLP_F32) return 0;
   int64_t tiles256 = 0, tiles128 = 0;
   for (int i = 0; i < count; ++i) {
-    if (R[i] < 1 || C[i] < 1 || pick_tile(dtype, R[i], C[i], Mred, 256, true) == TILE_MEDIUM) return 0;
+    if (R[i] < 1 || C[i] < 1 || pick_tile(dtype, R[i], C[i], Mred, 256) == TILE_MEDIUM) return 0;
     tiles256 += cdiv(R[i], 256) * cdiv(C[i], 256);
     tiles128 += cdiv(R[i], 128) * cdiv(C[i], 128);
   }
@@ -609,7 +608,7 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
     if (int rc = check_mult8(__func__, "R", R[i])) return rc;
     if (int rc = check_mult8(__func__, "C", C[i])) return rc;
     GMLP_REQUIRE_ALIGNED(lhs[i]); GMLP_REQUIRE_ALIGNED(rhs[i]); GMLP_REQUIRE_ALIGNED(dw[i]);
-    pipelined = pipelined && pick_tile(dtype, R[i], C[i], Mred, 256, true) != TILE_MEDIUM;
+    pipelined = pipelined && pick_tile(dtype, R[i], C[i], Mred, 256) != TILE_MEDIUM;
   }
   if (!pipelined) {
     for (int i = 0; i < count; ++i)
@@ -654,7 +653,7 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
       if (cols_fit && (!rows_fit || by_cols * tr <= by_rows * tc)) band_cols = C[last] - (tc - by_cols) * 256;
       else if (rows_fit) band_rows = R[last] - (tr - by_rows) * 256;
       const int64_t br = band_rows ? band_rows : R[last], bc = band_cols ? band_cols : C[last];
-      if ((band_rows || band_cols) && pick_tile(dtype, br, bc, Mred, 256, true) == TILE_MEDIUM) band_rows = band_cols = 0;
+      if ((band_rows || band_cols) && pick_tile(dtype, br, bc, Mred, 256) == TILE_MEDIUM) band_rows = band_cols = 0;
     }
   }
   hipError_t e = by_dtype(dtype, [&](auto tag) -> hipError_t {
@@ -684,7 +683,7 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
       ga.N = (int)(C[last] - c0);
       ga.group_m = pick_group(ga.M, ga.N);
       typename EpiStore<T>::Args ea = {(T*)dw[last] + r0 * C[last] + c0, nullptr, (int)C[last]};
-      return launch_dw<T>(pick_tile(dtype, ga.M, ga.N, Mred, 256, true), ga, ea, s);
+      return launch_dw<T>(pick_tile(dtype, ga.M, ga.N, Mred, 256), ga, ea, s);
     }
   });
   return hip_result(__func__, e);

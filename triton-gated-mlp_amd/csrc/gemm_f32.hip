@@ -159,19 +159,19 @@ static hipError_t launch_f32(const GemmArgs& ga, const typename Epi::Args& ea, h
 }
 
 template <>
-hipError_t launch_gateup<float>(int, const GemmArgs& ga, const EpiGateUp<float>::Args& ea, hipStream_t s) {
+hipError_t launch_gateup_kt<float, false>(int, const GemmArgs& ga, const EpiGateUp<float>::Args& ea, hipStream_t s) {
   return launch_f32<false, false, 2, EpiGateUp<float>>(ga, ea, s);
 }
 template <>
-hipError_t launch_linear<float>(int, const GemmArgs& ga, const EpiStore<float>::Args& ea, hipStream_t s) {
+hipError_t launch_linear_kt<float, false>(int, const GemmArgs& ga, const EpiStore<float>::Args& ea, hipStream_t s) {
   return launch_f32<false, false, 1, EpiStore<float>>(ga, ea, s);
 }
 template <>
-hipError_t launch_dh<float>(int, const GemmArgs& ga, const EpiDh<float>::Args& ea, hipStream_t s) {
+hipError_t launch_dh_kt<float, false>(int, const GemmArgs& ga, const EpiDh<float>::Args& ea, hipStream_t s) {
   return launch_f32<false, true, 1, EpiDh<float>>(ga, ea, s);
 }
 template <>
-hipError_t launch_dx<float>(int, const GemmArgs& ga, const EpiStore<float>::Args& ea, hipStream_t s) {
+hipError_t launch_dx_kt<float, false>(int, const GemmArgs& ga, const EpiStore<float>::Args& ea, hipStream_t s) {
   return launch_f32<false, true, 1, EpiStore<float>>(ga, ea, s);
 }
 template <>

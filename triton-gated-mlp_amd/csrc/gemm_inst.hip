@@ -1,5 +1,7 @@
-// One translation unit per (dtype, GEMM kind): compiled with -DGMLP_DT=<0|1> -DGMLP_KIND=<0..4>
-// so the kernels build in parallel.  Each unit instantiates every tile class.
+// One translation unit per (dtype, GEMM kind, reduction tail): compiled with -DGMLP_DT=<0|1>
+// -DGMLP_KIND=<0..4> -DGMLP_KT=<0|1> so the kernels build in parallel.  Each unit instantiates
+// every tile class; GMLP_KT=1 are the kernels for reduction lengths that are not a multiple of 64
+// (kinds with a reduction-contiguous operand, 0..3), which have no predicated class.
 #include "gemm_pipelined.hpp"
 #include "launch.hpp"
 
@@ -11,10 +13,12 @@ typedef f16 DT;
 typedef bf16 DT;
 #endif
 
+constexpr bool KT = GMLP_KT;
+
 #define GMLP_LARGE(AKS, BKS, NB, EPI, BN_L) \
-  launch_gemm_pipelined<DT, 256, BN_L, 16, 2, 2, AKS, BKS, NB, EPI<DT>>
+  launch_gemm_pipelined<DT, 256, BN_L, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M) \
-  launch_gemm_pipelined<DT, 128, BN_M, 16, 2, 2, AKS, BKS, NB, EPI<DT>>
+  launch_gemm_pipelined<DT, 128, BN_M, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_LARGE_GROUP \
   launch_gemm_group_pipelined<DT, 256, 256, 16, 2, 2, true, true, 1, EpiStore<DT>>
 #define GMLP_MEDIUM_GROUP \
@@ -23,11 +27,12 @@ typedef bf16 DT;
 #define GMLP_DISPATCH(AKS, BKS, NB, EPI, BN_L, BN_M)                                             \
   if (tile_class == TILE_LARGE) return GMLP_LARGE(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
   if (tile_class == TILE_MEDIUM_FULL) return GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M)(ga, ea, s);    \
-  return launch_gemm<DT, 128, BN_M, 64, 2, 2, AKS, BKS, NB, true, EPI<DT>>(ga, ea, s);
+  if constexpr (KT) return hipErrorInvalidValue; /* launch.hpp sends it to the other unit */       \
+  else return launch_gemm<DT, 128, BN_M, 64, 2, 2, AKS, BKS, NB, true, EPI<DT>>(ga, ea, s);
 
 #if GMLP_KIND == 0
 template <>
-hipError_t launch_gateup<DT>(int tile_class, const GemmArgs& ga, const EpiGateUp<DT>::Args& ea,
+hipError_t launch_gateup_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiGateUp<DT>::Args& ea,
                              hipStream_t s) {
   // the usual case (SiLU, no keep-mask output) has kernels of its own, see EpiGateUpPacked
   if (EpiGateUpPacked<DT>::packed_eligible(ea)) {
@@ -37,34 +42,34 @@ hipError_t launch_gateup<DT>(int tile_class, const GemmArgs& ga, const EpiGateUp
   GMLP_DISPATCH(false, false, 2, EpiGateUp, 128, 64)
 }
 template <>
-hipError_t launch_gateup_split<DT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
-  return launch_gemm_pipelined<DT, 128, 64, 16, 2, 2, false, false, 2, EpiPartial<DT>>(ga, ea, s);
+hipError_t launch_gateup_split_kt<DT, KT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+  return launch_gemm_pipelined<DT, 128, 64, 16, 2, 2, false, false, 2, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 1
 template <>
-hipError_t launch_linear<DT>(int tile_class, const GemmArgs& ga, const EpiStore<DT>::Args& ea,
+hipError_t launch_linear_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiStore<DT>::Args& ea,
                              hipStream_t s) {
   GMLP_DISPATCH(false, false, 1, EpiStore, 256, 128)
 }
 template <>
-hipError_t launch_linear_split<DT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
-  return launch_gemm_pipelined<DT, 128, 128, 16, 2, 2, false, false, 1, EpiPartial<DT>>(ga, ea, s);
+hipError_t launch_linear_split_kt<DT, KT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+  return launch_gemm_pipelined<DT, 128, 128, 16, 2, 2, false, false, 1, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 2
 template <>
-hipError_t launch_dh<DT>(int tile_class, const GemmArgs& ga, const EpiDh<DT>::Args& ea,
+hipError_t launch_dh_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiDh<DT>::Args& ea,
                          hipStream_t s) {
   GMLP_DISPATCH(false, true, 1, EpiDh, 256, 128)
 }
 #elif GMLP_KIND == 3
 template <>
-hipError_t launch_dx<DT>(int tile_class, const GemmArgs& ga, const EpiStore<DT>::Args& ea,
+hipError_t launch_dx_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiStore<DT>::Args& ea,
                          hipStream_t s) {
   GMLP_DISPATCH(false, true, 1, EpiStore, 256, 128)
 }
 template <>
-hipError_t launch_dx_split<DT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
-  return launch_gemm_pipelined<DT, 128, 128, 16, 2, 2, false, true, 1, EpiPartial<DT>>(ga, ea, s);
+hipError_t launch_dx_split_kt<DT, KT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+  return launch_gemm_pipelined<DT, 128, 128, 16, 2, 2, false, true, 1, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 4
 template <>

@@ -12,9 +12,12 @@
 //   * M and N need not be multiples of the tile: rows of a KC operand beyond the last one lie
 //     beyond its end; columns of a KS operand beyond the last one alias the next reduction row,
 //     which only feeds output rows/columns that the epilogue does not store.
-//   * K need not be a multiple of 64 when BOTH operands are KS (reduction rows beyond K lie beyond
-//     the end: the weight gradients, whose reduction runs over the tokens).  With a KC operand K
-//     must be a multiple of 64 (its tail would alias the next row); the host checks.
+//   * K need not be a multiple of 64: reduction rows of a KS operand beyond K lie beyond its end.
+//     The last reduction tile of a KC operand would alias the next row there; the kernels for such
+//     K (KT) push the 16-byte chunks beyond K out of the descriptor, so that they read as zero too
+//     (one v_and_or per load; instances of their own because the loop of the others is tuned to the
+//     instruction).  Against the predicated kernel of gemm.hpp, which such K took before, at
+//     M=1357, K=1160, N=3096 (bf16, us): gate/up 67 -> 51, down 57 -> 28, dH 67 -> 36, dX 125 -> 45.
 //
 // Per 512/MI-wide reduction step a wavefront issues G groups of TM MFMAs: group g multiplies one
 // B fragment (accumulator set b, column block j; G = NB * TN) with the step's TM A fragments.
@@ -87,7 +90,7 @@ struct PipeConfig {
 };
 
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
-          typename Epi, bool SK = false>
+          typename Epi, bool SK = false, bool KT = false>
 __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const typename Epi::Args& ea_in,
                                                     int pid, int nwg) {
   typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi>()> Cfg;
@@ -184,6 +187,29 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
   const buffer_rsrc rb[2] = {make_rsrc((const char*)ga.B[0] - DMA_BIAS, b_bytes),
                              make_rsrc((const char*)ga.B[1] - DMA_BIAS, b_bytes)};
 
+  // KT: chunks of 8 reduction elements beyond K in the last reduction tile of a KC operand.  A lane
+  // fetches chunk (lane % 8) ^ swz(row) of its row, and swz depends on the load's number only by
+  // its parity (8 rows per load), so two masks per lane say which of its loads to drop there:
+  // bit 31 puts an offset beyond the end of any operand (they are smaller than 2 GiB).
+  uint32_t oob[2] = {0u, 0u};
+  if constexpr (KT) {
+    const int kvalid = ga.K - (kt_seg - 1) * BK;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      oob[p] = ((lane & 7) ^ ((4 * p + (lane >> 4)) & 7)) * 8 >= kvalid ? 0x80000000u : 0u;
+  }
+  static_assert(!KT || (ATile::PER_WAVE % 2 == 0 && BTile::PER_WAVE % 2 == 0), "chunk masks go by the load's parity");
+  // Offset of load i of an operand: `soff` says whether the load state stands at the last
+  // reduction tile of the operand's rows, whose first tile is at `org`.
+  auto kt_offset = [&](uint32_t off, int i, uint32_t soff, uint32_t org) __attribute__((always_inline)) {
+    if constexpr (KT) {
+      const uint32_t at_tail = soff == org + (uint32_t)(kt_seg - 1) * (BK * 2) ? 0xFFFFFFFFu : 0u;
+      return off | (oob[i & 1] & at_tail);
+    } else {
+      return off;
+    }
+  };
+
   // Global->LDS load number x (0 .. L-1) of this wavefront for reduction tile kt_req: operand and
   // index within the operand's loads.
   auto load_index = [](int x) __attribute__((always_inline)) {
@@ -261,13 +287,13 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
     uint32_t voff, soff;
     if (x < ATile::PER_WAVE) {
       r = buffer_rsrc{(int)(uint32_t)ld_head_a, (int)(uint32_t)(ld_head_a >> 32), ra[0][2], ra[0][3]};
-      voff = aoff[x];
       soff = ld_soff_a;
+      voff = A_KS ? aoff[x] : kt_offset(aoff[x], x, soff, a_org);
     } else {
       int y = x - ATile::PER_WAVE, bsel = y / BTile::PER_WAVE, i = y % BTile::PER_WAVE;
       r = NB == 2 ? rb[bsel] : buffer_rsrc{(int)(uint32_t)ld_head_b, (int)(uint32_t)(ld_head_b >> 32), rb[0][2], rb[0][3]};
-      voff = boff[i];
       soff = ld_soff_b;
+      voff = B_KS ? boff[i] : kt_offset(boff[i], i, soff, b_org);
     }
     switch (load_index(x) & 3) {
       case 0: load16_to_lds_at<0>(r, voff, soff); break;
@@ -324,12 +350,12 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
     if (l3_is_b(z)) {
       const int bsel = z / BTile::PER_WAVE, i = z % BTile::PER_WAVE;
       r = NB == 2 ? rb[bsel] : buffer_rsrc{(int)(uint32_t)l3_head[1], (int)(uint32_t)(l3_head[1] >> 32), rb[0][2], rb[0][3]};
-      voff = boff[i];
       soff = l3_soff[1];
+      voff = B_KS ? boff[i] : kt_offset(boff[i], i, soff, b_org);
     } else {
       r = buffer_rsrc{(int)(uint32_t)l3_head[0], (int)(uint32_t)(l3_head[0] >> 32), ra[0][2], ra[0][3]};
-      voff = aoff[z - LDB];
       soff = l3_soff[0];
+      voff = A_KS ? aoff[z - LDB] : kt_offset(aoff[z - LDB], z - LDB, soff, a_org);
     }
     switch (l3_index(z) & 3) {
       case 0: load16_to_lds_at<0>(r, voff, soff); break;
@@ -848,19 +874,19 @@ __global__ void __launch_bounds__(WGM* WGN * 64) streamk_fixup_kernel(GemmArgs g
 }
 
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
-          typename Epi, bool SK = false>
+          typename Epi, bool SK = false, bool KT = false>
 __global__ void __launch_bounds__(WGM* WGN * 64)
     gemm_kernel_pipelined(GemmArgs ga, typename Epi::Args ea) {
-  gemm_pipelined_body<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, SK>(ga, ea, blockIdx.x, gridDim.x);
+  gemm_pipelined_body<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, SK, KT>(ga, ea, blockIdx.x, gridDim.x);
 }
 
 // The stream-K launches behind a launch that left ga.sk_tiles tiles out: the pieces, then the sums.
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
-          typename Epi>
+          typename Epi, bool KT>
 hipError_t launch_streamk_tail(const GemmArgs& ga, const typename Epi::Args& ea, hipStream_t s) {
   if constexpr (!Epi::SPLIT && BM == 256) {
     typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi>()> Cfg;
-    constexpr auto kern = gemm_kernel_pipelined<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, true>;
+    constexpr auto kern = gemm_kernel_pipelined<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, true, KT>;
     if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, Cfg::LDS_BYTES>, s)) return e;
     hipLaunchKernelGGL(kern, dim3(ga.sk_wgs), dim3(Cfg::NW * 64), Cfg::LDS_BYTES, s, ga, ea);
     if (hipError_t e = hipGetLastError()) return e;
@@ -890,10 +916,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64)
 }
 
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
-          typename Epi>
+          typename Epi, bool KT = false>
 hipError_t launch_gemm_pipelined(const GemmArgs& ga, const typename Epi::Args& ea, hipStream_t s) {
   typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi>()> Cfg;
-  constexpr auto kern = gemm_kernel_pipelined<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi>;
+  constexpr auto kern = gemm_kernel_pipelined<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, false, KT>;
   if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, Cfg::LDS_BYTES>, s)) return e;
   const int splits = Epi::SPLIT ? ga.splits : 1;
   const int tiles = ((ga.M + BM - 1) / BM) * ((ga.N + BN - 1) / BN);
@@ -903,7 +929,7 @@ hipError_t launch_gemm_pipelined(const GemmArgs& ga, const typename Epi::Args& e
     hipLaunchKernelGGL(kern, grid, block, Cfg::LDS_BYTES, s, ga, ea);
     if (hipError_t e = hipGetLastError()) return e;
   }
-  return sk ? launch_streamk_tail<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi>(ga, ea, s) : hipSuccess;
+  return sk ? launch_streamk_tail<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, KT>(ga, ea, s) : hipSuccess;
 }
 
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
@@ -925,7 +951,7 @@ hipError_t launch_gemm_group_pipelined(GemmGroup<typename Epi::Args>& grp, hipSt
   }
   for (int g = 0; g < grp.count; ++g) {
     if (grp.ga[g].sk_tiles <= 0) continue;
-    if (hipError_t e = launch_streamk_tail<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi>(grp.ga[g], grp.ea[g], s)) return e;
+    if (hipError_t e = launch_streamk_tail<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, false>(grp.ga[g], grp.ea[g], s)) return e;
   }
   return hipSuccess;
 }

@@ -6,25 +6,63 @@
 namespace gmlp {
 
 // Tile classes (all four wavefronts per workgroup, 64-wide reduction tiles).
-//   LARGE        256x256 output tiles, wavefronts of 128x128, pipelined kernel, whole tiles only
-//   MEDIUM_FULL  128x128 output tiles, wavefronts of 64x64, pipelined kernel, whole tiles only;
-//                two workgroups per CU, for problems with too few 256x256 tiles to fill the chip
-//   MEDIUM       128x128, predicated register-staged kernel: any M, N % 8, K % 8
+//   LARGE        256x256 output tiles, wavefronts of 128x128, pipelined kernel
+//   MEDIUM_FULL  128x128 output tiles, wavefronts of 64x64, pipelined kernel; two workgroups per CU,
+//                for problems with too few 256x256 tiles to fill the chip
+//   MEDIUM       128x128, predicated register-staged kernel, 64-bit addresses: operands too large for
+//                the pipelined kernels' 32-bit byte offsets
 enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2 };
 
-// kinds of GEMM the gated MLP needs; each is instantiated per dtype and tile class.
+// kinds of GEMM the gated MLP needs; each is instantiated per dtype and tile class, and for reduction
+// lengths that are (KT = false) or are not a multiple of 64, the width of a reduction tile.
+template <typename T, bool KT>
+hipError_t launch_gateup_kt(int tile_class, const GemmArgs& ga, const typename EpiGateUp<T>::Args& ea,
+                            hipStream_t s);  // A KC, B KC, two accumulator sets
+template <typename T, bool KT>
+hipError_t launch_linear_kt(int tile_class, const GemmArgs& ga, const typename EpiStore<T>::Args& ea,
+                            hipStream_t s);  // A KC, B KC
+template <typename T, bool KT>
+hipError_t launch_dh_kt(int tile_class, const GemmArgs& ga, const typename EpiDh<T>::Args& ea,
+                        hipStream_t s);  // A KC, B KS
+template <typename T, bool KT>
+hipError_t launch_dx_kt(int tile_class, const GemmArgs& ga, const typename EpiStore<T>::Args& ea,
+                        hipStream_t s);  // A KC, B KS, two reduction segments
+// Split-reduction variants (128x128 tiles): partial sums to a fp32 workspace, see splitk_reduce.
+template <typename T, bool KT>
+hipError_t launch_linear_split_kt(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
+template <typename T, bool KT>
+hipError_t launch_dx_split_kt(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
+template <typename T, bool KT>
+hipError_t launch_gateup_split_kt(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
+
+// The predicated class (and float32) has one kernel for every reduction length.
 template <typename T>
-hipError_t launch_gateup(int tile_class, const GemmArgs& ga, const typename EpiGateUp<T>::Args& ea,
-                         hipStream_t s);  // A KC, B KC, two accumulator sets
-template <typename T>
-hipError_t launch_linear(int tile_class, const GemmArgs& ga, const typename EpiStore<T>::Args& ea,
-                         hipStream_t s);  // A KC, B KC
-template <typename T>
-hipError_t launch_dh(int tile_class, const GemmArgs& ga, const typename EpiDh<T>::Args& ea,
-                     hipStream_t s);  // A KC, B KS
-template <typename T>
-hipError_t launch_dx(int tile_class, const GemmArgs& ga, const typename EpiStore<T>::Args& ea,
-                     hipStream_t s);  // A KC, B KS, two reduction segments
+bool reduction_tail(int tile_class, const GemmArgs& ga) {
+  return !std::is_same<T, float>::value && tile_class != TILE_MEDIUM && ga.K % 64 != 0;
+}
+#define GMLP_BY_TAIL(KIND, EPI)                                                                              \
+  template <typename T>                                                                                      \
+  hipError_t launch_##KIND(int tile_class, const GemmArgs& ga, const typename EPI<T>::Args& ea, hipStream_t s) { \
+    if constexpr (!std::is_same<T, float>::value)                                                            \
+      if (reduction_tail<T>(tile_class, ga)) return launch_##KIND##_kt<T, true>(tile_class, ga, ea, s);        \
+    return launch_##KIND##_kt<T, false>(tile_class, ga, ea, s);                                              \
+  }
+#define GMLP_SPLIT_BY_TAIL(KIND)                                                                             \
+  template <typename T>                                                                                      \
+  hipError_t launch_##KIND##_split(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s) {  \
+    return reduction_tail<T>(TILE_MEDIUM_FULL, ga) ? launch_##KIND##_split_kt<T, true>(ga, ea, s)              \
+                                                   : launch_##KIND##_split_kt<T, false>(ga, ea, s);            \
+  }
+GMLP_BY_TAIL(gateup, EpiGateUp)
+GMLP_BY_TAIL(linear, EpiStore)
+GMLP_BY_TAIL(dh, EpiDh)
+GMLP_BY_TAIL(dx, EpiStore)
+GMLP_SPLIT_BY_TAIL(gateup)
+GMLP_SPLIT_BY_TAIL(linear)
+GMLP_SPLIT_BY_TAIL(dx)
+#undef GMLP_BY_TAIL
+#undef GMLP_SPLIT_BY_TAIL
+
 template <typename T>
 hipError_t launch_dw(int tile_class, const GemmArgs& ga, const typename EpiStore<T>::Args& ea,
                      hipStream_t s);  // A KS, B KS
@@ -45,14 +83,6 @@ hipError_t launch_gemm(const GemmArgs& ga, const typename Epi::Args& ea, hipStre
   hipLaunchKernelGGL(kern, grid, block, Cfg::LDS_BYTES, s, ga, ea);
   return hipGetLastError();
 }
-
-// Split-reduction variants (128x128 tiles): partial sums to a fp32 workspace, see splitk_reduce.
-template <typename T>
-hipError_t launch_linear_split(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
-template <typename T>
-hipError_t launch_dx_split(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
-template <typename T>
-hipError_t launch_gateup_split(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
 
 // decode.hip
 template <typename T>
