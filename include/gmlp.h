@@ -10,8 +10,8 @@
  *   - All matrices are dense, row-major, contiguous, on the current HIP device, 16-byte aligned.
  *   - M = tokens (rows of x), K = hidden_size, N = intermediate_size.
  *     W_gate, W_up are [N,K]; W_down is [K,N]  (torch.nn.Linear [out,in] layout).
- *   - dtype: GMLP_F16 or GMLP_BF16 storage (the tuned kernels) or GMLP_F32 (compatibility path on
- *     fp32 MFMA, not tuned; not for gmlp_decode_fwd); accumulation and epilogue arithmetic are fp32.
+ *   - dtype: GMLP_F16 or GMLP_BF16 storage (the tuned kernels) or GMLP_F32 (fp32 MFMA; not for
+ *     gmlp_decode_fwd); accumulation and epilogue arithmetic are fp32.
  *   - Every call only ENQUEUES work on `stream` (a hipStream_t; NULL = default stream) and returns.
  *     The library never allocates or frees device memory and keeps no pointer past a call; the
  *     caller owns every buffer, including workspaces (sizes from gmlp_workspace_bytes).  The one
@@ -182,7 +182,7 @@ int gmlp_dw_bwd(const void* lhs, const void* rhs, void* dw, int64_t Mred, int64_
  * Same reference counterparts as gmlp_dw_bwd; one launch for dW_gate, dW_up and dW_down avoids
  * three partially filled last rounds of workgroups.
  * workspace (may be NULL): gmlp_dw_bwd_grouped_workspace_bytes(count, Mred, R, C, dtype) bytes (what
- * this set of problems uses, often 0), or the bound gmlp_workspace_bytes(GMLP_OP_DW_BWD_GROUPED, ...).
+ * this set of problems uses, often 0), or, 16-bit types, the bound gmlp_workspace_bytes(GMLP_OP_DW_BWD_GROUPED, ...).
  */
 size_t gmlp_dw_bwd_grouped_workspace_bytes(int count, int64_t Mred, const int64_t* R, const int64_t* C,
                                            int dtype);

@@ -1119,6 +1119,52 @@ def test_reduction_tails_every_operator_against_fp32_products(M, K, N):
     _close("dX", ops_bwd.dx_bwd(dg, du, wg, wu), f(dg) @ f(wg) + f(du) @ f(wu))
 
 
+@pytest.mark.parametrize(
+    "M,K,N",
+    [
+        (1, 8, 8),           # one tile, a quarter of a reduction tile
+        (65, 40, 136),       # one row and 8 columns beyond a 64x64 tile; reduction tails
+        (130, 1544, 264),    # few tiles, long reductions: split, ragged last split
+        (4100, 72, 200),     # long reduction of the weight gradients only: grouped launch, split
+        (2300, 1048, 4200),  # 128-row tiles (two reduction segments of unequal last tiles in dX)
+    ],
+)
+def test_fp32_every_operator_against_float64_products(M, K, N):
+    """float32 kernels: every tile class, split reductions, edges.  Bound: a sum of R products in float32,
+    in any order, is off by at most (R + 2) 2^-24 sum |a||b| (first order in 2^-24), element by element."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    print(f"fp32 operators: M={M} K={K} N={N}", flush=True)
+    g = torch.Generator().manual_seed(3)
+    rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g)).to(dev)
+    d = lambda t: t.double()
+
+    def check(name, got, pairs):
+        ref = sum(a @ b for a, b in pairs)
+        terms = sum(a.abs() @ b.abs() for a, b in pairs)
+        R = sum(a.shape[1] for a, _ in pairs)
+        assert torch.isfinite(got).all(), name
+        worst = ((got.double() - ref).abs() / ((R + 2) * 2.0**-24 * terms).clamp_min(1e-300)).max().item()
+        print(f"  {name}: largest error {worst:.3f} of its bound", flush=True)
+        assert worst <= 1.0, name
+
+    x, dy, h, dg, du = rnd(M, K), rnd(M, K), rnd(M, N), rnd(M, N), rnd(M, N)
+    wg, wu, wd = rnd(N, K, s=0.03), rnd(N, K, s=0.03), rnd(K, N, s=0.03)
+    hs = ops_fwd.gateup_fwd(x, wg, None, wu, None, save_activations=True)
+    check("G", hs.gate, [(d(x), d(wg).T)])
+    check("U", hs.up, [(d(x), d(wu).T)])
+    check("Y", ops_fwd.linear_fwd(h, wd), [(d(h), d(wd).T)])
+    ones = torch.ones_like(hs.up)
+    check("dH", ops_bwd.dh_bwd(dy, wd, ones, ones, act_fn="no_act")[1], [(d(dy), d(wd))])
+    check("dX", ops_bwd.dx_bwd(dg, du, wg, wu), [(d(dg), d(wg)), (d(du), d(wu))])
+    lhs_rhs = [(dg, x), (du, x), (dy, h)]
+    for name, got, (a, b) in zip(("dW_gate", "dW_up", "dW_down"), ops_bwd.dw_bwd_grouped(lhs_rhs), lhs_rhs):
+        check(name, got, [(d(a).T, d(b))])
+    check("dW alone", ops_bwd.dw_bwd(dy, h), [(d(dy).T, d(h))])
+
+
 def test_random_modules_through_the_one_call_entries_no_worse_than_torch_16bit():
     """Four dozen seeded random modules (token counts 1 to 6144, widths that are multiples of 8, 64
     or 256, both 16-bit dtypes, biases, dropout, five activations) through FusedGatedMLP, i.e. through

@@ -79,11 +79,51 @@ hipError_t launch_splitk_reduce(const float* ws, int splits, size_t split_stride
 #define GMLP_REDUCE_INST(T, EPI)                                                                    \
   template hipError_t launch_splitk_reduce<T, EPI<T>>(const float*, int, size_t, size_t,            \
                                                       const EPI<T>::Args&, int64_t, int64_t, hipStream_t);
+GMLP_REDUCE_INST(float, EpiStore)
+GMLP_REDUCE_INST(float, EpiGateUp)
+GMLP_REDUCE_INST(float, EpiDh)
+GMLP_REDUCE_INST(f16, EpiDh)
+GMLP_REDUCE_INST(bf16, EpiDh)
 GMLP_REDUCE_INST(f16, EpiStore)
 GMLP_REDUCE_INST(bf16, EpiStore)
 GMLP_REDUCE_INST(f16, EpiGateUp)
 GMLP_REDUCE_INST(bf16, EpiGateUp)
 #undef GMLP_REDUCE_INST
+
+// The same for the weight gradients of one pass (contiguous outputs without a bias): blockIdx.y
+// selects the problem.
+struct ReduceGroup {
+  const float* ws[GEMM_GROUP_MAX];
+  float* out[GEMM_GROUP_MAX];
+  size_t n[GEMM_GROUP_MAX];  // elements of an output, and between consecutive splits
+  int splits[GEMM_GROUP_MAX];
+};
+__global__ void __launch_bounds__(256) splitk_reduce_group_kernel(ReduceGroup g) {
+  const int p = blockIdx.y;
+  const float* __restrict__ ws = g.ws[p];
+  const size_t n = g.n[p], step = (size_t)gridDim.x * 256 * 4;
+  for (size_t e = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; e < n; e += step) {
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < g.splits[p]; ++i) s += *(const f32x4*)(ws + (size_t)i * n + e);
+    __builtin_nontemporal_store(s, (f32x4*)(g.out[p] + e));
+  }
+}
+hipError_t launch_splitk_reduce_group(const GemmGroup<EpiPartial<float>::Args>& part,
+                                      const GemmGroup<EpiStore<float>::Args>& out, hipStream_t s) {
+  ReduceGroup g = {};
+  size_t most = 0;
+  for (int i = 0; i < part.count; ++i) {
+    g.ws[i] = part.ea[i].ws;
+    g.out[i] = out.ea[i].out;
+    g.n[i] = part.ea[i].split_stride;
+    g.splits[i] = part.ga[i].splits;
+    if (g.n[i] > most) most = g.n[i];
+  }
+  size_t blocks = (most / 4 + 255) / 256;
+  if (blocks > 256 * 8) blocks = 256 * 8;
+  hipLaunchKernelGGL(splitk_reduce_group_kernel, dim3((unsigned)blocks, part.count), dim3(256), 0, s, g);
+  return hipGetLastError();
+}
 
 // Column sums in two fixed-order stages: COLSUM_SPLITS row ranges -> fp32 partials -> total.
 // Up to COLSUM_GROUP_MAX arrays with the same number of rows share the two launches (the bias

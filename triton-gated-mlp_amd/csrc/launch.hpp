@@ -11,7 +11,9 @@ namespace gmlp {
 //                for problems with too few 256x256 tiles to fill the chip
 //   MEDIUM       128x128, predicated register-staged kernel, 64-bit addresses: operands too large for
 //                the pipelined kernels' 32-bit byte offsets
-enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2 };
+//   F32_*        the float32 kernel's tiles (gemm_f32.hip): 128 x 128, 64 x 128, 64 x 64; with two
+//                accumulator sets 128 x 64 or 64 x 64
+enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2, TILE_F32_128 = 3, TILE_F32_64X128 = 4, TILE_F32_64 = 5 };
 
 // kinds of GEMM the gated MLP needs; each is instantiated per dtype and tile class, and for reduction
 // lengths that are (KT = false) or are not a multiple of 64, the width of a reduction tile.
@@ -67,9 +69,14 @@ template <typename T>
 hipError_t launch_dw(int tile_class, const GemmArgs& ga, const typename EpiStore<T>::Args& ea,
                      hipStream_t s);  // A KS, B KS
 
-// Several weight-gradient GEMMs of one pipelined tile class (LARGE or MEDIUM_FULL) as one grid.
+// Several weight-gradient GEMMs of one tile class (LARGE, MEDIUM_FULL or F32_*) as one grid.
 template <typename T>
 hipError_t launch_dw_group(int tile_class, GemmGroup<typename EpiStore<T>::Args>& grp, hipStream_t s);
+
+// The same with a split reduction, float32: every problem's ga.splits partial sums, then their totals.
+hipError_t launch_dw_group_split_f32(GemmGroup<EpiPartial<float>::Args>& grp, hipStream_t s);
+hipError_t launch_splitk_reduce_group(const GemmGroup<EpiPartial<float>::Args>& part,
+                                      const GemmGroup<EpiStore<float>::Args>& out, hipStream_t s);
 
 // Generic launcher used by the instantiation units.
 template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
