@@ -1122,6 +1122,45 @@ def test_reduction_tails_every_operator_against_fp32_products(M, K, N):
 @pytest.mark.parametrize(
     "M,K,N",
     [
+        (129, 4096, 14344),  # 128x256 tiles: one row beyond a tile, ragged columns; 8 to 16 splits
+        (200, 4104, 8200),   # the same with reduction tails
+        (1030, 2056, 5640),  # several rows of them, splits that end inside a tile
+        (3000, 256, 520),    # weight gradients with a split reduction (few tiles, many tokens)
+        (2500, 136, 72),     # the same, single tiles, ragged last split
+    ],
+)
+def test_wide_tiles_and_split_gradients_against_fp32_products(M, K, N):
+    """Grids that the planner gives to the 128x256 tiles (three ring entries of both operands), and split
+    reductions of dH and of the grouped weight gradients; twice, bit-identical."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    print(f"wide tiles, split gradients: M={M} K={K} N={N}", flush=True)
+    g = torch.Generator().manual_seed(8)
+    rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g)).bfloat16().to(dev)
+    f = lambda t: t.float()  # products in fp32 on the device: plain 2-D torch matmuls
+    x, dy, h, G, U = rnd(M, K), rnd(M, K), rnd(M, N), rnd(M, N), rnd(M, N)
+    wg, wu, wd = rnd(N, K, s=0.03), rnd(N, K, s=0.03), rnd(K, N, s=0.03)
+
+    def run():
+        hs = ops_fwd.gateup_fwd(x, wg, None, wu, None, save_activations=True)
+        dg, du = ops_bwd.dh_bwd(dy, wd, G, U)
+        return [hs.gate, hs.up, ops_fwd.linear_fwd(h, wd), dg, du, ops_bwd.dx_bwd(G, U, wg, wu),
+                *ops_bwd.dw_bwd_grouped([(G, x), (U, x), (dy, h)])]
+
+    got = run()
+    hb = oracle.hidden_backward(f(dy) @ f(wd), f(G), f(U), None, 0.0)
+    refs = [f(x) @ f(wg).T, f(x) @ f(wu).T, f(h) @ f(wd).T, hb["dG"], hb["dU"], f(G) @ f(wg) + f(U) @ f(wu),
+            f(G).T @ f(x), f(U).T @ f(x), f(dy).T @ f(h)]
+    for name, a, b in zip(("G", "U", "Y", "dG", "dU", "dX", "dW_gate", "dW_up", "dW_down"), got, refs):
+        _close(name, a, b)
+    assert all(torch.equal(a, b) for a, b in zip(got, run()))
+
+
+@pytest.mark.parametrize(
+    "M,K,N",
+    [
         (1, 8, 8),           # one tile, a quarter of a reduction tile
         (65, 40, 136),       # one row and 8 columns beyond a 64x64 tile; reduction tails
         (130, 1544, 264),    # few tiles, long reductions: split, ragged last split

@@ -116,18 +116,16 @@ int num_xcd() {
   return n < 1 ? 1 : n > 8 ? 8 : n;
 }
 
-// LARGE or MEDIUM_FULL for a grid of `large_tiles` large or `medium_tiles` small tiles, by
-// estimated time in rounds of workgroups (see pick_tile).
-int group_tile_class(int64_t large_tiles, int64_t medium_tiles) {
-  auto rounds = [](int64_t tiles, int64_t slots) {
-    double part = (double)(tiles % slots) / (double)slots;
-    return (double)(tiles / slots) + (part > 0.0 ? 0.6 + 0.4 * part : 0.0);
-  };
-  const int64_t cus = num_cu();
-  const double large_time = rounds(large_tiles, cus);
-  const double medium_time = rounds(medium_tiles, 2 * cus) * (2.0 / 3.0);
-  return large_time <= medium_time ? gmlp::TILE_LARGE : gmlp::TILE_MEDIUM_FULL;
-}
+// The GEMMs of a gated MLP (operand layouts, epilogues: launch.hpp).
+enum GemmKind { GATEUP, LINEAR, DH, DX, DW };
+
+// How a GEMM runs: tile class, and number of workgroups that share an output tile, each reducing a
+// contiguous range of reduction tiles (1: no split).
+struct GemmPlan {
+  int tile_class;
+  int splits;
+  double us;  // estimate
+};
 
 // float32: tile class and number of workgroups per tile (splits), by estimated time.  A launch takes
 // as long as the compute unit that gets the most workgroups, and a CU's workgroups share its matrix
@@ -139,15 +137,10 @@ int group_tile_class(int64_t large_tiles, int64_t medium_tiles) {
 // 128x128 tiles (128 of them) 180 us, 64x64 (512) 103; weight gradients at M=6974, K=256, N=768: 460
 // unsplit, 64x64 126, with 13 splits 85.  A split reduction (64x64 tiles, at least 4 reduction tiles
 // each) pays a second launch and the partial sums' round trip through the caches.
-struct PlanF32 {
-  int tile_class;
-  int splits;
-  double us;
-};
-PlanF32 plan_f32(int64_t tiles128, int64_t tiles64x128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes,
+GemmPlan plan_f32(int64_t tiles128, int64_t tiles64x128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes,
                  bool may_split) {
   static const double rate[3][3] = {{0.87, 0.88, 0.88}, {0.75, 0.78, 0.85}, {0.65, 0.76, 0.81}};  // by class, workgroups per CU
-  PlanF32 best = {gmlp::TILE_F32_128, 1, 1e30};
+  GemmPlan best = {gmlp::TILE_F32_128, 1, 1e30};
   const int64_t cus = num_cu();
   auto consider = [&](int tile_class, int64_t tiles, double weight, int64_t splits) {
     const int64_t per_cu = (tiles * splits + cus - 1) / cus;
@@ -155,7 +148,7 @@ PlanF32 plan_f32(int64_t tiles128, int64_t tiles64x128, int64_t tiles64, int64_t
     double us = (double)per_cu * weight * (double)((red_tiles + splits - 1) / splits + 1) * 0.445 /
                 rate[tile_class - gmlp::TILE_F32_128][per_cu >= 3 ? 2 : per_cu - 1];
     if (splits > 1) us += 5.0 + 2.0 * (double)splits * out_bytes * sets / 3e6;
-    if (us < best.us) best = PlanF32{tile_class, (int)splits, us};
+    if (us < best.us) best = GemmPlan{tile_class, (int)splits, us};
   };
   consider(gmlp::TILE_F32_128, tiles128, 4, 1);
   if (sets == 1) consider(gmlp::TILE_F32_64X128, tiles64x128, 2, 1);
@@ -164,69 +157,13 @@ PlanF32 plan_f32(int64_t tiles128, int64_t tiles64x128, int64_t tiles64, int64_t
     for (int64_t s = 2; s <= 16 && s * 4 <= red_tiles; ++s) consider(gmlp::TILE_F32_64, tiles64, sets, s);
   return best;
 }
-PlanF32 plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int sets, bool may_split) {
+GemmPlan plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int sets, bool may_split) {
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q; };
   return plan_f32(up(rows, 128) * up(cols, 128 / sets), up(rows, 64) * up(cols, 128), up(rows, 64) * up(cols, 64),
                   red_tiles, sets, (double)rows * (double)cols * 4.0, may_split);
 }
 
-// Tile class for an output of rows x cols with reduction length red (all in elements).
-// The pipelined kernels (LARGE: 256 x bn_large tiles, one workgroup per CU; MEDIUM_FULL: tiles of
-// half that in each direction, two per CU) take any rows and cols; they need 32-bit byte offsets
-// into the operands, padded to whole tiles.  Everything else runs on the predicated MEDIUM class.
-// Between the two pipelined classes the choice is estimated time in rounds of workgroups: a round
-// of small tiles (two per CU) takes 2/3 of a round of large ones (a quarter of the work at 75 % of
-// the throughput, two at a time), and a last round filled to the fraction f costs 0.6 + 0.4 f of
-// a full one (the busy CUs clock higher, but not in proportion; fitted to measurements).
-int pick_tile(int dtype, int64_t rows, int64_t cols, int64_t red, int bn_large) {
-  if (dtype == GMLP_F32) return plan_f32(rows, cols, (red + 31) / 32, bn_large == 128 ? 2 : 1, false).tile_class;
-  auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
-  // the buffer base sits up to 4 KB below the operand (shared-M0 loads)
-  const int64_t limit = ((int64_t)1 << 31) - 4096;
-  bool offsets_fit = up(rows, 256) * up(red, 64) * 2 < limit && up(cols, 256) * up(red, 64) * 2 < limit;
-  if (!offsets_fit) return gmlp::TILE_MEDIUM;
-  const int64_t large_tiles = (up(rows, 256) / 256) * (up(cols, bn_large) / bn_large);
-  const int64_t medium_tiles = (up(rows, 128) / 128) * (up(cols, bn_large / 2) / (bn_large / 2));
-  return group_tile_class(large_tiles, medium_tiles);
-}
-
-// Number of workgroups that should share one output tile of a rows x cols GEMM with `red_tiles`
-// 64-wide reduction tiles, or 1.  A GEMM with a few output tiles and a long reduction (down
-// projection and input gradient of a short batch) leaves most of the chip idle and is bound by
-// streaming the weights; splitting the reduction fills two 128-tile workgroups per CU.  Each split
-// keeps at least 8 reduction tiles.
-int pick_splits(int dtype, int64_t rows, int64_t cols, int64_t red, int64_t red_tiles, int bn_large = 256) {
-  if (dtype == GMLP_F32) {
-    const int64_t segments = red_tiles / ((red + 63) / 64), tiles = segments * ((red + 31) / 32);
-    const int64_t s = plan_f32(rows, cols, tiles, bn_large == 128 ? 2 : 1, true).splits;
-    const int64_t per = (tiles + s - 1) / s;  // drop the splits that rounding up leaves empty
-    return (int)((tiles + per - 1) / per);
-  }
-  if (pick_tile(dtype, rows, cols, red, bn_large) != gmlp::TILE_MEDIUM_FULL) return 1;
-  const int64_t bn = bn_large / 2;
-  const int64_t tiles = ((rows + 127) / 128) * ((cols + bn - 1) / bn);
-  int64_t s = 2 * num_cu() / tiles;
-  if (s > red_tiles / 8) s = red_tiles / 8;
-  if (s > 16) s = 16;
-  if (s < 2) return 1;
-  // the kernel gives every split ceil(red_tiles / s) reduction tiles: drop the splits that this
-  // leaves empty
-  const int64_t per = (red_tiles + s - 1) / s;
-  return (int)((red_tiles + per - 1) / per);
-}
-
-// For a rows x cols output on 256 x 256 tiles whose grid ends in a thinly filled round of
-// workgroups (at most half full): the number of tile ROWS that make whole rounds, or 0.  The
-// backward GEMMs read their weight operand reduction-strided, so they are cut along the rows of
-// the output (token rows: every other operand is row-major in them) where the forward GEMMs are cut
-// along the columns.
-int64_t whole_round_tile_rows(int dtype, int64_t rows, int64_t cols, int64_t red) {
-  if (dtype == GMLP_F32 || pick_tile(dtype, rows, cols, red, 256) != gmlp::TILE_LARGE) return 0;
-  const int64_t tiles_m = (rows + 255) / 256, tiles_n = (cols + 255) / 256, cus = num_cu();
-  const int64_t rounds = tiles_m * tiles_n / cus, tail = tiles_m * tiles_n % cus;
-  const int64_t whole = rounds * cus / tiles_n;
-  return rounds >= 1 && tail > 0 && 2 * tail <= cus && whole >= 1 && whole < tiles_m ? whole : 0;
-}
+int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Stream-K plan for a grid of `tiles` large output tiles with `kt` 64-wide reduction tiles each
 // (tiles of all problems of a grouped launch together).  The tiles beyond the last whole round of
@@ -235,11 +172,16 @@ int64_t whole_round_tile_rows(int dtype, int64_t rows, int64_t cols, int64_t red
 // (see pick_tile) against f with stream-K, plus the partial sums' round trip through memory and the
 // second launch (about 45 us, i.e. 30 reduction tiles' time): worth it when (1 - f) * kt > 50.
 // Every stream-K workgroup gets at least 8 reduction tiles.
+// A grid of less than one round that fills more than half of the chip is left alone unless its tiles
+// divide into whole pieces (`first_round`: false for the weight gradients, which keep the plan): even
+// ranges straddle tiles there, two partial stores per workgroup, and the busy CUs of the plain launch
+// clock higher.  Down projections of 160 tiles: 322 to 330 us shared out, 264 to 275 plain; 192
+// tiles: 313 / 292; dX of 192 tiles 362 / 327; 224 tiles 247 / 246.  (96 tiles: 324 / 495.)
 struct StreamK {
   int tiles = 0, wgs = 0, chunks = 0;
   size_t ws_bytes = 0;
 };
-StreamK plan_streamk(int dtype, int64_t tiles, int64_t kt) {
+StreamK plan_streamk(int dtype, int64_t tiles, int64_t kt, bool first_round = true) {
   StreamK p;
   const int64_t cus = num_cu(), tail = tiles % cus;
   if (dtype == GMLP_F32 || tail == 0 || kt < 8) return p;
@@ -257,6 +199,7 @@ StreamK plan_streamk(int dtype, int64_t tiles, int64_t kt) {
     p.chunks = (int)per_tile;
     p.wgs = (int)(per_tile * tail);
   }
+  if (first_round && tiles < cus && 2 * tiles > cus && p.chunks == 0) return StreamK{};
   p.ws_bytes = (size_t)(p.tiles + p.wgs) * 65536 * sizeof(float);  // 256 x 256 accumulators per slot
   return p;
 }
@@ -269,11 +212,139 @@ bool use_streamk(const StreamK& p, gmlp::GemmArgs& ga, void* workspace, size_t w
   ga.sk_ws = (float*)workspace;
   return true;
 }
-int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Output columns (per accumulator set) of a LARGE or WIDE tile; MEDIUM_FULL tiles have half.
+int tile_cols(int kind) { return kind == GATEUP ? 128 : 256; }
+int64_t red_tiles_of(int kind, int64_t red) { return (kind == DX ? 2 : 1) * cdiv(red, 64); }
+
+// 16-bit types: estimated time of a launch on a tile class, in rounds of workgroups (one per CU, two
+// for MEDIUM_FULL).  A round takes kt * r + e us: reduction tiles times the class's rate, and an
+// epilogue whose cost is its stores (and, dH, its loads).  A last round filled to the fraction f
+// costs base + (1 - base) f of a full one (busy CUs clock higher, but not in proportion; the small
+// tiles gain less once a CU has two: base + half up to f = 1/2, 1 at f = 1).  A split reduction adds a
+// second launch and the partial sums' round trip.  All constants are one least-squares fit to 3100
+// launches (five GEMMs of 89 random shapes, M 33 to 6000, widths 128 to 15000, every class and split;
+// standard deviation of the estimates 3 to 12 %); the class chosen costs 1.5 % over the fastest on
+// average.
+struct TileCost {
+  int tile_class;
+  int rows, col_div, per_cu;
+  double base, half;
+  double r[3];  // both operands reduction-contiguous (GATEUP, LINEAR); one (DH, DX); none (DW)
+  double e[6];  // by GemmKind; [5]: partial sums
+};
+const TileCost kLarge = {gmlp::TILE_LARGE, 256, 1, 1, 0.69, 0, {1.443, 1.477, 1.494}, {11.4, 6.1, 19.0, 6.8, 7.1, 12.0}};
+const TileCost kWide = {gmlp::TILE_WIDE, 128, 1, 1, 0.74, 0, {0.846, 0.940, 0.983}, {5.7, 2.7, 9.7, 3.3, 3.7, 2.0}};
+const TileCost kMedium = {gmlp::TILE_MEDIUM_FULL, 128, 2, 2, 0.46, 0.30, {0.967, 0.983, 1.094}, {3.4, 0.6, 8.4, 0.2, 2.4, 0.1}};
+
+double launch_us(const TileCost& c, int kind, int64_t tiles, int64_t kt, int splits, double out_elements) {
+  const int64_t slots = (int64_t)c.per_cu * num_cu(), wgs = tiles * splits;
+  const double f = (double)(wgs % slots) / (double)slots;
+  double rounds = (double)(wgs / slots);
+  if (f > 0.0)
+    rounds += c.half == 0.0 ? c.base + (1.0 - c.base) * f
+              : f <= 0.5    ? c.base + c.half * 2.0 * f
+                            : c.base + c.half + (1.0 - c.base - c.half) * (2.0 * f - 1.0);
+  double us = 3.1 + rounds * ((double)cdiv(kt, splits) * c.r[kind <= LINEAR ? 0 : kind <= DX ? 1 : 2] + c.e[splits > 1 ? 5 : kind]);
+  if (splits > 1) us += 4.0 + (double)splits * out_elements * 4.0 / 2.7e6;
+  return us;
+}
+
+// The classes and splits for a grid of this many tiles of each class (`wide` 0: class not built).  At
+// least 4 reduction tiles per split, at most 16 splits.
+GemmPlan cheapest(int kind, int64_t large, int64_t wide, int64_t medium, int64_t kt, double out_elements, bool may_split) {
+  GemmPlan best = {gmlp::TILE_LARGE, 1, launch_us(kLarge, kind, large, kt, 1, out_elements)};
+  auto consider = [&](const TileCost& c, int64_t tiles) {
+    const int64_t most = may_split ? std::max<int64_t>(1, std::min<int64_t>(16, kt / 4)) : 1;
+    for (int64_t s = 1; s <= most; ++s) {
+      if (s > 1 && cdiv(kt, cdiv(kt, s)) != s) continue;  // rounding up would leave splits empty
+      const double us = launch_us(c, kind, tiles, kt, (int)s, out_elements);
+      if (us < best.us) best = GemmPlan{c.tile_class, (int)s, us};
+    }
+  };
+  consider(kMedium, medium);
+  if (wide > 0) consider(kWide, wide);
+  return best;
+}
+int64_t tiles_of(const TileCost& c, int kind, int64_t rows, int64_t cols) {
+  return cdiv(rows, c.rows) * cdiv(cols, tile_cols(kind) / c.col_div);
+}
+
+// Large tiles with stream-K: behind whole rounds the launches take 0.9 of the sum of their parts
+// (eight shapes of 1.25 to 1.5 rounds, where they are up to 8 % ahead of the 128x256 tiles, 5 % behind
+// in one).  Grids of less than a round share out everything; inside a step, where their operands are
+// still cached and the partial sums' round trip is what is left, they come out a tenth slower than the
+// launch alone.
+double streamk_us(int kind, int64_t large, int64_t kt, double out_elements) {
+  const int64_t cus = num_cu();
+  const double pieces = (double)(large % cus) / (double)cus * (double)kt * 1.5;
+  if (large < cus) return 1.1 * (pieces + 43.0);
+  return 0.9 * (launch_us(kLarge, kind, large / cus * cus, kt, 1, out_elements) + pieces) + 40.0;
+}
+
+// A grid of large tiles that ends in a round filled to half or less can run its whole rounds and
+// the rest as two launches: cut along the output columns (forward) or the token rows (dH, dX: their
+// weight operand is reduction-strided, every other operand row-major in the rows).  Tile columns or
+// rows of the first part, or 0.
+int64_t whole_rounds(int kind, int64_t rows, int64_t cols) {
+  const int64_t tm = cdiv(rows, 256), tn = cdiv(cols, tile_cols(kind)), cus = num_cu();
+  const int64_t along = kind <= LINEAR ? tn : tm, across = kind <= LINEAR ? tm : tn;
+  const int64_t rounds = tm * tn / cus, tail = tm * tn % cus, whole = rounds * cus / across;
+  return rounds >= 1 && tail > 0 && 2 * tail <= cus && whole >= 1 && whole < along ? whole : 0;
+}
+
+// The pipelined kernels take any rows, cols and red but need 32-bit byte offsets into the operands,
+// padded to whole tiles; anything larger runs on the predicated MEDIUM class.
+GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red, bool may_split) {
+  if (dtype == GMLP_F32) {
+    // (the down projection of float32 modules asks for no workspace; callers rely on that)
+    const int64_t segments = kind == DX ? 2 : 1, tiles = segments * cdiv(red, 32);
+    GemmPlan p = plan_f32(rows, cols, tiles, kind == GATEUP ? 2 : 1, may_split && kind != LINEAR);
+    p.splits = (int)cdiv(tiles, cdiv(tiles, p.splits));  // drop the splits that rounding up leaves empty
+    return p;
+  }
+  auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
+  // the buffer base sits up to 4 KB below the operand (shared-M0 loads)
+  const int64_t limit = ((int64_t)1 << 31) - 4096;
+  if (up(rows, 256) * up(red, 64) * 2 >= limit || up(cols, 256) * up(red, 64) * 2 >= limit) return {gmlp::TILE_MEDIUM, 1, 0};
+  const int64_t kt = red_tiles_of(kind, red), large = tiles_of(kLarge, kind, rows, cols);
+  const double out = (double)rows * (double)cols * (kind == GATEUP ? 2 : 1);
+  GemmPlan p = cheapest(kind, large, kind == DW ? 0 : tiles_of(kWide, kind, rows, cols), tiles_of(kMedium, kind, rows, cols), kt,
+                        out, may_split);
+  if (p.tile_class == gmlp::TILE_LARGE) return p;
+  // large tiles whose thin last round is shared out (stream-K) or run by other tiles may still be ahead
+  const int64_t cus = num_cu(), whole = whole_rounds(kind, rows, cols);
+  double us = p.us;
+  if (plan_streamk(dtype, large, kt).tiles > 0) {
+    us = streamk_us(kind, large, kt, out);
+  } else if (whole > 0) {
+    const int64_t r = kind <= LINEAR ? rows : rows - whole * 256, c = kind <= LINEAR ? cols - whole * tile_cols(kind) : cols;
+    us = launch_us(kLarge, kind, large / cus * cus, kt, 1, out) +
+         cheapest(kind, tiles_of(kLarge, kind, r, c), tiles_of(kWide, kind, r, c), tiles_of(kMedium, kind, r, c), kt, 0, false).us;
+  }
+  return us < p.us ? GemmPlan{gmlp::TILE_LARGE, 1, us} : p;
+}
+
+// make_plan takes a few microseconds of estimating, as long as an enqueue: each host thread keeps the
+// plans of the last problems it saw (a function of the arguments and the device's compute units only).
+GemmPlan plan_gemm(int dtype, int kind, int64_t rows, int64_t cols, int64_t red, bool may_split) {
+  struct Entry {
+    int64_t key[4] = {-1, -1, -1, -1};
+    GemmPlan plan;
+  };
+  static thread_local Entry cache[64];
+  const int64_t key[4] = {rows, cols, red, (((int64_t)num_cu() * 8 + kind) * 4 + dtype) * 2 + (may_split ? 1 : 0)};
+  Entry& e = cache[(uint64_t)(rows * 0x9E3779B1 + cols * 0x85EBCA77 + red * 0xC2B2AE3D + key[3] * 0x27D4EB2F) >> 7 & 63];
+  if (!std::equal(key, key + 4, e.key)) {
+    e.plan = make_plan(dtype, kind, rows, cols, red, may_split);
+    std::copy(key, key + 4, e.key);
+  }
+  return e.plan;
+}
 
 // Weight gradients of float32 modules: all problems in one grid, on one tile class with one number of
 // splits; the problems' partial sums follow each other in the workspace.
-PlanF32 plan_dw_group_f32(int count, int64_t Mred, const int64_t* R, const int64_t* C) {
+GemmPlan plan_dw_group_f32(int count, int64_t Mred, const int64_t* R, const int64_t* C) {
   int64_t t128 = 0, t64x128 = 0, t64 = 0;
   double out_bytes = 0;
   for (int i = 0; i < count; ++i) {
@@ -282,30 +353,38 @@ PlanF32 plan_dw_group_f32(int count, int64_t Mred, const int64_t* R, const int64
     t64 += cdiv(R[i], 64) * cdiv(C[i], 64);
     out_bytes += (double)R[i] * (double)C[i] * 4.0;
   }
-  PlanF32 p = plan_f32(t128, t64x128, t64, cdiv(Mred, 32), 1, out_bytes, true);
+  GemmPlan p = plan_f32(t128, t64x128, t64, cdiv(Mred, 32), 1, out_bytes, true);
   const int64_t per = cdiv(cdiv(Mred, 32), p.splits);
   p.splits = (int)cdiv(cdiv(Mred, 32), per);  // drop the splits that rounding up leaves empty
   return p;
 }
-size_t dw_group_f32_bytes(int count, int64_t Mred, const int64_t* R, const int64_t* C) {
-  const PlanF32 p = plan_dw_group_f32(count, Mred, R, C);
+size_t dw_group_split_bytes(int count, int splits, const int64_t* R, const int64_t* C) {
   size_t n = 0;
-  if (p.splits > 1)
-    for (int i = 0; i < count; ++i) n += (size_t)p.splits * R[i] * C[i] * sizeof(float);
+  if (splits > 1)
+    for (int i = 0; i < count; ++i) n += (size_t)splits * R[i] * C[i] * sizeof(float);
   return n;
+}
+// Weight gradients of 16-bit modules: LARGE, or MEDIUM_FULL with or without a split reduction, chosen
+// for the problems together (their tiles share the rounds of workgroups).
+int64_t dw_group_tiles(const TileCost& c, int count, const int64_t* R, const int64_t* C) {
+  int64_t n = 0;
+  for (int i = 0; i < count; ++i) n += tiles_of(c, DW, R[i], C[i]);
+  return n;
+}
+GemmPlan plan_dw_group(int count, int64_t Mred, const int64_t* R, const int64_t* C) {
+  double out = 0;
+  for (int i = 0; i < count; ++i) out += (double)R[i] * (double)C[i];
+  const int64_t large = dw_group_tiles(kLarge, count, R, C), kt = cdiv(Mred, 64);
+  GemmPlan p = cheapest(DW, large, 0, dw_group_tiles(kMedium, count, R, C), kt, out, true);
+  if (p.tile_class != gmlp::TILE_LARGE && plan_streamk(GMLP_F16, large, kt, false).tiles > 0) {
+    const double us = streamk_us(DW, large, kt, out);
+    if (us < p.us) p = GemmPlan{gmlp::TILE_LARGE, 1, us};
+  }
+  return p;
 }
 
 size_t split_workspace_bytes(int splits, int64_t rows, int64_t cols, int accumulator_sets = 1) {
   return splits > 1 ? (size_t)splits * accumulator_sets * rows * cols * sizeof(float) : 0;
-}
-
-// The down projection of float32 modules asks for no workspace (callers rely on that).
-int pick_splits_linear(int dtype, int64_t M, int64_t cols, int64_t R) {
-  return dtype == GMLP_F32 ? 1 : pick_splits(dtype, M, cols, R, (R + 63) / 64);
-}
-// dH of float32 modules splits its reduction like the other GEMMs; the 16-bit kernels do not.
-int pick_splits_dh(int dtype, int64_t M, int64_t N, int64_t K) {
-  return dtype == GMLP_F32 ? pick_splits(dtype, M, N, K, (K + 63) / 64) : 1;
 }
 
 // A GEMM with a split reduction: `launch` leaves `sets` accumulator sets of fp32 partial sums per split
@@ -319,6 +398,33 @@ hipError_t run_split(gmlp::GemmArgs& ga, int splits, int sets, void* workspace, 
   const typename gmlp::EpiPartial<T>::Args pa = {(float*)workspace, sets * set, acc_stride, (int)cols};
   if (hipError_t err = launch(ga, pa)) return err;
   return gmlp::launch_splitk_reduce<T, Epi>((const float*)workspace, splits, sets * set, acc_stride, ea, rows, cols, s);
+}
+
+// Runs a GEMM as planned.  run(first, count, plan, sk) launches the output columns (forward) or rows
+// (dH, dX) [first, first + count); `sk`: the launch's stream-K plan, or null.
+template <typename Run>
+hipError_t run_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red, const void* workspace, size_t workspace_bytes,
+                    Run&& run) {
+  const int64_t all = kind <= LINEAR ? cols : rows;
+  GemmPlan p = plan_gemm(dtype, kind, rows, cols, red, true);
+  if (p.splits > 1 && (workspace == nullptr || workspace_bytes < split_workspace_bytes(p.splits, rows, cols, kind == GATEUP ? 2 : 1)))
+    p = plan_gemm(dtype, kind, rows, cols, red, false);
+  if (p.tile_class == gmlp::TILE_LARGE) {
+    // a thin last round behind a long reduction: its tiles are shared out by reduction range
+    const StreamK sk = plan_streamk(dtype, tiles_of(kLarge, kind, rows, cols), red_tiles_of(kind, red));
+    if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, all, p, &sk);
+    // behind a short one: the whole rounds, then the rest as a problem of its own, for which the planner
+    // usually picks smaller tiles (measured on the gate/up GEMM: 1.375 rounds 114 -> 95 us, 5.375
+    // rounds 627 -> 611 us, 3.5 rounds 416 -> 407 us)
+    const int64_t whole = whole_rounds(kind, rows, cols);
+    if (whole > 0) {
+      const int64_t first = whole * (kind <= LINEAR ? tile_cols(kind) : 256), rest = all - first;
+      if (hipError_t err = run(0, first, p, nullptr)) return err;
+      return run(first, rest, plan_gemm(dtype, kind, kind <= LINEAR ? rows : rest, kind <= LINEAR ? rest : cols, red, false),
+                 nullptr);
+    }
+  }
+  return run(0, all, p, nullptr);
 }
 
 std::mutex& lds_registry_mutex() {
@@ -372,29 +478,20 @@ size_t gmlp_workspace_bytes(int op, int64_t M, int64_t K, int64_t N, int dtype) 
   if (M < 1 || N < 1) return 0;
   if (op == GMLP_OP_COLSUM) return gmlp::colsum_workspace_bytes(M, N);
   if (K < 1) return 0;
-  // Each operation asks for the larger of what its split-reduction form (short batches) and its
-  // stream-K form (large tiles whose grid ends in a thinly filled round) would use.
-  auto larger = [](size_t a, size_t b) { return a > b ? a : b; };
-  auto sk = [&](int64_t rows, int64_t cols, int64_t red_tiles, int bn) -> size_t {
-    if (pick_tile(dtype, rows, cols, red_tiles * 64, bn) != gmlp::TILE_LARGE) return 0;
-    return plan_streamk(dtype, cdiv(rows, 256) * cdiv(cols, bn), red_tiles).ws_bytes;
+  // Each operation asks for what its plan uses: partial sums of a split reduction, or, large tiles whose
+  // grid ends in a thinly filled round, the stream-K slots.
+  auto bytes = [&](int kind, int64_t rows, int64_t cols, int64_t red) -> size_t {
+    const GemmPlan p = plan_gemm(dtype, kind, rows, cols, red, true);
+    if (p.tile_class == gmlp::TILE_LARGE)
+      return plan_streamk(dtype, tiles_of(kLarge, kind, rows, cols), red_tiles_of(kind, red)).ws_bytes;
+    return split_workspace_bytes(p.splits, rows, cols, kind == GATEUP ? 2 : 1);
   };
-  // gmlp_gateup_fwd(M, K, N): two accumulator sets [M,N], reduction K
-  if (op == GMLP_OP_GATEUP_FWD)
-    return larger(split_workspace_bytes(pick_splits(dtype, M, N, K, (K + 63) / 64, 128), M, N, 2),
-                  sk(M, N, cdiv(K, 64), 128));
-  // gmlp_linear_fwd(M, R = K, C = N): out [M,N], reduction K
-  if (op == GMLP_OP_LINEAR_FWD)
-    return larger(split_workspace_bytes(pick_splits_linear(dtype, M, N, K), M, N), sk(M, N, cdiv(K, 64), 256));
-  // gmlp_dx_bwd(M, K, N): out [M,K], reduction over two segments of N
-  if (op == GMLP_OP_DX_BWD)
-    return larger(split_workspace_bytes(pick_splits(dtype, M, K, N, 2 * ((N + 63) / 64)), M, K),
-                  sk(M, K, 2 * cdiv(N, 64), 256));
-  // gmlp_dh_bwd(M, K, N): out [M,N], reduction K
-  if (op == GMLP_OP_DH_BWD)
-    return larger(split_workspace_bytes(pick_splits_dh(dtype, M, N, K), M, N), sk(M, N, cdiv(K, 64), 256));
+  if (op == GMLP_OP_GATEUP_FWD) return bytes(GATEUP, M, N, K);  // gmlp_gateup_fwd(M, K, N)
+  if (op == GMLP_OP_LINEAR_FWD) return bytes(LINEAR, M, N, K);  // gmlp_linear_fwd(M, R = K, C = N)
+  if (op == GMLP_OP_DX_BWD) return bytes(DX, M, K, N);          // gmlp_dx_bwd(M, K, N): two segments of N
+  if (op == GMLP_OP_DH_BWD) return bytes(DH, M, N, K);          // gmlp_dh_bwd(M, K, N)
   // gmlp_dw_bwd(Mred = M, R = K, C = N): out [K,N], reduction over the M token rows
-  if (op == GMLP_OP_DW_BWD) return dtype == GMLP_F32 ? dw_group_f32_bytes(1, M, &K, &N) : sk(K, N, (M + 63) / 64, 256);
+  if (op == GMLP_OP_DW_BWD) return gmlp_dw_bwd_grouped_workspace_bytes(1, M, &K, &N, dtype);
   return 0;
 }
 
@@ -422,7 +519,7 @@ int gmlp_gateup_fwd(const void* x, const void* w_gate, const void* w_up, const v
     typedef decltype(tag) T;
     // The GEMM over output columns [col0, col0 + cols): every per-column pointer moves along, the
     // row pitch of the outputs stays N.
-    auto run = [&](int64_t col0, int64_t cols, bool may_split, int force_class, const StreamK* sk = nullptr) -> hipError_t {
+    auto run = [&](int64_t col0, int64_t cols, const GemmPlan& plan, const StreamK* sk) -> hipError_t {
       GemmArgs ga = {};
       ga.nxcd = num_xcd();
       if (sk) use_streamk(*sk, ga, workspace, workspace_bytes);
@@ -433,29 +530,12 @@ int gmlp_gateup_fwd(const void* x, const void* w_gate, const void* w_up, const v
       auto at = [&](const void* p) { return p ? (const T*)p + col0 : nullptr; };
       typename EpiGateUp<T>::Args ea = {(T*)at(h), (T*)at(g_save), (T*)at(u_save), mask_out ? mask_out + col0 : nullptr,
                                         at(b_gate), at(b_up), (int)N, act, d, (size_t)col0};
-      const int splits = may_split ? pick_splits(dtype, M, cols, K, (K + 63) / 64, 128) : 1;
-      if (splits > 1 && workspace != nullptr && workspace_bytes >= split_workspace_bytes(splits, M, cols, 2))
-        return run_split<T, EpiGateUp<T>>(ga, splits, 2, workspace, ea, M, cols, s,
-                                          [&](auto& g, auto& pa) { return launch_gateup_split<T>(g, pa, s); });
-      return launch_gateup<T>(force_class >= 0 ? force_class : pick_tile(dtype, M, cols, K, 128), ga, ea, s);
+      if (plan.splits > 1)
+        return run_split<T, EpiGateUp<T>>(ga, plan.splits, 2, workspace, ea, M, cols, s,
+                                          [&](auto& g, auto& pa) { return launch_gateup_split<T>(plan.tile_class, g, pa, s); });
+      return launch_gateup<T>(plan.tile_class, ga, ea, s);
     };
-    // A grid of large tiles that ends in a thinly filled round of workgroups runs as two launches:
-    // the tile columns that make whole rounds, and the remaining columns as a problem of their own,
-    // for which pick_tile usually chooses the small tiles (measured on the gate/up GEMM: 1.375
-    // rounds 114 -> 95 us, 5.375 rounds 627 -> 611 us, 3.5 rounds 416 -> 407 us).
-    if (dtype != GMLP_F32 && pick_tile(dtype, M, N, K, 128) == TILE_LARGE) {
-      const int64_t tiles_m = (M + 255) / 256, tiles_n = (N + 127) / 128, cus = num_cu();
-      // a long reduction: the tiles of the last round are shared out by reduction range instead
-      const StreamK sk = plan_streamk(dtype, tiles_m * tiles_n, cdiv(K, 64));
-      if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, N, false, TILE_LARGE, &sk);
-      const int64_t rounds = tiles_m * tiles_n / cus, tail = tiles_m * tiles_n % cus;
-      const int64_t whole_cols = rounds * cus / tiles_m;  // tile columns of the whole rounds
-      if (rounds >= 1 && tail > 0 && 2 * tail <= cus && whole_cols >= 1 && whole_cols < tiles_n) {
-        if (hipError_t err = run(0, whole_cols * 128, false, TILE_LARGE)) return err;
-        return run(whole_cols * 128, N - whole_cols * 128, false, -1);
-      }
-    }
-    return run(0, N, true, -1);
+    return run_plan(dtype, GATEUP, M, N, K, workspace, workspace_bytes, run);
   });
   return hip_result(__func__, e);
 }
@@ -475,7 +555,7 @@ int gmlp_linear_fwd(const void* a, const void* w, const void* bias, void* out, i
   hipError_t e = by_dtype(dtype, [&](auto tag) -> hipError_t {
     typedef decltype(tag) T;
     // The GEMM over output columns [col0, col0 + cols); the row pitch of `out` stays C.
-    auto run = [&](int64_t col0, int64_t cols, bool may_split, int force_class, const StreamK* sk = nullptr) -> hipError_t {
+    auto run = [&](int64_t col0, int64_t cols, const GemmPlan& plan, const StreamK* sk) -> hipError_t {
       GemmArgs ga = {};
       ga.nxcd = num_xcd();
       if (sk) use_streamk(*sk, ga, workspace, workspace_bytes);
@@ -484,26 +564,12 @@ int gmlp_linear_fwd(const void* a, const void* w, const void* bias, void* out, i
       ga.M = (int)M; ga.N = (int)cols; ga.K = (int)R; ga.lda = (int)R; ga.ldb = (int)R;
       ga.nseg = 1; ga.group_m = pick_group(M, cols); ga.rotate = M <= 512;
       typename EpiStore<T>::Args ea = {(T*)out + col0, bias ? (const T*)bias + col0 : nullptr, (int)C};
-      const int splits = may_split ? pick_splits_linear(dtype, M, cols, R) : 1;
-      if (splits > 1 && workspace != nullptr && workspace_bytes >= split_workspace_bytes(splits, M, cols))
-        return run_split<T, EpiStore<T>>(ga, splits, 1, workspace, ea, M, cols, s,
-                                         [&](auto& g, auto& pa) { return launch_linear_split<T>(g, pa, s); });
-      return launch_linear<T>(force_class >= 0 ? force_class : pick_tile(dtype, M, cols, R, 256), ga, ea, s);
+      if (plan.splits > 1)
+        return run_split<T, EpiStore<T>>(ga, plan.splits, 1, workspace, ea, M, cols, s,
+                                         [&](auto& g, auto& pa) { return launch_linear_split<T>(plan.tile_class, g, pa, s); });
+      return launch_linear<T>(plan.tile_class, ga, ea, s);
     };
-    // whole rounds of large tiles, then the remaining tile columns as a problem of their own (see
-    // gmlp_gateup_fwd)
-    if (dtype != GMLP_F32 && pick_tile(dtype, M, C, R, 256) == TILE_LARGE) {
-      const int64_t tiles_m = (M + 255) / 256, tiles_n = (C + 255) / 256, cus = num_cu();
-      const StreamK sk = plan_streamk(dtype, tiles_m * tiles_n, cdiv(R, 64));
-      if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, C, false, TILE_LARGE, &sk);
-      const int64_t rounds = tiles_m * tiles_n / cus, tail = tiles_m * tiles_n % cus;
-      const int64_t whole_cols = rounds * cus / tiles_m;
-      if (rounds >= 1 && tail > 0 && 2 * tail <= cus && whole_cols >= 1 && whole_cols < tiles_n) {
-        if (hipError_t err = run(0, whole_cols * 256, false, TILE_LARGE)) return err;
-        return run(whole_cols * 256, C - whole_cols * 256, false, -1);
-      }
-    }
-    return run(0, C, true, -1);
+    return run_plan(dtype, LINEAR, M, C, R, workspace, workspace_bytes, run);
   });
   return hip_result(__func__, e);
 }
@@ -530,7 +596,7 @@ int gmlp_dh_bwd(const void* dy, const void* w_down, const void* g, const void* u
   hipError_t e = by_dtype(dtype, [&](auto tag) -> hipError_t {
     typedef decltype(tag) T;
     // The GEMM over output rows [row0, row0 + rows): every per-row pointer moves along.
-    auto run = [&](int64_t row0, int64_t rows, int force_class, const StreamK* sk = nullptr) -> hipError_t {
+    auto run = [&](int64_t row0, int64_t rows, const GemmPlan& plan, const StreamK* sk) -> hipError_t {
       GemmArgs ga = {};
       ga.nxcd = num_xcd();
       if (sk) use_streamk(*sk, ga, workspace, workspace_bytes);
@@ -539,22 +605,12 @@ int gmlp_dh_bwd(const void* dy, const void* w_down, const void* g, const void* u
       ga.nseg = 1; ga.group_m = pick_group(rows, N);
       const size_t e0 = (size_t)row0 * N;
       typename EpiDh<T>::Args ea = {(const T*)g + e0, (const T*)u + e0, (T*)dg + e0, (T*)du + e0, (int)N, act, d, e0};
-      const int splits = force_class < 0 ? pick_splits_dh(dtype, rows, N, K) : 1;
-      if (splits > 1 && workspace != nullptr && workspace_bytes >= split_workspace_bytes(splits, rows, N))
-        return run_split<T, EpiDh<T>>(ga, splits, 1, workspace, ea, rows, N, s,
-                                      [&](auto& g, auto& pa) { return launch_dx_split<T>(g, pa, s); });  // one segment
-      return launch_dh<T>(force_class >= 0 ? force_class : pick_tile(dtype, rows, N, K, 256), ga, ea, s);
+      if (plan.splits > 1)  // (the partial sums' kernel of dX, with one reduction segment)
+        return run_split<T, EpiDh<T>>(ga, plan.splits, 1, workspace, ea, rows, N, s,
+                                      [&](auto& g, auto& pa) { return launch_dx_split<T>(plan.tile_class, g, pa, s); });
+      return launch_dh<T>(plan.tile_class, ga, ea, s);
     };
-    if (dtype != GMLP_F32 && pick_tile(dtype, M, N, K, 256) == TILE_LARGE) {
-      const StreamK sk = plan_streamk(dtype, cdiv(M, 256) * cdiv(N, 256), cdiv(K, 64));
-      if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, M, TILE_LARGE, &sk);
-    }
-    int64_t whole = whole_round_tile_rows(dtype, M, N, K);
-    if (whole > 0) {
-      if (hipError_t err = run(0, whole * 256, TILE_LARGE)) return err;
-      return run(whole * 256, M - whole * 256, -1);
-    }
-    return run(0, M, -1);
+    return run_plan(dtype, DH, M, N, K, workspace, workspace_bytes, run);
   });
   return hip_result(__func__, e);
 }
@@ -599,7 +655,7 @@ int gmlp_dx_bwd(const void* dg, const void* du, const void* w_gate, const void* 
   hipError_t e = by_dtype(dtype, [&](auto tag) -> hipError_t {
     typedef decltype(tag) T;
     // The GEMM over output rows [row0, row0 + rows).
-    auto run = [&](int64_t row0, int64_t rows, bool may_split, int force_class, const StreamK* sk = nullptr) -> hipError_t {
+    auto run = [&](int64_t row0, int64_t rows, const GemmPlan& plan, const StreamK* sk) -> hipError_t {
       GemmArgs ga = {};
       ga.nxcd = num_xcd();
       if (sk) use_streamk(*sk, ga, workspace, workspace_bytes);
@@ -609,22 +665,12 @@ int gmlp_dx_bwd(const void* dg, const void* du, const void* w_gate, const void* 
       // (no rotated reduction order here: a piece has room for one change of direction, and with
       // two reduction segments that is the step from dG·W_gate to dU·W_up)
       typename EpiStore<T>::Args ea = {(T*)dx + row0 * K, nullptr, (int)K};
-      const int splits = may_split ? pick_splits(dtype, rows, K, N, 2 * ((N + 63) / 64)) : 1;
-      if (splits > 1 && workspace != nullptr && workspace_bytes >= split_workspace_bytes(splits, rows, K))
-        return run_split<T, EpiStore<T>>(ga, splits, 1, workspace, ea, rows, K, s,
-                                         [&](auto& g, auto& pa) { return launch_dx_split<T>(g, pa, s); });
-      return launch_dx<T>(force_class >= 0 ? force_class : pick_tile(dtype, rows, K, N, 256), ga, ea, s);
+      if (plan.splits > 1)
+        return run_split<T, EpiStore<T>>(ga, plan.splits, 1, workspace, ea, rows, K, s,
+                                         [&](auto& g, auto& pa) { return launch_dx_split<T>(plan.tile_class, g, pa, s); });
+      return launch_dx<T>(plan.tile_class, ga, ea, s);
     };
-    if (dtype != GMLP_F32 && pick_tile(dtype, M, K, N, 256) == TILE_LARGE) {
-      const StreamK sk = plan_streamk(dtype, cdiv(M, 256) * cdiv(K, 256), 2 * cdiv(N, 64));
-      if (sk.tiles > 0 && workspace != nullptr && workspace_bytes >= sk.ws_bytes) return run(0, M, false, TILE_LARGE, &sk);
-    }
-    int64_t whole = whole_round_tile_rows(dtype, M, K, N);
-    if (whole > 0) {
-      if (hipError_t err = run(0, whole * 256, false, TILE_LARGE)) return err;
-      return run(whole * 256, M - whole * 256, false, -1);
-    }
-    return run(0, M, true, -1);
+    return run_plan(dtype, DX, M, K, N, workspace, workspace_bytes, run);
   });
   return hip_result(__func__, e);
 }
@@ -640,23 +686,7 @@ int gmlp_dw_bwd(const void* lhs, const void* rhs, void* dw, int64_t Mred, int64_
   GMLP_REQUIRE_ALIGNED(lhs); GMLP_REQUIRE_ALIGNED(rhs); GMLP_REQUIRE_ALIGNED(dw);
   GMLP_REQUIRE_ALIGNED(workspace);
 
-  if (dtype == GMLP_F32) return gmlp_dw_bwd_grouped(1, &lhs, &rhs, &dw, Mred, &R, &C, dtype, workspace, workspace_bytes, stream);
-
-  // dW[R,C] = lhs[Mred,R]ᵀ · rhs[Mred,C]: both operands reduction-strided.
-  GemmArgs ga = {};
-      ga.nxcd = num_xcd();
-  ga.A[0] = lhs; ga.A[1] = lhs; ga.B[0] = rhs; ga.B[1] = rhs;
-  ga.M = (int)R; ga.N = (int)C; ga.K = (int)Mred; ga.lda = (int)R; ga.ldb = (int)C;
-  ga.nseg = 1; ga.group_m = pick_group(R, C);
-  int tc = pick_tile(dtype, R, C, Mred, 256);
-  if (tc == TILE_LARGE) use_streamk(plan_streamk(dtype, cdiv(R, 256) * cdiv(C, 256), cdiv(Mred, 64)), ga, workspace, workspace_bytes);
-  hipStream_t s = (hipStream_t)stream;
-  hipError_t e = by_dtype(dtype, [&](auto tag) {
-    typedef decltype(tag) T;
-    typename EpiStore<T>::Args ea = {(T*)dw, nullptr, (int)C};
-    return launch_dw<T>(tc, ga, ea, s);
-  });
-  return hip_result(__func__, e);
+  return gmlp_dw_bwd_grouped(1, &lhs, &rhs, &dw, Mred, &R, &C, dtype, workspace, workspace_bytes, stream);
 }
 
 size_t gmlp_dw_bwd_grouped_workspace_bytes(int count, int64_t Mred, const int64_t* R, const int64_t* C, int dtype) {
@@ -665,17 +695,14 @@ size_t gmlp_dw_bwd_grouped_workspace_bytes(int count, int64_t Mred, const int64_
   if (dtype == GMLP_F32) {
     for (int i = 0; i < count; ++i)
       if (R[i] < 1 || C[i] < 1) return 0;
-    return dw_group_f32_bytes(count, Mred, R, C);
+    return dw_group_split_bytes(count, plan_dw_group_f32(count, Mred, R, C).splits, R, C);
   }
-  int64_t tiles256 = 0, tiles128 = 0;
-  for (int i = 0; i < count; ++i) {
-    if (R[i] < 1 || C[i] < 1 || pick_tile(dtype, R[i], C[i], Mred, 256) == TILE_MEDIUM) return 0;
-    tiles256 += cdiv(R[i], 256) * cdiv(C[i], 256);
-    tiles128 += cdiv(R[i], 128) * cdiv(C[i], 128);
-  }
-  if (group_tile_class(tiles256, tiles128) != TILE_LARGE) return 0;
-  const StreamK sk = plan_streamk(dtype, tiles256, cdiv(Mred, 64));
-  return sk.tiles > cdiv(R[count - 1], 256) * cdiv(C[count - 1], 256) ? 0 : sk.ws_bytes;
+  for (int i = 0; i < count; ++i)
+    if (R[i] < 1 || C[i] < 1 || plan_gemm(dtype, DW, R[i], C[i], Mred, false).tile_class == TILE_MEDIUM) return 0;
+  const GemmPlan p = plan_dw_group(count, Mred, R, C);
+  if (p.tile_class != TILE_LARGE) return dw_group_split_bytes(count, p.splits, R, C);
+  const StreamK sk = plan_streamk(dtype, dw_group_tiles(kLarge, count, R, C), cdiv(Mred, 64), false);
+  return sk.tiles > tiles_of(kLarge, DW, R[count - 1], C[count - 1]) ? 0 : sk.ws_bytes;
 }
 
 int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rhs, void* const* dw,
@@ -696,12 +723,7 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
     if (int rc = check_mult8(__func__, "R", R[i])) return rc;
     if (int rc = check_mult8(__func__, "C", C[i])) return rc;
     GMLP_REQUIRE_ALIGNED(lhs[i]); GMLP_REQUIRE_ALIGNED(rhs[i]); GMLP_REQUIRE_ALIGNED(dw[i]);
-    pipelined = pipelined && pick_tile(dtype, R[i], C[i], Mred, 256) != TILE_MEDIUM;
-  }
-  if (!pipelined) {
-    for (int i = 0; i < count; ++i)
-      if (int rc = gmlp_dw_bwd(lhs[i], rhs[i], dw[i], Mred, R[i], C[i], dtype, workspace, workspace_bytes, stream)) return rc;
-    return GMLP_OK;
+    pipelined = pipelined && plan_gemm(dtype, DW, R[i], C[i], Mred, false).tile_class != TILE_MEDIUM;
   }
   hipStream_t s = (hipStream_t)stream;
   auto fill = [&](GemmArgs& ga, int i) {
@@ -711,32 +733,42 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
     ga.M = (int)R[i]; ga.N = (int)C[i]; ga.K = (int)Mred; ga.lda = (int)R[i]; ga.ldb = (int)C[i];
     ga.nseg = 1; ga.group_m = pick_group(R[i], C[i]);
   };
-  if (dtype == GMLP_F32) {
-    PlanF32 plan = plan_dw_group_f32(count, Mred, R, C);
-    if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < dw_group_f32_bytes(count, Mred, R, C))) plan.splits = 1;
-    GemmGroup<EpiStore<float>::Args> grp = {};
-    GemmGroup<EpiPartial<float>::Args> part = {};
-    grp.count = part.count = count;
-    float* ws = (float*)workspace;
-    for (int i = 0; i < count; ++i) {
-      fill(grp.ga[i], i);
-      grp.ga[i].splits = plan.splits;
-      grp.ea[i] = {(float*)dw[i], nullptr, (int)C[i]};
-      part.ga[i] = grp.ga[i];
-      part.ea[i] = {ws, (size_t)R[i] * C[i], 0, (int)C[i]};
-      ws += (size_t)plan.splits * R[i] * C[i];
-    }
-    if (plan.splits == 1) return hip_result(__func__, launch_dw_group<float>(plan.tile_class, grp, s));
-    hipError_t e = launch_dw_group_split_f32(part, s);
-    if (e == hipSuccess) e = launch_splitk_reduce_group(part, grp, s);
+  if (!pipelined) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < count && e == hipSuccess; ++i)
+      e = by_dtype(dtype, [&](auto tag) {
+        typedef decltype(tag) T;
+        GemmArgs ga;
+        fill(ga, i);
+        const typename EpiStore<T>::Args ea = {(T*)dw[i], nullptr, (int)C[i]};
+        return launch_dw<T>(TILE_MEDIUM, ga, ea, s);
+      });
     return hip_result(__func__, e);
   }
-  int64_t tiles256 = 0, tiles128 = 0;
-  for (int i = 0; i < count; ++i) {
-    tiles256 += ((R[i] + 255) / 256) * ((C[i] + 255) / 256);
-    tiles128 += ((R[i] + 127) / 128) * ((C[i] + 127) / 128);
+  GemmPlan plan = dtype == GMLP_F32 ? plan_dw_group_f32(count, Mred, R, C) : plan_dw_group(count, Mred, R, C);
+  if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < dw_group_split_bytes(count, plan.splits, R, C))) plan.splits = 1;
+  if (dtype == GMLP_F32 || plan.splits > 1) {
+    return hip_result(__func__, by_dtype(dtype, [&](auto tag) -> hipError_t {
+      typedef decltype(tag) T;
+      GemmGroup<typename EpiStore<T>::Args> grp = {};
+      GemmGroup<typename EpiPartial<T>::Args> part = {};
+      grp.count = part.count = count;
+      float* ws = (float*)workspace;
+      for (int i = 0; i < count; ++i) {
+        fill(grp.ga[i], i);
+        grp.ga[i].splits = plan.splits;
+        grp.ea[i] = {(T*)dw[i], nullptr, (int)C[i]};
+        part.ga[i] = grp.ga[i];
+        part.ea[i] = {ws, (size_t)R[i] * C[i], 0, (int)C[i]};
+        ws += (size_t)plan.splits * R[i] * C[i];
+      }
+      if (plan.splits == 1) return launch_dw_group<T>(plan.tile_class, grp, s);
+      if (hipError_t err = launch_dw_group_split<T>(part, s)) return err;
+      return launch_splitk_reduce_group<T>(part, grp, s);
+    }));
   }
-  const int group_class = group_tile_class(tiles256, tiles128);
+  const int group_class = plan.tile_class;
+  const int64_t tiles256 = dw_group_tiles(kLarge, count, R, C);
   // A grid of large tiles that ends in a thinly filled round: the last problem gives up a band of
   // its output (whole tile rows or tile columns, whichever comes closer to the tiles of that last
   // round), which runs as a launch of its own on the tile class that suits it; the rest then makes
@@ -748,7 +780,7 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
   // by reduction range instead (stream-K), if the last problem has that many tiles.
   StreamK sk;
   if (group_class == TILE_LARGE) {
-    sk = plan_streamk(dtype, tiles256, cdiv(Mred, 64));
+    sk = plan_streamk(dtype, tiles256, cdiv(Mred, 64), false);
     if (sk.tiles > cdiv(R[last], 256) * cdiv(C[last], 256) || workspace == nullptr || workspace_bytes < sk.ws_bytes) sk = StreamK{};
   }
   if (group_class == TILE_LARGE && sk.tiles == 0) {
@@ -761,7 +793,7 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
       if (cols_fit && (!rows_fit || by_cols * tr <= by_rows * tc)) band_cols = C[last] - (tc - by_cols) * 256;
       else if (rows_fit) band_rows = R[last] - (tr - by_rows) * 256;
       const int64_t br = band_rows ? band_rows : R[last], bc = band_cols ? band_cols : C[last];
-      if ((band_rows || band_cols) && pick_tile(dtype, br, bc, Mred, 256) == TILE_MEDIUM) band_rows = band_cols = 0;
+      if ((band_rows || band_cols) && plan_gemm(dtype, DW, br, bc, Mred, false).tile_class == TILE_MEDIUM) band_rows = band_cols = 0;
     }
   }
   hipError_t e = by_dtype(dtype, [&](auto tag) -> hipError_t {
@@ -791,7 +823,7 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
       ga.N = (int)(C[last] - c0);
       ga.group_m = pick_group(ga.M, ga.N);
       typename EpiStore<T>::Args ea = {(T*)dw[last] + r0 * C[last] + c0, nullptr, (int)C[last]};
-      return launch_dw<T>(pick_tile(dtype, ga.M, ga.N, Mred, 256), ga, ea, s);
+      return launch_dw<T>(plan_gemm(dtype, DW, ga.M, ga.N, Mred, false).tile_class, ga, ea, s);
     }
   });
   return hip_result(__func__, e);

@@ -92,25 +92,33 @@ GMLP_REDUCE_INST(bf16, EpiGateUp)
 
 // The same for the weight gradients of one pass (contiguous outputs without a bias): blockIdx.y
 // selects the problem.
+template <typename T>
 struct ReduceGroup {
   const float* ws[GEMM_GROUP_MAX];
-  float* out[GEMM_GROUP_MAX];
+  T* out[GEMM_GROUP_MAX];
   size_t n[GEMM_GROUP_MAX];  // elements of an output, and between consecutive splits
   int splits[GEMM_GROUP_MAX];
 };
-__global__ void __launch_bounds__(256) splitk_reduce_group_kernel(ReduceGroup g) {
+template <typename T>
+__global__ void __launch_bounds__(256) splitk_reduce_group_kernel(ReduceGroup<T> g) {
   const int p = blockIdx.y;
   const float* __restrict__ ws = g.ws[p];
-  const size_t n = g.n[p], step = (size_t)gridDim.x * 256 * 4;
-  for (size_t e = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; e < n; e += step) {
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    for (int i = 0; i < g.splits[p]; ++i) s += *(const f32x4*)(ws + (size_t)i * n + e);
-    __builtin_nontemporal_store(s, (f32x4*)(g.out[p] + e));
+  const size_t n = g.n[p], step = (size_t)gridDim.x * 256 * 8;
+  for (size_t e = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8; e < n; e += step) {
+    f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+#pragma unroll 4
+    for (int i = 0; i < g.splits[p]; ++i) {
+      a += *(const f32x4*)(ws + (size_t)i * n + e);
+      b += *(const f32x4*)(ws + (size_t)i * n + e + 4);
+    }
+    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    store_w<T, 8, true>(g.out[p] + e, v);
   }
 }
-hipError_t launch_splitk_reduce_group(const GemmGroup<EpiPartial<float>::Args>& part,
-                                      const GemmGroup<EpiStore<float>::Args>& out, hipStream_t s) {
-  ReduceGroup g = {};
+template <typename T>
+hipError_t launch_splitk_reduce_group(const GemmGroup<typename EpiPartial<T>::Args>& part,
+                                      const GemmGroup<typename EpiStore<T>::Args>& out, hipStream_t s) {
+  ReduceGroup<T> g = {};
   size_t most = 0;
   for (int i = 0; i < part.count; ++i) {
     g.ws[i] = part.ea[i].ws;
@@ -119,11 +127,18 @@ hipError_t launch_splitk_reduce_group(const GemmGroup<EpiPartial<float>::Args>& 
     g.splits[i] = part.ga[i].splits;
     if (g.n[i] > most) most = g.n[i];
   }
-  size_t blocks = (most / 4 + 255) / 256;
+  size_t blocks = (most / 8 + 255) / 256;
   if (blocks > 256 * 8) blocks = 256 * 8;
-  hipLaunchKernelGGL(splitk_reduce_group_kernel, dim3((unsigned)blocks, part.count), dim3(256), 0, s, g);
+  hipLaunchKernelGGL(splitk_reduce_group_kernel<T>, dim3((unsigned)blocks, part.count), dim3(256), 0, s, g);
   return hipGetLastError();
 }
+#define GMLP_REDUCE_GROUP_INST(T)                                                                          \
+  template hipError_t launch_splitk_reduce_group<T>(const GemmGroup<EpiPartial<T>::Args>&,                 \
+                                                    const GemmGroup<EpiStore<T>::Args>&, hipStream_t);
+GMLP_REDUCE_GROUP_INST(f16)
+GMLP_REDUCE_GROUP_INST(bf16)
+GMLP_REDUCE_GROUP_INST(float)
+#undef GMLP_REDUCE_GROUP_INST
 
 // Column sums in two fixed-order stages: COLSUM_SPLITS row ranges -> fp32 partials -> total.
 // Up to COLSUM_GROUP_MAX arrays with the same number of rows share the two launches (the bias

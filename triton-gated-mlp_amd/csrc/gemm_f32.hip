@@ -323,15 +323,15 @@ hipError_t launch_dw<float>(int, const GemmArgs&, const EpiStore<float>::Args&, 
 }
 // Split reductions run on the smallest tile only (a grid of larger ones would be split further).
 template <>
-hipError_t launch_gateup_split_kt<float, false>(const GemmArgs& ga, const EpiPartial<float>::Args& ea, hipStream_t s) {
+hipError_t launch_gateup_split_kt<float, false>(int, const GemmArgs& ga, const EpiPartial<float>::Args& ea, hipStream_t s) {
   return launch_f32_tile<64, 64, false, false, 2, EpiPartial<float>>(ga, ea, s);
 }
 template <>
-hipError_t launch_linear_split_kt<float, false>(const GemmArgs&, const EpiPartial<float>::Args&, hipStream_t) {
+hipError_t launch_linear_split_kt<float, false>(int, const GemmArgs&, const EpiPartial<float>::Args&, hipStream_t) {
   return hipErrorInvalidValue;  // the float32 down projection does not split (pick_splits_linear)
 }
 template <>
-hipError_t launch_dx_split_kt<float, false>(const GemmArgs& ga, const EpiPartial<float>::Args& ea, hipStream_t s) {
+hipError_t launch_dx_split_kt<float, false>(int, const GemmArgs& ga, const EpiPartial<float>::Args& ea, hipStream_t s) {
   return launch_f32_tile<64, 64, false, true, 1, EpiPartial<float>>(ga, ea, s);
 }
 
@@ -355,7 +355,8 @@ hipError_t launch_dw_group<float>(int tc, GemmGroup<EpiStore<float>::Args>& grp,
   if (tc == TILE_F32_64X128) return launch_f32_group<64, 128, EpiStore<float>>(grp, s);
   return launch_f32_group<64, 64, EpiStore<float>>(grp, s);
 }
-hipError_t launch_dw_group_split_f32(GemmGroup<EpiPartial<float>::Args>& grp, hipStream_t s) {
+template <>
+hipError_t launch_dw_group_split<float>(GemmGroup<EpiPartial<float>::Args>& grp, hipStream_t s) {
   return launch_f32_group<64, 64, EpiPartial<float>>(grp, s);
 }
 

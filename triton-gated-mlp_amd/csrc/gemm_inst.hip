@@ -19,6 +19,8 @@ constexpr bool KT = GMLP_KT;
   launch_gemm_pipelined<DT, 256, BN_L, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M) \
   launch_gemm_pipelined<DT, 128, BN_M, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
+#define GMLP_WIDE(AKS, BKS, NB, EPI, BN_W) \
+  launch_gemm_pipelined<DT, 128, BN_W, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_LARGE_GROUP \
   launch_gemm_group_pipelined<DT, 256, 256, 16, 2, 2, true, true, 1, EpiStore<DT>>
 #define GMLP_MEDIUM_GROUP \
@@ -26,6 +28,8 @@ constexpr bool KT = GMLP_KT;
 
 #define GMLP_DISPATCH(AKS, BKS, NB, EPI, BN_L, BN_M)                                             \
   if (tile_class == TILE_LARGE) return GMLP_LARGE(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
+  if constexpr (!(AKS))                                                                          \
+    if (tile_class == TILE_WIDE) return GMLP_WIDE(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
   if (tile_class == TILE_MEDIUM_FULL) return GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M)(ga, ea, s);    \
   if constexpr (KT) return hipErrorInvalidValue; /* launch.hpp sends it to the other unit */       \
   else return launch_gemm<DT, 128, BN_M, 64, 2, 2, AKS, BKS, NB, true, EPI<DT>>(ga, ea, s);
@@ -37,12 +41,14 @@ hipError_t launch_gateup_kt<DT, KT>(int tile_class, const GemmArgs& ga, const Ep
   // the usual case (SiLU, no keep-mask output) has kernels of its own, see EpiGateUpPacked
   if (EpiGateUpPacked<DT>::packed_eligible(ea)) {
     if (tile_class == TILE_LARGE) return GMLP_LARGE(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
+    if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
     if (tile_class == TILE_MEDIUM_FULL) return GMLP_MEDIUM(false, false, 2, EpiGateUpPacked, 64)(ga, ea, s);
   }
   GMLP_DISPATCH(false, false, 2, EpiGateUp, 128, 64)
 }
 template <>
-hipError_t launch_gateup_split_kt<DT, KT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+hipError_t launch_gateup_split_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 2, EpiPartial, 128)(ga, ea, s);
   return launch_gemm_pipelined<DT, 128, 64, 16, 2, 2, false, false, 2, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 1
@@ -52,7 +58,8 @@ hipError_t launch_linear_kt<DT, KT>(int tile_class, const GemmArgs& ga, const Ep
   GMLP_DISPATCH(false, false, 1, EpiStore, 256, 128)
 }
 template <>
-hipError_t launch_linear_split_kt<DT, KT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+hipError_t launch_linear_split_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 1, EpiPartial, 256)(ga, ea, s);
   return launch_gemm_pipelined<DT, 128, 128, 16, 2, 2, false, false, 1, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 2
@@ -68,7 +75,8 @@ hipError_t launch_dx_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiSto
   GMLP_DISPATCH(false, true, 1, EpiStore, 256, 128)
 }
 template <>
-hipError_t launch_dx_split_kt<DT, KT>(const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+hipError_t launch_dx_split_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
+  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, true, 1, EpiPartial, 256)(ga, ea, s);
   return launch_gemm_pipelined<DT, 128, 128, 16, 2, 2, false, true, 1, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 4
@@ -80,6 +88,10 @@ hipError_t launch_dw<DT>(int tile_class, const GemmArgs& ga, const EpiStore<DT>:
 template <>
 hipError_t launch_dw_group<DT>(int tile_class, GemmGroup<EpiStore<DT>::Args>& grp, hipStream_t s) {
   return tile_class == TILE_LARGE ? GMLP_LARGE_GROUP(grp, s) : GMLP_MEDIUM_GROUP(grp, s);
+}
+template <>
+hipError_t launch_dw_group_split<DT>(GemmGroup<EpiPartial<DT>::Args>& grp, hipStream_t s) {
+  return launch_gemm_group_pipelined<DT, 128, 128, 16, 2, 2, true, true, 1, EpiPartial<DT>>(grp, s);
 }
 #endif
 

@@ -78,8 +78,9 @@ struct PipeConfig {
   // to back at the rate the texture addresser can take at best, which is where a load that misses
   // L2 backs the queue up into the issuing wavefronts (down projection: queue-full stalls 166 -> 10
   // clocks per tile, 2664 -> 2451 clocks per tile, -4 % run time; input gradient -2 %).
-  static constexpr bool A3 = RING_A3 && (BM == 256 || BM == 128) && !A_KS;
-  static constexpr int MAIN_BYTES = A3 ? 3 * ATile::BYTES + NS * NB * BTile::BYTES : NS * STAGE;
+  static constexpr bool B3 = BM == 128 && NB * BN == 256;
+  static constexpr bool A3 = B3 || (RING_A3 && (BM == 256 || BM == 128) && !A_KS);
+  static constexpr int MAIN_BYTES = A3 ? 3 * ATile::BYTES + (B3 ? 3 : NS) * NB * BTile::BYTES : NS * STAGE;
   static_assert(MAIN_BYTES <= 160 * 1024, "a workgroup has 160 KiB of LDS");
   static constexpr int LDS_BYTES = MAIN_BYTES > NW * EPI_WAVE_BYTES ? MAIN_BYTES : NW * EPI_WAVE_BYTES;
   static_assert(G >= 2 && TM >= 2 && TM % 2 == 0, "rolling scheme needs >= 2 groups and an even TM");
@@ -103,7 +104,7 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
   constexpr int KSTEPS = Cfg::KSTEPS, STAGE = Cfg::STAGE, L = Cfg::LOADS;
   constexpr int LOAD_SLOTS = LOAD_CYCLES / Cfg::MFMA_CYCLES;  // MFMA slots per load
   constexpr int TILE_SLOTS = KSTEPS * G * TM;                         // MFMA slots per tile
-  constexpr bool A3 = Cfg::A3;
+  constexpr bool A3 = Cfg::A3, B3 = Cfg::B3;
   constexpr int LA = B_LOOKAHEAD;
   static_assert(LA >= 2 && LA <= 3 && LA <= G, "B ring has 4 entries");
   constexpr int HEAD_SLOTS = LA * TM;  // slots between the retiring barrier and the tile's end
@@ -335,10 +336,10 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
   auto l3_starts_group = [&](int z) __attribute__((always_inline)) { return (l3_index(z) & 3) == 0; };
   // M0 for the group that load z starts; b_parity: ring entry of the B tile being filled,
   // a_off: ring offset of the A tile being filled.
-  auto l3_base = [&](int z, int b_parity, uint32_t a_off) __attribute__((always_inline)) {
+  auto l3_base = [&](int z, uint32_t b_off, uint32_t a_off) __attribute__((always_inline)) {
     if (l3_is_b(z)) {
       const int bsel = z / BTile::PER_WAVE, i = z % BTile::PER_WAVE;
-      set_lds_dma_base(lds_base + A_RING + b_parity * B_ENTRY + bsel * BTile::BYTES +
+      set_lds_dma_base(lds_base + A_RING + b_off + bsel * BTile::BYTES +
                        (wave * BTile::PER_WAVE + i) * 1024);
     } else {
       set_lds_dma_base(lds_base + a_off + (wave * ATile::PER_WAVE + (z - LDB)) * 1024);
@@ -388,8 +389,8 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
   auto fetch_a3 = [&](int bank, int i, uint32_t a_off, int ks) __attribute__((always_inline)) {
     af[bank][i] = ATile::template frag_mi<MI>(smem + a_off, wm * WTM + i * MI, ks, lane);
   };
-  auto fetch_b3 = [&](int entry, int g, int kt, int ks) __attribute__((always_inline)) {
-    const char* s = smem + A_RING + (kt & 1) * B_ENTRY;
+  auto fetch_b3 = [&](int entry, int g, uint32_t b_off, int ks) __attribute__((always_inline)) {
+    const char* s = smem + A_RING + b_off;
     const int bsel = g / TN, j = g % TN;
     bq[entry] = BTile::template frag_mi<MI>(s + bsel * BTile::BYTES, wn * WTN + j * MI, ks, lane);
   };
@@ -468,6 +469,9 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
     // its own made the register allocator move accumulators around inside the loop)
     const uint32_t a_rd = ((uint32_t)(kt - kt_first) % 3u) * (uint32_t)A_ENTRY;
     const uint32_t a_nxt = a3_next(a_rd), a_fill = a3_prev(a_rd);
+    const uint32_t b_rd = B3 ? ((uint32_t)(kt - kt_first) % 3u) * (uint32_t)B_ENTRY : (uint32_t)(kt & 1) * (uint32_t)B_ENTRY;
+    const uint32_t b_nxt = B3 ? (b_rd == 2u * B_ENTRY ? 0u : b_rd + B_ENTRY) : (uint32_t)B_ENTRY - b_rd;
+    const uint32_t b_fill = B3 ? (b_rd == 0u ? 2u * B_ENTRY : b_rd - B_ENTRY) : (uint32_t)B_ENTRY - b_rd;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       const bool last = ks == KSTEPS - 1;
@@ -475,7 +479,7 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
       for (int g = 0; g < G; ++g) {
         const bool handover = last && g >= G - LA;
         if (NEXT && last && g == G - LA) {
-          wait_vmem<LDA>();  // all but the A loads of the tile after next
+          wait_vmem<B3 ? L3 : LDA>();  // all but the (A) loads of the tile after next
           __syncthreads();
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -484,9 +488,9 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
           acc[g][i] = Traits<T>::mfma16(bq[(ks * G + g) % 4], af[ks & 1][i], acc[g][i]);
           if (i == 0) {
             const int g2 = g + LA;
-            if (g2 < G) fetch_b3((ks * G + g2) % 4, g2, kt, ks);
-            else if (!last) fetch_b3(((ks + 1) * G + g2 - G) % 4, g2 - G, kt, ks + 1);
-            else if (NEXT) fetch_b3((g2 - G) % 4, g2 - G, kt + 1, 0);
+            if (g2 < G) fetch_b3((ks * G + g2) % 4, g2, b_rd, ks);
+            else if (!last) fetch_b3(((ks + 1) * G + g2 - G) % 4, g2 - G, b_rd, ks + 1);
+            else if (NEXT) fetch_b3((g2 - G) % 4, g2 - G, b_nxt, 0);
           }
           if (!last) {
             if (i == 1 && g < TM) fetch_a3((ks + 1) & 1, g, a_rd, ks + 1);
@@ -500,10 +504,10 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
             // B entry being filled: behind this tile's barrier that of tile kt (with tile kt+2),
             // before it that of tile kt-1 (with tile kt+1); A entry: a_fill, tile kt+2, always
             // before the barrier.
-            const int b_parity = handover ? (kt & 1) : ((kt + 1) & 1);
+            const uint32_t b_off = handover ? b_rd : b_fill;
             if (slot % LSL == PH && slot / LSL < L3) l3_issue(slot / LSL);
             const int nz = (slot + 1) / LSL;
-            if ((slot + 1) % LSL == PH && nz < L3 && l3_starts_group(nz)) l3_base(nz, b_parity, a_fill);
+            if ((slot + 1) % LSL == PH && nz < L3 && l3_starts_group(nz)) l3_base(nz, b_off, a_fill);
             if (last && g == 0 && i == TM - 1) l3_advance(1);
             if (last && g == G - LA - 1 && i == TM - 1) l3_advance(0);
           }
@@ -571,37 +575,47 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
     constexpr int L3 = LDA + LDB, LSL3 = TILE_SLOTS / L3, PH3 = LSL3 >= 4 ? 2 : 0;
     constexpr int HEAD_B = (HEAD_SLOTS - PH3 + LSL3 - 1) / LSL3 < LDB ? (HEAD_SLOTS - PH3 + LSL3 - 1) / LSL3 : LDB;
     l3_start();
-    // tile 0 (A entry 0, B entry kt_first & 1), tile 1's A (entry 1) and the B loads of tile 1 that
+    // tile 0, tile 1's A (and B with three B entries), and the B loads of the tile behind those that
     // the handover slots of a tile before would have issued
+    const uint32_t b0 = B3 ? 0u : (uint32_t)(kt_first & 1) * (uint32_t)B_ENTRY;
+    const uint32_t b1 = (uint32_t)B_ENTRY - b0;
 #pragma unroll
     for (int z = LDB; z < L3; ++z) {
-      if (l3_starts_group(z)) l3_base(z, 0, 0u);
+      if (l3_starts_group(z)) l3_base(z, 0u, 0u);
       l3_issue(z);
     }
 #pragma unroll
     for (int z = 0; z < LDB; ++z) {
-      if (l3_starts_group(z)) l3_base(z, kt_first & 1, 0u);
+      if (l3_starts_group(z)) l3_base(z, b0, 0u);
       l3_issue(z);
     }
     l3_advance(0);
     l3_advance(1);
 #pragma unroll
     for (int z = LDB; z < L3; ++z) {
-      if (l3_starts_group(z)) l3_base(z, 0, (uint32_t)A_ENTRY);
+      if (l3_starts_group(z)) l3_base(z, 0u, (uint32_t)A_ENTRY);
       l3_issue(z);
+    }
+    if constexpr (B3) {
+#pragma unroll
+      for (int z = 0; z < LDB; ++z) {
+        if (l3_starts_group(z)) l3_base(z, b1, 0u);
+        l3_issue(z);
+      }
+      l3_advance(1);
     }
 #pragma unroll
     for (int z = 0; z < HEAD_B; ++z) {
-      if (l3_starts_group(z)) l3_base(z, (kt_first + 1) & 1, 0u);
+      if (l3_starts_group(z)) l3_base(z, B3 ? 2u * B_ENTRY : b1, 0u);
       l3_issue(z);
     }
     l3_advance(0);
-    wait_vmem<LDA + HEAD_B>();
+    wait_vmem<(B3 ? L3 : LDA) + HEAD_B>();
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < TM; ++i) fetch_a3(0, i, 0u, 0);
 #pragma unroll
-    for (int g = 0; g < LA; ++g) fetch_b3(g, g, kt_first, 0);
+    for (int g = 0; g < LA; ++g) fetch_b3(g, g, b0, 0);
   } else {
     load_state_start();
 #pragma unroll
@@ -942,7 +956,7 @@ hipError_t launch_gemm_group_pipelined(GemmGroup<typename Epi::Args>& grp, hipSt
   for (int g = 0; g < grp.count; ++g) {
     grp.first[g] = total;
     const int tiles = ((grp.ga[g].M + BM - 1) / BM) * ((grp.ga[g].N + BN - 1) / BN);
-    total += tiles - grp.ga[g].sk_tiles;
+    total += Epi::SPLIT ? tiles * grp.ga[g].splits : tiles - grp.ga[g].sk_tiles;
   }
   for (int g = grp.count; g <= GEMM_GROUP_MAX; ++g) grp.first[g] = total;
   if (total > 0) {  // (stream-K may have taken every tile of a single problem)

@@ -7,13 +7,19 @@ namespace gmlp {
 
 // Tile classes (all four wavefronts per workgroup, 64-wide reduction tiles).
 //   LARGE        256x256 output tiles, wavefronts of 128x128, pipelined kernel
+//   WIDE         128x256 output tiles, wavefronts of 64x128, pipelined kernel (not the weight gradients):
+//                one workgroup per CU, three ring entries of both operands.  Half of LARGE's work per
+//                workgroup at 5/6 of its throughput: for grids that LARGE fills badly and for short
+//                batches, where it reads the weights once per 128 token rows from L2 and needs fewer
+//                splits than MEDIUM_FULL
 //   MEDIUM_FULL  128x128 output tiles, wavefronts of 64x64, pipelined kernel; two workgroups per CU,
 //                for problems with too few 256x256 tiles to fill the chip
 //   MEDIUM       128x128, predicated register-staged kernel, 64-bit addresses: operands too large for
 //                the pipelined kernels' 32-bit byte offsets
 //   F32_*        the float32 kernel's tiles (gemm_f32.hip): 128 x 128, 64 x 128, 64 x 64; with two
 //                accumulator sets 128 x 64 or 64 x 64
-enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2, TILE_F32_128 = 3, TILE_F32_64X128 = 4, TILE_F32_64 = 5 };
+enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2, TILE_F32_128 = 3, TILE_F32_64X128 = 4, TILE_F32_64 = 5,
+                 TILE_WIDE = 6 };
 
 // kinds of GEMM the gated MLP needs; each is instantiated per dtype and tile class, and for reduction
 // lengths that are (KT = false) or are not a multiple of 64, the width of a reduction tile.
@@ -31,11 +37,11 @@ hipError_t launch_dx_kt(int tile_class, const GemmArgs& ga, const typename EpiSt
                         hipStream_t s);  // A KC, B KS, two reduction segments
 // Split-reduction variants (128x128 tiles): partial sums to a fp32 workspace, see splitk_reduce.
 template <typename T, bool KT>
-hipError_t launch_linear_split_kt(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
+hipError_t launch_linear_split_kt(int tile_class, const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
 template <typename T, bool KT>
-hipError_t launch_dx_split_kt(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
+hipError_t launch_dx_split_kt(int tile_class, const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
 template <typename T, bool KT>
-hipError_t launch_gateup_split_kt(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
+hipError_t launch_gateup_split_kt(int tile_class, const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s);
 
 // The predicated class (and float32) has one kernel for every reduction length.
 template <typename T>
@@ -51,9 +57,11 @@ bool reduction_tail(int tile_class, const GemmArgs& ga) {
   }
 #define GMLP_SPLIT_BY_TAIL(KIND)                                                                             \
   template <typename T>                                                                                      \
-  hipError_t launch_##KIND##_split(const GemmArgs& ga, const typename EpiPartial<T>::Args& ea, hipStream_t s) {  \
-    return reduction_tail<T>(TILE_MEDIUM_FULL, ga) ? launch_##KIND##_split_kt<T, true>(ga, ea, s)              \
-                                                   : launch_##KIND##_split_kt<T, false>(ga, ea, s);            \
+  hipError_t launch_##KIND##_split(int tile_class, const GemmArgs& ga, const typename EpiPartial<T>::Args& ea,  \
+                                   hipStream_t s) {                                                          \
+    if constexpr (!std::is_same<T, float>::value)                                                            \
+      if (reduction_tail<T>(tile_class, ga)) return launch_##KIND##_split_kt<T, true>(tile_class, ga, ea, s);  \
+    return launch_##KIND##_split_kt<T, false>(tile_class, ga, ea, s);                                        \
   }
 GMLP_BY_TAIL(gateup, EpiGateUp)
 GMLP_BY_TAIL(linear, EpiStore)
@@ -73,10 +81,13 @@ hipError_t launch_dw(int tile_class, const GemmArgs& ga, const typename EpiStore
 template <typename T>
 hipError_t launch_dw_group(int tile_class, GemmGroup<typename EpiStore<T>::Args>& grp, hipStream_t s);
 
-// The same with a split reduction, float32: every problem's ga.splits partial sums, then their totals.
-hipError_t launch_dw_group_split_f32(GemmGroup<EpiPartial<float>::Args>& grp, hipStream_t s);
-hipError_t launch_splitk_reduce_group(const GemmGroup<EpiPartial<float>::Args>& part,
-                                      const GemmGroup<EpiStore<float>::Args>& out, hipStream_t s);
+// The same with a split reduction (on MEDIUM_FULL or F32_64): every problem's ga.splits partial sums,
+// then their totals.
+template <typename T>
+hipError_t launch_dw_group_split(GemmGroup<typename EpiPartial<T>::Args>& grp, hipStream_t s);
+template <typename T>
+hipError_t launch_splitk_reduce_group(const GemmGroup<typename EpiPartial<T>::Args>& part,
+                                      const GemmGroup<typename EpiStore<T>::Args>& out, hipStream_t s);
 
 // Generic launcher used by the instantiation units.
 template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
