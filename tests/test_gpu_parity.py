@@ -1411,6 +1411,87 @@ def test_inference_forward_under_hip_graph_replay(M, K, N, streams):
             assert torch.equal(y, eager[rep]), f"replay with input {rep} differs from the eager forward"
 
 
+def test_native_autograd_nodes_keep_pytorchs_contracts():
+    """What torch.autograd.Function gives for free, from the native nodes: N-D and non-contiguous inputs,
+    partial gradients, errors on a second backward and on operands changed in place, saved-tensor hooks
+    (non-reentrant checkpointing), steps from several threads at once on streams of their own."""
+    import threading
+
+    from torch.utils.checkpoint import checkpoint
+    from triton_gated_mlp import FusedGatedMLP, FusedGatedMLPFunction
+
+    dev = _dev()
+    torch.manual_seed(6)
+    mlp = FusedGatedMLP(256, 512, bias=True).to(dev).half()
+    base = torch.randn(256, 3, 5, device=dev, dtype=torch.float16)
+    x = base.permute(2, 1, 0).detach().requires_grad_(True)  # [5, 3, 256], not contiguous
+    dy = torch.randn(5, 3, 256, device=dev, dtype=torch.float16)
+    y = mlp(x)
+    assert y.shape == x.shape and not y._is_view()
+    y.backward(dy, retain_graph=True)
+    ref = {n: p.grad.clone() for n, p in mlp.named_parameters()}
+    ref_x = x.grad.clone()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        with torch.no_grad():
+            mlp.up_proj.weight.mul_(1.0)
+        y.backward(dy)
+    y = mlp(x)
+    (gx,) = torch.autograd.grad(y, [x], dy)
+    assert gx.shape == x.shape and torch.equal(gx, ref_x)
+    with pytest.raises(RuntimeError, match="second time"):
+        y.backward(dy)
+    # frozen parameters get nothing, the others the same
+    for n, p in mlp.named_parameters():
+        p.requires_grad_(n.startswith("down"))
+        p.grad = None
+    mlp(x.detach()).backward(dy)
+    for n, p in mlp.named_parameters():
+        assert torch.equal(p.grad, ref[n]) if n.startswith("down") else p.grad is None
+        p.requires_grad_(True)
+        p.grad = None
+    # saved-tensor hooks: the whole node is recomputed, same gradients
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(tuple(t.shape)) or t, lambda t: t):
+        y = mlp(x)
+    assert (3, 15, 512) in packed  # G, U, H
+    y.backward(dy)
+    assert all(torch.equal(p.grad, ref[n]) for n, p in mlp.named_parameters())
+    for lean in (False, True):
+        mlp.recompute_activations = lean
+        mlp.zero_grad()
+        checkpoint(mlp, x, use_reentrant=False).backward(dy)
+        assert all(torch.equal(p.grad, ref[n]) for n, p in mlp.named_parameters())
+    # the hidden-state operator: dY of a sum is an expanded scalar
+    xs = x.detach().reshape(-1, 256).requires_grad_(True)
+    W = [mlp.up_proj.weight.detach().requires_grad_(True), mlp.gate_proj.weight.detach()]
+    FusedGatedMLPFunction.apply(xs, W[0], None, W[1], None).sum().backward()
+    assert xs.grad.shape == xs.shape and W[0].grad.shape == W[0].shape and W[1].grad is None
+    # two threads, a module and a stream each
+    results = {}
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            m = FusedGatedMLP(256, 512, bias=True).to(dev).half()
+            m.load_state_dict(mlp.state_dict())
+            t = x.detach().clone().requires_grad_(True)
+            for _ in range(20):
+                m.zero_grad()
+                t.grad = None
+                m(t).backward(dy)
+            torch.cuda.current_stream().synchronize()
+            results[k] = (t.grad, {n: p.grad for n, p in m.named_parameters()})
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(results) == 2
+    for gx, grads in results.values():
+        assert torch.equal(gx, ref_x) and all(torch.equal(g, ref[n]) for n, g in grads.items())
+
+
 def test_training_step_under_stream_capture_is_refused(monkeypatch):
     """A forward that records an autograd graph while its stream is being captured raises a
     RuntimeError (no kernel is enqueued, nothing is captured); the capture state is simulated on

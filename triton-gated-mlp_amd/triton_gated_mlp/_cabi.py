@@ -1,4 +1,5 @@
-"""ctypes binding of libgmlp.so (C ABI declared in include/gmlp.h).
+"""Bindings of libgmlp.so (C ABI declared in include/gmlp.h): ctypes for the per-operator wrappers, and
+the native autograd nodes of csrc/torch_binding.cpp for the module and the hidden-state operator.
 
 The library is the only implementation of the fused operators: if it cannot be found or loaded the
 import of the operators raises, there is no CPU or PyTorch fallback.
@@ -7,6 +8,8 @@ import of the operators raises, there is no CPU or PyTorch fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from pathlib import Path
 from typing import Optional
@@ -112,6 +115,28 @@ def lib() -> ctypes.CDLL:
             raise RuntimeError(f"libgmlp.so ABI version {got}, expected {ABI_VERSION}")
         _lib = handle
     return _lib
+
+
+_torch_binding = None
+
+
+def torch_binding():
+    """The extension module of csrc/torch_binding.cpp, bound to the loaded library; loaded once."""
+    global _torch_binding
+    if _torch_binding is None:
+        handle = lib()
+        path = Path(__file__).resolve().parent.parent / "lib" / "_gmlp_torch.so"
+        if not path.exists():
+            raise RuntimeError(
+                f"_gmlp_torch.so not found at {path}: build it with `make -C {path.parent.parent}`; the fused "
+                "gated-MLP module has no fallback path"
+            )
+        loader = importlib.machinery.ExtensionFileLoader("_gmlp_torch", str(path))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_gmlp_torch", path, loader=loader))
+        loader.exec_module(module)
+        module.bind([(n, ctypes.cast(getattr(handle, n), ctypes.c_void_p).value) for n in EXPORTED_SYMBOLS])
+        _torch_binding = module
+    return _torch_binding
 
 
 def check(status: int) -> None:

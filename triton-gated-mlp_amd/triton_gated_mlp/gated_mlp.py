@@ -21,7 +21,7 @@ import torch
 from torch import Tensor, nn
 from torch.autograd.function import Function
 
-from .ops import bwd as _bwd
+from . import _cabi
 from .ops import fwd as _fwd
 from .ops.bwd import mlp_hidden_states_bwd
 from .ops.fwd import mlp_hidden_states_fwd
@@ -111,96 +111,42 @@ def eager_bwd(x: Tensor, W_up: Tensor, W_gp: Tensor, grad_output: Tensor):
     return d_up @ W_up + d_gate @ W_gp, d_up.T @ x, d_gate.T @ x
 
 
+_U64 = (1 << 64) - 1
+
+
 class FusedGatedMLPFunction(Function):
     """Hidden-state operator hidden = dropout(act_fn(x·W_gpᵀ+b_gp) * (x·W_upᵀ+b_up)).
 
     Argument order (x, W_up, b_up, W_gp, b_gp) as in the reference; dropout_p, seed, offset and
-    act_fn (default "silu") are optional.
+    act_fn (default "silu") are optional.  `apply` records a native autograd node
+    (csrc/torch_binding.cpp) that keeps G and U.
     """
 
     @staticmethod
-    def forward(
-        ctx, x, W_up, b_up, W_gp, b_gp, dropout_p: float = 0.0, seed: int = 0, offset: int = 0, act_fn: str = "silu"
-    ):
-        needs_grad = any(ctx.needs_input_grad[:5])
-        out = _fwd.gateup_fwd(
-            x, W_gp, b_gp, W_up, b_up, dropout_p, seed, offset, save_activations=needs_grad, act_fn=act_fn
+    def apply(
+        x: Tensor, W_up: Tensor, b_up: Optional[Tensor], W_gp: Tensor, b_gp: Optional[Tensor], dropout_p: float = 0.0,
+        seed: int = 0, offset: int = 0, act_fn: str = "silu",
+    ) -> Tensor:
+        return _cabi.torch_binding().hidden(
+            x, W_up, b_up, W_gp, b_gp, float(dropout_p), int(seed) & _U64, int(offset) & _U64, _cabi.act_code(act_fn)
         )
-        if needs_grad:
-            ctx.save_for_backward(x, W_up, W_gp, out.gate, out.up)
-        ctx.act_fn = act_fn
-        ctx.dropout = (float(dropout_p), int(seed), int(offset))
-        ctx.has_bias = (b_up is not None, b_gp is not None)
-        return out.hidden
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        x, W_up, W_gp, gate, up = ctx.saved_tensors
-        p, seed, offset = ctx.dropout
-        need = ctx.needs_input_grad
-        dg, du = _bwd.gating_bwd(grad_output, gate, up, p, seed, offset, ctx.act_fn)
-        dx = _bwd.dx_bwd(dg, du, W_gp, W_up) if need[0] else None
-        dW_up = _bwd.dw_bwd(du, x) if need[1] else None
-        db_up = _bwd.colsum(du) if ctx.has_bias[0] and need[2] else None
-        dW_gp = _bwd.dw_bwd(dg, x) if need[3] else None
-        db_gp = _bwd.colsum(dg) if ctx.has_bias[1] and need[4] else None
-        grads = (dx, dW_up, db_up, dW_gp, db_gp, None, None, None, None)
-        return grads[: len(need)]  # apply() may have been called with the 5 reference arguments only
-
-
-_CU_COUNT = {}
-
-
-def _compute_units(device: torch.device) -> int:
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    if index not in _CU_COUNT:
-        _CU_COUNT[index] = torch.cuda.get_device_properties(index).multi_processor_count
-    return _CU_COUNT[index]
 
 
 class FusedGatedMLPFullFunction(Function):
-    """Whole MLP as one autograd node, so dY -> (dG, dU) is a single GEMM with a fused epilogue."""
+    """Whole MLP as one autograd node (native, csrc/torch_binding.cpp), so dY -> (dG, dU) is a single
+    GEMM with a fused epilogue.  With `recompute` the node keeps only the inputs (as the reference does,
+    gated_mlp.py:182) and runs the gate/up GEMM again in backward; the dropout mask is a function of
+    the seed."""
 
     @staticmethod
-    def forward(
-        ctx, x, W_gate, b_gate, W_up, b_up, W_down, b_down, dropout_p, seed, offset, recompute=False, act_fn="silu"
-    ):
-        needs_grad = any(ctx.needs_input_grad[:7])
-        keep = needs_grad and not recompute
-        # one library call enqueues the whole pass
-        y, hs = _fwd.mlp_fwd(
-            x, W_gate, b_gate, W_up, b_up, W_down, b_down, dropout_p, seed, offset, save_activations=keep, act_fn=act_fn
+    def apply(
+        x: Tensor, W_gate: Tensor, b_gate: Optional[Tensor], W_up: Tensor, b_up: Optional[Tensor], W_down: Tensor,
+        b_down: Optional[Tensor], dropout_p: float, seed: int, offset: int, recompute: bool = False, act_fn: str = "silu",
+    ) -> Tensor:
+        return _cabi.torch_binding().mlp_train(
+            x, W_gate, b_gate, W_up, b_up, W_down, b_down, float(dropout_p), int(seed) & _U64, int(offset) & _U64,
+            bool(recompute), _cabi.act_code(act_fn),
         )
-        if keep:
-            ctx.save_for_backward(x, W_gate, W_up, W_down, hs.gate, hs.up, hs.hidden)
-        elif needs_grad:
-            # memory-lean mode: keep the inputs only (as the reference does, gated_mlp.py:182) and
-            # run the gate/up GEMM again in backward; the dropout mask is a function of the seed
-            ctx.save_for_backward(x, W_gate, W_up, W_down, b_gate, b_up)
-        ctx.recompute = bool(recompute)
-        ctx.act_fn = act_fn
-        ctx.dropout = (float(dropout_p), int(seed), int(offset))
-        ctx.has_bias = (b_gate is not None, b_up is not None, b_down is not None)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        p, seed, offset = ctx.dropout
-        if ctx.recompute:
-            x, W_gate, W_up, W_down, b_gate, b_up = ctx.saved_tensors
-            hs = _fwd.gateup_fwd(
-                x, W_gate, b_gate, W_up, b_up, p, seed, offset, save_activations=True, act_fn=ctx.act_fn
-            )
-            gate, up, hidden = hs.gate, hs.up, hs.hidden
-        else:
-            x, W_gate, W_up, W_down, gate, up, hidden = ctx.saved_tensors
-        need = ctx.needs_input_grad
-        has = ctx.has_bias
-        want = (need[0], need[1], has[0] and need[2], need[3], has[1] and need[4], need[5], has[2] and need[6])
-        # one library call enqueues the whole pass: dH with the gating epilogue, dX, the three
-        # weight gradients as one grid, the bias gradients as one pair of launches
-        grads = _bwd.mlp_bwd(dy, x, W_gate, W_up, W_down, gate, up, hidden, want, p, seed, offset, ctx.act_fn)
-        return grads + (None, None, None, None, None)
 
 
 class FusedGatedMLP(_GatedMLPBase):
@@ -211,7 +157,7 @@ class FusedGatedMLP(_GatedMLPBase):
     set `dropout_seed` (int) for a fixed mask stream, otherwise each forward draws a seed from
     torch's default CPU generator (so `torch.manual_seed` makes runs repeatable).  The seed and
     offset of the last training forward are kept in `last_dropout_state`; a batch that ran as
-    several row chunks (see `_forward_2d`) drew one mask per chunk, and `last_dropout_states` lists
+    several row chunks (see `_forward_rows`) drew one mask per chunk, and `last_dropout_states` lists
     them all as (first row, rows, seed, offset), the mask of a chunk being that of a [rows, N] tensor.
 
     Under `torch.autocast("cuda")` the module casts its input and parameters to the autocast dtype
@@ -239,52 +185,45 @@ class FusedGatedMLP(_GatedMLPBase):
         return seed, offset
 
     def forward(self, x: Tensor) -> Tensor:
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
         p = float(self.dropout.p) if self.training else 0.0
-        gate, up, down = self.gate_proj, self.up_proj, self.down_proj
         self.last_dropout_states = []
-        if x2.is_cuda and torch.is_autocast_enabled("cuda"):
+        params = []
+        for layer in (self.gate_proj, self.up_proj, self.down_proj):
+            # (the usual parameters without a trip through nn.Module.__getattr__)
+            own = layer._parameters
+            params.append(own["weight"] if "weight" in own else layer.weight)
+            params.append(own["bias"] if "bias" in own else layer.bias)
+        if x.is_cuda and torch.is_autocast_enabled("cuda"):
             # Mixed precision as nn.Linear does it under torch.autocast: activations and (master)
             # weights are cast to the autocast dtype for the kernels; autograd casts the gradients back.
             with torch.autocast("cuda", enabled=False):
-                return self._forward_cast(x2, torch.get_autocast_dtype("cuda"), p).reshape(*lead, self.hidden_size)
-        return self._forward_2d(
-            x2, gate.weight, gate.bias, up.weight, up.bias, down.weight, down.bias, p
-        ).reshape(*lead, self.hidden_size)
+                dtype = torch.get_autocast_dtype("cuda")
+                return self._forward_rows(x.to(dtype), [t if t is None else t.to(dtype) for t in params], p)
+        return self._forward_rows(x, params, p)
 
-    def _forward_cast(self, x2: Tensor, dtype: torch.dtype, p: float) -> Tensor:
-        cast = lambda t: None if t is None else t.to(dtype)
-        g, u, d = self.gate_proj, self.up_proj, self.down_proj
-        return self._forward_2d(
-            cast(x2), cast(g.weight), cast(g.bias), cast(u.weight), cast(u.bias), cast(d.weight), cast(d.bias), p
-        )
-
-    def _forward_2d(self, x2, W_gate, b_gate, W_up, b_up, W_down, b_down, p: float, row0: int = 0) -> Tensor:
-        M, K = x2.shape
-        limit = _fwd.max_rows_32bit(K, self.intermediate_size, x2.dtype) if x2.is_cuda else None
+    def _forward_rows(self, x: Tensor, params, p: float, row0: int = 0) -> Tensor:
+        """x: [..., K]; params: weight and bias of gate, up and down."""
+        K = x.shape[-1]
+        M = x.numel() // K if K else 0
+        limit = _fwd.max_rows_32bit(K, self.intermediate_size, x.dtype) if x.is_cuda else None
         if limit is not None and M > limit:
             # Token rows are independent: a batch too tall for the pipelined kernels' 32-bit operand
             # offsets runs as near-equal row chunks (autograd sums the chunks' weight gradients; with
             # dropout every chunk draws its own mask, recorded in `last_dropout_states`).
             chunks = -(-M // limit)
             rows = -(-M // (chunks * 256)) * 256
+            x2 = x.reshape(-1, K)
             return torch.cat(
-                [
-                    self._forward_2d(x2[i : i + rows], W_gate, b_gate, W_up, b_up, W_down, b_down, p, row0 + i)
-                    for i in range(0, M, rows)
-                ]
+                [self._forward_rows(x2[i : i + rows], params, p, row0 + i) for i in range(0, M, rows)]
+            ).reshape(x.shape)
+        W_gate, b_gate, W_up, b_up, W_down, b_down = params
+        graph = torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in params))
+        if not graph and p == 0.0:
+            # Nothing to differentiate: the weight-streaming kernels for skinny M, no autograd node.
+            return _cabi.torch_binding().mlp_infer(
+                x, W_gate, b_gate, W_up, b_up, W_down, b_down, _cabi.act_code(self.act_fn)
             )
-        inference = not torch.is_grad_enabled() or not any(
-            t is not None and t.requires_grad for t in (x2, W_gate, b_gate, W_up, b_up, W_down, b_down)
-        )
-        if inference and p == 0.0 and x2.is_cuda:
-            # Nothing to differentiate: no autograd node (its bookkeeping costs more host time than a
-            # short batch's kernels take to enqueue), and the weight-streaming kernels for skinny M.
-            if _fwd.decode_preferred(M, K, self.intermediate_size, x2.dtype, _compute_units(x2.device)):
-                return _fwd.decode_fwd(x2, W_gate, b_gate, W_up, b_up, W_down, b_down, self.act_fn)
-            return _fwd.mlp_fwd(x2, W_gate, b_gate, W_up, b_up, W_down, b_down, act_fn=self.act_fn)[0]
-        if x2.is_cuda and torch.cuda.is_current_stream_capturing():
+        if x.is_cuda and torch.cuda.is_current_stream_capturing():
             # Capturing forward + backward with torch.cuda.graph has ended in a host-side crash inside
             # the runtime's end-of-capture call on ROCm 7.2; until its cause is known the module
             # refuses rather than take the process down.  Inference forwards capture fine.
@@ -296,5 +235,5 @@ class FusedGatedMLP(_GatedMLPBase):
         if p > 0.0:
             self.last_dropout_states.append((row0, M, seed, offset))
         return FusedGatedMLPFullFunction.apply(
-            x2, W_gate, b_gate, W_up, b_up, W_down, b_down, p, seed, offset, self.recompute_activations, self.act_fn
+            x, W_gate, b_gate, W_up, b_up, W_down, b_down, p, seed, offset, self.recompute_activations, self.act_fn
         )

@@ -221,9 +221,7 @@ def decode_preferred(M: int, K: int, N: int, dtype: torch.dtype = torch.float16,
     up; below that they tie or lose (2560 x 10240: -12 %), so the module asks for 14 rows of W_down
     per compute unit there.
     """
-    if M > DECODE_PREFERRED_MAX_M or not decode_supported(M, K, N, dtype) or K % 256 != 0 or N < 16 * num_cu:
-        return False
-    return K >= (8 if M <= 16 else 14) * num_cu
+    return decode_supported(M, K, N, dtype) and _cabi.torch_binding().decode_preferred(M, K, N, _cabi.dtype_code(dtype), num_cu)
 
 
 def decode_fwd(
