@@ -1158,6 +1158,37 @@ def test_wide_tiles_and_split_gradients_against_fp32_products(M, K, N):
     assert all(torch.equal(a, b) for a, b in zip(got, run()))
 
 
+def test_second_stages_against_float64():
+    """Sums of 2 to 16 partial results (every remainder of the groups that are in flight together) and
+    column sums at the edges of their row ranges and of a workgroup's 256 columns.  fp16 results of
+    float32 sums: half an ulp, 2^-11, beside the sums' own rounding."""
+    from triton_gated_mlp import _cabi
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(12)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).half().to(dev)
+    seen = set()
+    for red in range(512, 4608, 256):
+        M, C = 40, 520
+        a, w = rnd(M, red), rnd(C, red) * 0.03
+        nbytes = _cabi.lib().gmlp_workspace_bytes(_cabi.GMLP_OP_LINEAR_FWD, M, red, C, _cabi.dtype_code(a.dtype))
+        seen.add(nbytes // (4 * M * C))
+        ref = a.double() @ w.double().T
+        err = ((ops_fwd.linear_fwd(a, w).double() - ref).norm() / ref.norm()).item()
+        print(f"reduction {red}: {nbytes // (4 * M * C)} splits, rel {err:.2e}", flush=True)
+        assert err < 2.0**-11
+    assert len(seen) >= 4 and max(seen) >= 9, seen
+    for M, C in ((1, 8), (63, 264), (64, 256), (65, 248), (513, 1032), (1357, 3096)):
+        a = rnd(M, C)
+        ref = a.double().sum(0)
+        for out in ops_bwd.colsum_grouped([a, a, a]):
+            rel = ((out.double() - ref).norm() / ref.norm()).item()
+            print(f"column sums {M} x {C}: rel {rel:.2e}", flush=True)
+            assert rel < 2.0**-11
+
+
 @pytest.mark.parametrize(
     "M,K,N",
     [

@@ -40,39 +40,62 @@ template hipError_t launch_gating_bwd<float>(const float*, const float*, const f
 
 // Second stage of a split reduction: adds the partial results up in split order (deterministic)
 // and hands 8 consecutive columns of one row to the epilogue the unsplit GEMM would have run.
-template <typename T, typename Epi>
+// Outputs of short batches are a few thousand lanes' work, so the chain of a lane's loads decides: the
+// partial sums of 8 splits (4 with two accumulator sets) are in flight together, and small outputs go
+// out as workgroups of one wavefront, which spread over more CUs.  M=40, K=4096, N=14336: down
+// projection, 14 splits, 6.2 us -> 4.7; M=66,
+// K=3208, N=9568: down 6.3 -> 4.2, dX 6.6 -> 4.7.  (All 256 threads wide, the short ones stay at 5; one
+// wavefront wide, outputs of 65536 lanes or more gain nothing and large ones lose 1 us of 8.)
+template <typename T, typename Epi, int SETS>
 __global__ void __launch_bounds__(256)
     splitk_reduce_kernel(const float* __restrict__ ws, int splits, size_t split_stride, size_t acc_stride,
                          typename Epi::Args ea, size_t n8, int N) {
   size_t step = (size_t)gridDim.x * blockDim.x;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += step) {
     size_t e = i * 8;
-    alignas(16) float v0[8], v1[8];
+    alignas(16) float v[2][8];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) v0[r] = v1[r] = 0.f;
-    for (int s = 0; s < splits; ++s) {
-      const float* p = ws + (size_t)s * split_stride + e;
-      f32x4 a = *(const f32x4*)p, b = *(const f32x4*)(p + 4);
+    for (int r = 0; r < 8; ++r) v[0][r] = v[1][r] = 0.f;
+    int s = 0;
+    auto add = [&](auto count) __attribute__((always_inline)) {
+      constexpr int U = decltype(count)::value;
+      f32x4 t[U][SETS][2];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) { v0[r] += a[r]; v0[4 + r] += b[r]; }
-      if (acc_stride) {
-        f32x4 c = *(const f32x4*)(p + acc_stride), d = *(const f32x4*)(p + acc_stride + 4);
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) { v1[r] += c[r]; v1[4 + r] += d[r]; }
-      }
-    }
-    Epi::template apply<8>(ea, (int)(e / (size_t)N), (int)(e % (size_t)N), v0, v1);
+        for (int b = 0; b < SETS; ++b) {
+          const float* p = ws + (size_t)(s + u) * split_stride + (b ? acc_stride : 0) + e;
+          t[u][b][0] = *(const f32x4*)p;
+          t[u][b][1] = *(const f32x4*)(p + 4);
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int b = 0; b < SETS; ++b)
+#pragma unroll
+          for (int r = 0; r < 8; ++r) v[b][r] += t[u][b][r / 4][r % 4];
+      s += U;
+    };
+    if constexpr (SETS == 1)
+      while (s + 8 <= splits) add(std::integral_constant<int, 8>{});
+    while (s + 4 <= splits) add(std::integral_constant<int, 4>{});
+    if (s + 2 <= splits) add(std::integral_constant<int, 2>{});
+    if (s < splits) add(std::integral_constant<int, 1>{});
+    Epi::template apply<8>(ea, (int)(e / (size_t)N), (int)(e % (size_t)N), v[0], v[1]);
   }
 }
 
 template <typename T, typename Epi>
 hipError_t launch_splitk_reduce(const float* ws, int splits, size_t split_stride, size_t acc_stride,
                                 const typename Epi::Args& ea, int64_t M, int64_t N, hipStream_t s) {
+  constexpr int SETS = std::is_same<Epi, EpiGateUp<T>>::value ? 2 : 1;
+  if ((acc_stride != 0) != (SETS == 2)) return hipErrorInvalidValue;
   size_t n8 = (size_t)M * N / 8;
   if (n8 == 0) return hipSuccess;
-  size_t blocks = (n8 + 255) / 256;
+  const unsigned threads = n8 < 256 * 256 ? 64 : 256;
+  size_t blocks = (n8 + threads - 1) / threads;
   if (blocks > 256 * 8) blocks = 256 * 8;
-  hipLaunchKernelGGL((splitk_reduce_kernel<T, Epi>), dim3((unsigned)blocks), dim3(256), 0, s, ws, splits,
+  hipLaunchKernelGGL((splitk_reduce_kernel<T, Epi, SETS>), dim3((unsigned)blocks), dim3(threads), 0, s, ws, splits,
                      split_stride, acc_stride, ea, n8, (int)N);
   return hipGetLastError();
 }
@@ -176,14 +199,30 @@ __global__ void __launch_bounds__(256) colsum_partial_kernel(ColsumGroup<T> g, i
   *(f32x4*)(p + 4) = f32x4{s[4], s[5], s[6], s[7]};
 }
 
+// Each of a workgroup's four wavefronts adds up 16 of the 64 partial sums, all loads in flight
+// together, for the same 64 x 4 columns; the first one adds the four totals.  (One lane walking all 64
+// took 7.6 us at three arrays of 5632, 5632 and 2048 columns, this takes 4.8.)
 template <typename T>
 __global__ void __launch_bounds__(256) colsum_final_kernel(ColsumGroup<T> g) {
+  constexpr int WAVES = 4, PER = COLSUM_SPLITS / WAVES;
+  __shared__ f32x4 part[WAVES - 1][64];
   const float* __restrict__ ws = g.ws[blockIdx.z];
   const int64_t C = g.C[blockIdx.z];
-  int64_t c = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (c >= C) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t c = ((int64_t)blockIdx.x * 64 + lane) * 4;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < COLSUM_SPLITS; ++i) s += *(const f32x4*)(ws + (int64_t)i * C + c);
+  if (c < C) {
+    f32x4 t[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) t[i] = *(const f32x4*)(ws + (int64_t)(wave * PER + i) * C + c);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) s += t[i];
+  }
+  if (wave > 0) part[wave - 1][lane] = s;
+  __syncthreads();
+  if (wave > 0 || c >= C) return;
+#pragma unroll
+  for (int w = 0; w < WAVES - 1; ++w) s += part[w][lane];
   float t[4] = {s[0], s[1], s[2], s[3]};
   store_w<T, 4>(g.out[blockIdx.z] + c, t);
 }
@@ -194,7 +233,7 @@ template <typename T>
 hipError_t launch_colsum_group(const ColsumGroup<T>& g, int count, int64_t M, hipStream_t s) {
   int64_t cmax = 0;
   for (int i = 0; i < count; ++i) cmax = g.C[i] > cmax ? g.C[i] : cmax;
-  unsigned bx8 = (unsigned)((cmax / 8 + 255) / 256), bx4 = (unsigned)((cmax / 4 + 255) / 256);
+  unsigned bx8 = (unsigned)((cmax / 8 + 255) / 256), bx4 = (unsigned)((cmax / 4 + 63) / 64);
   hipLaunchKernelGGL(colsum_partial_kernel<T>, dim3(bx8, COLSUM_SPLITS, count), dim3(256), 0, s, g, M);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
