@@ -239,6 +239,14 @@ int gmlp_decode_fwd(const void* x, const void* w_gate, const void* w_up, const v
                     void* stream);
 
 /*
+ * The same on the LDS-ring streaming kernels alone, for any K and N that are multiples of 8, at least 768
+ * and K*N < 2^30 (M <= 32); anything else is refused.  h_scratch as above.
+ */
+int gmlp_decode_stream_fwd(const void* x, const void* w_gate, const void* w_up, const void* w_down,
+                           const void* b_gate, const void* b_up, const void* b_down, void* h_scratch,
+                           void* y, int64_t M, int64_t K, int64_t N, int dtype, int act, void* stream);
+
+/*
  * A whole pass of the MLP in one call: validates once and enqueues every launch of the pass, so a
  * host that drives the MLP from an interpreter pays for one foreign call per pass instead of one
  * per GEMM (a step of a small MLP is otherwise bound by the time it takes to enqueue it).

@@ -1373,6 +1373,64 @@ def test_decode_matches_general_path(dtype):
         _close(f"general Y M={M}", y_general, ref["Y"])
 
 
+@pytest.mark.parametrize(
+    "M,K,N",
+    [
+        (1, 776, 1032),      # least widths, one 16-byte piece in the last chunk of 256 and of 128
+        (3, 2200, 4608),     # tail in one operand only
+        (16, 4096, 4104),    # the other one; full tile of tokens
+        (11, 4496, 9472),    # H in fragment order; more than 16 rows of W_down per compute unit
+        (17, 1016, 888),     # two token tiles, last chunks short by one piece
+        (24, 4104, 1160),    # 32-row blocks of everything
+        (20, 2056, 8200),
+        (7, 5192, 1160),     # misaligned rows, 32-row blocks of W_down, one token tile
+        (29, 5192, 1160),    # and two
+        (32, 12568, 1032),   # 64-row blocks of W_down
+        (18, 12544, 1280),   # the same without tails
+    ],
+)
+def test_decode_streaming_kernels_at_any_width(M, K, N):
+    """Streaming kernels whose last chunk of a row is partly beyond it, where the next row begins with
+    large values, against float64 products; twice, bit-identical."""
+    from triton_gated_mlp import _cabi
+
+    dev = _dev()
+    print(f"decode, any width: M={M} K={K} N={N}", flush=True)
+    g = torch.Generator().manual_seed(21)
+    rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g)).half().to(dev)
+    x, wg, wu, wd = rnd(M, K, s=0.5), rnd(N, K, s=0.02), rnd(N, K, s=0.02), rnd(K, N, s=0.02)
+    bg, bu, bd = rnd(N, s=0.1), rnd(N, s=0.1), rnd(K, s=0.1)
+    x[:, :8] *= 16
+    for w in (wg, wu, wd):
+        w[:, :8] *= 16
+
+    def run():
+        h = torch.full((16 if M <= 16 else 32, N), float("nan"), dtype=x.dtype, device=dev)
+        y = torch.full((M, K), float("nan"), dtype=x.dtype, device=dev)
+        _cabi.check(_cabi.lib().gmlp_decode_stream_fwd(
+            *(t.data_ptr() for t in (x, wg, wu, wd, bg, bu, bd, h, y)), M, K, N, _cabi.dtype_code(x.dtype),
+            _cabi.act_code("silu"), _cabi.stream_ptr(dev)))
+        return y
+
+    y = run()
+    d = lambda t: t.double()
+    hidden = torch.nn.functional.silu(d(x) @ d(wg).T + d(bg)) * (d(x) @ d(wu).T + d(bu))
+    ref = hidden.half().double() @ d(wd).T + d(bd)
+    _close("Y", y, ref)
+    assert torch.equal(y, run())
+
+
+def test_decode_streaming_entry_refuses_what_its_kernels_do_not_take():
+    from triton_gated_mlp import _cabi
+
+    a = torch.zeros(4096, dtype=torch.float16, device=_dev())
+    call = lambda M, K, N, code=0: _cabi.lib().gmlp_decode_stream_fwd(
+        *[a.data_ptr()] * 4, None, None, None, a.data_ptr(), a.data_ptr(), M, K, N, code, 0, None)
+    for M, K, N in ((33, 1024, 1024), (0, 1024, 1024), (1, 760, 1024), (1, 1024, 760), (1, 1028, 1024), (1, 1024, 1028), (1, 32768, 32768)):
+        assert call(M, K, N) == -2, (M, K, N)
+    assert call(1, 1024, 1024, 2) == -2  # float32
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_decode_with_two_token_tiles(dtype):
     """16 < M <= 32 on the streaming kernels (two MFMAs per weight fragment, H for 32 token slots):

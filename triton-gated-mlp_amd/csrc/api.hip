@@ -885,39 +885,65 @@ int gmlp_colsum_grouped(int count, const void* const* a, void* const* out, void*
   return hip_result(__func__, e);
 }
 
+}  // extern "C"
+
+namespace {
+int run_decode(const char* fn, const void* x, const void* w_gate, const void* w_up, const void* w_down, const void* b_gate,
+               const void* b_up, const void* b_down, void* h_scratch, void* y, int64_t M, int64_t K, int64_t N, int dtype, int act,
+               void* stream) {
+  using namespace gmlp;
+  hipStream_t s = (hipStream_t)stream;
+  const hipError_t e = by_dtype(dtype, [&](auto tag) -> hipError_t {
+    typedef decltype(tag) T;
+    if constexpr (std::is_same<T, float>::value) return hipErrorInvalidValue;  // the callers refuse it
+    else
+      return launch_decode<T>((const T*)x, (const T*)w_gate, (const T*)w_up, (const T*)w_down, (const T*)b_gate, (const T*)b_up,
+                              (const T*)b_down, (T*)h_scratch, (T*)y, (int)M, (int)K, (int)N, act, s);
+  });
+  return hip_result(fn, e);
+}
+}  // namespace
+
+extern "C" {
+
+#define GMLP_DECODE_CHECKS()                                                                                           \
+  GMLP_REQUIRE_PTR(x); GMLP_REQUIRE_PTR(w_gate); GMLP_REQUIRE_PTR(w_up); GMLP_REQUIRE_PTR(w_down);                     \
+  GMLP_REQUIRE_PTR(h_scratch); GMLP_REQUIRE_PTR(y);                                                                    \
+  GMLP_REQUIRE_DTYPE(dtype);                                                                                           \
+  GMLP_REQUIRE_ACT(act);                                                                                               \
+  if (int rc = check_dims(__func__, M, K, N)) return rc;                                                               \
+  if (dtype == GMLP_F32) return fail(GMLP_ESHAPE, "%s: float32 is not supported by the skinny-M kernels", __func__)
+#define GMLP_DECODE_ALIGNED()                                                                                          \
+  GMLP_REQUIRE_ALIGNED(x); GMLP_REQUIRE_ALIGNED(w_gate); GMLP_REQUIRE_ALIGNED(w_up);                                   \
+  GMLP_REQUIRE_ALIGNED(w_down); GMLP_REQUIRE_ALIGNED(b_gate); GMLP_REQUIRE_ALIGNED(b_up);                              \
+  GMLP_REQUIRE_ALIGNED(b_down); GMLP_REQUIRE_ALIGNED(h_scratch); GMLP_REQUIRE_ALIGNED(y)
+
 int gmlp_decode_fwd(const void* x, const void* w_gate, const void* w_up, const void* w_down,
                     const void* b_gate, const void* b_up, const void* b_down, void* h_scratch,
                     void* y, void* workspace, int64_t M, int64_t K, int64_t N, int dtype, int act,
                     void* stream) {
-  using namespace gmlp;
   (void)workspace;
-  GMLP_REQUIRE_PTR(x); GMLP_REQUIRE_PTR(w_gate); GMLP_REQUIRE_PTR(w_up); GMLP_REQUIRE_PTR(w_down);
-  GMLP_REQUIRE_PTR(h_scratch); GMLP_REQUIRE_PTR(y);
-  GMLP_REQUIRE_DTYPE(dtype);
-  GMLP_REQUIRE_ACT(act);
-  if (int rc = check_dims(__func__, M, K, N)) return rc;
-  if (dtype == GMLP_F32) return fail(GMLP_ESHAPE, "%s: float32 is not supported by the skinny-M kernels", __func__);
-  if (M > 32 || (M > 16 && !decode_stream_supported((int)M, (int)K, (int)N)))
+  GMLP_DECODE_CHECKS();
+  if (M > 32 || (M > 16 && (K % 256 != 0 || !gmlp::decode_stream_supported((int)M, (int)K, (int)N))))
     return fail(GMLP_ESHAPE,
                 "%s: M = %lld exceeds the skinny-M limit (32 when K and N are multiples of 256, at least 768, "
                 "and K*N < 2^30; 16 otherwise)",
                 __func__, (long long)M);
   if (K % 32 != 0) return fail(GMLP_ESHAPE, "%s: K = %lld must be a multiple of 32", __func__, (long long)K);
   if (N % 256 != 0) return fail(GMLP_ESHAPE, "%s: N = %lld must be a multiple of 256", __func__, (long long)N);
-  GMLP_REQUIRE_ALIGNED(x); GMLP_REQUIRE_ALIGNED(w_gate); GMLP_REQUIRE_ALIGNED(w_up);
-  GMLP_REQUIRE_ALIGNED(w_down); GMLP_REQUIRE_ALIGNED(b_gate); GMLP_REQUIRE_ALIGNED(b_up);
-  GMLP_REQUIRE_ALIGNED(b_down); GMLP_REQUIRE_ALIGNED(h_scratch); GMLP_REQUIRE_ALIGNED(y);
-  hipStream_t s = (hipStream_t)stream;
-  hipError_t e =
-      dtype == GMLP_F16
-          ? launch_decode<f16>((const f16*)x, (const f16*)w_gate, (const f16*)w_up, (const f16*)w_down,
-                               (const f16*)b_gate, (const f16*)b_up, (const f16*)b_down,
-                               (f16*)h_scratch, (f16*)y, (int)M, (int)K, (int)N, act, s)
-          : launch_decode<bf16>((const bf16*)x, (const bf16*)w_gate, (const bf16*)w_up,
-                                (const bf16*)w_down, (const bf16*)b_gate, (const bf16*)b_up,
-                                (const bf16*)b_down, (bf16*)h_scratch, (bf16*)y, (int)M, (int)K,
-                                (int)N, act, s);
-  return hip_result(__func__, e);
+  GMLP_DECODE_ALIGNED();
+  return run_decode(__func__, x, w_gate, w_up, w_down, b_gate, b_up, b_down, h_scratch, y, M, K, N, dtype, act, stream);
+}
+
+int gmlp_decode_stream_fwd(const void* x, const void* w_gate, const void* w_up, const void* w_down,
+                           const void* b_gate, const void* b_up, const void* b_down, void* h_scratch,
+                           void* y, int64_t M, int64_t K, int64_t N, int dtype, int act, void* stream) {
+  GMLP_DECODE_CHECKS();
+  if (M > 32 || !gmlp::decode_stream_supported((int)M, (int)K, (int)N))
+    return fail(GMLP_ESHAPE, "%s: needs M <= 32, K and N multiples of 8 and at least 768, K*N < 2^30 (got %lld, %lld, %lld)", __func__,
+                (long long)M, (long long)K, (long long)N);
+  GMLP_DECODE_ALIGNED();
+  return run_decode(__func__, x, w_gate, w_up, w_down, b_gate, b_up, b_down, h_scratch, y, M, K, N, dtype, act, stream);
 }
 
 int gmlp_dropout_mask(uint8_t* mask, int64_t M, int64_t N, float dropout_p, uint64_t seed,

@@ -2,20 +2,23 @@
 // 512-byte (or 256-byte) row segments moved global -> LDS without passing through registers.
 //
 // One persistent workgroup of three wavefronts per CU.  The workgroup takes blocks of weight rows
-// that share one set of token operands: rows r..r+15 of W_gate and of W_up (GATED), or 32
-// consecutive rows of W_down (16 when a CU's share is no more than that); twice as many rows with
-// 256-byte segments.  Whole blocks go round-robin over the workgroups, the rows that do not fill a
-// last round are shared out evenly as one partly empty block each.  Its wavefronts split the
-// reduction range in near-equal runs of chunks (256 or 128 elements) and combine their partial
+// that share one set of token operands: 16 or 32 rows of W_gate and as many of W_up (GATED), or 16,
+// 32 or 64 consecutive rows of W_down.  Whole blocks go round-robin over the workgroups, the rows that
+// do not fill a last round are shared out evenly as one partly empty block each.  Its wavefronts split
+// the reduction range in near-equal runs of chunks (256 or 128 elements) and combine their partial
 // sums through LDS at the end of each block (fixed order, so the result is deterministic).  Each
 // wavefront runs a private ring of 3 or 4 LDS slots; a slot holds one stage = one chunk of the
-// block's weight rows, 8 KiB per matrix.  The matching token-row operands (x or H, L2-resident)
+// block's weight rows.  The matching token-row operands (x or H, L2-resident)
 // are fetched straight into registers, as many stages ahead: one 16-token tile for M <= 16, two
-// beyond (MT; the weight fragment read from LDS then feeds two MFMAs).  Achieved HBM bandwidth
-// follows the bytes in flight per CU, and LDS capacity bounds those: wavefronts x 3 slots x 16 KiB
-// fill 144 of the 160 KiB.  The stream of stages runs on across block boundaries, so the ring
-// never drains; loads past the end re-fetch the last stage into a free slot, which keeps the
-// in-flight count constant.
+// beyond (MT; the weight fragment read from LDS then feeds two MFMAs).  The stream of stages runs on
+// across block boundaries, so the ring never drains; loads past the end re-fetch the last stage into a
+// free slot, which keeps the in-flight count constant.
+//
+// Which block (chosen in launch_decode_stream; whole forward, us, fp16): the height decides what a
+// block costs in token operands and how well it fits a CU's share of the rows, the row segment of a
+// stage (SEGB) what is left of a chunk's imbalance between the wavefronts.  Bytes in flight no longer
+// decide at 96 KiB per CU: four, six and eight wavefronts with 128 to 144 KiB were no faster on any of
+// eleven widths.
 //
 //   GATED:   H[m, r] = act(x.W_gate[r] + b_gate[r]) * (x.W_up[r] + b_up[r])      (r over N)
 //   !GATED:  Y[m, r] = H.W_down[r] + b_down[r]                                   (r over K)
@@ -49,23 +52,11 @@ struct Mfma16x<bf16> {
   }
 };
 
-constexpr int DS_CH = 256;            // reduction elements per stage
-constexpr int DS_REGION = 16 * 512;   // bytes of one 16-row region
-// ring slots per wavefront (and stages in flight): 3 slots of two matrices, or 4 of one (3 where
-// two token tiles go with 512-byte segments: the token operands in flight are bounded by the
-// registers, see the kernel)
-constexpr int ds_ring_depth(int nmat, int mt, int segb) { return nmat == 2 || (mt == 2 && segb == 512) ? 3 : 4; }
-constexpr int DS_WAVES = 3;           // wavefronts per workgroup
-// buffers for the partial sums that change hands at the end of a block: two (alternating) where
-// LDS holds them beside the rings, else one
-constexpr int ds_part_buffers(int nmat, int mt, int segb) {
-  return DS_WAVES * ds_ring_depth(nmat, mt, segb) * nmat * DS_REGION + 2 * (DS_WAVES - 1) * nmat * (512 / segb) * mt * 1024 <=
-                 160 * 1024
-             ? 2
-             : 1;
-}
+constexpr int DS_MAX_LDS = 160 * 1024;
+constexpr int DS_WAVES = 3;                   // wavefronts per workgroup
+constexpr int DS_MIN_RED = 768;               // a chunk for every wavefront
 constexpr uint32_t DS_NOWHERE = 0x80000000u;  // voffset beyond any operand (operands are < 2 GiB)
-constexpr int DS_WIDE_SEGMENT_MAX_M = 20;     // two token tiles: 512-byte row segments up to here, 256 beyond
+constexpr int DS_WIDE_SEGMENT_MAX_M = 20;     // see ds_tall_gated
 constexpr int DS_H_TILED_MIN_M = 10;           // H goes out in fragment order above this many token rows
 
 struct StreamArgs {
@@ -95,36 +86,24 @@ __device__ __forceinline__ i32x4 load16_async(buffer_rsrc r, uint32_t voffset, u
 // to the same point.
 template <int N, int NX>
 __device__ __forceinline__ void wait_vmem_keep(i32x4 (&x)[NX]) {
-  static_assert(NX == 8 || NX == 16, "one or two token tiles");
-  asm volatile("s_waitcnt vmcnt(%8)"
-               : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]),
-                 "+v"(x[7])
-               : "n"(N)
-               : "memory");
-  if constexpr (NX == 16)
-    asm volatile(""
-                 : "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]),
-                   "+v"(x[14]), "+v"(x[15])
-                 :
-                 : "memory");
+  static_assert(NX % 4 == 0, "groups of four");
+  asm volatile("s_waitcnt vmcnt(%4)" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]) : "n"(N) : "memory");
+#pragma unroll
+  for (int i = 4; i < NX; i += 4) asm volatile("" : "+v"(x[i]), "+v"(x[i + 1]), "+v"(x[i + 2]), "+v"(x[i + 3]) : : "memory");
 }
 
-// NMAT: weight matrices / runs of rows per stage (GATED: W_gate and W_up; otherwise 1 or 2 runs of
-//       W_down rows).
+// HALVES: 16-row regions per matrix and stage.
 // MT:   tiles of 16 token slots (M <= 16 * MT).
-// SEGB: bytes of a weight row per stage, 512 or 256.  A stage always moves 8 KiB per matrix: 16
-//       rows x 512 bytes, or 32 rows x 256 bytes as two 16-row regions.  The second form halves
-//       the token operands fetched per weight byte (a stage spans half the reduction elements for
-//       twice the rows), which is what two token tiles need: with 16-row blocks their token
-//       operands cost as much L2 traffic as the weights cost HBM traffic.
-template <typename T, bool GATED, int NMAT, int MT, int SEGB>
+// SEGB: bytes of a weight row per stage, 512 or 256.
+// DS_RD: ring slots per wavefront and stages in flight.
+// TAIL: the reduction length need not be a multiple of the chunk (only of 8): the 16-byte pieces of the
+//       last chunk that lie beyond the row's end are pushed out of the descriptors, weights and token
+//       operands, and read as zeros.  An instance of its own: the others have no such selects.
+template <typename T, bool GATED, int HALVES, int MT, int SEGB, int DS_RD, bool TAIL>
 __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs a) {
   typedef typename Traits<T>::vec8 vec8;
-  static_assert(NMAT == 2 || (NMAT == 1 && !GATED), "gated blocks stream two matrices");
   static_assert(SEGB == 512 || SEGB == 256, "row segment of a stage");
-  constexpr int DS_RD = ds_ring_depth(NMAT, MT, SEGB);
-  constexpr int HALVES = 512 / SEGB;          // 16-row regions per matrix and stage
-  constexpr int NREG = NMAT * HALVES;         // 16-row regions per stage
+  constexpr int NREG = (GATED ? 2 : 1) * HALVES;  // 16-row regions per stage
   constexpr int REGION = 16 * SEGB;           // bytes of a region
   constexpr int CH = SEGB / 2;                // reduction elements per stage
   constexpr int KS = CH / 32;                 // MFMA steps per stage
@@ -135,7 +114,7 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
   // load instruction, before the data has arrived.
   static_assert(DS_RD * KS * MT * 4 <= 192, "token operands in flight must leave room in the VGPRs");
   // weight rows (per matrix) a block advances by
-  constexpr int BLOCK_ROWS = GATED ? 16 * HALVES : 16 * NREG;
+  constexpr int BLOCK_ROWS = 16 * HALVES;
   constexpr int SLOT = NREG * REGION;
   constexpr int LPS = KS * MT + NREG * LPR;  // load instructions per stage (token operands + weights)
   // A stage is complete when no more than the DS_RD - 1 younger stages are in flight.  vmcnt has 6
@@ -146,7 +125,7 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
   // Partial sums change hands through LDS in two alternating buffers, or, where LDS does not hold
   // two, in one buffer with a second barrier behind its readers.
   constexpr int PART_FLOATS = (DS_WAVES - 1) * NREG * MT * 256;
-  constexpr int PARITIES = ds_part_buffers(NMAT, MT, SEGB);
+  constexpr int PARITIES = DS_WAVES * DS_RD * SLOT + 2 * PART_FLOATS * 4 <= DS_MAX_LDS ? 2 : 1;
 
   extern __shared__ __align__(1024) char smem[];
   const int lane = threadIdx.x & 63;
@@ -177,7 +156,7 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
       valid = t_end - row0;
     }
   };
-  const int chunks = a.red / CH;
+  const int chunks = TAIL ? (a.red + CH - 1) / CH : a.red / CH;
   // wavefront w reduces chunks [c0, c0 + spb)
   const int c0 = (chunks * wave) / DS_WAVES;
   const int spb = (chunks * (wave + 1)) / DS_WAVES - c0;
@@ -194,10 +173,12 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
   const int r16 = lane & 15, kg = lane >> 4;
   uint32_t woff[LPR], xoff[MT];
   int wrow[LPR];  // row of the region that load q of this lane fetches
+  int wchunk[LPR];  // TAIL: and its 16-byte piece of the row's segment
 #pragma unroll
   for (int q = 0; q < LPR; ++q) {
     int row = (64 / CPR) * q + lane / CPR, pos = lane % CPR;
     wrow[q] = row;
+    wchunk[q] = pos ^ row;
     woff[q] = (uint32_t)(row * a.red + (pos ^ row) * 8) * 2u;
   }
   const bool tiled_x = !GATED && a.tiled;
@@ -236,10 +217,13 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
     // token operand of the stage's q-th MFMA step: 64 bytes further along each row of x, or the
     // next fragment of H (a stage of CH elements x 16 MT token slots)
     const uint32_t xstage = tiled_x ? koff * (16u * MT) : koff;
+    // TAIL: 16-byte pieces of this stage's segment that lie inside the row
+    const int pieces = TAIL ? (a.red - (c0 + c) * CH) / 8 : CPR;
 #pragma unroll
     for (int q = 0; q < KS; ++q)
 #pragma unroll
-      for (int t = 0; t < MT; ++t) xf[u][q * MT + t] = load16_async(rx, xoff[t], xstage + q * xq);
+      for (int t = 0; t < MT; ++t)
+        xf[u][q * MT + t] = load16_async(rx, !TAIL || q * 4 + kg < pieces ? xoff[t] : DS_NOWHERE, xstage + q * xq);
     uint32_t slot = lds_base + (uint32_t)u * SLOT;
     uint32_t woffs = (uint32_t)row0 * pitch + koff;
 #pragma unroll
@@ -248,7 +232,8 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
       const int valid_g = valid - first;
 #pragma unroll
       for (int q = 0; q < LPR; ++q)
-        load16_to_lds<true>(rw[GATED ? g / HALVES : 0], wrow[q] < valid_g ? woff[q] : DS_NOWHERE,
+        load16_to_lds<true>(rw[GATED ? g / HALVES : 0],
+                            wrow[q] < valid_g && (!TAIL || wchunk[q] < pieces) ? woff[q] : DS_NOWHERE,
                             woffs + (uint32_t)first * pitch, slot + g * REGION + q * 1024);
     }
   };
@@ -369,19 +354,23 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
   wait_vmem<0>();
 }
 
-template <typename T, bool GATED, int NMAT, int MT, int SEGB>
-static hipError_t launch_stream(const StreamArgs& a, int num_cu, hipStream_t s) {
-  constexpr int NREG = NMAT * (512 / SEGB);
-  constexpr int LDS = DS_WAVES * ds_ring_depth(NMAT, MT, SEGB) * NMAT * DS_REGION +
-                      ds_part_buffers(NMAT, MT, SEGB) * (DS_WAVES - 1) * NREG * MT * 256 * 4;
-  static_assert(LDS <= 160 * 1024, "a workgroup has 160 KiB of LDS");
-  constexpr auto kern = decode_stream_kernel<T, GATED, NMAT, MT, SEGB>;
+template <typename T, bool GATED, int HALVES, int MT, int SEGB, int RD, bool TAIL>
+static hipError_t launch_stream_tail(const StreamArgs& a, int num_cu, hipStream_t s) {
+  constexpr int NREG = (GATED ? 2 : 1) * HALVES, RING = DS_WAVES * RD * NREG * 16 * SEGB, PART = (DS_WAVES - 1) * NREG * MT * 1024;
+  constexpr int LDS = RING + (RING + 2 * PART <= DS_MAX_LDS ? 2 : 1) * PART;
+  static_assert(LDS <= DS_MAX_LDS, "a workgroup has 160 KiB of LDS");
+  constexpr auto kern = decode_stream_kernel<T, GATED, HALVES, MT, SEGB, RD, TAIL>;
   if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, LDS>, s)) return e;
   // one workgroup per CU, each with its share of the rows (a partly empty block when that is less
   // than a block); fewer workgroups when a share would be under 8 rows
   int grid = a.R / 8 < num_cu ? a.R / 8 : num_cu;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(DS_WAVES * 64), LDS, s, a);
   return hipGetLastError();
+}
+template <typename T, bool GATED, int HALVES, int MT, int SEGB, int RD>
+static hipError_t launch_stream(const StreamArgs& a, int num_cu, hipStream_t s) {
+  return a.red % (SEGB / 2) == 0 ? launch_stream_tail<T, GATED, HALVES, MT, SEGB, RD, false>(a, num_cu, s)
+                                 : launch_stream_tail<T, GATED, HALVES, MT, SEGB, RD, true>(a, num_cu, s);
 }
 
 // Layout of the intermediate H between the two kernels.  Row-major [M, N] costs the down projection
@@ -390,8 +379,23 @@ static hipError_t launch_stream(const StreamArgs& a, int num_cu, hipStream_t s) 
 static int ds_h_tiled(int M) { return M > DS_H_TILED_MIN_M ? 1 : 0; }
 
 bool decode_stream_supported(int M, int K, int N) {
-  return M >= 1 && M <= 32 && K % DS_CH == 0 && N % DS_CH == 0 && K >= DS_WAVES * DS_CH && N >= DS_WAVES * DS_CH &&
+  return M >= 1 && M <= 32 && K % 8 == 0 && N % 8 == 0 && K >= DS_MIN_RED && N >= DS_MIN_RED &&
          (int64_t)K * N * 2 < ((int64_t)1 << 31);
+}
+
+// Blocks of 32 rows of W_gate and W_up, 128 elements a stage (two stages' worth of 16-row blocks of 256
+// elements): half the token operands per weight byte.  M=24, K=4096, N=14336 73 us against 79, M=16,
+// K=5120, N=13824 80 / 85, M=1, K=6144, N=16384 98 / 101.  With one token tile or little more the
+// operands cost less than a block that a CU's share does not fill (M=1, K=2560, N=10240, 40 rows: 34.6
+// against 32.7; M=16, K=8192, N=28672, 112 rows: 228 / 224), so they are taken there only where the
+// share rounded up to 16 and to 32 rows is the same.  Rows that do not start on a 128-byte line take the
+// long segments throughout: a 256-byte one touches three lines instead of two (K=6712, N=24104, M=1 210 ->
+// 188 us; K=3592, N=8200, M=24 61 -> 56; M=32, K=3112, N=7000 is the one that loses, 46.4 -> 47.6).
+static bool ds_whole_lines(int red) { return red % 64 == 0; }
+static bool ds_tall_gated(int M, int K, int N, int num_cu) {
+  if (!ds_whole_lines(K)) return false;
+  const int rows = (N + num_cu - 1) / num_cu;
+  return M > DS_WIDE_SEGMENT_MAX_M || (rows + 15) / 16 % 2 == 0;
 }
 
 template <typename T>
@@ -405,23 +409,24 @@ hipError_t launch_decode_stream(const T* x, const T* wg, const T* wu, const T* w
   const int tiled = ds_h_tiled(M);
   StreamArgs a1 = {x, {wg, wu}, {bg, bu}, h, M, N, K, K, N, act, tiled};
   StreamArgs a2 = {h, {wd, wd}, {bd, bd}, y, M, K, N, N, K, ACT_IDENTITY, tiled};
-  // two runs of W_down rows per token-operand fetch halve the L2 traffic for H; worth it when a
-  // CU's share of the rows exceeds one run
-  const bool wide = K > 16 * num_cu;
+  const bool tall = ds_tall_gated(M, K, N, num_cu);
+  // W_down: 32 rows of 128 elements a stage, four stages deep, once a CU's share exceeds 16 rows (K=5120,
+  // N=13824, whole forward, against 32 rows of 256 three deep, or 64 of 128 from M = 21 up: M=1 72 -> 70
+  // us, M=16 80 -> 79, M=24 106 -> 98), 16 rows of 256 up to there (K=4096, N=11008, M=24, against 32
+  // half empty: 65 -> 64).  Two token tiles over 48 rows or more take 64 at a time: K=16384, N=53248, M=18
+  // 807 -> 783 us.  Misaligned rows take 256 elements at any height (K=6712, N=24104, M=1 188 -> 178).
+  const bool one = K <= 16 * num_cu, lines = ds_whole_lines(N), four = K > 48 * num_cu && lines;
   if (M <= 16) {
-    if (hipError_t e = launch_stream<T, true, 2, 1, 512>(a1, num_cu, s)) return e;
-    return wide ? launch_stream<T, false, 2, 1, 512>(a2, num_cu, s) : launch_stream<T, false, 1, 1, 512>(a2, num_cu, s);
+    if (hipError_t e = tall ? launch_stream<T, true, 2, 1, 256, 3>(a1, num_cu, s) : launch_stream<T, true, 1, 1, 512, 3>(a1, num_cu, s))
+      return e;
+    if (one) return launch_stream<T, false, 1, 1, 512, 4>(a2, num_cu, s);
+    return lines ? launch_stream<T, false, 2, 1, 256, 4>(a2, num_cu, s) : launch_stream<T, false, 2, 1, 512, 3>(a2, num_cu, s);
   }
-  // Two token tiles.  With 512-byte row segments the token operands cost as much L2 traffic as
-  // the weights cost HBM traffic, and the time grows by about 2 us per token at the 70B widths;
-  // 256-byte segments over twice the rows halve that but stream a few per cent slower from HBM.
-  // The two cross between M = 20 and M = 24 at every width measured.
-  if (M <= DS_WIDE_SEGMENT_MAX_M) {
-    if (hipError_t e = launch_stream<T, true, 2, 2, 512>(a1, num_cu, s)) return e;
-    return wide ? launch_stream<T, false, 2, 2, 512>(a2, num_cu, s) : launch_stream<T, false, 1, 2, 512>(a2, num_cu, s);
-  }
-  if (hipError_t e = launch_stream<T, true, 2, 2, 256>(a1, num_cu, s)) return e;
-  return wide ? launch_stream<T, false, 2, 2, 256>(a2, num_cu, s) : launch_stream<T, false, 1, 2, 256>(a2, num_cu, s);
+  if (hipError_t e = tall ? launch_stream<T, true, 2, 2, 256, 3>(a1, num_cu, s) : launch_stream<T, true, 1, 2, 512, 3>(a1, num_cu, s))
+    return e;
+  if (four) return launch_stream<T, false, 4, 2, 256, 3>(a2, num_cu, s);
+  if (one) return launch_stream<T, false, 1, 2, 512, 3>(a2, num_cu, s);
+  return lines ? launch_stream<T, false, 2, 2, 256, 4>(a2, num_cu, s) : launch_stream<T, false, 2, 2, 512, 3>(a2, num_cu, s);
 }
 
 template hipError_t launch_decode_stream<f16>(const f16*, const f16*, const f16*, const f16*,

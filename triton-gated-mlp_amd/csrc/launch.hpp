@@ -108,7 +108,7 @@ hipError_t launch_decode(const T* x, const T* wg, const T* wu, const T* wd, cons
                          const T* bu, const T* bd, T* h, T* y, int M, int K, int N, int act,
                          hipStream_t s);
 
-// decode_stream.hip: LDS-ring streaming variant for K % 256 == 0 and N % 256 == 0
+// decode_stream.hip: LDS-ring streaming variant for K and N from 768 up, any multiples of 8
 bool decode_stream_supported(int M, int K, int N);
 template <typename T>
 hipError_t launch_decode_stream(const T* x, const T* wg, const T* wu, const T* wd, const T* bg,

@@ -36,7 +36,7 @@ typedef std::optional<Tensor> OptTensor;
 
 #define GMLP_ENTRY_POINTS(X)                                                                     \
   X(gmlp_last_error) X(gmlp_workspace_bytes) X(gmlp_mlp_workspace_bytes) X(gmlp_mlp_fwd)         \
-  X(gmlp_mlp_bwd) X(gmlp_gateup_fwd) X(gmlp_decode_fwd) X(gmlp_gating_bwd) X(gmlp_dx_bwd)         \
+  X(gmlp_mlp_bwd) X(gmlp_gateup_fwd) X(gmlp_decode_fwd) X(gmlp_decode_stream_fwd) X(gmlp_gating_bwd) X(gmlp_dx_bwd) \
   X(gmlp_dw_bwd_grouped_workspace_bytes) X(gmlp_dw_bwd_grouped) X(gmlp_colsum_grouped)
 struct Library {
 #define GMLP_MEMBER(name) decltype(&::name) name = nullptr;
@@ -149,6 +149,16 @@ bool decode_preferred(int64_t M, int64_t K, int64_t N, int code, int64_t num_cu)
   if (M > 16 && !(K >= 768 && N >= 768 && K * N < ((int64_t)1 << 30))) return false;
   return K >= (M <= 16 ? 8 : 14) * num_cu;
 }
+// The widths that rule leaves out, on the same streaming kernels (two launches against the general path's
+// four, no partial sums in memory).  One token tile always wins: K=1024, N=2048 11 to 13 us against 16,
+// K=2200, N=4608 20 to 24 / 30, K=5168, N=20480 110 to 122 / 130 to 136.  With two, its operands' traffic
+// grows with the rows per compute unit: up to 32 rows of W_gate they win (K=1024, N=8192 27 / 28, K=3592,
+// N=8200 54 to 59 / 59 to 62), beyond they do not (K=2560, N=10240 49 / 46, K=4496, N=9472 68 / 67).
+bool narrow_decode_preferred(int64_t M, int64_t K, int64_t N, int code, int64_t num_cu) {
+  if (code == GMLP_F32 || M < 1 || M > 32 || K % 8 != 0 || N % 8 != 0) return false;
+  if (K < 768 || N < 768 || K * N >= ((int64_t)1 << 30)) return false;
+  return M <= 16 || N <= 33 * num_cu;
+}
 int64_t compute_units(int device) {
   static std::atomic<int> known[64];
   if (device < 0 || device >= 64) return 256;
@@ -181,10 +191,16 @@ Tensor mlp_infer(const Tensor& x_in, const Tensor& Wg_in, const OptTensor& bg_in
   const Tensor y = at::empty(x.sizes(), x.options());
   if (q.M == 0) return y;
   void* const stream = stream_of(x);
-  if (decode_preferred(q.M, q.K, q.N, q.code, compute_units(x.device().index()))) {
+  const int64_t cus = compute_units(x.device().index());
+  const bool decode = decode_preferred(q.M, q.K, q.N, q.code, cus);
+  if (decode || narrow_decode_preferred(q.M, q.K, q.N, q.code, cus)) {
     const Tensor h = at::empty({q.M <= 16 ? 16 : 32, q.N}, x.options());  // in the library's layout
-    check(lib.gmlp_decode_fwd(ptr(x), ptr(Wg), ptr(Wu), ptr(Wd), ptr(bg), ptr(bu), ptr(bd), out_ptr(h), out_ptr(y), nullptr, q.M,
-                              q.K, q.N, q.code, q.act, stream));
+    if (decode)
+      check(lib.gmlp_decode_fwd(ptr(x), ptr(Wg), ptr(Wu), ptr(Wd), ptr(bg), ptr(bu), ptr(bd), out_ptr(h), out_ptr(y), nullptr, q.M,
+                                q.K, q.N, q.code, q.act, stream));
+    else
+      check(lib.gmlp_decode_stream_fwd(ptr(x), ptr(Wg), ptr(Wu), ptr(Wd), ptr(bg), ptr(bu), ptr(bd), out_ptr(h), out_ptr(y), q.M,
+                                       q.K, q.N, q.code, q.act, stream));
     return y;
   }
   const Tensor h = at::empty({q.M, q.N}, x.options());

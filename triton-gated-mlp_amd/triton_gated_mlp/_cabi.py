@@ -70,6 +70,7 @@ _SIGNATURES = {
     "gmlp_colsum_static": (_int, [_c_ptr] * 2 + [_i64, _i64, _int, _c_ptr]),
     "gmlp_colsum_grouped": (_int, [_int, _c_ptr, _c_ptr, _c_ptr, _i64, _c_ptr, _int, _c_ptr]),
     "gmlp_decode_fwd": (_int, [_c_ptr] * 10 + [_i64, _i64, _i64, _int, _int, _c_ptr]),
+    "gmlp_decode_stream_fwd": (_int, [_c_ptr] * 9 + [_i64, _i64, _i64, _int, _int, _c_ptr]),
     "gmlp_dropout_mask": (_int, [_c_ptr, _i64, _i64, _f32, _u64, _u64, _c_ptr]),
     "gmlp_mlp_workspace_bytes": (ctypes.c_size_t, [_int, _i64, _i64, _i64, _int]),
     "gmlp_mlp_fwd": (

@@ -220,6 +220,9 @@ def decode_preferred(M: int, K: int, N: int, dtype: torch.dtype = torch.float16,
     kernels win by 4 to 17 % at M = 17 and by 0 to 10 % at M = 24 and 32 for hidden sizes from 3584
     up; below that they tie or lose (2560 x 10240: -12 %), so the module asks for 14 rows of W_down
     per compute unit there.
+
+    The module also takes them at narrower widths and at widths that are multiples of 8 only (entry point
+    `gmlp_decode_stream_fwd`, rule in csrc/torch_binding.cpp); this function answers for `decode_fwd`.
     """
     return decode_supported(M, K, N, dtype) and _cabi.torch_binding().decode_preferred(M, K, N, _cabi.dtype_code(dtype), num_cu)
 
