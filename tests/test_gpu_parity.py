@@ -1127,6 +1127,9 @@ def test_reduction_tails_every_operator_against_fp32_products(M, K, N):
         (1030, 2056, 5640),  # several rows of them, splits that end inside a tile
         (3000, 256, 520),    # weight gradients with a split reduction (few tiles, many tokens)
         (2500, 136, 72),     # the same, single tiles, ragged last split
+        (1345, 2264, 8120),  # 192-row tiles: gate/up and dH, one row beyond a tile, reduction tails
+        (2048, 2048, 5640),  # the same without tails, 10.7 tile rows, ragged columns
+        (5717, 1640, 6432),  # down and dX
     ],
 )
 def test_wide_tiles_and_split_gradients_against_fp32_products(M, K, N):

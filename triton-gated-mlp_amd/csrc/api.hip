@@ -235,6 +235,11 @@ struct TileCost {
 };
 const TileCost kLarge = {gmlp::TILE_LARGE, 256, 1, 1, 0.69, 0, {1.443, 1.477, 1.494}, {11.4, 6.1, 19.0, 6.8, 7.1, 12.0}};
 const TileCost kWide = {gmlp::TILE_WIDE, 128, 1, 1, 0.74, 0, {0.846, 0.940, 0.983}, {5.7, 2.7, 9.7, 3.3, 3.7, 2.0}};
+// (TALL: fitted the same way to 160 launches, four GEMMs of 40 shapes, standard deviation 7 %; it is the
+// fastest unsplit class in 55 of them, by up to 27 %: gate/up at M=1357, K=1160, N=3096 41.6 -> 30.4 us,
+// M=1346, K=2264, N=8120 117 -> 103, dH at M=2048, K=2048, N=5632 62 -> 54, down at M=5717, K=1640,
+// N=6432 124 -> 110.  Split reductions are left to the smaller classes.)
+const TileCost kTall = {gmlp::TILE_TALL, 192, 1, 1, 0.72, 0, {1.101, 1.156, 0}, {9.2, 3.9, 16.2, 0.4, 0, 0}};
 const TileCost kMedium = {gmlp::TILE_MEDIUM_FULL, 128, 2, 2, 0.46, 0.30, {0.967, 0.983, 1.094}, {3.4, 0.6, 8.4, 0.2, 2.4, 0.1}};
 
 double launch_us(const TileCost& c, int kind, int64_t tiles, int64_t kt, int splits, double out_elements) {
@@ -250,12 +255,12 @@ double launch_us(const TileCost& c, int kind, int64_t tiles, int64_t kt, int spl
   return us;
 }
 
-// The classes and splits for a grid of this many tiles of each class (`wide` 0: class not built).  At
+// The classes and splits for a grid of this many tiles of each class (`wide`, `tall` 0: not built).  At
 // least 4 reduction tiles per split, at most 16 splits.
-GemmPlan cheapest(int kind, int64_t large, int64_t wide, int64_t medium, int64_t kt, double out_elements, bool may_split) {
+GemmPlan cheapest(int kind, int64_t large, int64_t wide, int64_t tall, int64_t medium, int64_t kt, double out_elements, bool may_split) {
   GemmPlan best = {gmlp::TILE_LARGE, 1, launch_us(kLarge, kind, large, kt, 1, out_elements)};
   auto consider = [&](const TileCost& c, int64_t tiles) {
-    const int64_t most = may_split ? std::max<int64_t>(1, std::min<int64_t>(16, kt / 4)) : 1;
+    const int64_t most = may_split && c.tile_class != gmlp::TILE_TALL ? std::max<int64_t>(1, std::min<int64_t>(16, kt / 4)) : 1;
     for (int64_t s = 1; s <= most; ++s) {
       if (s > 1 && cdiv(kt, cdiv(kt, s)) != s) continue;  // rounding up would leave splits empty
       const double us = launch_us(c, kind, tiles, kt, (int)s, out_elements);
@@ -264,6 +269,7 @@ GemmPlan cheapest(int kind, int64_t large, int64_t wide, int64_t medium, int64_t
   };
   consider(kMedium, medium);
   if (wide > 0) consider(kWide, wide);
+  if (tall > 0) consider(kTall, tall);
   return best;
 }
 int64_t tiles_of(const TileCost& c, int kind, int64_t rows, int64_t cols) {
@@ -306,21 +312,24 @@ GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red,
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
   // the buffer base sits up to 4 KB below the operand (shared-M0 loads)
   const int64_t limit = ((int64_t)1 << 31) - 4096;
-  if (up(rows, 256) * up(red, 64) * 2 >= limit || up(cols, 256) * up(red, 64) * 2 >= limit) return {gmlp::TILE_MEDIUM, 1, 0};
+  if (std::max(up(rows, 256), up(rows, 192)) * up(red, 64) * 2 >= limit || up(cols, 256) * up(red, 64) * 2 >= limit) return {gmlp::TILE_MEDIUM, 1, 0};
   const int64_t kt = red_tiles_of(kind, red), large = tiles_of(kLarge, kind, rows, cols);
   const double out = (double)rows * (double)cols * (kind == GATEUP ? 2 : 1);
-  GemmPlan p = cheapest(kind, large, kind == DW ? 0 : tiles_of(kWide, kind, rows, cols), tiles_of(kMedium, kind, rows, cols), kt,
-                        out, may_split);
+  GemmPlan p = cheapest(kind, large, kind == DW ? 0 : tiles_of(kWide, kind, rows, cols), kind == DW ? 0 : tiles_of(kTall, kind, rows, cols),
+                        tiles_of(kMedium, kind, rows, cols), kt, out, may_split);
   if (p.tile_class == gmlp::TILE_LARGE) return p;
   // large tiles whose thin last round is shared out (stream-K) or run by other tiles may still be ahead
   const int64_t cus = num_cu(), whole = whole_rounds(kind, rows, cols);
   double us = p.us;
   if (plan_streamk(dtype, large, kt).tiles > 0) {
     us = streamk_us(kind, large, kt, out);
+    // (TALL's estimates differ from its times by 7 %: it has to be ahead by more than that)
+    if (p.tile_class == gmlp::TILE_TALL) us *= 0.9;
   } else if (whole > 0) {
     const int64_t r = kind <= LINEAR ? rows : rows - whole * 256, c = kind <= LINEAR ? cols - whole * tile_cols(kind) : cols;
     us = launch_us(kLarge, kind, large / cus * cus, kt, 1, out) +
-         cheapest(kind, tiles_of(kLarge, kind, r, c), tiles_of(kWide, kind, r, c), tiles_of(kMedium, kind, r, c), kt, 0, false).us;
+         cheapest(kind, tiles_of(kLarge, kind, r, c), tiles_of(kWide, kind, r, c), tiles_of(kTall, kind, r, c),
+                  tiles_of(kMedium, kind, r, c), kt, 0, false).us;
   }
   return us < p.us ? GemmPlan{gmlp::TILE_LARGE, 1, us} : p;
 }
@@ -375,7 +384,7 @@ GemmPlan plan_dw_group(int count, int64_t Mred, const int64_t* R, const int64_t*
   double out = 0;
   for (int i = 0; i < count; ++i) out += (double)R[i] * (double)C[i];
   const int64_t large = dw_group_tiles(kLarge, count, R, C), kt = cdiv(Mred, 64);
-  GemmPlan p = cheapest(DW, large, 0, dw_group_tiles(kMedium, count, R, C), kt, out, true);
+  GemmPlan p = cheapest(DW, large, 0, 0, dw_group_tiles(kMedium, count, R, C), kt, out, true);
   if (p.tile_class != gmlp::TILE_LARGE && plan_streamk(GMLP_F16, large, kt, false).tiles > 0) {
     const double us = streamk_us(DW, large, kt, out);
     if (us < p.us) p = GemmPlan{gmlp::TILE_LARGE, 1, us};

@@ -19,6 +19,8 @@ constexpr bool KT = GMLP_KT;
   launch_gemm_pipelined<DT, 256, BN_L, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M) \
   launch_gemm_pipelined<DT, 128, BN_M, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
+#define GMLP_TALL(AKS, BKS, NB, EPI, BN_T) \
+  launch_gemm_pipelined<DT, 192, BN_T, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_WIDE(AKS, BKS, NB, EPI, BN_W) \
   launch_gemm_pipelined<DT, 128, BN_W, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_LARGE_GROUP \
@@ -28,8 +30,10 @@ constexpr bool KT = GMLP_KT;
 
 #define GMLP_DISPATCH(AKS, BKS, NB, EPI, BN_L, BN_M)                                             \
   if (tile_class == TILE_LARGE) return GMLP_LARGE(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
-  if constexpr (!(AKS))                                                                          \
+  if constexpr (!(AKS)) {                                                                        \
     if (tile_class == TILE_WIDE) return GMLP_WIDE(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
+    if (tile_class == TILE_TALL) return GMLP_TALL(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
+  }                                                                                              \
   if (tile_class == TILE_MEDIUM_FULL) return GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M)(ga, ea, s);    \
   if constexpr (KT) return hipErrorInvalidValue; /* launch.hpp sends it to the other unit */       \
   else return launch_gemm<DT, 128, BN_M, 64, 2, 2, AKS, BKS, NB, true, EPI<DT>>(ga, ea, s);
@@ -42,6 +46,7 @@ hipError_t launch_gateup_kt<DT, KT>(int tile_class, const GemmArgs& ga, const Ep
   if (EpiGateUpPacked<DT>::packed_eligible(ea)) {
     if (tile_class == TILE_LARGE) return GMLP_LARGE(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
     if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
+    if (tile_class == TILE_TALL) return GMLP_TALL(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
     if (tile_class == TILE_MEDIUM_FULL) return GMLP_MEDIUM(false, false, 2, EpiGateUpPacked, 64)(ga, ea, s);
   }
   GMLP_DISPATCH(false, false, 2, EpiGateUp, 128, 64)

@@ -79,7 +79,7 @@ struct PipeConfig {
   // L2 backs the queue up into the issuing wavefronts (down projection: queue-full stalls 166 -> 10
   // clocks per tile, 2664 -> 2451 clocks per tile, -4 % run time; input gradient -2 %).
   static constexpr bool B3 = BM == 128 && NB * BN == 256;
-  static constexpr bool A3 = B3 || (RING_A3 && (BM == 256 || BM == 128) && !A_KS);
+  static constexpr bool A3 = B3 || (RING_A3 && (BM == 256 || BM == 192 || BM == 128) && !A_KS);
   static constexpr int MAIN_BYTES = A3 ? 3 * ATile::BYTES + (B3 ? 3 : NS) * NB * BTile::BYTES : NS * STAGE;
   static_assert(MAIN_BYTES <= 160 * 1024, "a workgroup has 160 KiB of LDS");
   static constexpr int LDS_BYTES = MAIN_BYTES > NW * EPI_WAVE_BYTES ? MAIN_BYTES : NW * EPI_WAVE_BYTES;
@@ -610,6 +610,7 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
       l3_issue(z);
     }
     l3_advance(0);
+    static_assert(HEAD_SLOTS % LSL3 != PH3 || HEAD_B % 4 != 0, "no handover slot leaves an M0 for the first load of a tile proper");
     wait_vmem<(B3 ? L3 : LDA) + HEAD_B>();
     __syncthreads();
 #pragma unroll
@@ -629,6 +630,9 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
       if (starts_group(x)) dma_base(kt_first + 1, x);
       issue_one(x);
     }
+    // (and the M0 that the last handover slot would have left for the next load: 192-row tiles)
+    if constexpr (HEAD_SLOTS % LOAD_SLOTS == LOAD_PHASE && L_HEAD < L)
+      if (starts_group(L_HEAD)) dma_base(kt_first + 1, L_HEAD);
     wait_vmem<L_HEAD>();
     __syncthreads();
 #pragma unroll

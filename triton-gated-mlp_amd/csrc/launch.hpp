@@ -12,6 +12,8 @@ namespace gmlp {
 //                workgroup at 5/6 of its throughput: for grids that LARGE fills badly and for short
 //                batches, where it reads the weights once per 128 token rows from L2 and needs fewer
 //                splits than MEDIUM_FULL
+//   TALL         192x256 output tiles, wavefronts of 96x128, pipelined kernel (not the weight gradients, no
+//                split reductions): three quarters of LARGE's work, for grids that LARGE fills badly
 //   MEDIUM_FULL  128x128 output tiles, wavefronts of 64x64, pipelined kernel; two workgroups per CU,
 //                for problems with too few 256x256 tiles to fill the chip
 //   MEDIUM       128x128, predicated register-staged kernel, 64-bit addresses: operands too large for
@@ -19,7 +21,7 @@ namespace gmlp {
 //   F32_*        the float32 kernel's tiles (gemm_f32.hip): 128 x 128, 64 x 128, 64 x 64; with two
 //                accumulator sets 128 x 64 or 64 x 64
 enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2, TILE_F32_128 = 3, TILE_F32_64X128 = 4, TILE_F32_64 = 5,
-                 TILE_WIDE = 6 };
+                 TILE_WIDE = 6, TILE_TALL = 7 };
 
 // kinds of GEMM the gated MLP needs; each is instantiated per dtype and tile class, and for reduction
 // lengths that are (KT = false) or are not a multiple of 64, the width of a reduction tile.
