@@ -385,17 +385,17 @@ bool decode_stream_supported(int M, int K, int N) {
 
 // Blocks of 32 rows of W_gate and W_up, 128 elements a stage (two stages' worth of 16-row blocks of 256
 // elements): half the token operands per weight byte.  M=24, K=4096, N=14336 73 us against 79, M=16,
-// K=5120, N=13824 80 / 85, M=1, K=6144, N=16384 98 / 101.  With one token tile or little more the
-// operands cost less than a block that a CU's share does not fill (M=1, K=2560, N=10240, 40 rows: 34.6
-// against 32.7; M=16, K=8192, N=28672, 112 rows: 228 / 224), so they are taken there only where the
-// share rounded up to 16 and to 32 rows is the same.  Rows that do not start on a 128-byte line take the
-// long segments throughout: a 256-byte one touches three lines instead of two (K=6712, N=24104, M=1 210 ->
-// 188 us; K=3592, N=8200, M=24 61 -> 56; M=32, K=3112, N=7000 is the one that loses, 46.4 -> 47.6).
+// K=5120, N=13824 80 / 85.  With one token tile or little more the operands cost less than a block that
+// a CU's share does not fill (M=16, K=8192, N=28672, 112 rows: 228 / 224), so they are taken there only
+// where the share rounded up to 16 and to 32 rows is the same, and up to 10 tokens not at all (M=5, K=3840,
+// N=6656 33.0 / 32.3).  Rows that do not start on a 128-byte line take the long segments throughout: a
+// 256-byte one touches three lines instead of two (K=6712, N=24104, M=1 210 -> 188 us; K=3592, N=8200,
+// M=24 61 -> 56; M=32, K=3112, N=7000 is the one that loses, 46.4 -> 47.6).
 static bool ds_whole_lines(int red) { return red % 64 == 0; }
 static bool ds_tall_gated(int M, int K, int N, int num_cu) {
   if (!ds_whole_lines(K)) return false;
   const int rows = (N + num_cu - 1) / num_cu;
-  return M > DS_WIDE_SEGMENT_MAX_M || (rows + 15) / 16 % 2 == 0;
+  return M > DS_WIDE_SEGMENT_MAX_M || (M > DS_H_TILED_MIN_M && (rows + 15) / 16 % 2 == 0);
 }
 
 template <typename T>
