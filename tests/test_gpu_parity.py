@@ -1584,6 +1584,41 @@ def test_native_autograd_nodes_keep_pytorchs_contracts():
         assert torch.equal(gx, ref_x) and all(torch.equal(g, ref[n]) for n, g in grads.items())
 
 
+def test_native_autograd_nodes_refuse_what_they_cannot_differentiate():
+    """Forward mode and functorch transforms raise (a result without its tangent would be wrong), unpack
+    hooks that change a saved tensor's type, size or device raise before a kernel reads it, and a
+    checkpoint that holds other operators beside the module recomputes them with autograd recording."""
+    import torch.autograd.forward_ad as fw
+    from torch.utils.checkpoint import checkpoint
+
+    from triton_gated_mlp import FusedGatedMLP, FusedGatedMLPFunction
+
+    dev = _dev()
+    torch.manual_seed(7)
+    mlp = FusedGatedMLP(256, 512, bias=True).to(dev).half()
+    x = torch.randn(24, 256, device=dev, dtype=torch.float16, requires_grad=True)
+    W = [mlp.up_proj.weight, mlp.gate_proj.weight]
+    calls = {256: mlp, 512: lambda t: FusedGatedMLPFunction.apply(t, W[0], None, W[1], None)}
+    for width, call in calls.items():
+        dy = torch.randn(24, width, device=dev, dtype=torch.float16)
+        with fw.dual_level(), pytest.raises(NotImplementedError, match="forward-mode"):
+            call(fw.make_dual(x, torch.ones_like(x)))
+        with pytest.raises(RuntimeError):
+            torch.vmap(call)(x[None])
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda t: call(t).sum())(x.detach())
+        for unpack in (lambda t: t.cpu(), lambda t: t.float(), lambda t: t.reshape(-1)[:-8]):
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+                y = call(x)
+            with pytest.raises(RuntimeError, match="saved tensor came back"):
+                y.backward(dy)
+        block = torch.nn.Linear(256, 256, bias=False).to(dev).half()
+        segment = lambda t: torch.tanh(call(torch.tanh(block(t))))
+        (want,) = torch.autograd.grad(segment(x), [x], dy)
+        (got,) = torch.autograd.grad(checkpoint(segment, x, use_reentrant=False), [x], dy)
+        assert torch.equal(got, want)
+
+
 def test_training_step_under_stream_capture_is_refused(monkeypatch):
     """A forward that records an autograd graph while its stream is being captured raises a
     RuntimeError (no kernel is enqueued, nothing is captured); the capture state is simulated on

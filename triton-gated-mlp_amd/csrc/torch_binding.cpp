@@ -121,6 +121,21 @@ Problem problem_of(const Tensor& x, const Tensor& W_up, int code, int64_t act) {
   return q;
 }
 
+// Neither node has a forward-mode derivative: a dual input would come out without its tangent.
+void refuse_forward_ad(std::initializer_list<std::reference_wrapper<const Tensor>> tensors) {
+  for (const Tensor& t : tensors)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(/*level=*/0).defined(),
+                                "the fused gated-MLP operators have no forward-mode derivative");
+}
+// A tensor that the kernels are about to read in a backward pass: saved-tensor hooks may hand back a tensor
+// on another device, of another type or size than was saved.
+Tensor readable(const Tensor& t, int64_t numel, const Tensor& grad) {
+  TORCH_CHECK(t.defined() && t.device() == grad.device() && t.scalar_type() == grad.scalar_type() && t.numel() == numel,
+              "a saved tensor came back as ", t.defined() ? c10::str(t.sizes(), " ", t.scalar_type(), " on ", t.device()) : "undefined",
+              ", expected ", numel, " elements of ", grad.scalar_type(), " on ", grad.device());
+  return t.contiguous();
+}
+
 Tensor scratch(size_t bytes, const Tensor& like) {
   return bytes > 0 ? at::empty({(int64_t)bytes}, like.options().dtype(at::kByte)) : Tensor();
 }
@@ -230,10 +245,14 @@ struct MlpBackward : public ag::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     ag::variable_list out(7);
     if (!grads[0].defined()) return out;
+    // first of all, while autograd still records: an unpack hook may run a whole forward (checkpointing)
+    const Tensor x_saved = x_.unpack(), Wg_saved = Wg_.unpack(), Wu_saved = Wu_.unpack(), Wd_saved = Wd_.unpack();
+    const Tensor acts_saved = acts_.unpack(), bg_saved = bg_.unpack(), bu_saved = bu_.unpack();
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(grads[0].device());
-    const Tensor dy = grads[0].contiguous(), x = x_.unpack().contiguous();
-    const Tensor Wg = Wg_.unpack().contiguous(), Wu = Wu_.unpack().contiguous(), Wd = Wd_.unpack().contiguous();
+    const Tensor dy = readable(grads[0], q.M * q.K, grads[0]), x = readable(x_saved, q.M * q.K, dy);
+    const Tensor Wg = readable(Wg_saved, q.N * q.K, dy), Wu = readable(Wu_saved, q.N * q.K, dy);
+    const Tensor Wd = readable(Wd_saved, q.K * q.N, dy);
     const bool want[7] = {true, true, has_bias[0], true, has_bias[1], true, has_bias[2]};
     const int64_t shape[7][2] = {{0, 0}, {q.N, q.K}, {q.N, 0}, {q.N, q.K}, {q.N, 0}, {q.K, q.N}, {q.K, 0}};
     for (int i = 0; i < 7; ++i) {
@@ -245,7 +264,8 @@ struct MlpBackward : public ag::Node {
     void* const stream = stream_of(dy);
     Tensor kept;
     if (recompute) {
-      const Tensor bg = contiguous(bg_.unpack()), bu = contiguous(bu_.unpack());
+      const Tensor bg = has_bias[0] ? readable(bg_saved, q.N, dy) : Tensor();
+      const Tensor bu = has_bias[1] ? readable(bu_saved, q.N, dy) : Tensor();
       kept = at::empty({3, q.M, q.N}, x.options());
       const Activations a(q, kept, true);
       const size_t bytes = lib.gmlp_workspace_bytes(GMLP_OP_GATEUP_FWD, q.M, q.K, q.N, q.code);
@@ -253,7 +273,7 @@ struct MlpBackward : public ag::Node {
       check(lib.gmlp_gateup_fwd(ptr(x), ptr(Wg), ptr(Wu), ptr(bg), ptr(bu), a.h, a.g, a.u, nullptr, q.M, q.K, q.N, q.code, q.act,
                                 (float)q.p, q.seed, q.offset, out_ptr(ws), bytes, stream));
     } else {
-      kept = acts_.unpack().contiguous();
+      kept = readable(acts_saved, 3 * q.M * q.N, dy);
     }
     const Activations a(q, kept, true);
     // dG, dU and the library's workspace share one scratch allocation that is dropped on return
@@ -274,6 +294,7 @@ Tensor mlp_train(const Tensor& x_in, const Tensor& Wg_in, const OptTensor& bg_in
                  int64_t act) {
   const Tensor &bg_o = or_undefined(bg_in), &bu_o = or_undefined(bu_in), &bd_o = or_undefined(bd_in);
   Problem q = check_mlp(x_in, Wg_in, bg_o, Wu_in, bu_o, Wd_in, bd_o, act);
+  refuse_forward_ad({x_in, Wg_in, bg_o, Wu_in, bu_o, Wd_in, bd_o});
   q.p = p;
   q.seed = seed;
   q.offset = offset;
@@ -335,10 +356,12 @@ struct HiddenBackward : public ag::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     ag::variable_list out(5);
     if (!grads[0].defined()) return out;
+    const Tensor x_saved = x_.unpack(), Wu_saved = Wu_.unpack(), Wg_saved = Wg_.unpack(), gate_up_saved = gate_up_.unpack();
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(grads[0].device());
-    const Tensor dh = grads[0].contiguous(), x = x_.unpack().contiguous();
-    const Tensor Wu = Wu_.unpack().contiguous(), Wg = Wg_.unpack().contiguous(), kept = gate_up_.unpack().contiguous();
+    const Tensor dh = readable(grads[0], q.M * q.N, grads[0]), x = readable(x_saved, q.M * q.K, dh);
+    const Tensor Wu = readable(Wu_saved, q.N * q.K, dh), Wg = readable(Wg_saved, q.N * q.K, dh);
+    const Tensor kept = readable(gate_up_saved, 2 * q.M * q.N, dh);
     const bool want[5] = {true, true, has_bias[0], true, has_bias[1]};
     const int64_t shape[5][2] = {{q.M, q.K}, {q.N, q.K}, {q.N, 0}, {q.N, q.K}, {q.N, 0}};
     for (int i = 0; i < 5; ++i) {
@@ -389,6 +412,7 @@ Tensor hidden(const Tensor& x_in, const Tensor& Wu_in, const OptTensor& bu_in, c
   TORCH_CHECK_VALUE(x_in.dim() == 2, "input tensor must be 2-D [M, K], got ", x_in.dim(), " dims");
   check_gate_up(x_in, Wg_in, bg_o, Wu_in, bu_o);
   Problem q = problem_of(x_in, Wu_in, require_gpu({x_in, Wg_in, bg_o, Wu_in, bu_o}), act);
+  refuse_forward_ad({x_in, Wg_in, bg_o, Wu_in, bu_o});
   q.p = p;
   q.seed = seed;
   q.offset = offset;

@@ -114,6 +114,12 @@ def eager_bwd(x: Tensor, W_up: Tensor, W_gp: Tensor, grad_output: Tensor):
 _U64 = (1 << 64) - 1
 
 
+def _refuse_functorch(operator: str) -> None:
+    # as torch.autograd.Function does for an operator without rules of its own
+    if torch._C._are_functorch_transforms_active():
+        raise RuntimeError(f"{operator} does not support functorch transforms (vmap, grad, jvp, jacrev, ...)")
+
+
 class FusedGatedMLPFunction(Function):
     """Hidden-state operator hidden = dropout(act_fn(x·W_gpᵀ+b_gp) * (x·W_upᵀ+b_up)).
 
@@ -127,6 +133,7 @@ class FusedGatedMLPFunction(Function):
         x: Tensor, W_up: Tensor, b_up: Optional[Tensor], W_gp: Tensor, b_gp: Optional[Tensor], dropout_p: float = 0.0,
         seed: int = 0, offset: int = 0, act_fn: str = "silu",
     ) -> Tensor:
+        _refuse_functorch("FusedGatedMLPFunction")
         return _cabi.torch_binding().hidden(
             x, W_up, b_up, W_gp, b_gp, float(dropout_p), int(seed) & _U64, int(offset) & _U64, _cabi.act_code(act_fn)
         )
@@ -143,6 +150,7 @@ class FusedGatedMLPFullFunction(Function):
         x: Tensor, W_gate: Tensor, b_gate: Optional[Tensor], W_up: Tensor, b_up: Optional[Tensor], W_down: Tensor,
         b_down: Optional[Tensor], dropout_p: float, seed: int, offset: int, recompute: bool = False, act_fn: str = "silu",
     ) -> Tensor:
+        _refuse_functorch("FusedGatedMLPFullFunction")
         return _cabi.torch_binding().mlp_train(
             x, W_gate, b_gate, W_up, b_up, W_down, b_down, float(dropout_p), int(seed) & _U64, int(offset) & _U64,
             bool(recompute), _cabi.act_code(act_fn),
