@@ -1619,6 +1619,46 @@ def test_native_autograd_nodes_refuse_what_they_cannot_differentiate():
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("grad", [True, False], ids=["records a graph", "nothing to differentiate"])
+def test_traced_forwards_run_the_kernels(grad):
+    """torch.jit.trace of the module and of the hidden-state operator records the call, not the allocation
+    of its output: the traced graph gives the eager result on other inputs and other numbers of tokens, bit
+    for bit, and the eager gradients; with dropout the mask of the seed that was drawn while tracing."""
+    from triton_gated_mlp import FusedGatedMLP, FusedGatedMLPFunction
+    from triton_gated_mlp.gated_mlp import FusedGatedMLPFullFunction
+
+    dev = _dev()
+    torch.manual_seed(9)
+    mlp = FusedGatedMLP(1024, 2048, bias=True).to(dev).half().requires_grad_(grad)
+    W = [mlp.up_proj.weight, mlp.gate_proj.weight]
+    hidden = lambda t, wu, wg: FusedGatedMLPFunction.apply(t, wu, None, wg, None)
+    example = torch.randn(2, 3, 1024, device=dev, dtype=torch.float16)  # without a graph: the decode kernels
+    traced = torch.jit.trace(mlp, (example,))
+    traced_hidden = torch.jit.trace(hidden, (example.flatten(0, 1), *W))
+    for shape in ((2, 3), (2, 3), (5, 40)):  # (the second and later runs are the executor's optimised graph)
+        x = torch.randn(*shape, 1024, device=dev, dtype=torch.float16)
+        got, want = traced(x), mlp(x)
+        assert got.requires_grad == grad and torch.equal(got, want)
+        got_h, want_h = (call(x.flatten(0, 1), *W) for call in (traced_hidden, hidden))
+        assert got_h.requires_grad == grad and torch.equal(got_h, want_h)
+        if grad:
+            dy, dh = torch.randn_like(want), torch.randn_like(want_h)
+            params = list(mlp.parameters())
+            for a, b in zip(torch.autograd.grad(got, params, dy), torch.autograd.grad(want, params, dy)):
+                assert torch.equal(a, b)
+            for a, b in zip(torch.autograd.grad(got_h, W, dh), torch.autograd.grad(want_h, W, dh)):
+                assert torch.equal(a, b)
+    if grad:
+        mlp.dropout.p = 0.25
+        traced = torch.jit.trace(mlp, (example,), check_trace=False)
+        seed, offset = mlp.last_dropout_state
+        x = torch.randn_like(example)
+        want = FusedGatedMLPFullFunction.apply(
+            x, W[1], mlp.gate_proj.bias, W[0], mlp.up_proj.bias, mlp.down_proj.weight, mlp.down_proj.bias, 0.25, seed, offset
+        )
+        assert torch.equal(traced(x), want)
+
+
 def test_training_step_under_stream_capture_is_refused(monkeypatch):
     """A forward that records an autograd graph while its stream is being captured raises a
     RuntimeError (no kernel is enqueued, nothing is captured); the capture state is simulated on

@@ -18,7 +18,9 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
+#include <torch/library.h>
 
 #include <algorithm>
 #include <atomic>
@@ -449,12 +451,60 @@ Tensor hidden(const Tensor& x_in, const Tensor& Wu_in, const OptTensor& bu_in, c
   return h;
 }
 
+// ------------------------------------------------------------------ torch.jit.trace
+// While a trace is being recorded a call goes through torch's dispatcher, as an operator with a schema: the
+// tracer then records the call itself.  Called directly it would record the only torch operation that it
+// sees, the output's at::empty, and the traced graph would return memory that nothing fills.  Whether an
+// autograd node is recorded is decided when the operator runs, as in the module.  Every other call goes
+// straight to the functions above.
+Tensor mlp_op(const Tensor& x, const Tensor& Wg, const OptTensor& bg, const Tensor& Wu, const OptTensor& bu, const Tensor& Wd,
+              const OptTensor& bd, double p, int64_t seed, int64_t offset, bool recompute, int64_t act) {
+  if (p == 0.0 && !ag::compute_requires_grad(x, Wg, or_undefined(bg), Wu, or_undefined(bu), Wd, or_undefined(bd)))
+    return mlp_infer(x, Wg, bg, Wu, bu, Wd, bd, act);
+  return mlp_train(x, Wg, bg, Wu, bu, Wd, bd, p, (uint64_t)seed, (uint64_t)offset, recompute, act);
+}
+Tensor hidden_op(const Tensor& x, const Tensor& Wu, const OptTensor& bu, const Tensor& Wg, const OptTensor& bg, double p,
+                 int64_t seed, int64_t offset, int64_t act) {
+  return hidden(x, Wu, bu, Wg, bg, p, (uint64_t)seed, (uint64_t)offset, act);
+}
+
+template <typename F>
+c10::TypedOperatorHandle<F> recorded_operator(const char* name, F*) {
+  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
+}
+
+// The entry points of the Python side (mlp_infer is not called while tracing).
+Tensor call_mlp_train(const Tensor& x, const Tensor& Wg, const OptTensor& bg, const Tensor& Wu, const OptTensor& bu,
+                      const Tensor& Wd, const OptTensor& bd, double p, uint64_t seed, uint64_t offset, bool recompute,
+                      int64_t act) {
+  if (torch::jit::tracer::isTracing()) {
+    static const auto op = recorded_operator("triton_gated_mlp::mlp", mlp_op);
+    return op.call(x, Wg, bg, Wu, bu, Wd, bd, p, (int64_t)seed, (int64_t)offset, recompute, act);
+  }
+  return mlp_train(x, Wg, bg, Wu, bu, Wd, bd, p, seed, offset, recompute, act);
+}
+Tensor call_hidden(const Tensor& x, const Tensor& Wu, const OptTensor& bu, const Tensor& Wg, const OptTensor& bg, double p,
+                   uint64_t seed, uint64_t offset, int64_t act) {
+  if (torch::jit::tracer::isTracing()) {
+    static const auto op = recorded_operator("triton_gated_mlp::hidden", hidden_op);
+    return op.call(x, Wu, bu, Wg, bg, p, (int64_t)seed, (int64_t)offset, act);
+  }
+  return hidden(x, Wu, bu, Wg, bg, p, seed, offset, act);
+}
+
 }  // namespace
+
+TORCH_LIBRARY(triton_gated_mlp, m) {
+  m.def("mlp(Tensor x, Tensor W_gate, Tensor? b_gate, Tensor W_up, Tensor? b_up, Tensor W_down, Tensor? b_down, "
+        "float dropout_p, int seed, int offset, bool recompute, int act) -> Tensor", mlp_op);
+  m.def("hidden(Tensor x, Tensor W_up, Tensor? b_up, Tensor W_gp, Tensor? b_gp, float dropout_p, int seed, int offset, "
+        "int act) -> Tensor", hidden_op);
+}
 
 PYBIND11_MODULE(_gmlp_torch, m) {
   m.def("bind", torch::wrap_pybind_function(bind));
   m.def("decode_preferred", torch::wrap_pybind_function(decode_preferred));
   m.def("mlp_infer", torch::wrap_pybind_function_no_gil(mlp_infer));
-  m.def("mlp_train", torch::wrap_pybind_function_no_gil(mlp_train));
-  m.def("hidden", torch::wrap_pybind_function_no_gil(hidden));
+  m.def("mlp_train", torch::wrap_pybind_function_no_gil(call_mlp_train));
+  m.def("hidden", torch::wrap_pybind_function_no_gil(call_hidden));
 }

@@ -226,8 +226,9 @@ class FusedGatedMLP(_GatedMLPBase):
             ).reshape(x.shape)
         W_gate, b_gate, W_up, b_up, W_down, b_down = params
         graph = torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in params))
-        if not graph and p == 0.0:
-            # Nothing to differentiate: the weight-streaming kernels for skinny M, no autograd node.
+        if not graph and p == 0.0 and not torch.jit.is_tracing():
+            # Nothing to differentiate: the weight-streaming kernels for skinny M, no autograd node.  (A trace
+            # records the operator below either way, which makes this choice whenever it runs.)
             return _cabi.torch_binding().mlp_infer(
                 x, W_gate, b_gate, W_up, b_up, W_down, b_down, _cabi.act_code(self.act_fn)
             )
