@@ -331,6 +331,23 @@ def test_max_rows_32bit_keeps_padded_operands_below_2_gib():
     assert max_rows_32bit(4096, 14336, torch.float32) is None
 
 
+def test_batches_of_the_row_limit_keep_the_pipelined_kernels():
+    """The largest batch the module hands out in one piece (max_rows_32bit) runs on the pipelined tile
+    classes, whatever the width: among the other operand's widths tried there is one whose grid ends in a thin
+    last round, for which they (and not the predicated class) ask for a workspace to share it out."""
+    from triton_gated_mlp.ops.fwd import max_rows_32bit
+
+    lib = _cabi.lib()
+    assert lib.gmlp_workspace_bytes(_cabi.GMLP_OP_LINEAR_FWD, 33536, 32000, 4096, 0) == 75497472
+    for width in range(4352, 32769, 256):  # (below, reductions are too short to share out)
+        M = max_rows_32bit(width, width, torch.float16)
+        others = [*range(256, 4097, 256)] + ([32512] if width <= 16384 else [])
+        for op in ("LINEAR_FWD", "GATEUP_FWD", "DH_BWD", "DX_BWD"):
+            dims = [(M, c, width) if op == "DX_BWD" else (M, width, c) for c in others]
+            asks = [lib.gmlp_workspace_bytes(getattr(_cabi, f"GMLP_OP_{op}"), *d, 0) for d in dims]
+            assert max(asks) > 0, (op, width, M)
+
+
 def test_decode_preferred_needs_widths_that_fill_the_chip():
     """Routing of M <= 16 inference between the streaming kernels and the general path."""
     from triton_gated_mlp.ops.fwd import decode_preferred

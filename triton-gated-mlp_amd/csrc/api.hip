@@ -312,10 +312,13 @@ GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red,
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
   // the buffer base sits up to 4 KB below the operand (shared-M0 loads)
   const int64_t limit = ((int64_t)1 << 31) - 4096;
-  if (std::max(up(rows, 256), up(rows, 192)) * up(red, 64) * 2 >= limit || up(cols, 256) * up(red, 64) * 2 >= limit) return {gmlp::TILE_MEDIUM, 1, 0};
+  auto fits = [&](int64_t elements) { return elements * up(red, 64) * 2 < limit; };
+  if (!fits(up(rows, 256)) || !fits(up(cols, 256))) return {gmlp::TILE_MEDIUM, 1, 0};
+  // (192-row tiles can reach further past the last row than the others: rows that are a multiple of 256)
+  auto tall = [&](int64_t r, int64_t c) { return kind != DW && fits(up(r, 192)) ? tiles_of(kTall, kind, r, c) : 0; };
   const int64_t kt = red_tiles_of(kind, red), large = tiles_of(kLarge, kind, rows, cols);
   const double out = (double)rows * (double)cols * (kind == GATEUP ? 2 : 1);
-  GemmPlan p = cheapest(kind, large, kind == DW ? 0 : tiles_of(kWide, kind, rows, cols), kind == DW ? 0 : tiles_of(kTall, kind, rows, cols),
+  GemmPlan p = cheapest(kind, large, kind == DW ? 0 : tiles_of(kWide, kind, rows, cols), tall(rows, cols),
                         tiles_of(kMedium, kind, rows, cols), kt, out, may_split);
   if (p.tile_class == gmlp::TILE_LARGE) return p;
   // large tiles whose thin last round is shared out (stream-K) or run by other tiles may still be ahead
@@ -328,7 +331,7 @@ GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red,
   } else if (whole > 0) {
     const int64_t r = kind <= LINEAR ? rows : rows - whole * 256, c = kind <= LINEAR ? cols - whole * tile_cols(kind) : cols;
     us = launch_us(kLarge, kind, large / cus * cus, kt, 1, out) +
-         cheapest(kind, tiles_of(kLarge, kind, r, c), tiles_of(kWide, kind, r, c), tiles_of(kTall, kind, r, c),
+         cheapest(kind, tiles_of(kLarge, kind, r, c), tiles_of(kWide, kind, r, c), tall(r, c),
                   tiles_of(kMedium, kind, r, c), kt, 0, false).us;
   }
   return us < p.us ? GemmPlan{gmlp::TILE_LARGE, 1, us} : p;
