@@ -1619,6 +1619,35 @@ def test_native_autograd_nodes_refuse_what_they_cannot_differentiate():
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("how", ["no_grad", "frozen"])
+def test_forward_mode_and_functorch_are_refused_where_reverse_mode_records_nothing(how):
+    """A dual tensor does not require grad and torch.no_grad() leaves forward mode on: an inference forward
+    that dropped its tangent would answer wrongly.  Where forward mode is off it is a plain forward."""
+    import torch.autograd.forward_ad as fw
+
+    from triton_gated_mlp import FusedGatedMLP
+
+    dev = _dev()
+    torch.manual_seed(8)
+    mlp = FusedGatedMLP(1024, 2048, bias=True).to(dev).half().requires_grad_(how == "no_grad")
+    for M in (4, 200):  # the streaming and the general kernels
+        x = torch.randn(M, 1024, device=dev, dtype=torch.float16)
+        with torch.set_grad_enabled(how != "no_grad"):
+            want = mlp(x)
+            with fw.dual_level():
+                dual = fw.make_dual(x, torch.ones_like(x))
+                with pytest.raises(NotImplementedError, match="forward-mode"):
+                    mlp(dual)
+                with torch.inference_mode():
+                    assert torch.equal(mlp(dual), want)
+            with fw.dual_level(), pytest.raises(NotImplementedError, match="forward-mode"):
+                bias = mlp.down_proj.bias
+                torch.func.functional_call(mlp, {"down_proj.bias": fw.make_dual(bias.detach(), torch.ones_like(bias))}, (x,))
+            for transform in (torch.vmap(mlp), lambda t: torch.func.jvp(mlp, (t,), (t,))):
+                with pytest.raises(RuntimeError, match="functorch"):
+                    transform(x[None])
+
+
 @pytest.mark.parametrize("grad", [True, False], ids=["records a graph", "nothing to differentiate"])
 def test_traced_forwards_run_the_kernels(grad):
     """torch.jit.trace of the module and of the hidden-state operator records the call, not the allocation

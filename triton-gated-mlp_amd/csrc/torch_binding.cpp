@@ -123,7 +123,8 @@ Problem problem_of(const Tensor& x, const Tensor& W_up, int code, int64_t act) {
   return q;
 }
 
-// Neither node has a forward-mode derivative: a dual input would come out without its tangent.
+// None of the operators has a forward-mode derivative: a dual input would come out without its tangent
+// (also where reverse mode records nothing: torch.no_grad() leaves forward mode on).
 void refuse_forward_ad(std::initializer_list<std::reference_wrapper<const Tensor>> tensors) {
   for (const Tensor& t : tensors)
     TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(/*level=*/0).defined(),
@@ -201,6 +202,7 @@ Problem check_mlp(const Tensor& x, const Tensor& W_gate, const Tensor& b_gate, c
 Tensor mlp_infer(const Tensor& x_in, const Tensor& Wg_in, const OptTensor& bg_in, const Tensor& Wu_in, const OptTensor& bu_in,
                  const Tensor& Wd_in, const OptTensor& bd_in, int64_t act) {
   const Problem q = check_mlp(x_in, Wg_in, or_undefined(bg_in), Wu_in, or_undefined(bu_in), Wd_in, or_undefined(bd_in), act);
+  refuse_forward_ad({x_in, Wg_in, or_undefined(bg_in), Wu_in, or_undefined(bu_in), Wd_in, or_undefined(bd_in)});
   at::AutoDispatchBelowADInplaceOrView below;
   const c10::DeviceGuard guard(x_in.device());
   const Tensor x = x_in.contiguous(), Wg = Wg_in.contiguous(), Wu = Wu_in.contiguous(), Wd = Wd_in.contiguous();

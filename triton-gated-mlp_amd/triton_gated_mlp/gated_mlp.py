@@ -229,6 +229,7 @@ class FusedGatedMLP(_GatedMLPBase):
         if not graph and p == 0.0 and not torch.jit.is_tracing():
             # Nothing to differentiate: the weight-streaming kernels for skinny M, no autograd node.  (A trace
             # records the operator below either way, which makes this choice whenever it runs.)
+            _refuse_functorch("FusedGatedMLP")
             return _cabi.torch_binding().mlp_infer(
                 x, W_gate, b_gate, W_up, b_up, W_down, b_down, _cabi.act_code(self.act_fn)
             )
