@@ -12,6 +12,7 @@ yardstick: torch's own fp16 module on the same inputs against the same oracle.
 """
 
 import contextlib
+import warnings
 
 import numpy as np
 import pytest
@@ -1646,6 +1647,45 @@ def test_forward_mode_and_functorch_are_refused_where_reverse_mode_records_nothi
             for transform in (torch.vmap(mlp), lambda t: torch.func.jvp(mlp, (t,), (t,))):
                 with pytest.raises(RuntimeError, match="functorch"):
                     transform(x[None])
+
+
+@pytest.mark.parametrize("which", ["module", "hidden"])
+def test_second_derivatives_raise_instead_of_being_dropped(which):
+    """create_graph: the gradients are the usual ones, and a derivative through them raises, whatever it is
+    asked for and whatever other terms a loss has (a penalty on the gradient would otherwise count as a
+    constant).  What does not pass through them is differentiated."""
+    from triton_gated_mlp import FusedGatedMLP, FusedGatedMLPFunction
+
+    dev = _dev()
+    torch.manual_seed(10)
+    mlp = FusedGatedMLP(256, 512, bias=True).to(dev).half()
+    W = [mlp.up_proj.weight, mlp.gate_proj.weight]
+    call = mlp if which == "module" else lambda t: FusedGatedMLPFunction.apply(t, W[0], None, W[1], None)
+    a = torch.randn(24, 256, device=dev, dtype=torch.float16, requires_grad=True)
+    scale = torch.ones((), device=dev, dtype=torch.float16, requires_grad=True)
+    x = a * 1.0
+    plain = torch.autograd.grad(call(x).sum(), [x, *W])
+    with_graph = torch.autograd.grad((call(x) * scale).sum(), [x, *W], create_graph=True)
+    assert all(torch.equal(g, h) and h.requires_grad for g, h in zip(plain, with_graph))
+    for gradient in with_graph:
+        penalty = gradient.float().square().sum()
+        for loss in (penalty, penalty + x.float().square().sum()):
+            for wanted in (a, x, W[0], scale):
+                with pytest.raises(RuntimeError, match="no second derivative"):
+                    torch.autograd.grad(loss, wanted, retain_graph=True, allow_unused=True)
+            with pytest.raises(RuntimeError, match="no second derivative"):
+                loss.backward(retain_graph=True)
+        # a weight of the other gradients only
+        factor = torch.ones_like(gradient, requires_grad=True)
+        assert torch.equal(torch.autograd.grad((gradient * factor).sum(), factor, retain_graph=True)[0], gradient)
+    # an optimiser step on gradients that carry a graph
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")  # torch's, once per process, that such gradients are a reference cycle
+        call(x).sum().backward(create_graph=True)
+    torch.optim.SGD(W, lr=0.0).step()
+    for w, g in zip(W, plain[1:]):
+        assert torch.equal(w.grad, g)
+        w.grad = None
 
 
 @pytest.mark.parametrize("grad", [True, False], ids=["records a graph", "nothing to differentiate"])

@@ -16,6 +16,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -137,6 +138,20 @@ Tensor readable(const Tensor& t, int64_t numel, const Tensor& grad) {
               "a saved tensor came back as ", t.defined() ? c10::str(t.sizes(), " ", t.scalar_type(), " on ", t.device()) : "undefined",
               ", expected ", numel, " elements of ", grad.scalar_type(), " on ", grad.device());
   return t.contiguous();
+}
+
+// The backward passes have no derivative themselves.  Where autograd records one (create_graph), its results
+// get a node in the place of the derivative that raises when it is differentiated through; results without
+// a graph would silently be taken for constants.  The node leads on to what a derivative would reach (the
+// operator's inputs and the incoming gradient), so that autograd comes by whichever of them is asked for.
+void refuse_second_derivative(const ag::Node& backward, const Tensor& grad, ag::variable_list& out) {
+  if (!at::GradMode::is_enabled()) return;
+  ag::edge_list next = backward.next_edges();
+  if (grad.requires_grad()) next.push_back(ag::impl::gradient_edge(grad));
+  const auto node = std::shared_ptr<ag::Error>(
+      new ag::Error("the fused gated-MLP operators have no second derivative", std::move(next)), ag::deleteNode);
+  for (Tensor& t : out)
+    if (t.defined()) ag::set_history(t, node);
 }
 
 Tensor scratch(size_t bytes, const Tensor& like) {
@@ -289,6 +304,7 @@ struct MlpBackward : public ag::Node {
                            out_ptr(out[1]), out_ptr(out[3]), out_ptr(out[5]), out_ptr(out[2]), out_ptr(out[4]), out_ptr(out[6]),
                            q.M, q.K, q.N, q.code, q.act, (float)q.p, q.seed, q.offset, bytes > 0 ? base + 2 * plane : nullptr,
                            bytes, stream));
+    refuse_second_derivative(*this, grads[0], out);
     return out;
   }
 };
@@ -406,6 +422,7 @@ struct HiddenBackward : public ag::Node {
     if (nw > 0) check(lib.gmlp_dw_bwd_grouped(nw, lhs, rhs, dw, q.M, R, C, q.code, ws, bytes, stream));
     const int64_t cols[2] = {q.N, q.N};
     if (nb > 0) check(lib.gmlp_colsum_grouped(nb, summed, db, ws, q.M, cols, q.code, stream));
+    refuse_second_derivative(*this, grads[0], out);
     return out;
   }
 };
