@@ -1649,6 +1649,35 @@ def test_forward_mode_and_functorch_are_refused_where_reverse_mode_records_nothi
                     transform(x[None])
 
 
+@pytest.mark.parametrize("recompute", [False, True])
+def test_missing_incoming_gradient_counts_as_zeros(recompute):
+    """An operator behind the module whose backward returns None for it: every gradient is zeros (as from a
+    torch.autograd.Function), not None, which an optimiser with momentum or weight decay would skip."""
+    from triton_gated_mlp import FusedGatedMLP, FusedGatedMLPFunction
+
+    class NoGradient(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            return t.clone()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    dev = _dev()
+    mlp = FusedGatedMLP(64, 128, bias=True).to(dev).half()
+    mlp.recompute_activations = recompute
+    x = torch.randn(2, 12, 64, device=dev, dtype=torch.float16, requires_grad=True)
+    leaves = [x, *mlp.parameters()]
+    NoGradient.apply(mlp(x)).sum().backward()
+    assert all(t.grad is not None and t.grad.shape == t.shape and not t.grad.any() for t in leaves)
+    up, gate = mlp.up_proj, mlp.gate_proj
+    leaves = [up.weight, up.bias, gate.weight, gate.bias]
+    mlp.zero_grad()
+    NoGradient.apply(FusedGatedMLPFunction.apply(x.flatten(0, 1), *leaves)).sum().backward()
+    assert all(t.grad is not None and not t.grad.any() for t in leaves)
+
+
 @pytest.mark.parametrize("which", ["module", "hidden"])
 def test_second_derivatives_raise_instead_of_being_dropped(which):
     """create_graph: the gradients are the usual ones, and a derivative through them raises, whatever it is

@@ -131,6 +131,11 @@ void refuse_forward_ad(std::initializer_list<std::reference_wrapper<const Tensor
     TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(/*level=*/0).defined(),
                                 "the fused gated-MLP operators have no forward-mode derivative");
 }
+// The incoming gradient, or zeros where what used the result has none for it (as torch.autograd.Function
+// does by default): the gradients are zeros then, not None.
+Tensor materialized(const Tensor& grad, at::IntArrayRef sizes, const at::TensorOptions& options) {
+  return grad.defined() ? grad : at::zeros(sizes, options);
+}
 // A tensor that the kernels are about to read in a backward pass: saved-tensor hooks may hand back a tensor
 // on another device, of another type or size than was saved.
 Tensor readable(const Tensor& t, int64_t numel, const Tensor& grad) {
@@ -251,6 +256,7 @@ struct MlpBackward : public ag::Node {
   bool recompute = false;
   bool has_bias[3] = {false, false, false};  // gate, up, down
   std::vector<int64_t> x_sizes;
+  at::TensorOptions options;  // of x
   ag::SavedVariable x_, Wg_, Wu_, Wd_;
   ag::SavedVariable acts_;      // G, U, H
   ag::SavedVariable bg_, bu_;   // recompute: G, U, H are computed again, from the inputs
@@ -263,13 +269,13 @@ struct MlpBackward : public ag::Node {
   ag::variable_list apply(ag::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     ag::variable_list out(7);
-    if (!grads[0].defined()) return out;
+    const Tensor grad = materialized(grads[0], x_sizes, options);
     // first of all, while autograd still records: an unpack hook may run a whole forward (checkpointing)
     const Tensor x_saved = x_.unpack(), Wg_saved = Wg_.unpack(), Wu_saved = Wu_.unpack(), Wd_saved = Wd_.unpack();
     const Tensor acts_saved = acts_.unpack(), bg_saved = bg_.unpack(), bu_saved = bu_.unpack();
     at::AutoDispatchBelowADInplaceOrView below;
-    const c10::DeviceGuard guard(grads[0].device());
-    const Tensor dy = readable(grads[0], q.M * q.K, grads[0]), x = readable(x_saved, q.M * q.K, dy);
+    const c10::DeviceGuard guard(grad.device());
+    const Tensor dy = readable(grad, q.M * q.K, grad), x = readable(x_saved, q.M * q.K, dy);
     const Tensor Wg = readable(Wg_saved, q.N * q.K, dy), Wu = readable(Wu_saved, q.N * q.K, dy);
     const Tensor Wd = readable(Wd_saved, q.K * q.N, dy);
     const bool want[7] = {true, true, has_bias[0], true, has_bias[1], true, has_bias[2]};
@@ -304,7 +310,7 @@ struct MlpBackward : public ag::Node {
                            out_ptr(out[1]), out_ptr(out[3]), out_ptr(out[5]), out_ptr(out[2]), out_ptr(out[4]), out_ptr(out[6]),
                            q.M, q.K, q.N, q.code, q.act, (float)q.p, q.seed, q.offset, bytes > 0 ? base + 2 * plane : nullptr,
                            bytes, stream));
-    refuse_second_derivative(*this, grads[0], out);
+    refuse_second_derivative(*this, grad, out);
     return out;
   }
 };
@@ -344,6 +350,7 @@ Tensor mlp_train(const Tensor& x_in, const Tensor& Wg_in, const OptTensor& bg_in
     node->has_bias[1] = bu_o.defined();
     node->has_bias[2] = bd_o.defined();
     node->x_sizes = x_in.sizes().vec();
+    node->options = y.options();
     node->x_ = ag::SavedVariable(x_in, false);
     node->Wg_ = ag::SavedVariable(Wg_in, false);
     node->Wu_ = ag::SavedVariable(Wu_in, false);
@@ -364,6 +371,7 @@ Tensor mlp_train(const Tensor& x_in, const Tensor& Wg_in, const OptTensor& bg_in
 struct HiddenBackward : public ag::Node {
   Problem q;
   bool has_bias[2] = {false, false};  // up, gate
+  at::TensorOptions options;          // of x
   ag::SavedVariable x_, Wu_, Wg_;
   ag::SavedVariable gate_up_;  // [2, M, N]
 
@@ -375,11 +383,11 @@ struct HiddenBackward : public ag::Node {
   ag::variable_list apply(ag::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     ag::variable_list out(5);
-    if (!grads[0].defined()) return out;
+    const Tensor grad = materialized(grads[0], {q.M, q.N}, options);
     const Tensor x_saved = x_.unpack(), Wu_saved = Wu_.unpack(), Wg_saved = Wg_.unpack(), gate_up_saved = gate_up_.unpack();
     at::AutoDispatchBelowADInplaceOrView below;
-    const c10::DeviceGuard guard(grads[0].device());
-    const Tensor dh = readable(grads[0], q.M * q.N, grads[0]), x = readable(x_saved, q.M * q.K, dh);
+    const c10::DeviceGuard guard(grad.device());
+    const Tensor dh = readable(grad, q.M * q.N, grad), x = readable(x_saved, q.M * q.K, dh);
     const Tensor Wu = readable(Wu_saved, q.N * q.K, dh), Wg = readable(Wg_saved, q.N * q.K, dh);
     const Tensor kept = readable(gate_up_saved, 2 * q.M * q.N, dh);
     const bool want[5] = {true, true, has_bias[0], true, has_bias[1]};
@@ -422,7 +430,7 @@ struct HiddenBackward : public ag::Node {
     if (nw > 0) check(lib.gmlp_dw_bwd_grouped(nw, lhs, rhs, dw, q.M, R, C, q.code, ws, bytes, stream));
     const int64_t cols[2] = {q.N, q.N};
     if (nb > 0) check(lib.gmlp_colsum_grouped(nb, summed, db, ws, q.M, cols, q.code, stream));
-    refuse_second_derivative(*this, grads[0], out);
+    refuse_second_derivative(*this, grad, out);
     return out;
   }
 };
@@ -461,6 +469,7 @@ Tensor hidden(const Tensor& x_in, const Tensor& Wu_in, const OptTensor& bu_in, c
     node->q = q;
     node->has_bias[0] = bu_o.defined();
     node->has_bias[1] = bg_o.defined();
+    node->options = h.options();
     node->x_ = ag::SavedVariable(x_in, false);
     node->Wu_ = ag::SavedVariable(Wu_in, false);
     node->Wg_ = ag::SavedVariable(Wg_in, false);
