@@ -1348,6 +1348,23 @@ def test_grouped_weight_gradients_equal_single_launches():
         _close("dW_gate grouped", grouped[0], dg.float().cpu().T @ x.float().cpu())
 
 
+def test_grouped_weight_gradients_of_mixed_sizes_equal_single_launches():
+    """One problem of a group beyond the pipelined kernels' 32-bit operand offsets takes the predicated
+    kernel alone: the others run as they do by themselves (here with a split reduction), bit for bit."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+
+    dev = _dev()
+    g = torch.Generator(device=dev).manual_seed(13)
+    rnd = lambda *shape: torch.empty(shape, dtype=torch.float16, device=dev).normal_(generator=g)
+    M = 66048
+    big, small, thin = rnd(M, 16384), rnd(M, 520), rnd(M, 8)  # 2.16e9 bytes, 69 MB, 1 MB
+    pairs = [(small, rnd(M, 520)), (big, thin), (thin, small)]
+    got = ops_bwd.dw_bwd_grouped(pairs)
+    for (a, b), dw in zip(pairs, got):
+        assert torch.equal(dw, ops_bwd.dw_bwd(a, b)), (a.shape, b.shape)
+        _close("dW", dw, sum(p.float().T @ q.float() for p, q in zip(a.split(8256), b.split(8256))))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_decode_matches_general_path(dtype):
     """Skinny-M kernels against the oracle and the general path: both layouts of the intermediate H

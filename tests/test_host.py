@@ -348,6 +348,19 @@ def test_batches_of_the_row_limit_keep_the_pipelined_kernels():
             assert max(asks) > 0, (op, width, M)
 
 
+def test_grouped_workspace_covers_the_separate_launches_of_mixed_sizes():
+    """A group with a problem that the pipelined kernels cannot address runs as separate launches: the
+    workspace is the largest that one of them uses."""
+    lib = _cabi.lib()
+    I64 = ctypes.c_int64 * 3
+    size = lambda n, R, C: lib.gmlp_dw_bwd_grouped_workspace_bytes(
+        n, 66048, ctypes.cast(I64(*R), ctypes.c_void_p), ctypes.cast(I64(*C), ctypes.c_void_p), 0)
+    alone = size(1, (520, 0, 0), (520, 0, 0))
+    assert alone > 0 and size(1, (16384, 0, 0), (8, 0, 0)) == 0  # operand of 2.16e9 bytes
+    assert size(2, (520, 16384, 0), (520, 8, 0)) == alone
+    assert size(3, (16384, 8, 520), (8, 8, 520)) == max(alone, size(1, (8, 0, 0), (8, 0, 0)))
+
+
 def test_decode_preferred_needs_widths_that_fill_the_chip():
     """Routing of M <= 16 inference between the streaming kernels and the general path."""
     from triton_gated_mlp.ops.fwd import decode_preferred

@@ -709,8 +709,17 @@ size_t gmlp_dw_bwd_grouped_workspace_bytes(int count, int64_t Mred, const int64_
       if (R[i] < 1 || C[i] < 1) return 0;
     return dw_group_split_bytes(count, plan_dw_group_f32(count, Mred, R, C).splits, R, C);
   }
-  for (int i = 0; i < count; ++i)
-    if (R[i] < 1 || C[i] < 1 || plan_gemm(dtype, DW, R[i], C[i], Mred, false).tile_class == TILE_MEDIUM) return 0;
+  bool pipelined = true;
+  for (int i = 0; i < count; ++i) {
+    if (R[i] < 1 || C[i] < 1) return 0;
+    pipelined = pipelined && plan_gemm(dtype, DW, R[i], C[i], Mred, false).tile_class != TILE_MEDIUM;
+  }
+  if (!pipelined) {  // separate launches, one after the other
+    size_t most = 0;
+    for (int i = 0; i < count && count > 1; ++i)
+      most = std::max(most, gmlp_dw_bwd_grouped_workspace_bytes(1, Mred, R + i, C + i, dtype));
+    return most;
+  }
   const GemmPlan p = plan_dw_group(count, Mred, R, C);
   if (p.tile_class != TILE_LARGE) return dw_group_split_bytes(count, p.splits, R, C);
   const StreamK sk = plan_streamk(dtype, dw_group_tiles(kLarge, count, R, C), cdiv(Mred, 64), false);
@@ -745,18 +754,20 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
     ga.M = (int)R[i]; ga.N = (int)C[i]; ga.K = (int)Mred; ga.lda = (int)R[i]; ga.ldb = (int)C[i];
     ga.nseg = 1; ga.group_m = pick_group(R[i], C[i]);
   };
-  if (!pipelined) {
-    hipError_t e = hipSuccess;
-    for (int i = 0; i < count && e == hipSuccess; ++i)
-      e = by_dtype(dtype, [&](auto tag) {
-        typedef decltype(tag) T;
-        GemmArgs ga;
-        fill(ga, i);
-        const typename EpiStore<T>::Args ea = {(T*)dw[i], nullptr, (int)C[i]};
-        return launch_dw<T>(TILE_MEDIUM, ga, ea, s);
-      });
-    return hip_result(__func__, e);
+  if (!pipelined && count > 1) {  // each problem on the class that suits it
+    for (int i = 0; i < count; ++i)
+      if (int rc = gmlp_dw_bwd_grouped(1, lhs + i, rhs + i, dw + i, Mred, R + i, C + i, dtype, workspace, workspace_bytes, stream))
+        return rc;
+    return GMLP_OK;
   }
+  if (!pipelined)
+    return hip_result(__func__, by_dtype(dtype, [&](auto tag) {
+      typedef decltype(tag) T;
+      GemmArgs ga;
+      fill(ga, 0);
+      const typename EpiStore<T>::Args ea = {(T*)dw[0], nullptr, (int)C[0]};
+      return launch_dw<T>(TILE_MEDIUM, ga, ea, s);
+    }));
   GemmPlan plan = dtype == GMLP_F32 ? plan_dw_group_f32(count, Mred, R, C) : plan_dw_group(count, Mred, R, C);
   if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < dw_group_split_bytes(count, plan.splits, R, C))) plan.splits = 1;
   if (dtype == GMLP_F32 || plan.splits > 1) {
