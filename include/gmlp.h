@@ -271,7 +271,10 @@ int gmlp_decode_stream_fwd(const void* x, const void* w_gate, const void* w_up, 
  * workspace: gmlp_mlp_workspace_bytes(GMLP_PASS_FWD or GMLP_PASS_BWD, M, K, N, dtype) bytes (may be
  * NULL or smaller for a pass without bias gradients: launches then take their plain form, with the
  * same results up to the order of fp32 additions; bias gradients need it and fail with GMLP_EINVAL
- * without).
+ * without).  GMLP_PASS_BWD answers for a pass that computes every gradient.  One or two of the weight
+ * gradients by themselves may use more (fewer tiles, more splits); such a pass uses the largest of
+ * gmlp_workspace_bytes of GMLP_OP_DH_BWD and GMLP_OP_DX_BWD, gmlp_dw_bwd_grouped_workspace_bytes of
+ * its weight gradients in the order above, and the sum of GMLP_OP_COLSUM over its bias gradients.
  */
 enum gmlp_pass { GMLP_PASS_FWD = 0, GMLP_PASS_BWD = 1 };
 size_t gmlp_mlp_workspace_bytes(int pass, int64_t M, int64_t K, int64_t N, int dtype);

@@ -1348,6 +1348,47 @@ def test_grouped_weight_gradients_equal_single_launches():
         _close("dW_gate grouped", grouped[0], dg.float().cpu().T @ x.float().cpu())
 
 
+@pytest.mark.parametrize(
+    "M,K,N,dtype,trained",
+    [
+        (380, 152, 136, torch.float32, ("gate_proj", "up_proj")),
+        (708, 96, 912, torch.float16, ("gate_proj", "down_proj")),
+        (5857, 1752, 6576, torch.float16, ("gate_proj", "up_proj")),  # stream-K
+        (3776, 2720, 136, torch.bfloat16, ("gate_proj",)),
+        (3115, 64, 7328, torch.float16, ("down_proj",)),
+    ],
+)
+def test_some_weight_gradients_run_as_planned_for_them(M, K, N, dtype, trained):
+    """A step that trains some of the weights gives their gradients the workspace that they use by
+    themselves, which here is more than that of a step that trains all: bit-identical to the grouped launch
+    (whose plan's order of additions differs from the one that a smaller workspace forces)."""
+    from triton_gated_mlp import FusedGatedMLP, _cabi
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    torch.manual_seed(14)
+    mlp = FusedGatedMLP(K, N, bias=False).to(dev).to(dtype)
+    mlp.requires_grad_(False)
+    weights = [getattr(mlp, name).weight.requires_grad_(True) for name in trained]
+    x, dy = torch.randn(M, K, device=dev).to(dtype), torch.randn(M, K, device=dev).to(dtype)
+    Wg, Wu, Wd = mlp.gate_proj.weight, mlp.up_proj.weight, mlp.down_proj.weight
+    with torch.no_grad():
+        hs = ops_fwd.gateup_fwd(x, Wg, None, Wu, None, save_activations=True)
+        dg, du = ops_bwd.dh_bwd(dy, Wd, hs.gate, hs.up)
+        operands = {"gate_proj": (dg, x), "up_proj": (du, x), "down_proj": (dy, hs.hidden)}
+        want = ops_bwd.dw_bwd_grouped([operands[name] for name in trained])
+        need = [False] * 7
+        for name in trained:
+            need[{"gate_proj": 1, "up_proj": 3, "down_proj": 5}[name]] = True
+        used = ops_bwd._mlp_bwd_workspace_bytes(M, K, N, _cabi.dtype_code(dtype), need)
+        assert used > _cabi.lib().gmlp_mlp_workspace_bytes(_cabi.GMLP_PASS_BWD, M, K, N, _cabi.dtype_code(dtype))
+        one_call = ops_bwd.mlp_bwd(dy, x, Wg, Wu, Wd, hs.gate, hs.up, hs.hidden, need)
+    mlp(x).backward(dy)
+    for w, a, b in zip(weights, want, (t for t in one_call if t is not None)):
+        assert torch.equal(w.grad, a) and torch.equal(b, a)
+
+
 def test_grouped_weight_gradients_of_mixed_sizes_equal_single_launches():
     """One problem of a group beyond the pipelined kernels' 32-bit operand offsets takes the predicated
     kernel alone: the others run as they do by themselves (here with a split reduction), bit for bit."""

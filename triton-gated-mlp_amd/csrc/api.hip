@@ -995,25 +995,17 @@ struct BwdWorkspace {
   size_t colsum = 0;  // gmlp_colsum_grouped
   size_t total() const { return std::max(act, std::max(dw, colsum)); }
 };
-BwdWorkspace plan_bwd_workspace(int64_t M, int64_t K, int64_t N, int dtype, bool gate, bool up, bool down,
-                                bool bias_gate, bool bias_up, bool bias_down) {
+BwdWorkspace plan_bwd_workspace(int64_t M, int64_t K, int64_t N, int dtype, bool hidden, bool dx, bool gate, bool up,
+                                bool down, bool bias_gate, bool bias_up, bool bias_down) {
   BwdWorkspace w;
-  const size_t dh = gmlp_workspace_bytes(GMLP_OP_DH_BWD, M, K, N, dtype);
-  const size_t dx = gmlp_workspace_bytes(GMLP_OP_DX_BWD, M, K, N, dtype);
-  w.act = dh > dx ? dh : dx;
+  if (hidden) w.act = gmlp_workspace_bytes(GMLP_OP_DH_BWD, M, K, N, dtype);
+  if (dx) w.act = std::max(w.act, gmlp_workspace_bytes(GMLP_OP_DX_BWD, M, K, N, dtype));
   int64_t R[3], C[3];
   int n = 0;
   if (gate) { R[n] = N; C[n] = K; ++n; }
   if (up) { R[n] = N; C[n] = K; ++n; }
   if (down) { R[n] = K; C[n] = N; ++n; }
   if (n > 0) w.dw = gmlp_dw_bwd_grouped_workspace_bytes(n, M, R, C, dtype);
-  // without stream-K a problem that takes the single-launch path may still ask for its own
-  if (n > 0 && w.dw == 0) {
-    for (int i = 0; i < n; ++i) {
-      const size_t one = gmlp_workspace_bytes(GMLP_OP_DW_BWD, M, R[i], C[i], dtype);
-      if (one > w.dw) w.dw = one;
-    }
-  }
   if (bias_gate) w.colsum += gmlp::colsum_workspace_bytes(M, N);
   if (bias_up) w.colsum += gmlp::colsum_workspace_bytes(M, N);
   if (bias_down) w.colsum += gmlp::colsum_workspace_bytes(M, K);
@@ -1031,7 +1023,7 @@ size_t gmlp_mlp_workspace_bytes(int pass, int64_t M, int64_t K, int64_t N, int d
     const size_t b = gmlp_workspace_bytes(GMLP_OP_LINEAR_FWD, M, N, K, dtype);
     return a > b ? a : b;
   }
-  if (pass == GMLP_PASS_BWD) return plan_bwd_workspace(M, K, N, dtype, true, true, true, true, true, true).total();
+  if (pass == GMLP_PASS_BWD) return plan_bwd_workspace(M, K, N, dtype, true, true, true, true, true, true, true, true).total();
   return 0;
 }
 
@@ -1085,7 +1077,7 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
   GMLP_REQUIRE_ALIGNED(dw_up); GMLP_REQUIRE_ALIGNED(dw_down); GMLP_REQUIRE_ALIGNED(db_gate); GMLP_REQUIRE_ALIGNED(db_up);
   GMLP_REQUIRE_ALIGNED(db_down); GMLP_REQUIRE_ALIGNED(workspace);
 
-  const BwdWorkspace need = plan_bwd_workspace(M, K, N, dtype, dw_gate, dw_up, dw_down, db_gate, db_up, db_down);
+  const BwdWorkspace need = plan_bwd_workspace(M, K, N, dtype, hidden, dx, dw_gate, dw_up, dw_down, db_gate, db_up, db_down);
   // Every launch gets the caller's buffer when it is large enough for that launch, and none
   // otherwise (same results from the plain form of the launch).  Bias gradients cannot do without.
   auto fits = [&](size_t bytes) { return workspace != nullptr && bytes > 0 && bytes <= workspace_bytes; };

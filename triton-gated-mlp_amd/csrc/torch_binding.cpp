@@ -266,6 +266,22 @@ struct MlpBackward : public ag::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     for (ag::SavedVariable* v : {&x_, &Wg_, &Wu_, &Wd_, &acts_, &bg_, &bu_}) v->reset_data();
   }
+  // What the launches for the gradients asked for use, one after the other: some of the weight gradients by
+  // themselves may take more than all three together (fewer tiles, more splits).
+  size_t workspace_of(const ag::variable_list& out) const {
+    const bool hidden = out[0].defined() || out[1].defined() || out[2].defined() || out[3].defined() || out[4].defined();
+    size_t bytes = hidden ? lib.gmlp_workspace_bytes(GMLP_OP_DH_BWD, q.M, q.K, q.N, q.code) : 0;
+    if (out[0].defined()) bytes = std::max(bytes, lib.gmlp_workspace_bytes(GMLP_OP_DX_BWD, q.M, q.K, q.N, q.code));
+    int64_t R[3], C[3];
+    int n = 0;
+    for (int i = 1; i <= 5; i += 2)
+      if (out[i].defined()) R[n] = i < 5 ? q.N : q.K, C[n] = i < 5 ? q.K : q.N, ++n;
+    if (n > 0) bytes = std::max(bytes, lib.gmlp_dw_bwd_grouped_workspace_bytes(n, q.M, R, C, q.code));
+    size_t sums = 0;
+    for (int i = 2; i <= 6; i += 2)
+      if (out[i].defined()) sums += lib.gmlp_workspace_bytes(GMLP_OP_COLSUM, q.M, 0, i < 6 ? q.N : q.K, q.code);
+    return std::max(bytes, sums);
+  }
   ag::variable_list apply(ag::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     ag::variable_list out(7);
@@ -303,7 +319,7 @@ struct MlpBackward : public ag::Node {
     const Activations a(q, kept, true);
     // dG, dU and the library's workspace share one scratch allocation that is dropped on return
     const size_t plane = ((size_t)(q.M * q.N) * dy.element_size() + 255) / 256 * 256;
-    const size_t bytes = lib.gmlp_mlp_workspace_bytes(GMLP_PASS_BWD, q.M, q.K, q.N, q.code);
+    const size_t bytes = workspace_of(out);
     const Tensor arena = scratch(2 * plane + bytes, x);
     char* const base = (char*)out_ptr(arena);
     check(lib.gmlp_mlp_bwd(ptr(dy), ptr(x), ptr(Wg), ptr(Wu), ptr(Wd), a.g, a.u, a.h, base, base + plane, out_ptr(out[0]),

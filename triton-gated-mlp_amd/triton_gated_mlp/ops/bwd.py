@@ -243,6 +243,30 @@ def colsum_grouped(arrays):
     return outs
 
 
+def _mlp_bwd_workspace_bytes(M: int, K: int, N: int, code: int, need) -> int:
+    """What mlp_bwd's launches for the gradients in `need` use, one after the other: some of the weight
+    gradients by themselves may take more than all three together (fewer tiles, more splits)."""
+    import ctypes
+
+    lib = _cabi.lib()
+    dx, dwg, dbg, dwu, dbu, dwd, dbd = need
+    sizes = [0]
+    if any(need[:5]):
+        sizes.append(lib.gmlp_workspace_bytes(_cabi.GMLP_OP_DH_BWD, M, K, N, code))
+    if dx:
+        sizes.append(lib.gmlp_workspace_bytes(_cabi.GMLP_OP_DX_BWD, M, K, N, code))
+    problems = [p for p, wanted in (((N, K), dwg), ((N, K), dwu), ((K, N), dwd)) if wanted]
+    if problems:
+        I64Arr = ctypes.c_int64 * len(problems)
+        R, C = (I64Arr(*dims) for dims in zip(*problems))
+        sizes.append(lib.gmlp_dw_bwd_grouped_workspace_bytes(
+            len(problems), M, ctypes.cast(R, ctypes.c_void_p), ctypes.cast(C, ctypes.c_void_p), code
+        ))
+    sums = [c for c, wanted in ((N, dbg), (N, dbu), (K, dbd)) if wanted]
+    sizes.append(sum(lib.gmlp_workspace_bytes(_cabi.GMLP_OP_COLSUM, M, 0, c, code) for c in sums))
+    return max(sizes)
+
+
 def mlp_bwd(
     dy: Tensor,
     x: Tensor,
@@ -281,7 +305,7 @@ def mlp_bwd(
     outs = [torch.empty(s, dtype=dy.dtype, device=dev) if n else None for s, n in zip(shapes, need)]
     dx, dwg, dbg, dwu, dbu, dwd, dbd = outs
     with torch.cuda.device(dev):
-        nbytes = _cabi.mlp_workspace_bytes(_cabi.GMLP_PASS_BWD, M, K, N, code, dev)
+        nbytes = _mlp_bwd_workspace_bytes(M, K, N, code, need)
         plane = (M * N * dy.element_size() + 255) // 256 * 256
         arena = torch.empty((2 * plane + nbytes,), dtype=torch.uint8, device=dev)
         base = arena.data_ptr()
