@@ -93,8 +93,9 @@ int gmlp_init(void);
  * (M, K, N) as the entry point of that name takes them: GMLP_OP_COLSUM (M, 0, C),
  * GMLP_OP_LINEAR_FWD (M, R, C), GMLP_OP_DX_BWD (M, K, N), GMLP_OP_GATEUP_FWD (M, K, N),
  * GMLP_OP_DECODE_FWD (M, K, N), GMLP_OP_DH_BWD (M, K, N), GMLP_OP_DW_BWD (Mred, R, C),
- * GMLP_OP_DW_BWD_GROUPED (arguments ignored: an upper bound for any set of problems, 128 MiB on a
- * whole MI355X).  The values are enumerators, not flags: ask per operation; one buffer of the
+ * GMLP_OP_DW_BWD_GROUPED (sizes ignored: the most that stream-K takes for any set of problems, 128 MiB
+ * on a whole MI355X, and 0 for float32, which has none; split reductions may take more, see
+ * gmlp_dw_bwd_grouped_workspace_bytes).  The values are enumerators, not flags: ask per operation; one buffer of the
  * largest answer serves every call of a forward or backward pass (calls on one stream are ordered).
  * Two things use a workspace, and without one (NULL, 0) every entry point computes the same result
  * more slowly on the shapes concerned: split reductions for short batches (see gmlp_linear_fwd),
@@ -182,7 +183,9 @@ int gmlp_dw_bwd(const void* lhs, const void* rhs, void* dw, int64_t Mred, int64_
  * Same reference counterparts as gmlp_dw_bwd; one launch for dW_gate, dW_up and dW_down avoids
  * three partially filled last rounds of workgroups.
  * workspace (may be NULL): gmlp_dw_bwd_grouped_workspace_bytes(count, Mred, R, C, dtype) bytes (what
- * this set of problems uses, often 0), or, 16-bit types, the bound gmlp_workspace_bytes(GMLP_OP_DW_BWD_GROUPED, ...).
+ * this set of problems uses, often 0).  With less the fastest form that fits runs; 16-bit types: with
+ * gmlp_workspace_bytes(GMLP_OP_DW_BWD_GROUPED, ...) bytes that is the planned one unless the partial sums of
+ * its split reductions are larger (M=42136, K=120, N=23416: 1.26 times that size).
  */
 size_t gmlp_dw_bwd_grouped_workspace_bytes(int count, int64_t Mred, const int64_t* R, const int64_t* C,
                                            int dtype);

@@ -1389,6 +1389,37 @@ def test_some_weight_gradients_run_as_planned_for_them(M, K, N, dtype, trained):
         assert torch.equal(w.grad, a) and torch.equal(b, a)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(4100, 72, 200), (9000, 264, 520)])
+def test_grouped_weight_gradients_use_what_fits_of_a_smaller_workspace(M, K, N, dtype):
+    """A workspace that does not hold the planned partial sums is used for as many splits as it holds, never
+    beyond its end, and none is needed."""
+    import ctypes
+
+    from triton_gated_mlp import _cabi
+
+    dev, lib, code = _dev(), _cabi.lib(), _cabi.dtype_code(dtype)
+    g = torch.Generator(device=dev).manual_seed(15)
+    rnd = lambda *shape: torch.empty(shape, device=dev).normal_(generator=g).to(dtype)
+    pairs = [(rnd(M, N), rnd(M, K)), (rnd(M, N), rnd(M, K)), (rnd(M, K), rnd(M, N))]
+    outs = [torch.empty(a.shape[1], b.shape[1], device=dev, dtype=dtype) for a, b in pairs]
+    array = lambda kind, values: ctypes.cast((kind * 3)(*values), ctypes.c_void_p)
+    lhs, rhs, dws = (array(ctypes.c_void_p, [t.data_ptr() for t in ts]) for ts in (*zip(*pairs), outs))
+    R, C = array(ctypes.c_int64, [N, N, K]), array(ctypes.c_int64, [K, K, N])
+    need = lib.gmlp_dw_bwd_grouped_workspace_bytes(3, M, R, C, code)
+    one_split = 4 * 3 * N * K
+    assert need >= 4 * one_split and need % one_split == 0
+    for nbytes in (need, need - one_split, need // 2, 2 * one_split, 2 * one_split - 16, 0):
+        buffer = torch.full((need,), 0xA5, device=dev, dtype=torch.uint8)
+        _cabi.check(lib.gmlp_dw_bwd_grouped(
+            3, lhs, rhs, dws, M, R, C, code, buffer.data_ptr() if nbytes else None, nbytes, _cabi.stream_ptr(dev)))
+        assert (buffer[nbytes:] == 0xA5).all(), nbytes
+        used = nbytes - int((buffer[:nbytes] == 0xA5).all()) * nbytes
+        assert (used > 0) == (nbytes >= 2 * one_split), nbytes
+        for (a, b), dw in zip(pairs, outs):
+            _close(f"dW with {nbytes} of {need} bytes", dw, a.float().T @ b.float())
+
+
 def test_grouped_weight_gradients_of_mixed_sizes_equal_single_launches():
     """One problem of a group beyond the pipelined kernels' 32-bit operand offsets takes the predicated
     kernel alone: the others run as they do by themselves (here with a split reduction), bit for bit."""

@@ -119,6 +119,8 @@ int num_xcd() {
 // The GEMMs of a gated MLP (operand layouts, epilogues: launch.hpp).
 enum GemmKind { GATEUP, LINEAR, DH, DX, DW };
 
+const int64_t kMaxSplits = 16;
+
 // How a GEMM runs: tile class, and number of workgroups that share an output tile, each reducing a
 // contiguous range of reduction tiles (1: no split).
 struct GemmPlan {
@@ -138,7 +140,7 @@ struct GemmPlan {
 // unsplit, 64x64 126, with 13 splits 85.  A split reduction (64x64 tiles, at least 4 reduction tiles
 // each) pays a second launch and the partial sums' round trip through the caches.
 GemmPlan plan_f32(int64_t tiles128, int64_t tiles64x128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes,
-                 bool may_split) {
+                 int64_t max_splits) {
   static const double rate[3][3] = {{0.87, 0.88, 0.88}, {0.75, 0.78, 0.85}, {0.65, 0.76, 0.81}};  // by class, workgroups per CU
   GemmPlan best = {gmlp::TILE_F32_128, 1, 1e30};
   const int64_t cus = num_cu();
@@ -153,14 +155,13 @@ GemmPlan plan_f32(int64_t tiles128, int64_t tiles64x128, int64_t tiles64, int64_
   consider(gmlp::TILE_F32_128, tiles128, 4, 1);
   if (sets == 1) consider(gmlp::TILE_F32_64X128, tiles64x128, 2, 1);
   consider(gmlp::TILE_F32_64, tiles64, sets, 1);
-  if (may_split)
-    for (int64_t s = 2; s <= 16 && s * 4 <= red_tiles; ++s) consider(gmlp::TILE_F32_64, tiles64, sets, s);
+  for (int64_t s = 2; s <= max_splits && s * 4 <= red_tiles; ++s) consider(gmlp::TILE_F32_64, tiles64, sets, s);
   return best;
 }
-GemmPlan plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int sets, bool may_split) {
+GemmPlan plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int sets, int64_t max_splits) {
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q; };
   return plan_f32(up(rows, 128) * up(cols, 128 / sets), up(rows, 64) * up(cols, 128), up(rows, 64) * up(cols, 64),
-                  red_tiles, sets, (double)rows * (double)cols * 4.0, may_split);
+                  red_tiles, sets, (double)rows * (double)cols * 4.0, max_splits);
 }
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -256,11 +257,11 @@ double launch_us(const TileCost& c, int kind, int64_t tiles, int64_t kt, int spl
 }
 
 // The classes and splits for a grid of this many tiles of each class (`wide`, `tall` 0: not built).  At
-// least 4 reduction tiles per split, at most 16 splits.
-GemmPlan cheapest(int kind, int64_t large, int64_t wide, int64_t tall, int64_t medium, int64_t kt, double out_elements, bool may_split) {
+// least 4 reduction tiles per split, at most max_splits splits.
+GemmPlan cheapest(int kind, int64_t large, int64_t wide, int64_t tall, int64_t medium, int64_t kt, double out_elements, int64_t max_splits) {
   GemmPlan best = {gmlp::TILE_LARGE, 1, launch_us(kLarge, kind, large, kt, 1, out_elements)};
   auto consider = [&](const TileCost& c, int64_t tiles) {
-    const int64_t most = may_split && c.tile_class != gmlp::TILE_TALL ? std::max<int64_t>(1, std::min<int64_t>(16, kt / 4)) : 1;
+    const int64_t most = c.tile_class != gmlp::TILE_TALL ? std::max<int64_t>(1, std::min(max_splits, kt / 4)) : 1;
     for (int64_t s = 1; s <= most; ++s) {
       if (s > 1 && cdiv(kt, cdiv(kt, s)) != s) continue;  // rounding up would leave splits empty
       const double us = launch_us(c, kind, tiles, kt, (int)s, out_elements);
@@ -305,7 +306,7 @@ GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red,
   if (dtype == GMLP_F32) {
     // (the down projection of float32 modules asks for no workspace; callers rely on that)
     const int64_t segments = kind == DX ? 2 : 1, tiles = segments * cdiv(red, 32);
-    GemmPlan p = plan_f32(rows, cols, tiles, kind == GATEUP ? 2 : 1, may_split && kind != LINEAR);
+    GemmPlan p = plan_f32(rows, cols, tiles, kind == GATEUP ? 2 : 1, may_split && kind != LINEAR ? kMaxSplits : 1);
     p.splits = (int)cdiv(tiles, cdiv(tiles, p.splits));  // drop the splits that rounding up leaves empty
     return p;
   }
@@ -319,7 +320,7 @@ GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red,
   const int64_t kt = red_tiles_of(kind, red), large = tiles_of(kLarge, kind, rows, cols);
   const double out = (double)rows * (double)cols * (kind == GATEUP ? 2 : 1);
   GemmPlan p = cheapest(kind, large, kind == DW ? 0 : tiles_of(kWide, kind, rows, cols), tall(rows, cols),
-                        tiles_of(kMedium, kind, rows, cols), kt, out, may_split);
+                        tiles_of(kMedium, kind, rows, cols), kt, out, may_split ? kMaxSplits : 1);
   if (p.tile_class == gmlp::TILE_LARGE) return p;
   // large tiles whose thin last round is shared out (stream-K) or run by other tiles may still be ahead
   const int64_t cus = num_cu(), whole = whole_rounds(kind, rows, cols);
@@ -332,7 +333,7 @@ GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red,
     const int64_t r = kind <= LINEAR ? rows : rows - whole * 256, c = kind <= LINEAR ? cols - whole * tile_cols(kind) : cols;
     us = launch_us(kLarge, kind, large / cus * cus, kt, 1, out) +
          cheapest(kind, tiles_of(kLarge, kind, r, c), tiles_of(kWide, kind, r, c), tall(r, c),
-                  tiles_of(kMedium, kind, r, c), kt, 0, false).us;
+                  tiles_of(kMedium, kind, r, c), kt, 0, 1).us;
   }
   return us < p.us ? GemmPlan{gmlp::TILE_LARGE, 1, us} : p;
 }
@@ -354,9 +355,16 @@ GemmPlan plan_gemm(int dtype, int kind, int64_t rows, int64_t cols, int64_t red,
   return e.plan;
 }
 
+// Splits whose partial sums of `out_bytes` each fit a workspace.
+int64_t splits_that_fit(size_t workspace_bytes, double out_bytes) {
+  const double n = (double)workspace_bytes / out_bytes;
+  return n < 1.0 ? 1 : n < (double)kMaxSplits ? (int64_t)n : kMaxSplits;
+}
+
 // Weight gradients of float32 modules: all problems in one grid, on one tile class with one number of
-// splits; the problems' partial sums follow each other in the workspace.
-GemmPlan plan_dw_group_f32(int count, int64_t Mred, const int64_t* R, const int64_t* C) {
+// splits; the problems' partial sums follow each other in the workspace.  (workspace_bytes: plan for
+// what a workspace of that size can hold.)
+GemmPlan plan_dw_group_f32(int count, int64_t Mred, const int64_t* R, const int64_t* C, size_t workspace_bytes = SIZE_MAX) {
   int64_t t128 = 0, t64x128 = 0, t64 = 0;
   double out_bytes = 0;
   for (int i = 0; i < count; ++i) {
@@ -365,7 +373,7 @@ GemmPlan plan_dw_group_f32(int count, int64_t Mred, const int64_t* R, const int6
     t64 += cdiv(R[i], 64) * cdiv(C[i], 64);
     out_bytes += (double)R[i] * (double)C[i] * 4.0;
   }
-  GemmPlan p = plan_f32(t128, t64x128, t64, cdiv(Mred, 32), 1, out_bytes, true);
+  GemmPlan p = plan_f32(t128, t64x128, t64, cdiv(Mred, 32), 1, out_bytes, splits_that_fit(workspace_bytes, out_bytes));
   const int64_t per = cdiv(cdiv(Mred, 32), p.splits);
   p.splits = (int)cdiv(cdiv(Mred, 32), per);  // drop the splits that rounding up leaves empty
   return p;
@@ -383,12 +391,13 @@ int64_t dw_group_tiles(const TileCost& c, int count, const int64_t* R, const int
   for (int i = 0; i < count; ++i) n += tiles_of(c, DW, R[i], C[i]);
   return n;
 }
-GemmPlan plan_dw_group(int count, int64_t Mred, const int64_t* R, const int64_t* C) {
+GemmPlan plan_dw_group(int count, int64_t Mred, const int64_t* R, const int64_t* C, size_t workspace_bytes = SIZE_MAX) {
   double out = 0;
   for (int i = 0; i < count; ++i) out += (double)R[i] * (double)C[i];
   const int64_t large = dw_group_tiles(kLarge, count, R, C), kt = cdiv(Mred, 64);
-  GemmPlan p = cheapest(DW, large, 0, 0, dw_group_tiles(kMedium, count, R, C), kt, out, true);
-  if (p.tile_class != gmlp::TILE_LARGE && plan_streamk(GMLP_F16, large, kt, false).tiles > 0) {
+  GemmPlan p = cheapest(DW, large, 0, 0, dw_group_tiles(kMedium, count, R, C), kt, out, splits_that_fit(workspace_bytes, 4.0 * out));
+  const StreamK sk = plan_streamk(GMLP_F16, large, kt, false);
+  if (p.tile_class != gmlp::TILE_LARGE && sk.tiles > 0 && sk.ws_bytes <= workspace_bytes) {
     const double us = streamk_us(DW, large, kt, out);
     if (us < p.us) p = GemmPlan{gmlp::TILE_LARGE, 1, us};
   }
@@ -483,9 +492,9 @@ int gmlp_init(void) {
 }
 
 size_t gmlp_workspace_bytes(int op, int64_t M, int64_t K, int64_t N, int dtype) {
-  // gmlp_dw_bwd_grouped: any set of problems (the plan depends on all of them together): the most
-  // a plan can take, a slot per compute unit for the shared-out tiles and for the workgroups
-  // (float32: gmlp_dw_bwd_grouped_workspace_bytes knows what its split reductions use)
+  // gmlp_dw_bwd_grouped, any set of problems (the plan depends on all of them together): the most that
+  // shared-out tiles can take, a slot per compute unit for them and one for the workgroups.  Split reductions
+  // of long batches can take more, see gmlp_dw_bwd_grouped_workspace_bytes.
   if (op == GMLP_OP_DW_BWD_GROUPED) return dtype == GMLP_F32 ? 0 : (size_t)2 * num_cu() * 65536 * sizeof(float);
   if (M < 1 || N < 1) return 0;
   if (op == GMLP_OP_COLSUM) return gmlp::colsum_workspace_bytes(M, N);
@@ -768,8 +777,12 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
       const typename EpiStore<T>::Args ea = {(T*)dw[0], nullptr, (int)C[0]};
       return launch_dw<T>(TILE_MEDIUM, ga, ea, s);
     }));
-  GemmPlan plan = dtype == GMLP_F32 ? plan_dw_group_f32(count, Mred, R, C) : plan_dw_group(count, Mred, R, C);
-  if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < dw_group_split_bytes(count, plan.splits, R, C))) plan.splits = 1;
+  auto plan_group = [&](size_t bytes) {
+    return dtype == GMLP_F32 ? plan_dw_group_f32(count, Mred, R, C, bytes) : plan_dw_group(count, Mred, R, C, bytes);
+  };
+  GemmPlan plan = plan_group(SIZE_MAX);
+  if (plan.splits > 1 && (workspace == nullptr || workspace_bytes < dw_group_split_bytes(count, plan.splits, R, C)))
+    plan = plan_group(workspace == nullptr ? 0 : workspace_bytes);
   if (dtype == GMLP_F32 || plan.splits > 1) {
     return hip_result(__func__, by_dtype(dtype, [&](auto tag) -> hipError_t {
       typedef decltype(tag) T;
