@@ -1466,51 +1466,89 @@ def test_decode_matches_general_path(dtype):
         _close(f"general Y M={M}", y_general, ref["Y"])
 
 
-@pytest.mark.parametrize(
-    "M,K,N",
-    [
-        (1, 776, 1032),      # least widths, one 16-byte piece in the last chunk of 256 and of 128
-        (3, 2200, 4608),     # tail in one operand only
-        (16, 4096, 4104),    # the other one; full tile of tokens
-        (11, 4496, 9472),    # H in fragment order; more than 16 rows of W_down per compute unit
-        (17, 1016, 888),     # two token tiles, last chunks short by one piece
-        (24, 4104, 1160),    # 32-row blocks of everything
-        (20, 2056, 8200),
-        (7, 5192, 1160),     # misaligned rows, 32-row blocks of W_down, one token tile
-        (29, 5192, 1160),    # and two
-        (32, 12568, 1032),   # 64-row blocks of W_down
-        (18, 12544, 1280),   # the same without tails
-    ],
-)
-def test_decode_streaming_kernels_at_any_width(M, K, N):
+# Streaming kernels by (16-row regions per matrix, token tiles, bytes of a row per stage); what a case names
+# is what its launches are held to.  K and N with a row tail unless marked: of 512-byte stages a width that
+# is not a multiple of 256 elements, of 256-byte ones (rows of whole 128-byte lines only) 64 mod 128.
+_DECODE_CASES = [
+    # M, K, N, gate/up, down
+    (1, 776, 1032, (1, 1, 512), (1, 1, 512)),      # least widths, one 16-byte piece in the last chunk of each
+    (3, 2200, 4608, (1, 1, 512), (1, 1, 512)),     # no tail in the down projection
+    (16, 4096, 4104, (2, 1, 256), (1, 1, 512)),    # none in gate/up; full tile of tokens
+    (11, 4496, 9472, (1, 1, 512), (2, 1, 256)),    # H in fragment order; no tail in the down projection
+    (17, 1016, 888, (1, 2, 512), (1, 2, 512)),     # last chunks short by one piece
+    (24, 4104, 1160, (1, 2, 512), (2, 2, 512)),
+    (20, 2056, 8200, (1, 2, 512), (1, 2, 512)),
+    (7, 5192, 1160, (1, 1, 512), (2, 1, 512)),
+    (29, 5192, 1160, (1, 2, 512), (2, 2, 512)),
+    (32, 12568, 1032, (1, 2, 512), (2, 2, 512)),
+    (18, 12544, 1280, (1, 2, 512), (4, 2, 256)),   # no tails
+    (12, 1088, 4160, (2, 1, 256), (1, 1, 512)),
+    (12, 4160, 1088, (1, 1, 512), (2, 1, 256)),
+    (24, 4160, 4160, (2, 2, 256), (2, 2, 256)),
+    (24, 4160, 1088, (2, 2, 256), (2, 2, 256)),
+    (18, 12352, 1088, (1, 2, 512), (4, 2, 256)),
+]
+
+
+def _decode_tails():
+    width = lambda kernel: kernel[2] // 2
+    return {("gate/up", g) for _, K, _, g, _ in _DECODE_CASES if K % width(g)} | {
+        ("down", d) for _, _, N, _, d in _DECODE_CASES if N % width(d)}
+
+
+@pytest.mark.parametrize("bias", [True, False], ids=["biases", "plain"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("M,K,N,gated,down", _DECODE_CASES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_decode_streaming_kernels_at_any_width(M, K, N, gated, down, dtype, bias):
     """Streaming kernels whose last chunk of a row is partly beyond it, where the next row begins with
-    large values, against float64 products; twice, bit-identical."""
+    large values, against float64 products; twice, bit-identical, the second time with the launched kernels'
+    names (on a whole MI355X: the choice goes by rows per compute unit)."""
+    import re
+
+    from torch.profiler import ProfilerActivity, profile
     from triton_gated_mlp import _cabi
 
     dev = _dev()
-    print(f"decode, any width: M={M} K={K} N={N}", flush=True)
-    g = torch.Generator().manual_seed(21)
-    rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g)).half().to(dev)
+    print(f"decode, any width: M={M} K={K} N={N} {dtype} bias={bias}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(21)
+    rnd = lambda *shape, s=1.0: torch.empty(shape, device=dev).normal_(0.0, s, generator=g).to(dtype)
     x, wg, wu, wd = rnd(M, K, s=0.5), rnd(N, K, s=0.02), rnd(N, K, s=0.02), rnd(K, N, s=0.02)
-    bg, bu, bd = rnd(N, s=0.1), rnd(N, s=0.1), rnd(K, s=0.1)
+    bg, bu, bd = (rnd(N, s=0.1), rnd(N, s=0.1), rnd(K, s=0.1)) if bias else (None, None, None)
     x[:, :8] *= 16
     for w in (wg, wu, wd):
         w[:, :8] *= 16
 
     def run():
-        h = torch.full((16 if M <= 16 else 32, N), float("nan"), dtype=x.dtype, device=dev)
-        y = torch.full((M, K), float("nan"), dtype=x.dtype, device=dev)
+        h = torch.full((16 if M <= 16 else 32, N), float("nan"), dtype=dtype, device=dev)
+        y = torch.full((M, K), float("nan"), dtype=dtype, device=dev)
         _cabi.check(_cabi.lib().gmlp_decode_stream_fwd(
-            *(t.data_ptr() for t in (x, wg, wu, wd, bg, bu, bd, h, y)), M, K, N, _cabi.dtype_code(x.dtype),
+            *(_cabi.ptr(t) for t in (x, wg, wu, wd, bg, bu, bd, h, y)), M, K, N, _cabi.dtype_code(dtype),
             _cabi.act_code("silu"), _cabi.stream_ptr(dev)))
         return y
 
     y = run()
-    d = lambda t: t.double()
+    d = lambda t: 0.0 if t is None else t.double()
     hidden = torch.nn.functional.silu(d(x) @ d(wg).T + d(bg)) * (d(x) @ d(wu).T + d(bu))
-    ref = hidden.half().double() @ d(wd).T + d(bd)
+    ref = hidden.to(dtype).double() @ d(wd).T + d(bd)
     _close("Y", y, ref)
-    assert torch.equal(y, run())
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as prof:
+        again = run()
+        torch.cuda.synchronize()
+    assert torch.equal(y, again)
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        # (names come mangled or, bfloat16's, halfway demangled)
+        name = r"decode_stream_kernel.*?(?:ELi|, )(\d+)(?:ELi|, )(\d+)(?:ELi|, )(\d+)(?:ELi|, )\d+(?:ELb|, )(0|1|false|true)"
+        found = [m.groups() for m in (re.search(name, e.name) for e in prof.events()) if m]
+        launched = [(*map(int, g[:3]), g[3] in ("1", "true")) for g in found]
+        tail = lambda kernel, red: red % (kernel[2] // 2) != 0
+        assert launched == [(*gated, tail(gated, K)), (*down, tail(down, N))], launched
+
+
+def test_decode_cases_cover_every_row_tail():
+    """Every block shape that launch_decode_stream chooses among occurs with a row tail."""
+    assert _decode_tails() == {("gate/up", (h, t, s)) for h, s in ((1, 512), (2, 256)) for t in (1, 2)} | {
+        ("down", k) for k in ((1, 1, 512), (2, 1, 256), (2, 1, 512), (1, 2, 512), (2, 2, 256), (2, 2, 512), (4, 2, 256))}
 
 
 def test_decode_streaming_entry_refuses_what_its_kernels_do_not_take():
