@@ -13,8 +13,10 @@
 #include <ATen/ops/empty.h>
 #include <ATen/ops/zeros.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -125,8 +127,13 @@ Problem problem_of(const Tensor& x, const Tensor& W_up, int code, int64_t act) {
 }
 
 // None of the operators has a forward-mode derivative: a dual input would come out without its tangent
-// (also where reverse mode records nothing: torch.no_grad() leaves forward mode on).
-void refuse_forward_ad(std::initializer_list<std::reference_wrapper<const Tensor>> tensors) {
+// (also where reverse mode records nothing: torch.no_grad() leaves forward mode on).  Nor rules for
+// functorch: refused as torch.autograd.Function does for an operator without rules of its own.
+void refuse_transforms(const char* name, std::initializer_list<std::reference_wrapper<const Tensor>> tensors) {
+  // (the key is included while a transform is active)
+  TORCH_CHECK(!c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode), name,
+              " does not support functorch transforms (vmap, grad, jvp, jacrev, ...)");
+  if (ag::ForwardADLevel::try_get_by_idx(0) == nullptr) return;  // outside forward mode nothing is dual
   for (const Tensor& t : tensors)
     TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(/*level=*/0).defined(),
                                 "the fused gated-MLP operators have no forward-mode derivative");
@@ -221,8 +228,8 @@ Problem check_mlp(const Tensor& x, const Tensor& W_gate, const Tensor& b_gate, c
 
 Tensor mlp_infer(const Tensor& x_in, const Tensor& Wg_in, const OptTensor& bg_in, const Tensor& Wu_in, const OptTensor& bu_in,
                  const Tensor& Wd_in, const OptTensor& bd_in, int64_t act) {
+  refuse_transforms("FusedGatedMLP", {x_in, Wg_in, or_undefined(bg_in), Wu_in, or_undefined(bu_in), Wd_in, or_undefined(bd_in)});
   const Problem q = check_mlp(x_in, Wg_in, or_undefined(bg_in), Wu_in, or_undefined(bu_in), Wd_in, or_undefined(bd_in), act);
-  refuse_forward_ad({x_in, Wg_in, or_undefined(bg_in), Wu_in, or_undefined(bu_in), Wd_in, or_undefined(bd_in)});
   at::AutoDispatchBelowADInplaceOrView below;
   const c10::DeviceGuard guard(x_in.device());
   const Tensor x = x_in.contiguous(), Wg = Wg_in.contiguous(), Wu = Wu_in.contiguous(), Wd = Wd_in.contiguous();
@@ -335,8 +342,8 @@ Tensor mlp_train(const Tensor& x_in, const Tensor& Wg_in, const OptTensor& bg_in
                  const Tensor& Wd_in, const OptTensor& bd_in, double p, uint64_t seed, uint64_t offset, bool recompute,
                  int64_t act) {
   const Tensor &bg_o = or_undefined(bg_in), &bu_o = or_undefined(bu_in), &bd_o = or_undefined(bd_in);
+  refuse_transforms("FusedGatedMLPFullFunction", {x_in, Wg_in, bg_o, Wu_in, bu_o, Wd_in, bd_o});
   Problem q = check_mlp(x_in, Wg_in, bg_o, Wu_in, bu_o, Wd_in, bd_o, act);
-  refuse_forward_ad({x_in, Wg_in, bg_o, Wu_in, bu_o, Wd_in, bd_o});
   q.p = p;
   q.seed = seed;
   q.offset = offset;
@@ -454,10 +461,10 @@ struct HiddenBackward : public ag::Node {
 Tensor hidden(const Tensor& x_in, const Tensor& Wu_in, const OptTensor& bu_in, const Tensor& Wg_in, const OptTensor& bg_in,
               double p, uint64_t seed, uint64_t offset, int64_t act) {
   const Tensor &bu_o = or_undefined(bu_in), &bg_o = or_undefined(bg_in);
+  refuse_transforms("FusedGatedMLPFunction", {x_in, Wg_in, bg_o, Wu_in, bu_o});
   TORCH_CHECK_VALUE(x_in.dim() == 2, "input tensor must be 2-D [M, K], got ", x_in.dim(), " dims");
   check_gate_up(x_in, Wg_in, bg_o, Wu_in, bu_o);
   Problem q = problem_of(x_in, Wu_in, require_gpu({x_in, Wg_in, bg_o, Wu_in, bu_o}), act);
-  refuse_forward_ad({x_in, Wg_in, bg_o, Wu_in, bu_o});
   q.p = p;
   q.seed = seed;
   q.offset = offset;

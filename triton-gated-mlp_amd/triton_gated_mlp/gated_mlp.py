@@ -114,12 +114,6 @@ def eager_bwd(x: Tensor, W_up: Tensor, W_gp: Tensor, grad_output: Tensor):
 _U64 = (1 << 64) - 1
 
 
-def _refuse_functorch(operator: str) -> None:
-    # as torch.autograd.Function does for an operator without rules of its own
-    if torch._C._are_functorch_transforms_active():
-        raise RuntimeError(f"{operator} does not support functorch transforms (vmap, grad, jvp, jacrev, ...)")
-
-
 class FusedGatedMLPFunction(Function):
     """Hidden-state operator hidden = dropout(act_fn(x·W_gpᵀ+b_gp) * (x·W_upᵀ+b_up)).
 
@@ -133,7 +127,6 @@ class FusedGatedMLPFunction(Function):
         x: Tensor, W_up: Tensor, b_up: Optional[Tensor], W_gp: Tensor, b_gp: Optional[Tensor], dropout_p: float = 0.0,
         seed: int = 0, offset: int = 0, act_fn: str = "silu",
     ) -> Tensor:
-        _refuse_functorch("FusedGatedMLPFunction")
         return _cabi.torch_binding().hidden(
             x, W_up, b_up, W_gp, b_gp, float(dropout_p), int(seed) & _U64, int(offset) & _U64, _cabi.act_code(act_fn)
         )
@@ -150,7 +143,6 @@ class FusedGatedMLPFullFunction(Function):
         x: Tensor, W_gate: Tensor, b_gate: Optional[Tensor], W_up: Tensor, b_up: Optional[Tensor], W_down: Tensor,
         b_down: Optional[Tensor], dropout_p: float, seed: int, offset: int, recompute: bool = False, act_fn: str = "silu",
     ) -> Tensor:
-        _refuse_functorch("FusedGatedMLPFullFunction")
         return _cabi.torch_binding().mlp_train(
             x, W_gate, b_gate, W_up, b_up, W_down, b_down, float(dropout_p), int(seed) & _U64, int(offset) & _U64,
             bool(recompute), _cabi.act_code(act_fn),
@@ -226,10 +218,9 @@ class FusedGatedMLP(_GatedMLPBase):
             ).reshape(x.shape)
         W_gate, b_gate, W_up, b_up, W_down, b_down = params
         graph = torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in params))
-        if not graph and p == 0.0 and not torch.jit.is_tracing():
+        if not graph and p == 0.0 and not torch._C._is_tracing():
             # Nothing to differentiate: the weight-streaming kernels for skinny M, no autograd node.  (A trace
             # records the operator below either way, which makes this choice whenever it runs.)
-            _refuse_functorch("FusedGatedMLP")
             return _cabi.torch_binding().mlp_infer(
                 x, W_gate, b_gate, W_up, b_up, W_down, b_down, _cabi.act_code(self.act_fn)
             )
