@@ -233,8 +233,9 @@ int gmlp_colsum_grouped(int count, const void* const* a, void* const* out, void*
  * workspace: unused by the current kernels (gmlp_workspace_bytes(GMLP_OP_DECODE_FWD, ...) is 0): pass
  * NULL.  The argument is kept so that the signature does not change.  No dropout (inference).
  * Same math as EagerGatedMLP.forward in eval mode (src/triton_gated_mlp/gated_mlp.py:92-98).
- * Requires K % 32 == 0 and N % 256 == 0 (the LDS-ring streaming kernels run when K % 256 == 0 too,
- * K >= 768, N >= 768 and K*N < 2^30; 16 < M <= 32 is accepted only then).
+ * Requires K % 32 == 0 and N % 256 == 0; 16 < M <= 32 is accepted only with K % 256 == 0, K >= 768,
+ * N >= 768 and K*N < 2^30.  The LDS-ring streaming kernels run when K and N are at least 768 and K*N <
+ * 2^30, plainer ones otherwise.
  */
 int gmlp_decode_fwd(const void* x, const void* w_gate, const void* w_up, const void* w_down,
                     const void* b_gate, const void* b_up, const void* b_down, void* h_scratch,

@@ -170,8 +170,9 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // (tiles of all problems of a grouped launch together).  The tiles beyond the last whole round of
 // workgroups (one per compute unit) are shared out by reduction range when that beats running them
 // as a thinly filled round: a round filled to the fraction f costs about 0.6 + 0.4 f of a full one
-// (see pick_tile) against f with stream-K, plus the partial sums' round trip through memory and the
-// second launch (about 45 us, i.e. 30 reduction tiles' time): worth it when (1 - f) * kt > 50.
+// (kLarge has the later fit, 0.69 + 0.31 f) against f with stream-K, plus the partial sums' round trip
+// through memory and the second launch (about 45 us, i.e. 30 reduction tiles' time): worth it when
+// (1 - f) * kt > 50.
 // Every stream-K workgroup gets at least 8 reduction tiles.
 // A grid of less than one round that fills more than half of the chip is left alone unless its tiles
 // divide into whole pieces (`first_round`: false for the weight gradients, which keep the plan): even
@@ -237,9 +238,10 @@ struct TileCost {
 const TileCost kLarge = {gmlp::TILE_LARGE, 256, 1, 1, 0.69, 0, {1.443, 1.477, 1.494}, {11.4, 6.1, 19.0, 6.8, 7.1, 12.0}};
 const TileCost kWide = {gmlp::TILE_WIDE, 128, 1, 1, 0.74, 0, {0.846, 0.940, 0.983}, {5.7, 2.7, 9.7, 3.3, 3.7, 2.0}};
 // (TALL: fitted the same way to 160 launches, four GEMMs of 40 shapes, standard deviation 7 %; it is the
-// fastest unsplit class in 55 of them, by up to 27 %: gate/up at M=1357, K=1160, N=3096 41.6 -> 30.4 us,
-// M=1346, K=2264, N=8120 117 -> 103, dH at M=2048, K=2048, N=5632 62 -> 54, down at M=5717, K=1640,
-// N=6432 124 -> 110.  Split reductions are left to the smaller classes.)
+// fastest unsplit class in 55 of them, by up to 27 %.  bf16, back to back, without and with the class:
+// gate/up with biases, G and U kept, at M=1357, K=1160, N=3096 44.1 -> 35.3 us (gelu 44.1 -> 37.5, silu
+// without G and U 37.6 -> 28.8), M=1346, K=2264, N=8120 111 -> 106, dH at M=2048, K=2048, N=5632 60 -> 54,
+// down at M=5717, K=1640, N=6432 122 -> 110.  Split reductions are left to the smaller classes.)
 const TileCost kTall = {gmlp::TILE_TALL, 192, 1, 1, 0.72, 0, {1.101, 1.156, 0}, {9.2, 3.9, 16.2, 0.4, 0, 0}};
 const TileCost kMedium = {gmlp::TILE_MEDIUM_FULL, 128, 2, 2, 0.46, 0.30, {0.967, 0.983, 1.094}, {3.4, 0.6, 8.4, 0.2, 2.4, 0.1}};
 

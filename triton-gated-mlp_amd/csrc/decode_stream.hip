@@ -412,8 +412,8 @@ hipError_t launch_decode_stream(const T* x, const T* wg, const T* wu, const T* w
   const bool tall = ds_tall_gated(M, K, N, num_cu);
   // W_down: 32 rows of 128 elements a stage, four stages deep, once a CU's share exceeds 16 rows (K=5120,
   // N=13824, whole forward, against 32 rows of 256 three deep, or 64 of 128 from M = 21 up: M=1 72 -> 70
-  // us, M=16 80 -> 79, M=24 106 -> 98), 16 rows of 256 up to there (K=4096, N=11008, M=24, against 32
-  // half empty: 65 -> 64).  Two token tiles over 48 rows or more take 64 at a time: K=16384, N=53248, M=18
+  // us, M=16 80 -> 79, M=24 106 -> 98), 16 rows of 256 up to there (K=4096, N=11008, M=24: 64 us
+  // either way; 32 rows would be half empty).  Two token tiles over 48 rows or more take 64 at a time: K=16384, N=53248, M=18
   // 807 -> 783 us.  Misaligned rows take 256 elements at any height (K=6712, N=24104, M=1 188 -> 178).
   const bool one = K <= 16 * num_cu, lines = ds_whole_lines(N), four = K > 48 * num_cu && lines;
   if (M <= 16) {

@@ -328,7 +328,7 @@ hipError_t launch_gateup_split_kt<float, false>(int, const GemmArgs& ga, const E
 }
 template <>
 hipError_t launch_linear_split_kt<float, false>(int, const GemmArgs&, const EpiPartial<float>::Args&, hipStream_t) {
-  return hipErrorInvalidValue;  // the float32 down projection does not split (pick_splits_linear)
+  return hipErrorInvalidValue;  // the float32 down projection does not split (make_plan)
 }
 template <>
 hipError_t launch_dx_split_kt<float, false>(int, const GemmArgs& ga, const EpiPartial<float>::Args& ea, hipStream_t s) {
