@@ -273,8 +273,8 @@ int gmlp_decode_stream_fwd(const void* x, const void* w_gate, const void* w_up, 
  *   Every launch goes to `stream`, in that order.
  *
  * workspace: gmlp_mlp_workspace_bytes(GMLP_PASS_FWD or GMLP_PASS_BWD, M, K, N, dtype) bytes (may be
- * NULL or smaller for a pass without bias gradients: launches then take their plain form, with the
- * same results up to the order of fp32 additions; bias gradients need it and fail with GMLP_EINVAL
+ * NULL or smaller for a pass without bias gradients: launches then use what it holds, with the same
+ * results up to the order of fp32 additions; bias gradients need it and fail with GMLP_EINVAL
  * without).  GMLP_PASS_BWD answers for a pass that computes every gradient.  One or two of the weight
  * gradients by themselves may use more (fewer tiles, more splits); such a pass uses the largest of
  * gmlp_workspace_bytes of GMLP_OP_DH_BWD and GMLP_OP_DX_BWD, gmlp_dw_bwd_grouped_workspace_bytes of

@@ -1389,6 +1389,31 @@ def test_some_weight_gradients_run_as_planned_for_them(M, K, N, dtype, trained):
         assert torch.equal(w.grad, a) and torch.equal(b, a)
 
 
+def test_one_call_backward_hands_its_launches_whatever_workspace_there_is():
+    """gmlp_mlp_bwd for one weight gradient with the workspace of a pass that computes all three, which holds
+    some of its ten splits: the value of gmlp_dw_bwd with that workspace, not the one of an unsplit launch
+    (another order of additions)."""
+    from triton_gated_mlp import _cabi
+
+    dev, lib = _dev(), _cabi.lib()
+    M, K, N, code = 3776, 2720, 136, _cabi.GMLP_BF16
+    g = torch.Generator(device=dev).manual_seed(16)
+    rnd = lambda *shape: torch.empty(shape, device=dev).normal_(generator=g).bfloat16()
+    dy, x, wd, G, U = rnd(M, K), rnd(M, K), rnd(K, N) * 0.02, rnd(M, N), rnd(M, N)
+    dg, du, dw, alone, unsplit = rnd(M, N), rnd(M, N), rnd(N, K), rnd(N, K), rnd(N, K)
+    nbytes = lib.gmlp_mlp_workspace_bytes(_cabi.GMLP_PASS_BWD, M, K, N, code)
+    assert 2 * 4 * N * K <= nbytes < lib.gmlp_workspace_bytes(_cabi.GMLP_OP_DW_BWD, M, N, K, code)
+    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    p, stream = (lambda t: t.data_ptr()), _cabi.stream_ptr(dev)
+    _cabi.check(lib.gmlp_mlp_bwd(
+        p(dy), p(x), None, None, p(wd), p(G), p(U), None, p(dg), p(du), None, p(dw), None, None, None, None, None,
+        M, K, N, code, _cabi.act_code("silu"), 0.0, 0, 0, p(ws), nbytes, stream))
+    _cabi.check(lib.gmlp_dw_bwd(p(dg), p(x), p(alone), M, N, K, code, p(ws), nbytes, stream))
+    _cabi.check(lib.gmlp_dw_bwd(p(dg), p(x), p(unsplit), M, N, K, code, None, 0, stream))
+    assert torch.equal(dw, alone) and not torch.equal(dw, unsplit)
+    _close("dW_gate", dw, dg.float().T @ x.float())
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,K,N", [(4100, 72, 200), (9000, 264, 520)])
 def test_grouped_weight_gradients_use_what_fits_of_a_smaller_workspace(M, K, N, dtype):

@@ -1002,29 +1002,16 @@ int gmlp_dropout_mask(uint8_t* mask, int64_t M, int64_t N, float dropout_p, uint
 // ---------------------------------------------------------------- whole passes in one call
 namespace {
 
+size_t bias_workspace_bytes(int64_t M, int64_t K, int64_t N, bool gate, bool up, bool down) {
+  return (gate + up) * gmlp::colsum_workspace_bytes(M, N) + down * gmlp::colsum_workspace_bytes(M, K);
+}
+
 // Workspace of a backward pass: what its launches ask for, one after the other on one stream, so
 // one buffer of the largest request serves them all.
-struct BwdWorkspace {
-  size_t act = 0;     // gmlp_dh_bwd, then gmlp_dx_bwd
-  size_t dw = 0;      // gmlp_dw_bwd_grouped
-  size_t colsum = 0;  // gmlp_colsum_grouped
-  size_t total() const { return std::max(act, std::max(dw, colsum)); }
-};
-BwdWorkspace plan_bwd_workspace(int64_t M, int64_t K, int64_t N, int dtype, bool hidden, bool dx, bool gate, bool up,
-                                bool down, bool bias_gate, bool bias_up, bool bias_down) {
-  BwdWorkspace w;
-  if (hidden) w.act = gmlp_workspace_bytes(GMLP_OP_DH_BWD, M, K, N, dtype);
-  if (dx) w.act = std::max(w.act, gmlp_workspace_bytes(GMLP_OP_DX_BWD, M, K, N, dtype));
-  int64_t R[3], C[3];
-  int n = 0;
-  if (gate) { R[n] = N; C[n] = K; ++n; }
-  if (up) { R[n] = N; C[n] = K; ++n; }
-  if (down) { R[n] = K; C[n] = N; ++n; }
-  if (n > 0) w.dw = gmlp_dw_bwd_grouped_workspace_bytes(n, M, R, C, dtype);
-  if (bias_gate) w.colsum += gmlp::colsum_workspace_bytes(M, N);
-  if (bias_up) w.colsum += gmlp::colsum_workspace_bytes(M, N);
-  if (bias_down) w.colsum += gmlp::colsum_workspace_bytes(M, K);
-  return w;
+size_t bwd_workspace_bytes(int64_t M, int64_t K, int64_t N, int dtype) {
+  const int64_t R[3] = {N, N, K}, C[3] = {K, K, N};
+  return std::max({gmlp_workspace_bytes(GMLP_OP_DH_BWD, M, K, N, dtype), gmlp_workspace_bytes(GMLP_OP_DX_BWD, M, K, N, dtype),
+                   gmlp_dw_bwd_grouped_workspace_bytes(3, M, R, C, dtype), bias_workspace_bytes(M, K, N, true, true, true)});
 }
 
 }  // namespace
@@ -1038,7 +1025,7 @@ size_t gmlp_mlp_workspace_bytes(int pass, int64_t M, int64_t K, int64_t N, int d
     const size_t b = gmlp_workspace_bytes(GMLP_OP_LINEAR_FWD, M, N, K, dtype);
     return a > b ? a : b;
   }
-  if (pass == GMLP_PASS_BWD) return plan_bwd_workspace(M, K, N, dtype, true, true, true, true, true, true, true, true).total();
+  if (pass == GMLP_PASS_BWD) return bwd_workspace_bytes(M, K, N, dtype);
   return 0;
 }
 
@@ -1092,17 +1079,13 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
   GMLP_REQUIRE_ALIGNED(dw_up); GMLP_REQUIRE_ALIGNED(dw_down); GMLP_REQUIRE_ALIGNED(db_gate); GMLP_REQUIRE_ALIGNED(db_up);
   GMLP_REQUIRE_ALIGNED(db_down); GMLP_REQUIRE_ALIGNED(workspace);
 
-  const BwdWorkspace need = plan_bwd_workspace(M, K, N, dtype, hidden, dx, dw_gate, dw_up, dw_down, db_gate, db_up, db_down);
-  // Every launch gets the caller's buffer when it is large enough for that launch, and none
-  // otherwise (same results from the plain form of the launch).  Bias gradients cannot do without.
-  auto fits = [&](size_t bytes) { return workspace != nullptr && bytes > 0 && bytes <= workspace_bytes; };
-  void* const ws_cs = fits(need.colsum) ? workspace : nullptr;
-  void* const ws_dw = fits(need.dw) ? workspace : nullptr;
-  void* const ws_act = fits(need.act) ? workspace : nullptr;
-  const size_t n_dw = ws_dw ? workspace_bytes : 0, n_act = ws_act ? workspace_bytes : 0;
-  if (need.colsum > 0 && ws_cs == nullptr)
+  // Every launch gets the caller's buffer and uses what it holds (same results from the plainer form that
+  // a smaller one leaves).  Bias gradients cannot do without.
+  const size_t ws_bytes = workspace != nullptr ? workspace_bytes : 0;
+  const size_t sums = bias_workspace_bytes(M, K, N, db_gate, db_up, db_down);
+  if (sums > ws_bytes)
     return fail(GMLP_EINVAL, "%s: bias gradients need a workspace of at least %zu bytes (gmlp_mlp_workspace_bytes)",
-                __func__, need.colsum);
+                __func__, sums);
 
   const void* lhs[3]; const void* rhs[3]; void* dws[3]; int64_t R[3], C[3];
   int n = 0;
@@ -1116,7 +1099,7 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
   if (db_down) { cs_in[nb] = dy; cs_out[nb] = db_down; cs_c[nb] = K; ++nb; }
 
   if (hidden)
-    if (int rc = gmlp_dh_bwd(dy, w_down, g, u, dg, du, M, K, N, dtype, act, dropout_p, seed, offset, ws_act, n_act, stream))
+    if (int rc = gmlp_dh_bwd(dy, w_down, g, u, dg, du, M, K, N, dtype, act, dropout_p, seed, offset, workspace, ws_bytes, stream))
       return rc;
   // Everything on the caller's stream, one launch after the other.  Running the weight gradients
   // on a second stream next to dX was measured and is not done: two grids that each fill the chip
@@ -1124,9 +1107,9 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
   // grids under-fill the chip (M=2048, K=2048, N=5632) the two event waits that fork and join the
   // streams cost what the overlap gains.
   int rc = GMLP_OK;
-  if (dx) rc = gmlp_dx_bwd(dg, du, w_gate, w_up, dx, M, K, N, dtype, ws_act, n_act, stream);
-  if (rc == GMLP_OK && n > 0) rc = gmlp_dw_bwd_grouped(n, lhs, rhs, dws, M, R, C, dtype, ws_dw, n_dw, stream);
-  if (rc == GMLP_OK && nb > 0) rc = gmlp_colsum_grouped(nb, cs_in, cs_out, ws_cs, M, cs_c, dtype, stream);
+  if (dx) rc = gmlp_dx_bwd(dg, du, w_gate, w_up, dx, M, K, N, dtype, workspace, ws_bytes, stream);
+  if (rc == GMLP_OK && n > 0) rc = gmlp_dw_bwd_grouped(n, lhs, rhs, dws, M, R, C, dtype, workspace, ws_bytes, stream);
+  if (rc == GMLP_OK && nb > 0) rc = gmlp_colsum_grouped(nb, cs_in, cs_out, workspace, M, cs_c, dtype, stream);
   return rc;
 }
 
