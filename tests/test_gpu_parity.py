@@ -1239,6 +1239,68 @@ def test_fp32_every_operator_against_float64_products(M, K, N):
     check("dW alone", ops_bwd.dw_bwd(dy, h), [(d(dy).T, d(h))])
 
 
+@pytest.mark.parametrize("M,K,N", [(72, 40, 136), (130, 1544, 264)])  # one 64-row tile and a bit; split reductions
+def test_fp32_extreme_operands_against_float64_products(M, K, N):
+    """Operands that three bf16 parts of 2^16 x do not hold (infinities, NaNs, 2^111 and more), products
+    that overflow on the way, and subnormal ones, in rows and columns of their own beside ordinary ones: NaNs
+    and infinities where IEEE sums in float32 have them, and everything finite within the bound of a float32
+    sum, (R + 2) 2^-24 sum |a||b|, beside half the spacing of subnormal results per term."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(17)
+    rnd = lambda *shape: torch.randn(*shape, generator=g)
+    inf, nan = float("inf"), float("nan")
+
+    def extreme(t):
+        """t [rows, red]: extremes in rows 3 to 13, at the start and at the end of the reduction."""
+        t = t.clone()
+        t[3, 1], t[4, -1], t[5, 2], t[5, -2] = inf, -inf, inf, -inf
+        t[6, 0], t[7, 3], t[8, -1] = nan, 3.4e38, -(2.0**112)
+        t[9] = 2.0**-140 * t[9].sign()
+        t[10] *= 2.0**-120
+        t[11] *= 2.0**100
+        t[12] = 0.0
+        t[13] = 2.0**-149
+        return t
+
+    def check(name, got, pairs):
+        ref = sum(a.double() @ b.double() for a, b in pairs)
+        terms = sum(a.double().abs() @ b.double().abs() for a, b in pairs)
+        # what float32 makes of the float64 sum: out of range is infinite (no sum here is within rounding of it)
+        ref = torch.where(ref.abs() >= 3.4028236e38, ref.sign() * inf, ref)
+        got = got.double().cpu()
+        assert torch.equal(torch.isnan(got), torch.isnan(ref)), name
+        assert torch.equal(torch.isinf(got), torch.isinf(ref)) and torch.equal(got[torch.isinf(ref)], ref[torch.isinf(ref)]), name
+        R = sum(a.shape[1] for a, _ in pairs)
+        ok = torch.isfinite(ref)
+        bound = (R + 2) * (2.0**-24 * terms + 2.0**-149)
+        worst = ((got - ref).abs()[ok] / bound[ok]).max().item()
+        print(f"  {name}: largest error {worst:.3f} of its bound, {int((~ok).sum())} not finite", flush=True)
+        assert worst <= 1.0, name
+
+    print(f"fp32 extremes: M={M} K={K} N={N}", flush=True)
+    # weights that bf16 holds exactly (their second and third parts are zero), zeros among them
+    exact = lambda *shape: (rnd(*shape) * 2).round() / 2
+    d = lambda t: t.to(dev)
+    x, w = extreme(rnd(M, K)), exact(N, K)
+    hs = ops_fwd.gateup_fwd(d(x), d(w), None, d(exact(N, K)), None, save_activations=True)
+    check("G", hs.gate, [(x, w.T)])
+    h, wd = extreme(rnd(M, N)), exact(K, N)
+    check("Y", ops_fwd.linear_fwd(d(h), d(wd)), [(h, wd.T)])
+    a, we = exact(M, N), extreme(rnd(K, N))
+    check("Y, extreme weights", ops_fwd.linear_fwd(d(a), d(we)), [(a, we.T)])
+    ones = torch.ones(M, N)
+    check("dH", ops_bwd.dh_bwd(d(x), d(wd), d(ones), d(ones), act_fn="no_act")[1], [(x, wd)])
+    wg, wu = exact(N, K), exact(N, K)
+    h2 = rnd(M, N)
+    check("dX", ops_bwd.dx_bwd(d(h), d(h2), d(wg), d(wu)), [(h, wg), (h2, wu)])
+    lhs = extreme(rnd(N, M)).T.contiguous()  # reduction over the rows: extremes in columns
+    e = exact(M, K)
+    check("dW", ops_bwd.dw_bwd(d(lhs), d(e)), [(lhs.T, e)])
+
+
 def test_random_modules_through_the_one_call_entries_no_worse_than_torch_16bit():
     """Four dozen seeded random modules (token counts 1 to 6144, widths that are multiples of 8, 64
     or 256, both 16-bit dtypes, biases, dropout, five activations) through FusedGatedMLP, i.e. through

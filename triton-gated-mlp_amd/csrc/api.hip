@@ -129,42 +129,47 @@ struct GemmPlan {
   double us;  // estimate
 };
 
-// float32: tile class and number of workgroups per tile (splits), by estimated time.  A launch takes
-// as long as the compute unit that gets the most workgroups, and a CU's workgroups share its matrix
-// cores: per_cu workgroups of `weight` 64x64 tiles' work each, 0.445 us per 64x64x32 (16 MFMAs per
-// wavefront x 64 clocks at 2.3 GHz), at the fraction of the matrix cores' rate that the tile reaches
-// with one, two, or more workgroups per CU.  Fractions fitted to sweeps of all classes over the five
-// GEMMs of eight shapes (M 128 to 6974, K 256 to 3712, N 256 to 6144), where the estimate picks a
-// class within 5 % of the fastest.  What that is worth, down projection at M=2048, K=1024, N=2816:
-// 128x128 tiles (128 of them) 180 us, 64x64 (512) 103; weight gradients at M=6974, K=256, N=768: 460
-// unsplit, 64x64 126, with 13 splits 85.  A split reduction (64x64 tiles, at least 4 reduction tiles
-// each) pays a second launch and the partial sums' round trip through the caches.
-GemmPlan plan_f32(int64_t tiles128, int64_t tiles64x128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes,
-                 int64_t max_splits) {
-  static const double rate[3][3] = {{0.87, 0.88, 0.88}, {0.75, 0.78, 0.85}, {0.65, 0.76, 0.81}};  // by class, workgroups per CU
+int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// float32: tile class and number of workgroups per tile (splits), by estimated time: rounds of 2
+// (128x128 tiles) or 3 (64x64; 2 with two accumulator sets) workgroups per CU, each reduction tile at what
+// it takes with that many workgroups on a CU, a last round as long as the CUs with the most, a little
+// less where they are few.  A split reduction pays a second launch and the partial sums' round trip
+// through the caches.  One least-squares fit to the launches of five GEMMs of 70 shapes (M 32 to 6000,
+// widths 40 to 14400, both classes, 1 to 16 splits): standard deviation of the estimates 6 %, what it picks
+// costs 1.2 % over the fastest on average.  What that is worth at M=2048, K=1024, N=2816: down projection
+// on 128x128 tiles (128 of them) unsplit 136 us, in 4 splits 74, 64x64 unsplit 90; dX 258 / 128 / 169.
+GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes, int64_t max_splits) {
   GemmPlan best = {gmlp::TILE_F32_128, 1, 1e30};
   const int64_t cus = num_cu();
-  auto consider = [&](int tile_class, int64_t tiles, double weight, int64_t splits) {
-    const int64_t per_cu = (tiles * splits + cus - 1) / cus;
-    // (one reduction tile's time for the prologue and the epilogue)
-    double us = (double)per_cu * weight * (double)((red_tiles + splits - 1) / splits + 1) * 0.445 /
-                rate[tile_class - gmlp::TILE_F32_128][per_cu >= 3 ? 2 : per_cu - 1];
-    if (splits > 1) us += 5.0 + 2.0 * (double)splits * out_bytes * sets / 3e6;
+  auto consider = [&](int tile_class, int64_t tiles, int64_t splits) {
+    // us per reduction tile with 1, 2, 3 workgroups on a CU; us of an epilogue
+    static const double r128[] = {1.568, 2.482}, r64[] = {0.696, 1.015, 1.334}, r64x2[] = {1.140, 1.663};
+    const bool big = tile_class == gmlp::TILE_F32_128;
+    const double* r = big ? r128 : sets == 2 ? r64x2 : r64;
+    const int64_t cap = big || sets == 2 ? 2 : 3, wgs = tiles * splits, k = cdiv(red_tiles, splits), rest = wgs % (cus * cap);
+    const double e = big ? 1.414 : 0.168;
+    double us = 5.3 + (double)(wgs / (cus * cap)) * ((double)k * r[cap - 1] + e);
+    if (rest > 0) {
+      const int64_t per = cdiv(rest, cus);
+      const double f = (double)rest / (double)cus - (double)(per - 1);
+      us += (double)k * (r[per - 1] - 0.129 * (1.0 - f) * (r[per - 1] - (per > 1 ? r[per - 2] : 0.0))) + e;
+    }
+    // (1.6 on the GPU; the rest is what the second launch costs the host, which bounds passes this small)
+    if (splits > 1) us += 4.6 + 0.382e-6 * (double)splits * out_bytes * sets;
     if (us < best.us) best = GemmPlan{tile_class, (int)splits, us};
   };
-  consider(gmlp::TILE_F32_128, tiles128, 4, 1);
-  if (sets == 1) consider(gmlp::TILE_F32_64X128, tiles64x128, 2, 1);
-  consider(gmlp::TILE_F32_64, tiles64, sets, 1);
-  for (int64_t s = 2; s <= max_splits && s * 4 <= red_tiles; ++s) consider(gmlp::TILE_F32_64, tiles64, sets, s);
+  for (int64_t s = 1; s <= std::max<int64_t>(1, std::min(max_splits, red_tiles / 4)); ++s) {
+    if (s > 1 && cdiv(red_tiles, cdiv(red_tiles, s)) != s) continue;  // rounding up would leave splits empty
+    consider(gmlp::TILE_F32_128, tiles128, s);
+    consider(gmlp::TILE_F32_64, tiles64, s);
+  }
   return best;
 }
 GemmPlan plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int sets, int64_t max_splits) {
-  auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q; };
-  return plan_f32(up(rows, 128) * up(cols, 128 / sets), up(rows, 64) * up(cols, 128), up(rows, 64) * up(cols, 64),
-                  red_tiles, sets, (double)rows * (double)cols * 4.0, max_splits);
+  return plan_f32(cdiv(rows, 128) * cdiv(cols, 128 / sets), cdiv(rows, 64) * cdiv(cols, 64), red_tiles, sets,
+                  (double)rows * (double)cols * 4.0, max_splits);
 }
-
-int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Stream-K plan for a grid of `tiles` large output tiles with `kt` 64-wide reduction tiles each
 // (tiles of all problems of a grouped launch together).  The tiles beyond the last whole round of
@@ -306,11 +311,9 @@ int64_t whole_rounds(int kind, int64_t rows, int64_t cols) {
 // padded to whole tiles; anything larger runs on the predicated MEDIUM class.
 GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red, bool may_split) {
   if (dtype == GMLP_F32) {
-    // (the down projection of float32 modules asks for no workspace; callers rely on that)
-    const int64_t segments = kind == DX ? 2 : 1, tiles = segments * cdiv(red, 32);
-    GemmPlan p = plan_f32(rows, cols, tiles, kind == GATEUP ? 2 : 1, may_split && kind != LINEAR ? kMaxSplits : 1);
-    p.splits = (int)cdiv(tiles, cdiv(tiles, p.splits));  // drop the splits that rounding up leaves empty
-    return p;
+    // (a down projection of at most 64 rows asks for no workspace in float32: its callers rely on that)
+    return plan_f32(rows, cols, (kind == DX ? 2 : 1) * cdiv(red, 32), kind == GATEUP ? 2 : 1,
+                    may_split && (kind != LINEAR || rows > 64) ? kMaxSplits : 1);
   }
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
   // the buffer base sits up to 4 KB below the operand (shared-M0 loads)
@@ -367,18 +370,14 @@ int64_t splits_that_fit(size_t workspace_bytes, double out_bytes) {
 // splits; the problems' partial sums follow each other in the workspace.  (workspace_bytes: plan for
 // what a workspace of that size can hold.)
 GemmPlan plan_dw_group_f32(int count, int64_t Mred, const int64_t* R, const int64_t* C, size_t workspace_bytes = SIZE_MAX) {
-  int64_t t128 = 0, t64x128 = 0, t64 = 0;
+  int64_t t128 = 0, t64 = 0;
   double out_bytes = 0;
   for (int i = 0; i < count; ++i) {
     t128 += cdiv(R[i], 128) * cdiv(C[i], 128);
-    t64x128 += cdiv(R[i], 64) * cdiv(C[i], 128);
     t64 += cdiv(R[i], 64) * cdiv(C[i], 64);
     out_bytes += (double)R[i] * (double)C[i] * 4.0;
   }
-  GemmPlan p = plan_f32(t128, t64x128, t64, cdiv(Mred, 32), 1, out_bytes, splits_that_fit(workspace_bytes, out_bytes));
-  const int64_t per = cdiv(cdiv(Mred, 32), p.splits);
-  p.splits = (int)cdiv(cdiv(Mred, 32), per);  // drop the splits that rounding up leaves empty
-  return p;
+  return plan_f32(t128, t64, cdiv(Mred, 32), 1, out_bytes, splits_that_fit(workspace_bytes, out_bytes));
 }
 size_t dw_group_split_bytes(int count, int splits, const int64_t* R, const int64_t* C) {
   size_t n = 0;
@@ -801,7 +800,7 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
         ws += (size_t)plan.splits * R[i] * C[i];
       }
       if (plan.splits == 1) return launch_dw_group<T>(plan.tile_class, grp, s);
-      if (hipError_t err = launch_dw_group_split<T>(part, s)) return err;
+      if (hipError_t err = launch_dw_group_split<T>(plan.tile_class, part, s)) return err;
       return launch_splitk_reduce_group<T>(part, grp, s);
     }));
   }

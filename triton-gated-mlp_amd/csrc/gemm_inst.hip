@@ -95,7 +95,7 @@ hipError_t launch_dw_group<DT>(int tile_class, GemmGroup<EpiStore<DT>::Args>& gr
   return tile_class == TILE_LARGE ? GMLP_LARGE_GROUP(grp, s) : GMLP_MEDIUM_GROUP(grp, s);
 }
 template <>
-hipError_t launch_dw_group_split<DT>(GemmGroup<EpiPartial<DT>::Args>& grp, hipStream_t s) {
+hipError_t launch_dw_group_split<DT>(int, GemmGroup<EpiPartial<DT>::Args>& grp, hipStream_t s) {
   return launch_gemm_group_pipelined<DT, 128, 128, 16, 2, 2, true, true, 1, EpiPartial<DT>>(grp, s);
 }
 #endif

@@ -18,10 +18,10 @@ namespace gmlp {
 //                for problems with too few 256x256 tiles to fill the chip
 //   MEDIUM       128x128, predicated register-staged kernel, 64-bit addresses: operands too large for
 //                the pipelined kernels' 32-bit byte offsets
-//   F32_*        the float32 kernel's tiles (gemm_f32.hip): 128 x 128, 64 x 128, 64 x 64; with two
-//                accumulator sets 128 x 64 or 64 x 64
-enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2, TILE_F32_128 = 3, TILE_F32_64X128 = 4, TILE_F32_64 = 5,
-                 TILE_WIDE = 6, TILE_TALL = 7 };
+//   F32_*        the float32 kernel's tiles (gemm_f32.hip): 128 x 128 or 64 x 64; with two accumulator
+//                sets 128 x 64 or 64 x 64
+enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2, TILE_F32_128 = 3, TILE_F32_64 = 4, TILE_WIDE = 5,
+                 TILE_TALL = 6 };
 
 // kinds of GEMM the gated MLP needs; each is instantiated per dtype and tile class, and for reduction
 // lengths that are (KT = false) or are not a multiple of 64, the width of a reduction tile.
@@ -83,10 +83,10 @@ hipError_t launch_dw(int tile_class, const GemmArgs& ga, const typename EpiStore
 template <typename T>
 hipError_t launch_dw_group(int tile_class, GemmGroup<typename EpiStore<T>::Args>& grp, hipStream_t s);
 
-// The same with a split reduction (on MEDIUM_FULL or F32_64): every problem's ga.splits partial sums,
+// The same with a split reduction (on MEDIUM_FULL, F32_128 or F32_64): every problem's ga.splits partial sums,
 // then their totals.
 template <typename T>
-hipError_t launch_dw_group_split(GemmGroup<typename EpiPartial<T>::Args>& grp, hipStream_t s);
+hipError_t launch_dw_group_split(int tile_class, GemmGroup<typename EpiPartial<T>::Args>& grp, hipStream_t s);
 template <typename T>
 hipError_t launch_splitk_reduce_group(const GemmGroup<typename EpiPartial<T>::Args>& part,
                                       const GemmGroup<typename EpiStore<T>::Args>& out, hipStream_t s);
