@@ -1638,6 +1638,27 @@ def test_decode_cases_cover_every_row_tail():
         ("down", k) for k in ((1, 1, 512), (2, 1, 256), (2, 1, 512), (1, 2, 512), (2, 2, 256), (2, 2, 512), (4, 2, 256))}
 
 
+@pytest.mark.parametrize(
+    "M,K,N,gated,down",  # on a whole MI355X, as above; rows per compute unit in brackets
+    [
+        (1, 768, 2048, (1, 1, 128), (1, 1, 128)),      # fewer stages than ring slots, half a block [8] and a quarter [3]
+        (16, 1024, 5632, (2, 1, 128), (1, 1, 128)),    # [22] H in fragment order
+        (5, 4352, 2112, (1, 1, 128), (2, 1, 256)),     # [8.25] K [17]; N no multiple of 256
+        (9, 4352, 2048, (1, 1, 128), (2, 1, 128)),
+        (17, 1280, 3904, (1, 2, 128), (1, 2, 512)),    # [15.25]
+        (24, 768, 8256, (3, 2, 128), (1, 2, 512)),     # [32.25]
+        (32, 768, 7744, (2, 2, 128), (1, 2, 512)),     # [30.25]
+        (20, 768, 14336, (4, 2, 128), (1, 2, 512)),    # [56]
+        (32, 768, 18944, (5, 2, 128), (1, 2, 512)),    # [74]
+        (32, 768, 45056, (4, 2, 128), (1, 2, 512)),    # [176]: two whole blocks and most of a third
+    ],
+)
+def test_decode_streaming_kernels_short_segments(M, K, N, gated, down):
+    """Every block height of the kernels that stream 128-byte segments, with partly empty blocks, against
+    float64 products; twice, bit-identical, the second time with the launched kernels' names."""
+    test_decode_streaming_kernels_at_any_width(M, K, N, gated, down, torch.bfloat16 if M % 2 else torch.float16, M > 16)
+
+
 def test_decode_streaming_entry_refuses_what_its_kernels_do_not_take():
     from triton_gated_mlp import _cabi
 

@@ -1,31 +1,34 @@
 // Skinny-M (M <= 32) weight-streaming kernels, HBM-bound: every weight byte is fetched once, in
-// 512-byte (or 256-byte) row segments moved global -> LDS without passing through registers.
+// row segments of 128, 256 or 512 bytes moved global -> LDS without passing through registers.
 //
 // One persistent workgroup of three wavefronts per CU.  The workgroup takes blocks of weight rows
-// that share one set of token operands: 16 or 32 rows of W_gate and as many of W_up (GATED), or 16,
+// that share one set of token operands: 16 to 80 rows of W_gate and as many of W_up (GATED), or 16,
 // 32 or 64 consecutive rows of W_down.  Whole blocks go round-robin over the workgroups, the rows that
 // do not fill a last round are shared out evenly as one partly empty block each.  Its wavefronts split
-// the reduction range in near-equal runs of chunks (256 or 128 elements) and combine their partial
+// the reduction range in near-equal runs of chunks (64 to 256 elements) and combine their partial
 // sums through LDS at the end of each block (fixed order, so the result is deterministic).  Each
-// wavefront runs a private ring of 3 or 4 LDS slots; a slot holds one stage = one chunk of the
+// wavefront runs a private ring of 2 to 8 LDS slots; a slot holds one stage = one chunk of the
 // block's weight rows.  The matching token-row operands (x or H, L2-resident)
 // are fetched straight into registers, as many stages ahead: one 16-token tile for M <= 16, two
 // beyond (MT; the weight fragment read from LDS then feeds two MFMAs).  The stream of stages runs on
 // across block boundaries, so the ring never drains; loads past the end re-fetch the last stage into a
 // free slot, which keeps the in-flight count constant.
 //
-// Which block (chosen in launch_decode_stream; whole forward, us, fp16): the height decides what a
-// block costs in token operands and how well it fits a CU's share of the rows, the row segment of a
-// stage (SEGB) what is left of a chunk's imbalance between the wavefronts.  Bytes in flight no longer
-// decide at 96 KiB per CU: four, six and eight wavefronts with 128 to 144 KiB were no faster on any of
-// eleven widths.
+// Which block (chosen in launch_decode_stream; kernel times, us, fp16): the height decides what a block
+// costs in token operands and how well it fits a CU's share of the rows; the row segment of a stage (SEGB)
+// how evenly the chunks divide over the wavefronts (16 chunks of 256 elements at K = 4096: 6, 5 and 5; 64 of
+// 64: 22, 21 and 21), how soon the first MFMA can start, and how finely the ring's slots take up what the
+// loads in flight leave.  512- -> 128-byte segments, W_gate / W_up, 16 rows a block: K=2048, N=8192 M=8
+// 17.4 -> 14.6, M=16 19.1 -> 15.4; K=1024, N=4096 9.3 -> 7.1, 10.1 -> 7.6.  Bytes in flight do not decide at
+// 96 KiB per CU: four, six and eight wavefronts with 128 to 144 KiB were no faster on any of eleven
+// widths.
 //
 //   GATED:   H[m, r] = act(x.W_gate[r] + b_gate[r]) * (x.W_up[r] + b_up[r])      (r over N)
 //   !GATED:  Y[m, r] = H.W_down[r] + b_down[r]                                   (r over K)
 //
-// LDS layout of a slot: regions of 16 rows x SEGB bytes (SEGB = 512 or 256); the 16-byte chunk c
-// of row r is stored at position c ^ r, so the 16 lanes that read one chunk index of 16 different
-// rows for v_mfma_f32_16x16x32 hit 16 different bank groups.
+// LDS layout of a slot: regions of 16 rows x SEGB bytes; the 16-byte chunk c of row r is stored at
+// position c ^ r (128-byte segments, two rows to all banks: c ^ (r / 2)), so the 16 lanes that read one
+// chunk index of 16 different rows for v_mfma_f32_16x16x32 hit 16 different bank groups.
 //
 // All vector-memory loads of the main loop are written as assembly and ordered by explicit
 // s_waitcnt vmcnt(N): the compiler does not see them, so it cannot serialise them either (the
@@ -56,7 +59,7 @@ constexpr int DS_MAX_LDS = 160 * 1024;
 constexpr int DS_WAVES = 3;                   // wavefronts per workgroup
 constexpr int DS_MIN_RED = 768;               // a chunk for every wavefront
 constexpr uint32_t DS_NOWHERE = 0x80000000u;  // voffset beyond any operand (operands are < 2 GiB)
-constexpr int DS_WIDE_SEGMENT_MAX_M = 20;     // see ds_tall_gated
+constexpr int DS_WIDE_SEGMENT_MAX_M = 20;     // see ds_tall_gated, ds_short_segments
 constexpr int DS_H_TILED_MIN_M = 10;           // H goes out in fragment order above this many token rows
 
 struct StreamArgs {
@@ -80,21 +83,20 @@ __device__ __forceinline__ i32x4 load16_async(buffer_rsrc r, uint32_t voffset, u
                : "memory");
   return v;
 }
-// s_waitcnt vmcnt(N) that also "defines" the registers a stage's token operands arrive in (8 per
-// token tile), so no use of them can be scheduled above the wait.  The second statement issues no
-// instruction: volatile asm statements keep their order, so it ties the second tile's registers
-// to the same point.
+// s_waitcnt vmcnt(N) that also "defines" the registers a stage's token operands arrive in, so no use
+// of them can be scheduled above the wait.  The other statements issue no instruction: volatile asm
+// statements keep their order, so they tie the other registers to the same point.
 template <int N, int NX>
 __device__ __forceinline__ void wait_vmem_keep(i32x4 (&x)[NX]) {
-  static_assert(NX % 4 == 0, "groups of four");
-  asm volatile("s_waitcnt vmcnt(%4)" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]) : "n"(N) : "memory");
+  static_assert(NX % 2 == 0, "pairs");
+  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(x[0]), "+v"(x[1]) : "n"(N) : "memory");
 #pragma unroll
-  for (int i = 4; i < NX; i += 4) asm volatile("" : "+v"(x[i]), "+v"(x[i + 1]), "+v"(x[i + 2]), "+v"(x[i + 3]) : : "memory");
+  for (int i = 2; i < NX; i += 2) asm volatile("" : "+v"(x[i]), "+v"(x[i + 1]) : : "memory");
 }
 
 // HALVES: 16-row regions per matrix and stage.
 // MT:   tiles of 16 token slots (M <= 16 * MT).
-// SEGB: bytes of a weight row per stage, 512 or 256.
+// SEGB: bytes of a weight row per stage, 512, 256 or 128.
 // DS_RD: ring slots per wavefront and stages in flight.
 // TAIL: the reduction length need not be a multiple of the chunk (only of 8): the 16-byte pieces of the
 //       last chunk that lie beyond the row's end are pushed out of the descriptors, weights and token
@@ -102,7 +104,8 @@ __device__ __forceinline__ void wait_vmem_keep(i32x4 (&x)[NX]) {
 template <typename T, bool GATED, int HALVES, int MT, int SEGB, int DS_RD, bool TAIL>
 __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs a) {
   typedef typename Traits<T>::vec8 vec8;
-  static_assert(SEGB == 512 || SEGB == 256, "row segment of a stage");
+  static_assert(SEGB == 512 || SEGB == 256 || SEGB == 128, "row segment of a stage");
+  auto swz = [](int r) __attribute__((always_inline)) { return SEGB == 128 ? r >> 1 : r; };
   constexpr int NREG = (GATED ? 2 : 1) * HALVES;  // 16-row regions per stage
   constexpr int REGION = 16 * SEGB;           // bytes of a region
   constexpr int CH = SEGB / 2;                // reduction elements per stage
@@ -178,8 +181,8 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
   for (int q = 0; q < LPR; ++q) {
     int row = (64 / CPR) * q + lane / CPR, pos = lane % CPR;
     wrow[q] = row;
-    wchunk[q] = pos ^ row;
-    woff[q] = (uint32_t)(row * a.red + (pos ^ row) * 8) * 2u;
+    wchunk[q] = pos ^ swz(row);
+    woff[q] = (uint32_t)(row * a.red + (pos ^ swz(row)) * 8) * 2u;
   }
   const bool tiled_x = !GATED && a.tiled;
 #pragma unroll
@@ -257,7 +260,7 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_stream_kernel(StreamArgs
         const char* slot = ring + u * SLOT;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          int pos = ((ks * 4 + kg) ^ r16) << 4;
+          int pos = ((ks * 4 + kg) ^ swz(r16)) << 4;
 #pragma unroll
           for (int g = 0; g < NREG; ++g) {
             vec8 wf = *(const vec8*)(slot + g * REGION + r16 * SEGB + pos);
@@ -369,8 +372,9 @@ static hipError_t launch_stream_tail(const StreamArgs& a, int num_cu, hipStream_
 }
 template <typename T, bool GATED, int HALVES, int MT, int SEGB, int RD>
 static hipError_t launch_stream(const StreamArgs& a, int num_cu, hipStream_t s) {
-  return a.red % (SEGB / 2) == 0 ? launch_stream_tail<T, GATED, HALVES, MT, SEGB, RD, false>(a, num_cu, s)
-                                 : launch_stream_tail<T, GATED, HALVES, MT, SEGB, RD, true>(a, num_cu, s);
+  if constexpr (SEGB > 128)  // (rows of whole 128-byte lines are a multiple of 64 elements)
+    if (a.red % (SEGB / 2) != 0) return launch_stream_tail<T, GATED, HALVES, MT, SEGB, RD, true>(a, num_cu, s);
+  return launch_stream_tail<T, GATED, HALVES, MT, SEGB, RD, false>(a, num_cu, s);
 }
 
 // Layout of the intermediate H between the two kernels.  Row-major [M, N] costs the down projection
@@ -383,10 +387,45 @@ bool decode_stream_supported(int M, int K, int N) {
          (int64_t)K * N * 2 < ((int64_t)1 << 31);
 }
 
-// Blocks of 32 rows of W_gate and W_up, 128 elements a stage (two stages' worth of 16-row blocks of 256
-// elements): half the token operands per weight byte.  M=24, K=4096, N=14336 73 us against 79, M=16,
-// K=5120, N=13824 80 / 85.  With one token tile or little more the operands cost less than a block that
-// a CU's share does not fill (M=16, K=8192, N=28672, 112 rows: 228 / 224), so they are taken there only
+// Segments of 128 bytes: reduction lengths that are a multiple of 256 and rows that are one of 64, the
+// widths that models have and that this was measured on.  (Never rows that do not start on a 128-byte
+// line: every segment touches one line more than it fills, see ds_tall_gated.)  Long segments stream a few
+// per cent faster from HBM once a kernel runs long enough for that to count and the token operands cost
+// little.  One token tile, whole forward, long -> short: K=1024, N=4096 M=1 14.8 -> 13.8, M=8 16.2 -> 14.0;
+// K=4096, N=14336 61.7 -> 61.7, 63.3 -> 59.5; K=6144, N=16384 99.5 -> 101.9, 97.3 -> 97.9; K=2048, N=8192
+// 26.9 -> 27.6, 29.6 -> 28.3.  Two: K=8192, N=28672 M=17 230 -> 232, M=32 243 -> 234.
+static bool ds_short_segments(int M, int rows, int red) {
+  if (red % 256 != 0 || rows % 64 != 0) return false;
+  const int64_t elements = (int64_t)rows * red;
+  if (M > 16) return M > DS_WIDE_SEGMENT_MAX_M || elements <= ((int64_t)128 << 20);
+  return elements <= ((int64_t)(M <= 4 ? 12 : 64) << 20);
+}
+
+// Height of a block of W_gate and W_up rows, in units of 16, for segments of 128 bytes: the one whose blocks
+// cost a CU's share least, a block costing its rows (the partly empty last one all of them: its missing rows
+// leave slots of the ring unused) and its token operands (0.2 of a row of weights per token with two token
+// tiles; 0.05 with one).  One tile: 16 or 32 rows (N = 13824, K = 5120, 54 rows per CU, M = 8 47.8 / 46.6;
+// N = 11008, K = 4096, 43 rows 30.1 / 33.0), two: up to 80.  M = 32, rows per CU, us at 16 / 32 / 48 / 64 / 80: N = 11008,
+// K = 4096, 43 rows 41 / 40 / 34 / 34 / 36; N = 14336, 56 rows 51 / 44 / 51 / 41 / 42; N = 28672, K = 8192,
+// 112 rows 179 / 158 / 172 / 150 / 162; N = 18944, K = 3584, 74 rows 65 / 59 / 53 / 61 / 52.  Over 25
+// widths and M = 17, 24, 32 the kernel takes 0.89 of the time of the blocks of 16 rows of 256 elements or 32 of 128
+// that it took before, M = 6, 10, 16 0.92.
+static int ds_gated_height(int M, int N, int num_cu) {
+  const bool two = M > 16;
+  int best = 1;
+  double least = 1e30;
+  for (int h = 1; h <= (two ? 5 : 2); ++h) {
+    const int rows = 16 * h, full = N / rows / num_cu, rest = N - full * num_cu * rows;
+    const int blocks = full + (rest + num_cu * rows - 1) / (num_cu * rows);
+    const double cost = blocks * (rows + (two ? 0.2 : 0.05) * M);
+    if (cost < least) least = cost, best = h;
+  }
+  return best;
+}
+
+// The other widths.  Blocks of 32 rows of W_gate and W_up, 128 elements a stage (two stages' worth of 16-row
+// blocks of 256 elements): half the token operands per weight byte.  With one token tile or little more
+// the operands cost less than a block that a CU's share does not fill, so they are taken there only
 // where the share rounded up to 16 and to 32 rows is the same, and up to 10 tokens not at all (M=5, K=3840,
 // N=6656 33.0 / 32.3).  Rows that do not start on a 128-byte line take the long segments throughout: a
 // 256-byte one touches three lines instead of two (K=6712, N=24104, M=1 210 -> 188 us; K=3592, N=8200,
@@ -409,21 +448,38 @@ hipError_t launch_decode_stream(const T* x, const T* wg, const T* wu, const T* w
   const int tiled = ds_h_tiled(M);
   StreamArgs a1 = {x, {wg, wu}, {bg, bu}, h, M, N, K, K, N, act, tiled};
   StreamArgs a2 = {h, {wd, wd}, {bd, bd}, y, M, K, N, N, K, ACT_IDENTITY, tiled};
-  const bool tall = ds_tall_gated(M, K, N, num_cu);
-  // W_down: 32 rows of 128 elements a stage, four stages deep, once a CU's share exceeds 16 rows (K=5120,
-  // N=13824, whole forward, against 32 rows of 256 three deep, or 64 of 128 from M = 21 up: M=1 72 -> 70
-  // us, M=16 80 -> 79, M=24 106 -> 98), 16 rows of 256 up to there (K=4096, N=11008, M=24: 64 us
-  // either way; 32 rows would be half empty).  Two token tiles over 48 rows or more take 64 at a time: K=16384, N=53248, M=18
-  // 807 -> 783 us.  Misaligned rows take 256 elements at any height (K=6712, N=24104, M=1 188 -> 178).
+  // Ring depths: what 160 KiB hold (and, two token tiles, what the operands in flight leave in the VGPRs).
+  auto gated = [&]() -> hipError_t {
+    if (!ds_short_segments(M, N, K) || N < 8 * num_cu) {
+      const bool tall = ds_tall_gated(M, K, N, num_cu);
+      if (M <= 16) return tall ? launch_stream<T, true, 2, 1, 256, 3>(a1, num_cu, s) : launch_stream<T, true, 1, 1, 512, 3>(a1, num_cu, s);
+      return tall ? launch_stream<T, true, 2, 2, 256, 3>(a1, num_cu, s) : launch_stream<T, true, 1, 2, 512, 3>(a1, num_cu, s);
+    }
+    const int height = ds_gated_height(M, N, num_cu);
+    if (M <= 16) return height == 1 ? launch_stream<T, true, 1, 1, 128, 8>(a1, num_cu, s) : launch_stream<T, true, 2, 1, 128, 6>(a1, num_cu, s);
+    switch (height) {
+      case 1: return launch_stream<T, true, 1, 2, 128, 8>(a1, num_cu, s);
+      case 2: return launch_stream<T, true, 2, 2, 128, 6>(a1, num_cu, s);
+      case 3: return launch_stream<T, true, 3, 2, 128, 3>(a1, num_cu, s);
+      case 4: return launch_stream<T, true, 4, 2, 128, 2>(a1, num_cu, s);
+      default: return launch_stream<T, true, 5, 2, 128, 2>(a1, num_cu, s);
+    }
+  };
+  if (hipError_t e = gated()) return e;
+  // W_down: 32 rows a block once a CU's share exceeds 16 rows, 16 up to there.  One token tile: segments of
+  // 128 bytes, eight stages deep (against 512 / 256 bytes, M = 6 to 16, 25 widths: 0.91 of the time);
+  // otherwise 256 elements a stage up to 16 rows and on misaligned rows, 128 beyond (K=6712,
+  // N=24104, M=1, 256 elements for 128 188 -> 178 us).  Two tiles: H's operands are as many bytes as the
+  // weights, and shorter stages only add instructions (K=2048, N=8192, M=24 128- against 512-byte segments
+  // 16.0 / 14.9), so 256 elements up to 16 rows, 128 beyond, and 64 rows at a time from 48 rows (K=16384,
+  // N=53248, M=18 807 -> 783 us for the whole forward).
   const bool one = K <= 16 * num_cu, lines = ds_whole_lines(N), four = K > 48 * num_cu && lines;
   if (M <= 16) {
-    if (hipError_t e = tall ? launch_stream<T, true, 2, 1, 256, 3>(a1, num_cu, s) : launch_stream<T, true, 1, 1, 512, 3>(a1, num_cu, s))
-      return e;
+    if (ds_short_segments(M, K, N))
+      return one ? launch_stream<T, false, 1, 1, 128, 8>(a2, num_cu, s) : launch_stream<T, false, 2, 1, 128, 8>(a2, num_cu, s);
     if (one) return launch_stream<T, false, 1, 1, 512, 4>(a2, num_cu, s);
     return lines ? launch_stream<T, false, 2, 1, 256, 4>(a2, num_cu, s) : launch_stream<T, false, 2, 1, 512, 3>(a2, num_cu, s);
   }
-  if (hipError_t e = tall ? launch_stream<T, true, 2, 2, 256, 3>(a1, num_cu, s) : launch_stream<T, true, 1, 2, 512, 3>(a1, num_cu, s))
-    return e;
   if (four) return launch_stream<T, false, 4, 2, 256, 3>(a2, num_cu, s);
   if (one) return launch_stream<T, false, 1, 2, 512, 3>(a2, num_cu, s);
   return lines ? launch_stream<T, false, 2, 2, 256, 4>(a2, num_cu, s) : launch_stream<T, false, 2, 2, 512, 3>(a2, num_cu, s);

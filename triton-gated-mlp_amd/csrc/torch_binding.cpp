@@ -198,11 +198,14 @@ bool decode_preferred(int64_t M, int64_t K, int64_t N, int code, int64_t num_cu)
 // four, no partial sums in memory).  One token tile always wins: K=1024, N=2048 11 to 13 us against 16,
 // K=2200, N=4608 20 to 24 / 30, K=5168, N=20480 110 to 122 / 130 to 136.  With two, its operands' traffic
 // grows with the rows per compute unit: up to 32 rows of W_gate they win (K=1024, N=8192 27 / 28, K=3592,
-// N=8200 54 to 59 / 59 to 62), beyond they do not (K=2560, N=10240 49 / 46, K=4496, N=9472 68 / 67).
+// N=8200 54 to 59 / 59 to 62), and beyond where the blocks are high enough for the share (rows of whole lines,
+// K from 8 rows per unit up: K=2560, N=10240 44 / 47, K=3072, N=12288 55 / 60, K=2048, N=16384 M=24 52 / 56;
+// K=3328, N=13312 M=20 64 / 62, M=24 60 / 62; K=1024, N=16384 41 / 39; K=4800, N=14400 89 / 89).
 bool narrow_decode_preferred(int64_t M, int64_t K, int64_t N, int code, int64_t num_cu) {
   if (code == GMLP_F32 || M < 1 || M > 32 || K % 8 != 0 || N % 8 != 0) return false;
   if (K < 768 || N < 768 || K * N >= ((int64_t)1 << 30)) return false;
-  return M <= 16 || N <= 33 * num_cu;
+  if (M <= 16 || N <= 33 * num_cu) return true;
+  return K % 256 == 0 && N % 64 == 0 && K >= 8 * num_cu && (M > 20 || N <= 48 * num_cu);
 }
 int64_t compute_units(int device) {
   static std::atomic<int> known[64];
