@@ -218,7 +218,7 @@ int gmlp_colsum(const void* a, void* out, void* workspace, int64_t M, int64_t C,
 int gmlp_colsum_static(const void* a, void* out, int64_t M, int64_t C, int dtype, void* stream);
 
 /*
- * Up to 3 bias gradients of one backward pass in one pair of launches: out[i][C[i]] = Σ_m a[i][m,C[i]].
+ * Up to 3 bias gradients of one backward pass in one launch or two: out[i][C[i]] = Σ_m a[i][m,C[i]].
  * workspace: the sum over i of gmlp_workspace_bytes(GMLP_OP_COLSUM, M, 0, C[i], dtype) bytes.
  * Same reference counterpart as gmlp_colsum.
  */

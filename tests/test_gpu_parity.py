@@ -1239,6 +1239,24 @@ def test_fp32_every_operator_against_float64_products(M, K, N):
     check("dW alone", ops_bwd.dw_bwd(dy, h), [(d(dy).T, d(h))])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 700, 2560, 2561])  # row ranges empty, of one row, uneven; one launch and two
+def test_column_sums_against_float64(M, dtype):
+    """Column sums of three arrays, one strip of 64 columns to several with a ragged last one.  Bound: a
+    float32 sum of M terms in any order, (M + 2) 2^-24 sum |a|, and half a unit of the stored type."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(M)
+    arrays = [torch.randn(M, C, generator=g).to(dtype).to(dev) for C in (8, 72, 264)]
+    half_unit = {torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8, torch.float32: 2.0**-24}[dtype]
+    for a, got in zip(arrays, ops_bwd.colsum_grouped(arrays)):
+        ref = a.double().sum(0)
+        bound = (M + 2) * 2.0**-24 * a.double().abs().sum(0) + half_unit * ref.abs()
+        assert ((got.double() - ref).abs() <= bound * (1 + half_unit) + 2.0**-25).all(), (M, a.shape[1], dtype)
+        assert torch.equal(got, ops_bwd.colsum(a))
+
+
 @pytest.mark.parametrize("M,K,N", [(72, 40, 136), (130, 1544, 264)])  # one 64-row tile and a bit; split reductions
 def test_fp32_extreme_operands_against_float64_products(M, K, N):
     """Operands that three bf16 parts of 2^16 x do not hold (infinities, NaNs, 2^111 and more), products
