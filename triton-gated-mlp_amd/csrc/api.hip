@@ -139,7 +139,8 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // widths 40 to 14400, both classes, 1 to 16 splits): standard deviation of the estimates 6 %, what it picks
 // costs 1.2 % over the fastest on average.  What that is worth at M=2048, K=1024, N=2816: down projection
 // on 128x128 tiles (128 of them) unsplit 136 us, in 4 splits 74, 64x64 unsplit 90; dX 258 / 128 / 169.
-GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes, int64_t max_splits) {
+GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes, int64_t max_splits,
+                  double split_us) {
   GemmPlan best = {gmlp::TILE_F32_128, 1, 1e30};
   const int64_t cus = num_cu();
   auto consider = [&](int tile_class, int64_t tiles, int64_t splits) {
@@ -155,8 +156,7 @@ GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets
       const double f = (double)rest / (double)cus - (double)(per - 1);
       us += (double)k * (r[per - 1] - 0.129 * (1.0 - f) * (r[per - 1] - (per > 1 ? r[per - 2] : 0.0))) + e;
     }
-    // (1.6 on the GPU; the rest is what the second launch costs the host, which bounds passes this small)
-    if (splits > 1) us += 4.6 + 0.382e-6 * (double)splits * out_bytes * sets;
+    if (splits > 1) us += split_us + 0.382e-6 * (double)splits * out_bytes * sets;
     if (us < best.us) best = GemmPlan{tile_class, (int)splits, us};
   };
   for (int64_t s = 1; s <= std::max<int64_t>(1, std::min(max_splits, red_tiles / 4)); ++s) {
@@ -166,9 +166,14 @@ GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets
   }
   return best;
 }
-GemmPlan plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int sets, int64_t max_splits) {
+// What a split costs beside its traffic: 1.6 us on the GPU, and the rest is what the second launch costs the
+// host, which bounds passes this small.  A forward down projection pays that twice: nothing else in its
+// pass is split at such sizes (training step at M=K=N=512 89.4 us with one launch, 92.4 with two).
+const double kSplitF32 = 4.6, kSplitF32Linear = 8.6;
+GemmPlan plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int kind, int64_t max_splits) {
+  const int sets = kind == GATEUP ? 2 : 1;
   return plan_f32(cdiv(rows, 128) * cdiv(cols, 128 / sets), cdiv(rows, 64) * cdiv(cols, 64), red_tiles, sets,
-                  (double)rows * (double)cols * 4.0, max_splits);
+                  (double)rows * (double)cols * 4.0, max_splits, kind == LINEAR ? kSplitF32Linear : kSplitF32);
 }
 
 // Stream-K plan for a grid of `tiles` large output tiles with `kt` 64-wide reduction tiles each
@@ -312,8 +317,7 @@ int64_t whole_rounds(int kind, int64_t rows, int64_t cols) {
 GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red, bool may_split) {
   if (dtype == GMLP_F32) {
     // (a down projection of at most 64 rows asks for no workspace in float32: its callers rely on that)
-    return plan_f32(rows, cols, (kind == DX ? 2 : 1) * cdiv(red, 32), kind == GATEUP ? 2 : 1,
-                    may_split && (kind != LINEAR || rows > 64) ? kMaxSplits : 1);
+    return plan_f32(rows, cols, (kind == DX ? 2 : 1) * cdiv(red, 32), kind, may_split && (kind != LINEAR || rows > 64) ? kMaxSplits : 1);
   }
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
   // the buffer base sits up to 4 KB below the operand (shared-M0 loads)
@@ -377,7 +381,7 @@ GemmPlan plan_dw_group_f32(int count, int64_t Mred, const int64_t* R, const int6
     t64 += cdiv(R[i], 64) * cdiv(C[i], 64);
     out_bytes += (double)R[i] * (double)C[i] * 4.0;
   }
-  return plan_f32(t128, t64, cdiv(Mred, 32), 1, out_bytes, splits_that_fit(workspace_bytes, out_bytes));
+  return plan_f32(t128, t64, cdiv(Mred, 32), 1, out_bytes, splits_that_fit(workspace_bytes, out_bytes), kSplitF32);
 }
 size_t dw_group_split_bytes(int count, int splits, const int64_t* R, const int64_t* C) {
   size_t n = 0;
