@@ -1033,6 +1033,38 @@ def test_whole_pass_entry_points_equal_the_separate_launches(M, K, N, dtype, bia
             assert a is None or torch.equal(a, ref[n]), f"{n} differs for subset {want}"
 
 
+# dX beside the weight gradients in one grid: 128x128 tiles for both (a single tile each, remainders in every
+# direction, few rows), 256x256 tiles beside a split and an unsplit dX, 192-row and 128-row tiles of dX, reduction lengths
+# that are not a multiple of the 64 of a reduction tile; last, shapes next to these that keep launches of their own
+# (split weight gradients, shared-out tiles).
+@pytest.mark.parametrize(
+    "M,K,N",
+    [(1, 8, 8), (129, 136, 264), (33, 512, 1528), (512, 512, 1536), (1024, 1024, 2816), (1000, 1024, 2824), (3000, 1536, 4096),
+     (2999, 1528, 4104), (384, 1984, 5440), (271, 2456, 6600), (6656, 1472, 1472), (3456, 384, 1536), (842, 5032, 13520)],
+)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
+    """gmlp_mlp_bwd may run dX and whichever weight gradients are wanted as one grid: the same sums in the same order
+    as the entry points of their own (held against the oracle elsewhere), hence equal bit for bit."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+
+    g = torch.Generator(device=_dev()).manual_seed(M + N)
+    rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g, device=_dev())).to(dtype)
+    x, wg, wu, wd, dy = rnd(M, K), rnd(N, K, s=0.03), rnd(N, K, s=0.03), rnd(K, N, s=0.03), rnd(M, K)
+    gate, up, hidden = rnd(M, N), rnd(M, N), rnd(M, N)
+    dg, du = ops_bwd.dh_bwd(dy, wd, gate, up)
+    dx = ops_bwd.dx_bwd(dg, du, wg, wu)
+    pairs = [(dg, x), (du, x), (dy, hidden)]
+    for wanted in ((1, 1, 1), (1, 0, 0), (0, 1, 1), (0, 0, 1)):
+        dws = iter(ops_bwd.dw_bwd_grouped([p for p, w in zip(pairs, wanted) if w]))
+        got = ops_bwd.mlp_bwd(dy, x, wg, wu, wd, gate, up, hidden, (True, *(bool(w) and i == 0 for w in wanted for i in (0, 1))))
+        assert torch.equal(got[0], dx), f"dX differs beside {wanted}"
+        for w, a in zip(wanted, got[1::2]):
+            assert torch.equal(a, next(dws)) if w else a is None, f"a weight gradient differs for {wanted}"
+    torch.cuda.synchronize()
+
+
+
 def test_random_shapes_every_operator_against_fp32_products():
     """Two dozen seeded random shapes through the five GEMM operators: token counts from 1 to a few
     thousand, widths that are multiples of 64 (tuned kernels: large, medium, two-launch, split and

@@ -409,6 +409,21 @@ GemmPlan plan_dw_group(int count, int64_t Mred, const int64_t* R, const int64_t*
   return p;
 }
 
+// Estimated time of a GEMM as run_plan launches it (16-bit types, no stream-K).
+double planned_us(int kind, int64_t rows, int64_t cols, int64_t red, const GemmPlan& p) {
+  const int64_t kt = red_tiles_of(kind, red), whole = whole_rounds(kind, rows, cols);
+  if (p.tile_class != gmlp::TILE_LARGE || whole == 0) return p.us;
+  const int64_t r = kind <= LINEAR ? rows : rows - whole * 256, c = kind <= LINEAR ? cols - whole * tile_cols(kind) : cols;
+  return launch_us(kLarge, kind, tiles_of(kLarge, kind, rows, cols) / num_cu() * num_cu(), kt, 1, 0) +
+         plan_gemm(GMLP_F16, kind, r, c, red, false).us;
+}
+// ... and of grouped weight gradients: a thin last round runs as a launch of its own.
+double planned_dw_group_us(int64_t Mred, int64_t large, const GemmPlan& p) {
+  const int64_t cus = num_cu(), rounds = large / cus, tail = large % cus, kt = cdiv(Mred, 64);
+  if (p.tile_class != gmlp::TILE_LARGE || rounds < 1 || rounds > 4 || tail == 0 || 2 * tail > cus) return p.us;
+  return launch_us(kLarge, DW, rounds * cus, kt, 1, 0) + launch_us(kMedium, DW, 4 * tail, kt, 1, 0);
+}
+
 size_t split_workspace_bytes(int splits, int64_t rows, int64_t cols, int accumulator_sets = 1) {
   return splits > 1 ? (size_t)splits * accumulator_sets * rows * cols * sizeof(float) : 0;
 }
@@ -451,6 +466,98 @@ hipError_t run_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red
     }
   }
   return run(0, all, p, nullptr);
+}
+
+// dX and the weight gradients as one grid.  Behind each other both end in a round that does not fill the
+// chip; in one grid the workgroups with the longer tiles come first and the others fill what those leave.
+// Estimated by dealing the workgroups out to the CUs in that order, each at what its class takes in a full
+// round, and taken where that is ahead of the separate launches' estimates: mostly below about 4000 rows
+// (4096x4096x14336 and 7431x2208x3296 stay as they are: many rounds, 0.999 to 1.001 of the time either way).
+// dX keeps the number of splits that it has by itself, so that the results are the same bit for
+// bit; shared-out tiles (stream-K) and split weight gradients keep launches of their own.
+struct DxDwPlan {
+  bool merged = false, dx_first = true;
+  int x_class = 0, splits = 1;
+};
+// When `slots` that take the next workgroup as they get free are through with n0 workgroups of d0 us and then n1 of d1 us.
+double makespan_us(int64_t slots, int64_t n0, double d0, int64_t n1, double d1) {
+  const int64_t late_slots = n0 % slots;  // these get free a round later than the others
+  const double early = (double)(n0 / slots) * d0, late = late_slots ? early + d0 : early;
+  const double work = ((double)n0 * d0 + (double)n1 * d1) / (double)slots;
+  auto done_by = [&](double t) {
+    auto each = [&](double from) { return (int64_t)std::max(0.0, std::floor((t - from) / d1 + 1e-6)); };
+    return late_slots * each(late) + (slots - late_slots) * each(early);
+  };
+  auto end_from = [&](double from) {  // (the last one ends a whole number of d1 after one of the two moments)
+    double t = from + std::max(0.0, std::floor((work - from) / d1)) * d1;
+    while (done_by(t) < n1) t += d1;
+    return t;
+  };
+  return std::max(late, std::min(end_from(early), end_from(late)));
+}
+DxDwPlan make_plan_dx_dw(int dtype, int64_t M, int64_t K, int64_t N, int count, const int64_t* R, const int64_t* C,
+                         size_t workspace_bytes) {
+  DxDwPlan p;
+  GemmPlan px = plan_gemm(dtype, DX, M, K, N, true);
+  if (px.splits > 1 && workspace_bytes < split_workspace_bytes(px.splits, M, K)) px = plan_gemm(dtype, DX, M, K, N, false);
+  if (px.tile_class == gmlp::TILE_MEDIUM) return p;
+  for (int i = 0; i < count; ++i)
+    if (plan_gemm(dtype, DW, R[i], C[i], M, false).tile_class == gmlp::TILE_MEDIUM) return p;
+  GemmPlan pw = plan_dw_group(count, M, R, C);
+  if (pw.splits > 1) return p;  // (also where the workspace does not hold them)
+  const int64_t ktx = red_tiles_of(DX, N), ktw = cdiv(M, 64), large = dw_group_tiles(kLarge, count, R, C);
+  if (px.tile_class == gmlp::TILE_LARGE && plan_streamk(dtype, tiles_of(kLarge, DX, M, K), ktx).tiles > 0) return p;
+  if (pw.tile_class == gmlp::TILE_LARGE && plan_streamk(dtype, large, ktw, false).tiles > 0) return p;
+  double best = planned_us(DX, M, K, N, px) + planned_dw_group_us(M, large, pw);
+  const int64_t kt = cdiv(ktx, px.splits), cus = num_cu();
+  const double second = px.splits > 1 ? 4.0 + (double)px.splits * (double)M * (double)K * 4.0 / 2.7e6 : 0.0;
+  auto consider = [&](const TileCost& cx, const TileCost& cw, double measured) {
+    const int64_t slots = cx.per_cu * cus, nx = tiles_of(cx, DX, M, K) * px.splits, nw = dw_group_tiles(cw, count, R, C);
+    double dx = (double)kt * cx.r[1] + cx.e[px.splits > 1 ? 5 : DX], dw = (double)ktw * cw.r[2] + cw.e[DW];
+    if (nx + nw < slots) {  // (a partly filled round, see launch_us)
+      const double f = (double)(nx + nw) / (double)slots;
+      const double fill = cx.half == 0.0 ? cx.base + (1.0 - cx.base) * f
+                          : f <= 0.5     ? cx.base + cx.half * 2.0 * f
+                                         : cx.base + cx.half + (1.0 - cx.base - cx.half) * (2.0 * f - 1.0);
+      dx *= fill;
+      dw *= fill;
+    }
+    const bool dx_first = dx >= dw;
+    const double us = measured * (3.1 + second + (dx_first ? makespan_us(slots, nx, dx, nw, dw) : makespan_us(slots, nw, dw, nx, dx)));
+    if (us < best) {
+      best = us;
+      p.merged = true;
+      p.dx_first = dx_first;
+      p.x_class = cx.tile_class;
+      p.splits = px.splits;
+    }
+  };
+  // (times as measured against this estimate: CUs that are at different places of their tiles get a larger share
+  // of the bandwidth each.  Chosen with these factors, a backward pass with its dH takes 0.89 times as long over
+  // 60 shapes of 32 to 8192 rows and 32 to 5000 inputs, at worst 1.017 with runs of one side 2.5 % apart.)
+  consider(kLarge, kLarge, 0.96);
+  consider(kWide, kLarge, 1.02);
+  // (a 192-row tile can reach further past the last row than the others: see make_plan)
+  if (px.splits == 1 && cdiv(M, 192) * 192 * (cdiv(N, 64) * 64) * 2 < ((int64_t)1 << 31) - 4096) consider(kTall, kLarge, 1.0);
+  consider(kMedium, kMedium, 0.98);
+  return p;
+}
+DxDwPlan plan_dx_dw(int dtype, int64_t M, int64_t K, int64_t N, int count, const int64_t* R, const int64_t* C,
+                    size_t workspace_bytes) {
+  struct Entry {
+    int64_t key[6] = {-1, -1, -1, -1, -1, -1};
+    DxDwPlan plan;
+  };
+  static thread_local Entry cache[32];
+  int64_t wide = 0;  // which of the weights: the gradients are [N, K] or [K, N]
+  for (int i = 0; i < count; ++i) wide = wide * 2 + (R[i] == K);
+  const int64_t key[6] = {M, K, N, ((int64_t)num_cu() * 4 + dtype) * 8 + count, wide, (int64_t)workspace_bytes};
+  Entry& e = cache[(uint64_t)(M * 0x9E3779B1 + K * 0x85EBCA77 + N * 0xC2B2AE3D + key[3] * 0x27D4EB2F + wide) >> 7 & 31];
+  if (!std::equal(key, key + 6, e.key)) {
+    e.plan = make_plan_dx_dw(dtype, M, K, N, count, R, C, workspace_bytes);
+    std::copy(key, key + 6, e.key);
+  }
+  return e.plan;
 }
 
 std::mutex& lds_registry_mutex() {
@@ -1005,6 +1112,63 @@ int gmlp_dropout_mask(uint8_t* mask, int64_t M, int64_t N, float dropout_p, uint
 // ---------------------------------------------------------------- whole passes in one call
 namespace {
 
+// dX and the weight gradients lhs[i]^T . rhs[i] of a pass whose arguments have been checked.
+int run_dx_dw(const char* fn, const void* dg, const void* du, const void* w_gate, const void* w_up, void* dx, int count,
+              const void* const* lhs, const void* const* rhs, void* const* dws, int64_t M, int64_t K, int64_t N, const int64_t* R,
+              const int64_t* C, int dtype, void* workspace, size_t ws_bytes, void* stream) {
+  using namespace gmlp;
+  DxDwPlan plan;
+  if (dx && count > 0 && dtype != GMLP_F32) plan = plan_dx_dw(dtype, M, K, N, count, R, C, workspace ? ws_bytes : 0);
+  if (!plan.merged) {
+    int rc = GMLP_OK;
+    if (dx) rc = gmlp_dx_bwd(dg, du, w_gate, w_up, dx, M, K, N, dtype, workspace, ws_bytes, stream);
+    if (rc == GMLP_OK && count > 0) rc = gmlp_dw_bwd_grouped(count, lhs, rhs, dws, M, R, C, dtype, workspace, ws_bytes, stream);
+    return rc;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  hipError_t e = by_dtype(dtype, [&](auto tag) -> hipError_t {
+    typedef decltype(tag) T;
+    if constexpr (std::is_same<T, float>::value) {
+      return hipErrorInvalidValue;  // not reached
+    } else {
+      const typename EpiStore<T>::Args store = {(T*)dx, nullptr, (int)K};
+      auto launch = [&](auto& grp, auto&& kernel) -> hipError_t {
+        GemmArgs& ga = grp.gx;
+        ga.nxcd = num_xcd();
+        ga.A[0] = dg; ga.A[1] = du; ga.B[0] = w_gate; ga.B[1] = w_up;
+        ga.M = (int)M; ga.N = (int)K; ga.K = (int)N; ga.lda = (int)N; ga.ldb = (int)K;
+        ga.nseg = 2; ga.group_m = pick_group(M, K); ga.splits = plan.splits;
+        grp.w.count = count;
+        for (int i = 0; i < count; ++i) {
+          GemmArgs& gw = grp.w.ga[i];
+          gw.nxcd = num_xcd();
+          gw.A[0] = gw.A[1] = lhs[i]; gw.B[0] = gw.B[1] = rhs[i];
+          gw.M = (int)R[i]; gw.N = (int)C[i]; gw.K = (int)M; gw.lda = (int)R[i]; gw.ldb = (int)C[i];
+          gw.nseg = 1; gw.group_m = pick_group(R[i], C[i]);
+          grp.w.ea[i] = {(T*)dws[i], nullptr, (int)C[i]};
+        }
+        return kernel(grp);
+      };
+      const bool tail = N % 64 != 0;
+      if (plan.splits == 1) {
+        DxDwGroup<T, EpiStore<T>> grp = {};
+        grp.ex = store;
+        return launch(grp, [&](auto& g) {
+          return tail ? launch_dx_dw_kt<T, true>(plan.x_class, g, plan.dx_first, s) : launch_dx_dw_kt<T, false>(plan.x_class, g, plan.dx_first, s);
+        });
+      }
+      DxDwGroup<T, EpiPartial<T>> grp = {};
+      grp.ex = {(float*)workspace, (size_t)M * K, 0, (int)K};
+      if (hipError_t err = launch(grp, [&](auto& g) {
+            return tail ? launch_dx_dw_split_kt<T, true>(plan.x_class, g, plan.dx_first, s) : launch_dx_dw_split_kt<T, false>(plan.x_class, g, plan.dx_first, s);
+          }))
+        return err;
+      return launch_splitk_reduce<T, EpiStore<T>>((const float*)workspace, plan.splits, (size_t)M * K, 0, store, M, K, s);
+    }
+  });
+  return hip_result(fn, e);
+}
+
 size_t bias_workspace_bytes(int64_t M, int64_t K, int64_t N, bool gate, bool up, bool down) {
   return (gate + up) * gmlp::colsum_workspace_bytes(M, N) + down * gmlp::colsum_workspace_bytes(M, K);
 }
@@ -1109,9 +1273,7 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
   // run 2.5 to 4 % slower side by side than one after the other (M=8192, K=4096, N=14336), and where
   // grids under-fill the chip (M=2048, K=2048, N=5632) the two event waits that fork and join the
   // streams cost what the overlap gains.
-  int rc = GMLP_OK;
-  if (dx) rc = gmlp_dx_bwd(dg, du, w_gate, w_up, dx, M, K, N, dtype, workspace, ws_bytes, stream);
-  if (rc == GMLP_OK && n > 0) rc = gmlp_dw_bwd_grouped(n, lhs, rhs, dws, M, R, C, dtype, workspace, ws_bytes, stream);
+  int rc = run_dx_dw(__func__, dg, du, w_gate, w_up, dx, n, lhs, rhs, dws, M, K, N, R, C, dtype, workspace, ws_bytes, stream);
   if (rc == GMLP_OK && nb > 0) rc = gmlp_colsum_grouped(nb, cs_in, cs_out, workspace, M, cs_c, dtype, stream);
   return rc;
 }

@@ -1,7 +1,7 @@
 // One translation unit per (dtype, GEMM kind, reduction tail): compiled with -DGMLP_DT=<0|1>
-// -DGMLP_KIND=<0..4> -DGMLP_KT=<0|1> so the kernels build in parallel.  Each unit instantiates
+// -DGMLP_KIND=<0..6> -DGMLP_KT=<0|1> so the kernels build in parallel.  Each unit instantiates
 // every tile class; GMLP_KT=1 are the kernels for reduction lengths that are not a multiple of 64
-// (kinds with a reduction-contiguous operand, 0..3), which have no predicated class.
+// (kinds with a reduction-contiguous operand, all but 4), which have no predicated class.
 #include "gemm_pipelined.hpp"
 #include "launch.hpp"
 
@@ -97,6 +97,21 @@ hipError_t launch_dw_group<DT>(int tile_class, GemmGroup<EpiStore<DT>::Args>& gr
 template <>
 hipError_t launch_dw_group_split<DT>(int, GemmGroup<EpiPartial<DT>::Args>& grp, hipStream_t s) {
   return launch_gemm_group_pipelined<DT, 128, 128, 16, 2, 2, true, true, 1, EpiPartial<DT>>(grp, s);
+}
+#elif GMLP_KIND == 5
+template <>
+hipError_t launch_dx_dw_kt<DT, KT>(int x_class, DxDwGroup<DT, EpiStore<DT>>& grp, bool dx_first, hipStream_t s) {
+  if (x_class == TILE_LARGE) return launch_dx_dw_pipelined<DT, 256, 256, 256, EpiStore<DT>, KT>(grp, dx_first, s);
+  if (x_class == TILE_TALL) return launch_dx_dw_pipelined<DT, 192, 256, 256, EpiStore<DT>, KT>(grp, dx_first, s);
+  if (x_class == TILE_WIDE) return launch_dx_dw_pipelined<DT, 128, 256, 256, EpiStore<DT>, KT>(grp, dx_first, s);
+  return launch_dx_dw_pipelined<DT, 128, 128, 128, EpiStore<DT>, KT>(grp, dx_first, s);
+}
+#elif GMLP_KIND == 6
+template <>
+hipError_t launch_dx_dw_split_kt<DT, KT>(int x_class, DxDwGroup<DT, EpiPartial<DT>>& grp, bool dx_first, hipStream_t s) {
+  if (x_class == TILE_LARGE) return launch_dx_dw_pipelined<DT, 256, 256, 256, EpiPartial<DT>, KT>(grp, dx_first, s);
+  if (x_class == TILE_WIDE) return launch_dx_dw_pipelined<DT, 128, 256, 256, EpiPartial<DT>, KT>(grp, dx_first, s);
+  return launch_dx_dw_pipelined<DT, 128, 128, 128, EpiPartial<DT>, KT>(grp, dx_first, s);
 }
 #endif
 

@@ -933,6 +933,53 @@ __global__ void __launch_bounds__(WGM* WGN * 64)
       ga, ea, (int)blockIdx.x - grp.first[g], grp.first[g + 1] - grp.first[g]);
 }
 
+// The input gradient and the weight gradients of a pass as one grid: workgroups [x0, x0 + dx_wgs) compute
+// dX (EpiPartial: its split reduction's partial sums) on BMX-row tiles, the others the weight gradients on
+// BMW-row tiles.  Matrix-core bound like the grids it stands for; what it takes away is a launch (about 4 us of
+// GPU time) and a partly filled last round.  A backward pass, dH included, before and after, bfloat16: 512x512x512
+// 30.5 -> 22.1 us, 1024x1024x2816 77.7 -> 66.8, 2048x2048x5632 322 -> 313, 3000x1536x4096 276 -> 222.
+// Registers and LDS are those of the larger of the two bodies: pairs that run at the same number of
+// workgroups a CU.
+template <typename T, int BMX, int BNX, int BMW, typename EpiX, bool KT>
+__global__ void __launch_bounds__(256) gemm_dx_dw_kernel_pipelined(DxDwGroup<T, EpiX> grp) {
+  int pid = (int)blockIdx.x;
+  if (pid >= grp.x0 && pid < grp.x0 + grp.dx_wgs) {
+    gemm_pipelined_body<T, BMX, BNX, 16, 2, 2, false, true, 1, EpiX, false, KT>(grp.gx, grp.ex, pid - grp.x0, grp.dx_wgs);
+    return;
+  }
+  if (pid >= grp.x0 + grp.dx_wgs) pid -= grp.dx_wgs;
+  int g = 0;
+#pragma unroll
+  for (int i = 1; i < GEMM_GROUP_MAX; ++i)
+    if (i < grp.w.count && pid >= grp.w.first[i]) g = i;
+  GemmArgs ga = grp.w.ga[0];
+  typename EpiStore<T>::Args ea = grp.w.ea[0];
+#pragma unroll
+  for (int i = 1; i < GEMM_GROUP_MAX; ++i)
+    if (g == i) { ga = grp.w.ga[i]; ea = grp.w.ea[i]; }
+  gemm_pipelined_body<T, BMW, BMW, 16, 2, 2, true, true, 1, EpiStore<T>>(ga, ea, pid - grp.w.first[g],
+                                                                         grp.w.first[g + 1] - grp.w.first[g]);
+}
+
+template <typename T, int BMX, int BNX, int BMW, typename EpiX, bool KT>
+hipError_t launch_dx_dw_pipelined(DxDwGroup<T, EpiX>& grp, bool dx_first, hipStream_t s) {
+  typedef PipeConfig<T, BMX, BNX, 16, 2, 2, false, true, 1, wants_ring_a3<T, EpiX>()> CfgX;
+  typedef PipeConfig<T, BMW, BMW, 16, 2, 2, true, true, 1, wants_ring_a3<T, EpiStore<T>>()> CfgW;
+  constexpr int LDS = CfgX::LDS_BYTES > CfgW::LDS_BYTES ? CfgX::LDS_BYTES : CfgW::LDS_BYTES;
+  constexpr auto kern = gemm_dx_dw_kernel_pipelined<T, BMX, BNX, BMW, EpiX, KT>;
+  if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, LDS>, s)) return e;
+  int total = 0;
+  for (int g = 0; g < grp.w.count; ++g) {
+    grp.w.first[g] = total;
+    total += ((grp.w.ga[g].M + BMW - 1) / BMW) * ((grp.w.ga[g].N + BMW - 1) / BMW);
+  }
+  for (int g = grp.w.count; g <= GEMM_GROUP_MAX; ++g) grp.w.first[g] = total;
+  grp.dx_wgs = ((grp.gx.M + BMX - 1) / BMX) * ((grp.gx.N + BNX - 1) / BNX) * (EpiX::SPLIT ? grp.gx.splits : 1);
+  grp.x0 = dx_first ? 0 : total;
+  hipLaunchKernelGGL(kern, dim3(total + grp.dx_wgs), dim3(256), LDS, s, grp);
+  return hipGetLastError();
+}
+
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
           typename Epi, bool KT = false>
 hipError_t launch_gemm_pipelined(const GemmArgs& ga, const typename Epi::Args& ea, hipStream_t s) {

@@ -126,4 +126,14 @@ struct GemmGroup {
   int count;
 };
 
+// The input gradient and the weight gradients of a pass in a single launch: workgroups [x0, x0 + dx_wgs)
+// belong to the input gradient.
+template <typename T, typename EpiX>
+struct DxDwGroup {
+  GemmArgs gx;
+  typename EpiX::Args ex;
+  GemmGroup<typename EpiStore<T>::Args> w;
+  int x0, dx_wgs;
+};
+
 }  // namespace gmlp

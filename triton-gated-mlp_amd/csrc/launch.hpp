@@ -91,6 +91,14 @@ template <typename T>
 hipError_t launch_splitk_reduce_group(const GemmGroup<typename EpiPartial<T>::Args>& part,
                                       const GemmGroup<typename EpiStore<T>::Args>& out, hipStream_t s);
 
+// dX and up to three weight gradients as one grid: dX on `x_class` (LARGE, TALL, WIDE beside large tiles of
+// the weight gradients, MEDIUM_FULL beside MEDIUM_FULL ones; a split reduction with EpiPartial, not TALL).
+// The workgroups of the problem that takes longer per tile should come first.
+template <typename T, bool KT>
+hipError_t launch_dx_dw_kt(int x_class, DxDwGroup<T, EpiStore<T>>& grp, bool dx_first, hipStream_t s);
+template <typename T, bool KT>
+hipError_t launch_dx_dw_split_kt(int x_class, DxDwGroup<T, EpiPartial<T>>& grp, bool dx_first, hipStream_t s);
+
 // Generic launcher used by the instantiation units.
 template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
           bool EDGE, typename Epi>
