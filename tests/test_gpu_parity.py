@@ -1036,7 +1036,7 @@ def test_whole_pass_entry_points_equal_the_separate_launches(M, K, N, dtype, bia
 # dX beside the weight gradients in one grid: 128x128 tiles for both (a single tile each, remainders in every
 # direction, few rows), 256x256 tiles beside a split and an unsplit dX, 192-row and 128-row tiles of dX, reduction lengths
 # that are not a multiple of the 64 of a reduction tile; last, shapes next to these that keep launches of their own
-# (split weight gradients, shared-out tiles).
+# (split weight gradients, shared-out tiles).  Bias gradients take their place behind the tiles.
 @pytest.mark.parametrize(
     "M,K,N",
     [(1, 8, 8), (129, 136, 264), (33, 512, 1528), (512, 512, 1536), (1024, 1024, 2816), (1000, 1024, 2824), (3000, 1536, 4096),
@@ -1044,8 +1044,8 @@ def test_whole_pass_entry_points_equal_the_separate_launches(M, K, N, dtype, bia
 )
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
-    """gmlp_mlp_bwd may run dX and whichever weight gradients are wanted as one grid: the same sums in the same order
-    as the entry points of their own (held against the oracle elsewhere), hence equal bit for bit."""
+    """gmlp_mlp_bwd may run dX, whichever weight gradients are wanted and the bias gradients as one grid: the same sums in
+    the same order as the entry points of their own (held against the oracle elsewhere), hence equal bit for bit."""
     from triton_gated_mlp.ops import bwd as ops_bwd
 
     g = torch.Generator(device=_dev()).manual_seed(M + N)
@@ -1055,14 +1055,16 @@ def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
     dg, du = ops_bwd.dh_bwd(dy, wd, gate, up)
     dx = ops_bwd.dx_bwd(dg, du, wg, wu)
     pairs = [(dg, x), (du, x), (dy, hidden)]
-    for wanted in ((1, 1, 1), (1, 0, 0), (0, 1, 1), (0, 0, 1)):
+    for want_dx, wanted, biases in ((1, (1, 1, 1), 1), (1, (1, 0, 0), 0), (1, (0, 1, 1), 1), (1, (0, 0, 1), 0), (0, (1, 1, 1), 1)):
         dws = iter(ops_bwd.dw_bwd_grouped([p for p, w in zip(pairs, wanted) if w]))
-        got = ops_bwd.mlp_bwd(dy, x, wg, wu, wd, gate, up, hidden, (True, *(bool(w) and i == 0 for w in wanted for i in (0, 1))))
-        assert torch.equal(got[0], dx), f"dX differs beside {wanted}"
-        for w, a in zip(wanted, got[1::2]):
+        dbs = iter(ops_bwd.colsum_grouped([p[0] for p, w in zip(pairs, wanted) if w]) if biases else ())
+        need = (bool(want_dx), *(bool(w and (i == 0 or biases)) for w in wanted for i in (0, 1)))
+        got = ops_bwd.mlp_bwd(dy, x, wg, wu, wd, gate, up, hidden, need)
+        assert torch.equal(got[0], dx) if want_dx else got[0] is None, f"dX differs beside {wanted}"
+        for w, a, b in zip(wanted, got[1::2], got[2::2]):
             assert torch.equal(a, next(dws)) if w else a is None, f"a weight gradient differs for {wanted}"
+            assert torch.equal(b, next(dbs)) if w and biases else b is None, f"a bias gradient differs for {wanted}"
     torch.cuda.synchronize()
-
 
 
 def test_random_shapes_every_operator_against_fp32_products():

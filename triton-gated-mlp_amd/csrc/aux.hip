@@ -174,58 +174,13 @@ GMLP_REDUCE_GROUP_INST(float)
 // 5.2 -> 3.5, M=200, N=704, K=256 5.3 -> 3.5, M=1357, N=3096, K=1160 8.8 -> 8.4, M=2048, N=5632, K=2048
 // 13.8 -> 11.8; M=5000, N=600, K=200 9.9 -> 14.3, M=8192, N=8192, K=2048 75 -> 83.  (And one launch less for
 // the host, 3 to 4 us of passes that it bounds.)
-constexpr int COLSUM_SPLITS = 64, COLSUM_COLS = 64;
 constexpr int64_t COLSUM_ONE_LAUNCH_MAX_M = 2560;  // 40 rows, five batches of loads, to a range
 
 template <typename T>
 __global__ void __launch_bounds__(COLSUM_SPLITS * 8) colsum_kernel(ColsumGroup<T> g, int64_t M) {
-  constexpr int RUNS = 4, PER = COLSUM_SPLITS / RUNS;
-  __shared__ __align__(16) float part[COLSUM_SPLITS][COLSUM_COLS + 4];
-  const T* __restrict__ a = g.a[blockIdx.y];
-  const int64_t C = g.C[blockIdx.y], c0 = (int64_t)blockIdx.x * COLSUM_COLS;
-  if (c0 >= C) return;
-  const int range = threadIdx.x / 8, col = threadIdx.x % 8 * 8;
-  const int64_t rows = (M + COLSUM_SPLITS - 1) / COLSUM_SPLITS;
-  const int64_t r0 = range * rows, r1 = r0 + rows < M ? r0 + rows : M;
-  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (c0 + col < C) {
-    const T* p = a + r0 * C + c0 + col;
-    int64_t r = r0;
-    auto add = [&](auto count) __attribute__((always_inline)) {  // that many independent loads in flight
-      constexpr int U = decltype(count)::value;
-      typename Traits<T>::vec8 t[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) t[u] = *(const typename Traits<T>::vec8*)(p + u * C);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) s[q] += Traits<T>::to_f32(t[u][q]);
-      p += U * C;
-      r += U;
-    };
-    while (r + 8 <= r1) add(std::integral_constant<int, 8>{});
-    if (r + 4 <= r1) add(std::integral_constant<int, 4>{});
-    if (r + 2 <= r1) add(std::integral_constant<int, 2>{});
-    if (r < r1) add(std::integral_constant<int, 1>{});
-  }
-  *(f32x4*)&part[range][col] = f32x4{s[0], s[1], s[2], s[3]};
-  *(f32x4*)&part[range][col + 4] = f32x4{s[4], s[5], s[6], s[7]};
-  __syncthreads();
-  // the first wavefront: 16 lanes to a run, 4 columns each
-  const int run = threadIdx.x / 16, c = threadIdx.x % 16 * 4;
-  f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  if (run < RUNS) {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) v += *(const f32x4*)&part[run * PER + i][c];
-  }
-  __syncthreads();
-  if (run < RUNS) *(f32x4*)&part[run][c] = v;
-  __syncthreads();
-  if (run > 0 || c0 + c >= C) return;
-#pragma unroll
-  for (int i = 1; i < RUNS; ++i) v += *(const f32x4*)&part[i][c];
-  const float t[4] = {v[0], v[1], v[2], v[3]};
-  store_w<T, 4>(g.out[blockIdx.y] + c0 + c, t);
+  __shared__ __align__(16) char lds[COLSUM_LDS_BYTES];
+  const int64_t c0 = (int64_t)blockIdx.x * COLSUM_COLS;
+  if (c0 < g.C[blockIdx.y]) colsum_body<T, COLSUM_SPLITS * 8>(g.a[blockIdx.y], g.out[blockIdx.y], g.C[blockIdx.y], c0, M, lds);
 }
 
 template <typename T>

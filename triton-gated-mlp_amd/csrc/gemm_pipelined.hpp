@@ -933,16 +933,35 @@ __global__ void __launch_bounds__(WGM* WGN * 64)
       ga, ea, (int)blockIdx.x - grp.first[g], grp.first[g + 1] - grp.first[g]);
 }
 
-// The input gradient and the weight gradients of a pass as one grid: workgroups [x0, x0 + dx_wgs) compute
+// The input gradient, the weight gradients and the bias gradients of a pass as one grid: workgroups [x0, x0 + dx_wgs) compute
 // dX (EpiPartial: its split reduction's partial sums) on BMX-row tiles, the others the weight gradients on
 // BMW-row tiles.  Matrix-core bound like the grids it stands for; what it takes away is a launch (about 4 us of
 // GPU time) and a partly filled last round.  A backward pass, dH included, before and after, bfloat16: 512x512x512
 // 30.5 -> 22.1 us, 1024x1024x2816 77.7 -> 66.8, 2048x2048x5632 322 -> 313, 3000x1536x4096 276 -> 222.
-// Registers and LDS are those of the larger of the two bodies: pairs that run at the same number of
+// The bias gradients, memory bound, come last, on CUs that the last round of tiles leaves free: with them
+// 310x416x1248 36.0 -> 26.3 us, 2048x2048x5632 320 -> 295, 3762x1848x7392 730 -> 635, and beside the weight gradients
+// alone 1357x1160x3096 128.6 -> 121.5.
+// Registers and LDS are those of the larger of the bodies: pairs that run at the same number of
 // workgroups a CU.
 template <typename T, int BMX, int BNX, int BMW, typename EpiX, bool KT>
 __global__ void __launch_bounds__(256) gemm_dx_dw_kernel_pipelined(DxDwGroup<T, EpiX> grp) {
   int pid = (int)blockIdx.x;
+  if (grp.nsums > 0 && pid >= grp.sum_first[0]) {
+    extern __shared__ __align__(1024) char smem_raw[];
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < COLSUM_GROUP_MAX; ++k)
+      if (k < grp.nsums && pid >= grp.sum_first[k]) i = k;
+    const T* a = grp.sums.a[0];
+    T* out = grp.sums.out[0];
+    int64_t C = grp.sums.C[0];
+    int first = grp.sum_first[0];
+#pragma unroll
+    for (int k = 1; k < COLSUM_GROUP_MAX; ++k)
+      if (i == k) { a = grp.sums.a[k]; out = grp.sums.out[k]; C = grp.sums.C[k]; first = grp.sum_first[k]; }
+    colsum_body<T, 256>(a, out, C, (int64_t)(pid - first) * COLSUM_COLS, grp.sum_rows, smem_raw);
+    return;
+  }
   if (pid >= grp.x0 && pid < grp.x0 + grp.dx_wgs) {
     gemm_pipelined_body<T, BMX, BNX, 16, 2, 2, false, true, 1, EpiX, false, KT>(grp.gx, grp.ex, pid - grp.x0, grp.dx_wgs);
     return;
@@ -974,9 +993,16 @@ hipError_t launch_dx_dw_pipelined(DxDwGroup<T, EpiX>& grp, bool dx_first, hipStr
     total += ((grp.w.ga[g].M + BMW - 1) / BMW) * ((grp.w.ga[g].N + BMW - 1) / BMW);
   }
   for (int g = grp.w.count; g <= GEMM_GROUP_MAX; ++g) grp.w.first[g] = total;
+  // (no rows: dX not wanted, or in a launch of its own)
   grp.dx_wgs = ((grp.gx.M + BMX - 1) / BMX) * ((grp.gx.N + BNX - 1) / BNX) * (EpiX::SPLIT ? grp.gx.splits : 1);
   grp.x0 = dx_first ? 0 : total;
-  hipLaunchKernelGGL(kern, dim3(total + grp.dx_wgs), dim3(256), LDS, s, grp);
+  total += grp.dx_wgs;
+  static_assert(LDS >= COLSUM_LDS_BYTES, "the sums' workgroups use the same allocation");
+  for (int i = 0; i < grp.nsums; ++i) {
+    grp.sum_first[i] = total;
+    total += (int)((grp.sums.C[i] + COLSUM_COLS - 1) / COLSUM_COLS);
+  }
+  hipLaunchKernelGGL(kern, dim3(total), dim3(256), LDS, s, grp);
   return hipGetLastError();
 }
 

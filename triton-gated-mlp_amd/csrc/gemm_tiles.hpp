@@ -11,6 +11,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "colsum.hpp"
 #include "gemm.hpp"
 #include "lds_dma.hpp"
 
@@ -126,14 +127,16 @@ struct GemmGroup {
   int count;
 };
 
-// The input gradient and the weight gradients of a pass in a single launch: workgroups [x0, x0 + dx_wgs)
-// belong to the input gradient.
+// The input gradient, the weight gradients and the bias gradients of a pass in a single launch: workgroups
+// [x0, x0 + dx_wgs) belong to the input gradient, those from sum_first[i] on to column sum i.
 template <typename T, typename EpiX>
 struct DxDwGroup {
   GemmArgs gx;
   typename EpiX::Args ex;
   GemmGroup<typename EpiStore<T>::Args> w;
-  int x0, dx_wgs;
+  ColsumGroup<T> sums;
+  int64_t sum_rows;
+  int x0, dx_wgs, nsums, sum_first[COLSUM_GROUP_MAX];
 };
 
 }  // namespace gmlp

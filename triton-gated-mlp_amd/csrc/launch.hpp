@@ -1,5 +1,6 @@
 // Host-side launch interface between the C ABI (api.hip) and the kernel translation units.
 #pragma once
+#include "colsum.hpp"
 #include "gemm.hpp"
 #include "gemm_tiles.hpp"
 
@@ -134,14 +135,6 @@ hipError_t launch_gating_bwd(const T* dh, const T* g, const T* u, T* dg, T* du, 
 template <typename T, typename Epi>
 hipError_t launch_splitk_reduce(const float* ws, int splits, size_t split_stride, size_t acc_stride,
                                 const typename Epi::Args& ea, int64_t M, int64_t N, hipStream_t s);
-constexpr int COLSUM_GROUP_MAX = 3;
-template <typename T>
-struct ColsumGroup {
-  const T* a[COLSUM_GROUP_MAX];   // [M, C[i]]
-  T* out[COLSUM_GROUP_MAX];       // [C[i]]
-  float* ws[COLSUM_GROUP_MAX];    // colsum_workspace_bytes(M, C[i]) bytes each
-  int64_t C[COLSUM_GROUP_MAX];
-};
 template <typename T>
 hipError_t launch_colsum_group(const ColsumGroup<T>& g, int count, int64_t M, hipStream_t s);
 size_t colsum_workspace_bytes(int64_t M, int64_t C);
