@@ -270,7 +270,7 @@ int gmlp_decode_stream_fwd(const void* x, const void* w_gate, const void* w_up, 
  *   caller provides (they hold dG and dU on return).  Any output pointer may be NULL: that gradient
  *   is not computed, and what only it needs is not read (with dx, dw_gate, dw_up, db_gate and
  *   db_up all NULL nothing behind dG, dU runs and w_down, g, u, dg, du may be NULL too).
- *   Every launch goes to `stream`, in that order.
+ *   Every launch goes to `stream`, in that order; dx, the weight gradients and the bias gradients may share one.
  *
  * workspace: gmlp_mlp_workspace_bytes(GMLP_PASS_FWD or GMLP_PASS_BWD, M, K, N, dtype) bytes (may be
  * NULL or smaller for a pass without bias gradients: launches then use what it holds, with the same
@@ -279,6 +279,8 @@ int gmlp_decode_stream_fwd(const void* x, const void* w_gate, const void* w_up, 
  * gradients by themselves may use more (fewer tiles, more splits); such a pass uses the largest of
  * gmlp_workspace_bytes of GMLP_OP_DH_BWD and GMLP_OP_DX_BWD, gmlp_dw_bwd_grouped_workspace_bytes of
  * its weight gradients in the order above, and the sum of GMLP_OP_COLSUM over its bias gradients.
+ * Where that holds the partial sums of dx and of the weight gradients side by side (GMLP_OP_DX_BWD's bytes plus
+ * those of the weight gradients always do) they can share launches: the same results, sooner.
  */
 enum gmlp_pass { GMLP_PASS_FWD = 0, GMLP_PASS_BWD = 1 };
 size_t gmlp_mlp_workspace_bytes(int pass, int64_t M, int64_t K, int64_t N, int dtype);

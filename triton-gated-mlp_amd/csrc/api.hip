@@ -471,13 +471,17 @@ hipError_t run_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red
 // dX and the weight gradients as one grid.  Behind each other both end in a round that does not fill the
 // chip; in one grid the workgroups with the longer tiles come first and the others fill what those leave.
 // Estimated by dealing the workgroups out to the CUs in that order, each at what its class takes in a full
-// round, and taken where that is ahead of the separate launches' estimates: mostly below about 4000 rows
-// (4096x4096x14336 and 7431x2208x3296 stay as they are: many rounds, 0.999 to 1.001 of the time either way).
-// dX keeps the number of splits that it has by itself, so that the results are the same bit for
-// bit; shared-out tiles (stream-K) and split weight gradients keep launches of their own.
+// round (and a fifth of it at a perfect deal: CUs that are at different places of their tiles get a larger share
+// of the bandwidth each), and taken where that is ahead of the separate launches' estimates: mostly below about
+// 4000 rows (4096x4096x14336 and 7431x2208x3296 stay as they are: many rounds, 0.999 to 1.001 of the time
+// either way).  Fitted over 116 shapes of 64 to 8192 rows and 128 to 4700 inputs, each on all four pairs of
+// classes and separately: backward passes take 0.907 of the time with this choice, 0.898 with the best one, at worst 1.02.
+// Both keep the number of splits that they have by themselves, so that the results are the same bit for bit, and
+// one launch adds up the partial sums of both; shared-out tiles (stream-K) keep launches of their own.
 struct DxDwPlan {
   bool merged = false, dx_first = true;  // dX in the grid
   int x_class = 0, splits = 1;           // ... its tiles
+  int dw_splits = 1;                     // ... and of the weight gradients
   int dw_class = -1;                     // the weight gradients' tiles in one grid of their own, or -1: not one grid
 };
 // When `slots` that take the next workgroup as they get free are through with n0 workgroups of d0 us and then n1 of d1 us.
@@ -502,21 +506,24 @@ DxDwPlan make_plan_dx_dw(int dtype, int64_t M, int64_t K, int64_t N, int count, 
   for (int i = 0; i < count; ++i)
     if (plan_gemm(dtype, DW, R[i], C[i], M, false).tile_class == gmlp::TILE_MEDIUM) return p;
   const GemmPlan pw = plan_dw_group(count, M, R, C);
-  if (pw.splits > 1) return p;  // (also where the workspace does not hold them)
+  const size_t dw_bytes = dw_group_split_bytes(count, pw.splits, R, C);
+  if (dw_bytes > workspace_bytes) return p;
   const int64_t ktx = red_tiles_of(DX, N), ktw = cdiv(M, 64), large = dw_group_tiles(kLarge, count, R, C);
   if (pw.tile_class == gmlp::TILE_LARGE && plan_streamk(dtype, large, ktw, false).tiles > 0) return p;
   const double dw_us = planned_dw_group_us(M, large, pw);
-  if (dw_us == pw.us) p.dw_class = pw.tile_class;
+  if (pw.splits == 1 && dw_us == pw.us) p.dw_class = pw.tile_class;
   GemmPlan px = plan_gemm(dtype, DX, M, K, N, true);
   if (px.splits > 1 && workspace_bytes < split_workspace_bytes(px.splits, M, K)) px = plan_gemm(dtype, DX, M, K, N, false);
-  if (px.tile_class == gmlp::TILE_MEDIUM) return p;
+  const size_t dx_bytes = split_workspace_bytes(px.splits, M, K);
+  if (px.tile_class == gmlp::TILE_MEDIUM || dx_bytes + dw_bytes > workspace_bytes) return p;
   if (px.tile_class == gmlp::TILE_LARGE && plan_streamk(dtype, tiles_of(kLarge, DX, M, K), ktx).tiles > 0) return p;
   double best = planned_us(DX, M, K, N, px) + dw_us;
-  const int64_t kt = cdiv(ktx, px.splits), cus = num_cu();
-  const double second = px.splits > 1 ? 4.0 + (double)px.splits * (double)M * (double)K * 4.0 / 2.7e6 : 0.0;
-  auto consider = [&](const TileCost& cx, const TileCost& cw, double measured) {
-    const int64_t slots = cx.per_cu * cus, nx = tiles_of(cx, DX, M, K) * px.splits, nw = dw_group_tiles(cw, count, R, C);
-    double dx = (double)kt * cx.r[1] + cx.e[px.splits > 1 ? 5 : DX], dw = (double)ktw * cw.r[2] + cw.e[DW];
+  const int64_t kt = cdiv(ktx, px.splits), kt_dw = cdiv(ktw, pw.splits), cus = num_cu();
+  // (the splits' partial sums are written while other workgroups compute, and are read from the cache)
+  const double second = dx_bytes + dw_bytes > 0 ? 1.5 + (double)(dx_bytes + dw_bytes) / 1.8e7 : 0.0;
+  auto consider = [&](const TileCost& cx, const TileCost& cw) {
+    const int64_t slots = cx.per_cu * cus, nx = tiles_of(cx, DX, M, K) * px.splits, nw = dw_group_tiles(cw, count, R, C) * pw.splits;
+    double dx = (double)kt * cx.r[1] + cx.e[px.splits > 1 ? 5 : DX], dw = (double)kt_dw * cw.r[2] + cw.e[pw.splits > 1 ? 5 : DW];
     if (nx + nw < slots) {  // (a partly filled round, see launch_us)
       const double f = (double)(nx + nw) / (double)slots;
       const double fill = cx.half == 0.0 ? cx.base + (1.0 - cx.base) * f
@@ -526,23 +533,23 @@ DxDwPlan make_plan_dx_dw(int dtype, int64_t M, int64_t K, int64_t N, int count, 
       dw *= fill;
     }
     const bool dx_first = dx >= dw;
-    const double us = measured * (3.1 + second + (dx_first ? makespan_us(slots, nx, dx, nw, dw) : makespan_us(slots, nw, dw, nx, dx)));
+    const double makespan = dx_first ? makespan_us(slots, nx, dx, nw, dw) : makespan_us(slots, nw, dw, nx, dx);
+    const double us = 7.5 + 0.8 * makespan + 0.2 * ((double)nx * dx + (double)nw * dw) / (double)slots + second;
     if (us < best) {
       best = us;
       p.merged = true;
       p.dx_first = dx_first;
       p.x_class = cx.tile_class;
       p.splits = px.splits;
+      p.dw_splits = pw.splits;
     }
   };
-  // (times as measured against this estimate: CUs that are at different places of their tiles get a larger share
-  // of the bandwidth each.  Chosen with these factors, a backward pass with its dH takes 0.89 times as long over
-  // 60 shapes of 32 to 8192 rows and 32 to 5000 inputs, at worst 1.017 with runs of one side 2.5 % apart.)
-  consider(kLarge, kLarge, 0.96);
-  consider(kWide, kLarge, 1.02);
+  consider(kMedium, kMedium);
+  if (pw.splits > 1) return p;
+  consider(kLarge, kLarge);
+  consider(kWide, kLarge);
   // (a 192-row tile can reach further past the last row than the others: see make_plan)
-  if (px.splits == 1 && cdiv(M, 192) * 192 * (cdiv(N, 64) * 64) * 2 < ((int64_t)1 << 31) - 4096) consider(kTall, kLarge, 1.0);
-  consider(kMedium, kMedium, 0.98);
+  if (px.splits == 1 && cdiv(M, 192) * 192 * (cdiv(N, 64) * 64) * 2 < ((int64_t)1 << 31) - 4096) consider(kTall, kLarge);
   return p;
 }
 DxDwPlan plan_dx_dw(int dtype, int64_t M, int64_t K, int64_t N, int count, const int64_t* R, const int64_t* C,
@@ -903,7 +910,8 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
       typedef decltype(tag) T;
       GemmGroup<typename EpiStore<T>::Args> grp = {};
       GemmGroup<typename EpiPartial<T>::Args> part = {};
-      grp.count = part.count = count;
+      ReduceGroup<T> sum = {};
+      grp.count = part.count = sum.count = count;
       float* ws = (float*)workspace;
       for (int i = 0; i < count; ++i) {
         fill(grp.ga[i], i);
@@ -911,11 +919,15 @@ int gmlp_dw_bwd_grouped(int count, const void* const* lhs, const void* const* rh
         grp.ea[i] = {(T*)dw[i], nullptr, (int)C[i]};
         part.ga[i] = grp.ga[i];
         part.ea[i] = {ws, (size_t)R[i] * C[i], 0, (int)C[i]};
+        sum.ws[i] = ws;
+        sum.out[i] = (T*)dw[i];
+        sum.n[i] = (size_t)R[i] * C[i];
+        sum.splits[i] = plan.splits;
         ws += (size_t)plan.splits * R[i] * C[i];
       }
       if (plan.splits == 1) return launch_dw_group<T>(plan.tile_class, grp, s);
       if (hipError_t err = launch_dw_group_split<T>(plan.tile_class, part, s)) return err;
-      return launch_splitk_reduce_group<T>(part, grp, s);
+      return launch_splitk_reduce_group<T>(sum, s);
     }));
   }
   const int group_class = plan.tile_class;
@@ -1119,7 +1131,7 @@ namespace {
 // lhs[i]^T . rhs[i] and the column sums.  The sums run as workgroups at the end of the grid that computes the
 // weight gradients, on CUs that its last round leaves free and without a launch (or two) of their own; unsplit weight
 // gradients in a single grid without dX take them along too.  Backward passes with three bias gradients over
-// 43 shapes of 33 to 8192 rows: 0.867 of the time of separate launches, none above 1.01.
+// 46 shapes of 75 to 8192 rows: 0.73 of the time of separate launches (without biases 0.84), none above 1.02.
 int run_gradients(const char* fn, const void* dg, const void* du, const void* w_gate, const void* w_up, void* dx, int count,
                   const void* const* lhs, const void* const* rhs, void* const* dws, int64_t M, int64_t K, int64_t N, const int64_t* R,
                   const int64_t* C, int nsums, const void* const* sum_in, void* const* sum_out, const int64_t* sum_cols, int dtype,
@@ -1142,20 +1154,35 @@ int run_gradients(const char* fn, const void* dg, const void* du, const void* w_
     if constexpr (std::is_same<T, float>::value) {
       return hipErrorInvalidValue;  // not reached
     } else {
-      auto fill = [&](auto& grp) {
+      ReduceGroup<T> sum = {};
+      float* ws = (float*)workspace;
+      auto partial = [&](int splits, void* out, int64_t rows, int64_t cols) {  // where the partial sums of an output go
+        const typename EpiPartial<T>::Args ea = {ws, (size_t)rows * cols, 0, (int)cols};
+        sum.ws[sum.count] = ws;
+        sum.out[sum.count] = (T*)out;
+        sum.n[sum.count] = (size_t)rows * cols;
+        sum.splits[sum.count++] = splits;
+        ws += (size_t)splits * rows * cols;
+        return ea;
+      };
+      auto launch = [&](auto grp) -> hipError_t {
         GemmArgs& ga = grp.gx;
         ga.nxcd = num_xcd();
         ga.A[0] = dg; ga.A[1] = du; ga.B[0] = w_gate; ga.B[1] = w_up;
         ga.M = dx_inside ? (int)M : 0; ga.N = (int)K; ga.K = (int)N; ga.lda = (int)N; ga.ldb = (int)K;
         ga.nseg = 2; ga.group_m = pick_group(M, K); ga.splits = plan.splits;
+        if constexpr (std::is_same<decltype(grp.ex), typename EpiPartial<T>::Args>::value) grp.ex = partial(plan.splits, dx, M, K);
+        else grp.ex = {(T*)dx, nullptr, (int)K};
         grp.w.count = count;
         for (int i = 0; i < count; ++i) {
           GemmArgs& gw = grp.w.ga[i];
           gw.nxcd = num_xcd();
           gw.A[0] = gw.A[1] = lhs[i]; gw.B[0] = gw.B[1] = rhs[i];
           gw.M = (int)R[i]; gw.N = (int)C[i]; gw.K = (int)M; gw.lda = (int)R[i]; gw.ldb = (int)C[i];
-          gw.nseg = 1; gw.group_m = pick_group(R[i], C[i]);
-          grp.w.ea[i] = {(T*)dws[i], nullptr, (int)C[i]};
+          gw.nseg = 1; gw.group_m = pick_group(R[i], C[i]); gw.splits = plan.dw_splits;
+          if constexpr (std::is_same<decltype(grp.w), GemmGroup<typename EpiPartial<T>::Args>>::value)
+            grp.w.ea[i] = partial(plan.dw_splits, dws[i], R[i], C[i]);
+          else grp.w.ea[i] = {(T*)dws[i], nullptr, (int)C[i]};
         }
         grp.nsums = nsums;
         grp.sum_rows = M;
@@ -1164,23 +1191,16 @@ int run_gradients(const char* fn, const void* dg, const void* du, const void* w_
           grp.sums.out[i] = (T*)sum_out[i];
           grp.sums.C[i] = sum_cols[i];
         }
-      };
-      const bool tail = N % 64 != 0;
-      const typename EpiStore<T>::Args store = {(T*)dx, nullptr, (int)K};
-      if (!dx_inside || plan.splits == 1) {
-        DxDwGroup<T, EpiStore<T>> grp = {};
-        fill(grp);
-        grp.ex = store;
         const int x_class = dx_inside ? plan.x_class : plan.dw_class;
-        return tail ? launch_dx_dw_kt<T, true>(x_class, grp, plan.dx_first, s) : launch_dx_dw_kt<T, false>(x_class, grp, plan.dx_first, s);
-      }
-      DxDwGroup<T, EpiPartial<T>> grp = {};
-      fill(grp);
-      grp.ex = {(float*)workspace, (size_t)M * K, 0, (int)K};
-      if (hipError_t err = tail ? launch_dx_dw_split_kt<T, true>(plan.x_class, grp, plan.dx_first, s)
-                                : launch_dx_dw_split_kt<T, false>(plan.x_class, grp, plan.dx_first, s))
-        return err;
-      return launch_splitk_reduce<T, EpiStore<T>>((const float*)workspace, plan.splits, (size_t)M * K, 0, store, M, K, s);
+        if (hipError_t err = N % 64 != 0 ? launch_dx_dw_kt<T, true>(x_class, grp, plan.dx_first, s)
+                                         : launch_dx_dw_kt<T, false>(x_class, grp, plan.dx_first, s))
+          return err;
+        return sum.count > 0 ? launch_splitk_reduce_group<T>(sum, s) : hipSuccess;
+      };
+      const bool dx_split = dx_inside && plan.splits > 1;
+      if (dx_inside && plan.dw_splits > 1)
+        return dx_split ? launch(DxDwGroup<T, EpiPartial<T>, EpiPartial<T>>{}) : launch(DxDwGroup<T, EpiStore<T>, EpiPartial<T>>{});
+      return dx_split ? launch(DxDwGroup<T, EpiPartial<T>>{}) : launch(DxDwGroup<T, EpiStore<T>>{});
     }
   });
   return hip_result(fn, e);

@@ -113,15 +113,7 @@ GMLP_REDUCE_INST(f16, EpiGateUp)
 GMLP_REDUCE_INST(bf16, EpiGateUp)
 #undef GMLP_REDUCE_INST
 
-// The same for the weight gradients of one pass (contiguous outputs without a bias): blockIdx.y
-// selects the problem.
-template <typename T>
-struct ReduceGroup {
-  const float* ws[GEMM_GROUP_MAX];
-  T* out[GEMM_GROUP_MAX];
-  size_t n[GEMM_GROUP_MAX];  // elements of an output, and between consecutive splits
-  int splits[GEMM_GROUP_MAX];
-};
+// The same for the gradients of one pass (contiguous outputs without a bias): blockIdx.y selects the problem.
 template <typename T>
 __global__ void __launch_bounds__(256) splitk_reduce_group_kernel(ReduceGroup<T> g) {
   const int p = blockIdx.y;
@@ -139,25 +131,16 @@ __global__ void __launch_bounds__(256) splitk_reduce_group_kernel(ReduceGroup<T>
   }
 }
 template <typename T>
-hipError_t launch_splitk_reduce_group(const GemmGroup<typename EpiPartial<T>::Args>& part,
-                                      const GemmGroup<typename EpiStore<T>::Args>& out, hipStream_t s) {
-  ReduceGroup<T> g = {};
+hipError_t launch_splitk_reduce_group(const ReduceGroup<T>& g, hipStream_t s) {
   size_t most = 0;
-  for (int i = 0; i < part.count; ++i) {
-    g.ws[i] = part.ea[i].ws;
-    g.out[i] = out.ea[i].out;
-    g.n[i] = part.ea[i].split_stride;
-    g.splits[i] = part.ga[i].splits;
+  for (int i = 0; i < g.count; ++i)
     if (g.n[i] > most) most = g.n[i];
-  }
   size_t blocks = (most / 8 + 255) / 256;
   if (blocks > 256 * 8) blocks = 256 * 8;
-  hipLaunchKernelGGL(splitk_reduce_group_kernel<T>, dim3((unsigned)blocks, part.count), dim3(256), 0, s, g);
+  hipLaunchKernelGGL(splitk_reduce_group_kernel<T>, dim3((unsigned)blocks, g.count), dim3(256), 0, s, g);
   return hipGetLastError();
 }
-#define GMLP_REDUCE_GROUP_INST(T)                                                                          \
-  template hipError_t launch_splitk_reduce_group<T>(const GemmGroup<EpiPartial<T>::Args>&,                 \
-                                                    const GemmGroup<EpiStore<T>::Args>&, hipStream_t);
+#define GMLP_REDUCE_GROUP_INST(T) template hipError_t launch_splitk_reduce_group<T>(const ReduceGroup<T>&, hipStream_t);
 GMLP_REDUCE_GROUP_INST(f16)
 GMLP_REDUCE_GROUP_INST(bf16)
 GMLP_REDUCE_GROUP_INST(float)

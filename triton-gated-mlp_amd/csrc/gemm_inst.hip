@@ -101,17 +101,25 @@ hipError_t launch_dw_group_split<DT>(int, GemmGroup<EpiPartial<DT>::Args>& grp, 
 #elif GMLP_KIND == 5
 template <>
 hipError_t launch_dx_dw_kt<DT, KT>(int x_class, DxDwGroup<DT, EpiStore<DT>>& grp, bool dx_first, hipStream_t s) {
-  if (x_class == TILE_LARGE) return launch_dx_dw_pipelined<DT, 256, 256, 256, EpiStore<DT>, KT>(grp, dx_first, s);
-  if (x_class == TILE_TALL) return launch_dx_dw_pipelined<DT, 192, 256, 256, EpiStore<DT>, KT>(grp, dx_first, s);
-  if (x_class == TILE_WIDE) return launch_dx_dw_pipelined<DT, 128, 256, 256, EpiStore<DT>, KT>(grp, dx_first, s);
-  return launch_dx_dw_pipelined<DT, 128, 128, 128, EpiStore<DT>, KT>(grp, dx_first, s);
+  if (x_class == TILE_LARGE) return launch_dx_dw_pipelined<DT, 256, 256, 256, KT>(grp, dx_first, s);
+  if (x_class == TILE_TALL) return launch_dx_dw_pipelined<DT, 192, 256, 256, KT>(grp, dx_first, s);
+  if (x_class == TILE_WIDE) return launch_dx_dw_pipelined<DT, 128, 256, 256, KT>(grp, dx_first, s);
+  return launch_dx_dw_pipelined<DT, 128, 128, 128, KT>(grp, dx_first, s);
+}
+template <>
+hipError_t launch_dx_dw_kt<DT, KT>(int, DxDwGroup<DT, EpiStore<DT>, EpiPartial<DT>>& grp, bool dx_first, hipStream_t s) {
+  return launch_dx_dw_pipelined<DT, 128, 128, 128, KT>(grp, dx_first, s);
 }
 #elif GMLP_KIND == 6
 template <>
-hipError_t launch_dx_dw_split_kt<DT, KT>(int x_class, DxDwGroup<DT, EpiPartial<DT>>& grp, bool dx_first, hipStream_t s) {
-  if (x_class == TILE_LARGE) return launch_dx_dw_pipelined<DT, 256, 256, 256, EpiPartial<DT>, KT>(grp, dx_first, s);
-  if (x_class == TILE_WIDE) return launch_dx_dw_pipelined<DT, 128, 256, 256, EpiPartial<DT>, KT>(grp, dx_first, s);
-  return launch_dx_dw_pipelined<DT, 128, 128, 128, EpiPartial<DT>, KT>(grp, dx_first, s);
+hipError_t launch_dx_dw_kt<DT, KT>(int x_class, DxDwGroup<DT, EpiPartial<DT>>& grp, bool dx_first, hipStream_t s) {
+  if (x_class == TILE_LARGE) return launch_dx_dw_pipelined<DT, 256, 256, 256, KT>(grp, dx_first, s);
+  if (x_class == TILE_WIDE) return launch_dx_dw_pipelined<DT, 128, 256, 256, KT>(grp, dx_first, s);
+  return launch_dx_dw_pipelined<DT, 128, 128, 128, KT>(grp, dx_first, s);
+}
+template <>
+hipError_t launch_dx_dw_kt<DT, KT>(int, DxDwGroup<DT, EpiPartial<DT>, EpiPartial<DT>>& grp, bool dx_first, hipStream_t s) {
+  return launch_dx_dw_pipelined<DT, 128, 128, 128, KT>(grp, dx_first, s);
 }
 #endif
 

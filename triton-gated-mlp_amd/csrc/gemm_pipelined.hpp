@@ -934,17 +934,18 @@ __global__ void __launch_bounds__(WGM* WGN * 64)
 }
 
 // The input gradient, the weight gradients and the bias gradients of a pass as one grid: workgroups [x0, x0 + dx_wgs) compute
-// dX (EpiPartial: its split reduction's partial sums) on BMX-row tiles, the others the weight gradients on
-// BMW-row tiles.  Matrix-core bound like the grids it stands for; what it takes away is a launch (about 4 us of
+// dX (EpiPartial: its split reduction's partial sums) on BMX-row tiles, the others the weight gradients (EpiPartial: as
+// with dX) on BMW-row tiles.  Matrix-core bound like the grids it stands for; what it takes away is a launch (about 4 us of
 // GPU time) and a partly filled last round.  A backward pass, dH included, before and after, bfloat16: 512x512x512
 // 30.5 -> 22.1 us, 1024x1024x2816 77.7 -> 66.8, 2048x2048x5632 322 -> 313, 3000x1536x4096 276 -> 222.
 // The bias gradients, memory bound, come last, on CUs that the last round of tiles leaves free: with them
 // 310x416x1248 36.0 -> 26.3 us, 2048x2048x5632 320 -> 295, 3762x1848x7392 730 -> 635, and beside the weight gradients
-// alone 1357x1160x3096 128.6 -> 121.5.
+// alone 1357x1160x3096 128.6 -> 121.5.  Split weight gradients (long batches, small weights) add up with dX's
+// partial sums in one launch: 2334x232x616 54 -> 34, 3968x384x832 71 -> 42.
 // Registers and LDS are those of the larger of the bodies: pairs that run at the same number of
 // workgroups a CU.
-template <typename T, int BMX, int BNX, int BMW, typename EpiX, bool KT>
-__global__ void __launch_bounds__(256) gemm_dx_dw_kernel_pipelined(DxDwGroup<T, EpiX> grp) {
+template <typename T, int BMX, int BNX, int BMW, typename EpiX, typename EpiW, bool KT>
+__global__ void __launch_bounds__(256) gemm_dx_dw_kernel_pipelined(DxDwGroup<T, EpiX, EpiW> grp) {
   int pid = (int)blockIdx.x;
   if (grp.nsums > 0 && pid >= grp.sum_first[0]) {
     extern __shared__ __align__(1024) char smem_raw[];
@@ -972,25 +973,25 @@ __global__ void __launch_bounds__(256) gemm_dx_dw_kernel_pipelined(DxDwGroup<T, 
   for (int i = 1; i < GEMM_GROUP_MAX; ++i)
     if (i < grp.w.count && pid >= grp.w.first[i]) g = i;
   GemmArgs ga = grp.w.ga[0];
-  typename EpiStore<T>::Args ea = grp.w.ea[0];
+  typename EpiW::Args ea = grp.w.ea[0];
 #pragma unroll
   for (int i = 1; i < GEMM_GROUP_MAX; ++i)
     if (g == i) { ga = grp.w.ga[i]; ea = grp.w.ea[i]; }
-  gemm_pipelined_body<T, BMW, BMW, 16, 2, 2, true, true, 1, EpiStore<T>>(ga, ea, pid - grp.w.first[g],
-                                                                         grp.w.first[g + 1] - grp.w.first[g]);
+  gemm_pipelined_body<T, BMW, BMW, 16, 2, 2, true, true, 1, EpiW>(ga, ea, pid - grp.w.first[g],
+                                                                  grp.w.first[g + 1] - grp.w.first[g]);
 }
 
-template <typename T, int BMX, int BNX, int BMW, typename EpiX, bool KT>
-hipError_t launch_dx_dw_pipelined(DxDwGroup<T, EpiX>& grp, bool dx_first, hipStream_t s) {
+template <typename T, int BMX, int BNX, int BMW, bool KT, typename EpiX, typename EpiW>
+hipError_t launch_dx_dw_pipelined(DxDwGroup<T, EpiX, EpiW>& grp, bool dx_first, hipStream_t s) {
   typedef PipeConfig<T, BMX, BNX, 16, 2, 2, false, true, 1, wants_ring_a3<T, EpiX>()> CfgX;
-  typedef PipeConfig<T, BMW, BMW, 16, 2, 2, true, true, 1, wants_ring_a3<T, EpiStore<T>>()> CfgW;
+  typedef PipeConfig<T, BMW, BMW, 16, 2, 2, true, true, 1, wants_ring_a3<T, EpiW>()> CfgW;
   constexpr int LDS = CfgX::LDS_BYTES > CfgW::LDS_BYTES ? CfgX::LDS_BYTES : CfgW::LDS_BYTES;
-  constexpr auto kern = gemm_dx_dw_kernel_pipelined<T, BMX, BNX, BMW, EpiX, KT>;
+  constexpr auto kern = gemm_dx_dw_kernel_pipelined<T, BMX, BNX, BMW, EpiX, EpiW, KT>;
   if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, LDS>, s)) return e;
   int total = 0;
   for (int g = 0; g < grp.w.count; ++g) {
     grp.w.first[g] = total;
-    total += ((grp.w.ga[g].M + BMW - 1) / BMW) * ((grp.w.ga[g].N + BMW - 1) / BMW);
+    total += ((grp.w.ga[g].M + BMW - 1) / BMW) * ((grp.w.ga[g].N + BMW - 1) / BMW) * (EpiW::SPLIT ? grp.w.ga[g].splits : 1);
   }
   for (int g = grp.w.count; g <= GEMM_GROUP_MAX; ++g) grp.w.first[g] = total;
   // (no rows: dX not wanted, or in a launch of its own)

@@ -129,11 +129,11 @@ struct GemmGroup {
 
 // The input gradient, the weight gradients and the bias gradients of a pass in a single launch: workgroups
 // [x0, x0 + dx_wgs) belong to the input gradient, those from sum_first[i] on to column sum i.
-template <typename T, typename EpiX>
+template <typename T, typename EpiX, typename EpiW = EpiStore<T>>
 struct DxDwGroup {
   GemmArgs gx;
   typename EpiX::Args ex;
-  GemmGroup<typename EpiStore<T>::Args> w;
+  GemmGroup<typename EpiW::Args> w;
   ColsumGroup<T> sums;
   int64_t sum_rows;
   int x0, dx_wgs, nsums, sum_first[COLSUM_GROUP_MAX];

@@ -89,16 +89,28 @@ hipError_t launch_dw_group(int tile_class, GemmGroup<typename EpiStore<T>::Args>
 template <typename T>
 hipError_t launch_dw_group_split(int tile_class, GemmGroup<typename EpiPartial<T>::Args>& grp, hipStream_t s);
 template <typename T>
-hipError_t launch_splitk_reduce_group(const GemmGroup<typename EpiPartial<T>::Args>& part,
-                                      const GemmGroup<typename EpiStore<T>::Args>& out, hipStream_t s);
+struct ReduceGroup {
+  const float* ws[GEMM_GROUP_MAX + 1];
+  T* out[GEMM_GROUP_MAX + 1];
+  size_t n[GEMM_GROUP_MAX + 1];  // elements of an output, and between consecutive splits
+  int splits[GEMM_GROUP_MAX + 1];
+  int count;
+};
+template <typename T>
+hipError_t launch_splitk_reduce_group(const ReduceGroup<T>& g, hipStream_t s);
 
 // dX and up to three weight gradients as one grid: dX on `x_class` (LARGE, TALL, WIDE beside large tiles of
-// the weight gradients, MEDIUM_FULL beside MEDIUM_FULL ones; a split reduction with EpiPartial, not TALL).
+// the weight gradients, MEDIUM_FULL beside MEDIUM_FULL ones; a split dX, EpiPartial, not TALL; split weight
+// gradients MEDIUM_FULL beside MEDIUM_FULL).
 // The workgroups of the problem that takes longer per tile should come first.
 template <typename T, bool KT>
 hipError_t launch_dx_dw_kt(int x_class, DxDwGroup<T, EpiStore<T>>& grp, bool dx_first, hipStream_t s);
 template <typename T, bool KT>
-hipError_t launch_dx_dw_split_kt(int x_class, DxDwGroup<T, EpiPartial<T>>& grp, bool dx_first, hipStream_t s);
+hipError_t launch_dx_dw_kt(int x_class, DxDwGroup<T, EpiPartial<T>>& grp, bool dx_first, hipStream_t s);
+template <typename T, bool KT>
+hipError_t launch_dx_dw_kt(int x_class, DxDwGroup<T, EpiStore<T>, EpiPartial<T>>& grp, bool dx_first, hipStream_t s);
+template <typename T, bool KT>
+hipError_t launch_dx_dw_kt(int x_class, DxDwGroup<T, EpiPartial<T>, EpiPartial<T>>& grp, bool dx_first, hipStream_t s);
 
 // Generic launcher used by the instantiation units.
 template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool A_KS, bool B_KS, int NB,

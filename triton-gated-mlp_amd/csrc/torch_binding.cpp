@@ -276,21 +276,21 @@ struct MlpBackward : public ag::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     for (ag::SavedVariable* v : {&x_, &Wg_, &Wu_, &Wd_, &acts_, &bg_, &bu_}) v->reset_data();
   }
-  // What the launches for the gradients asked for use, one after the other: some of the weight gradients by
-  // themselves may take more than all three together (fewer tiles, more splits).
+  // What the launches for the gradients asked for use, one after the other, dX and the weight gradients side by
+  // side: some of the weight gradients by themselves may take more than all three together (fewer tiles, more splits).
   size_t workspace_of(const ag::variable_list& out) const {
     const bool hidden = out[0].defined() || out[1].defined() || out[2].defined() || out[3].defined() || out[4].defined();
     size_t bytes = hidden ? lib.gmlp_workspace_bytes(GMLP_OP_DH_BWD, q.M, q.K, q.N, q.code) : 0;
-    if (out[0].defined()) bytes = std::max(bytes, lib.gmlp_workspace_bytes(GMLP_OP_DX_BWD, q.M, q.K, q.N, q.code));
+    size_t grads = out[0].defined() ? lib.gmlp_workspace_bytes(GMLP_OP_DX_BWD, q.M, q.K, q.N, q.code) : 0;
     int64_t R[3], C[3];
     int n = 0;
     for (int i = 1; i <= 5; i += 2)
       if (out[i].defined()) R[n] = i < 5 ? q.N : q.K, C[n] = i < 5 ? q.K : q.N, ++n;
-    if (n > 0) bytes = std::max(bytes, lib.gmlp_dw_bwd_grouped_workspace_bytes(n, q.M, R, C, q.code));
+    if (n > 0) grads += lib.gmlp_dw_bwd_grouped_workspace_bytes(n, q.M, R, C, q.code);
     size_t sums = 0;
     for (int i = 2; i <= 6; i += 2)
       if (out[i].defined()) sums += lib.gmlp_workspace_bytes(GMLP_OP_COLSUM, q.M, 0, i < 6 ? q.N : q.K, q.code);
-    return std::max(bytes, sums);
+    return std::max({bytes, grads, sums});
   }
   ag::variable_list apply(ag::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
