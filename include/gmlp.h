@@ -294,6 +294,17 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
                  int64_t N, int dtype, int act, float dropout_p, uint64_t seed, uint64_t offset, void* workspace,
                  size_t workspace_bytes, void* stream);
 
+/*
+ * gmlp_hidden_bwd: the backward pass of the hidden states alone, from dh [M,N]: dG, dU (gmlp_gating_bwd), then dx, dw_gate,
+ *   dw_up, db_gate, db_up as in gmlp_mlp_bwd (any of them may be NULL), the same values as the separate
+ *   calls give.  Stands behind the operator's autograd backward (src/triton_gated_mlp/ops/bwd.py:466-602).
+ * workspace: as for gmlp_mlp_bwd, without GMLP_OP_DH_BWD and the down projection's gradients.
+ */
+int gmlp_hidden_bwd(const void* dh, const void* x, const void* w_gate, const void* w_up, const void* g, const void* u,
+                    void* dg, void* du, void* dx, void* dw_gate, void* dw_up, void* db_gate, void* db_up, int64_t M,
+                    int64_t K, int64_t N, int dtype, int act, float dropout_p, uint64_t seed, uint64_t offset,
+                    void* workspace, size_t workspace_bytes, void* stream);
+
 /* Writes the dropout keep mask (1 = keep) for an [M,N] tensor; the test oracle of the generator. */
 int gmlp_dropout_mask(uint8_t* mask, int64_t M, int64_t N, float dropout_p, uint64_t seed,
                       uint64_t offset, void* stream);

@@ -1047,6 +1047,7 @@ def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
     """gmlp_mlp_bwd may run dX, whichever weight gradients are wanted and the bias gradients as one grid: the same sums in
     the same order as the entry points of their own (held against the oracle elsewhere), hence equal bit for bit."""
     from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
 
     g = torch.Generator(device=_dev()).manual_seed(M + N)
     rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g, device=_dev())).to(dtype)
@@ -1064,6 +1065,18 @@ def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
         for w, a, b in zip(wanted, got[1::2], got[2::2]):
             assert torch.equal(a, next(dws)) if w else a is None, f"a weight gradient differs for {wanted}"
             assert torch.equal(b, next(dbs)) if w and biases else b is None, f"a bias gradient differs for {wanted}"
+    # ... and the hidden-state operator's backward, whose grid has no down projection
+    from triton_gated_mlp import FusedGatedMLPFunction
+
+    leaves = [t.detach().clone().requires_grad_(True) for t in (x, wu, rnd(N), wg, rnd(N))]
+    grad = rnd(M, N)
+    FusedGatedMLPFunction.apply(*leaves).backward(grad)
+    hs = ops_fwd.gateup_fwd(x, wg, leaves[4].detach(), wu, leaves[2].detach(), save_activations=True)
+    dg, du = ops_bwd.gating_bwd(grad, hs.gate, hs.up)
+    dwu, dwg = ops_bwd.dw_bwd_grouped([(du, x), (dg, x)])
+    dbu, dbg = ops_bwd.colsum_grouped([du, dg])
+    for t, want in zip(leaves, (ops_bwd.dx_bwd(dg, du, wg, wu), dwu, dbu, dwg, dbg)):
+        assert torch.equal(t.grad, want)
     torch.cuda.synchronize()
 
 

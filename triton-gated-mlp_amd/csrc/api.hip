@@ -1314,4 +1314,36 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
                        workspace, ws_bytes, stream);
 }
 
+int gmlp_hidden_bwd(const void* dh, const void* x, const void* w_gate, const void* w_up, const void* g, const void* u,
+                    void* dg, void* du, void* dx, void* dw_gate, void* dw_up, void* db_gate, void* db_up, int64_t M,
+                    int64_t K, int64_t N, int dtype, int act, float dropout_p, uint64_t seed, uint64_t offset,
+                    void* workspace, size_t workspace_bytes, void* stream) {
+  GMLP_REQUIRE_DTYPE(dtype);
+  if (int rc = check_dims(__func__, M, K, N)) return rc;
+  if (int rc = check_mult8(__func__, "K", K)) return rc;
+  if (int rc = check_mult8(__func__, "N", N)) return rc;
+  if (dx) { GMLP_REQUIRE_PTR(w_gate); GMLP_REQUIRE_PTR(w_up); }
+  if (dw_gate || dw_up) GMLP_REQUIRE_PTR(x);
+  GMLP_REQUIRE_ALIGNED(x); GMLP_REQUIRE_ALIGNED(w_gate); GMLP_REQUIRE_ALIGNED(w_up); GMLP_REQUIRE_ALIGNED(dx);
+  GMLP_REQUIRE_ALIGNED(dw_gate); GMLP_REQUIRE_ALIGNED(dw_up); GMLP_REQUIRE_ALIGNED(db_gate); GMLP_REQUIRE_ALIGNED(db_up);
+  GMLP_REQUIRE_ALIGNED(workspace);
+  const size_t ws_bytes = workspace != nullptr ? workspace_bytes : 0;
+  const size_t sums = bias_workspace_bytes(M, K, N, db_gate, db_up, false);
+  if (sums > ws_bytes)
+    return fail(GMLP_EINVAL, "%s: bias gradients need a workspace of at least %zu bytes", __func__, sums);
+  if (int rc = gmlp_gating_bwd(dh, g, u, dg, du, M, N, dtype, act, dropout_p, seed, offset, stream)) return rc;
+
+  const void* lhs[2]; const void* rhs[2] = {x, x}; void* dws[2];
+  const int64_t R[2] = {N, N}, C[2] = {K, K};
+  int n = 0;
+  if (dw_gate) { lhs[n] = dg; dws[n] = dw_gate; ++n; }
+  if (dw_up) { lhs[n] = du; dws[n] = dw_up; ++n; }
+  const void* cs_in[2]; void* cs_out[2];
+  int nb = 0;
+  if (db_gate) { cs_in[nb] = dg; cs_out[nb] = db_gate; ++nb; }
+  if (db_up) { cs_in[nb] = du; cs_out[nb] = db_up; ++nb; }
+  return run_gradients(__func__, dg, du, w_gate, w_up, dx, n, lhs, rhs, dws, M, K, N, R, C, nb, cs_in, cs_out, R, dtype,
+                       workspace, ws_bytes, stream);
+}
+
 }  // extern "C"

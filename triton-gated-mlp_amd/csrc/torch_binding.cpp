@@ -41,8 +41,8 @@ typedef std::optional<Tensor> OptTensor;
 
 #define GMLP_ENTRY_POINTS(X)                                                                     \
   X(gmlp_last_error) X(gmlp_workspace_bytes) X(gmlp_mlp_workspace_bytes) X(gmlp_mlp_fwd)         \
-  X(gmlp_mlp_bwd) X(gmlp_gateup_fwd) X(gmlp_decode_fwd) X(gmlp_decode_stream_fwd) X(gmlp_gating_bwd) X(gmlp_dx_bwd) \
-  X(gmlp_dw_bwd_grouped_workspace_bytes) X(gmlp_dw_bwd_grouped) X(gmlp_colsum_grouped)
+  X(gmlp_mlp_bwd) X(gmlp_gateup_fwd) X(gmlp_decode_fwd) X(gmlp_decode_stream_fwd) X(gmlp_hidden_bwd) \
+  X(gmlp_dw_bwd_grouped_workspace_bytes)
 struct Library {
 #define GMLP_MEMBER(name) decltype(&::name) name = nullptr;
   GMLP_ENTRY_POINTS(GMLP_MEMBER)
@@ -424,38 +424,21 @@ struct HiddenBackward : public ag::Node {
       out[i] = q.M == 0 ? at::zeros(sizes, dh.options()) : at::empty(sizes, dh.options());
     }
     if (q.M == 0) return out;
-    // the weight gradients as one grid, the bias gradients as one pair of launches
-    const void *lhs[2], *rhs[2], *summed[2];
-    void *dw[2], *db[2];
-    int64_t R[2], C[2];
-    int nw = 0, nb = 0;
+    // dG, dU and the library's workspace (dX and the weight gradients side by side, see MlpBackward) share one
+    // scratch allocation
     const size_t plane = ((size_t)(q.M * q.N) * dh.element_size() + 255) / 256 * 256;
-    for (int i = 1; i <= 4; i += 2)
-      if (out[i].defined()) R[nw] = q.N, C[nw] = q.K, ++nw;
-    const size_t dx_bytes = out[0].defined() ? lib.gmlp_workspace_bytes(GMLP_OP_DX_BWD, q.M, q.K, q.N, q.code) : 0;
-    const size_t dw_bytes = nw > 0 ? lib.gmlp_dw_bwd_grouped_workspace_bytes(nw, q.M, R, C, q.code) : 0;
-    size_t db_bytes = 0;
-    for (int i = 2; i <= 4; i += 2)
-      if (out[i].defined()) db_bytes += lib.gmlp_workspace_bytes(GMLP_OP_COLSUM, q.M, 0, q.N, q.code);
-    const size_t bytes = std::max(dx_bytes, std::max(dw_bytes, db_bytes));
+    const int64_t R[2] = {q.N, q.N}, C[2] = {q.K, q.K};
+    const int nw = (int)out[1].defined() + (int)out[3].defined(), nb = (int)out[2].defined() + (int)out[4].defined();
+    size_t bytes = out[0].defined() ? lib.gmlp_workspace_bytes(GMLP_OP_DX_BWD, q.M, q.K, q.N, q.code) : 0;
+    if (nw > 0) bytes += lib.gmlp_dw_bwd_grouped_workspace_bytes(nw, q.M, R, C, q.code);
+    if (nb > 0) bytes = std::max(bytes, nb * lib.gmlp_workspace_bytes(GMLP_OP_COLSUM, q.M, 0, q.N, q.code));
     const Tensor arena = scratch(2 * plane + bytes, x);
     char *const dg = (char*)out_ptr(arena), *const du = dg + plane, *const ws = bytes > 0 ? du + plane : nullptr;
-    nw = 0;
-    for (int i = 1; i <= 4; ++i) {
-      if (!out[i].defined()) continue;
-      const char* from = i <= 2 ? du : dg;
-      if (i % 2 == 1) lhs[nw] = from, rhs[nw] = ptr(x), dw[nw] = out_ptr(out[i]), ++nw;
-      else summed[nb] = from, db[nb] = out_ptr(out[i]), ++nb;
-    }
-    void* const stream = stream_of(dh);
     const char* g = (const char*)ptr(kept);
     const char* u = g + q.M * q.N * (int64_t)kept.element_size();
-    check(lib.gmlp_gating_bwd(ptr(dh), g, u, dg, du, q.M, q.N, q.code, q.act, (float)q.p, q.seed, q.offset, stream));
-    if (out[0].defined())
-      check(lib.gmlp_dx_bwd(dg, du, ptr(Wg), ptr(Wu), out_ptr(out[0]), q.M, q.K, q.N, q.code, ws, bytes, stream));
-    if (nw > 0) check(lib.gmlp_dw_bwd_grouped(nw, lhs, rhs, dw, q.M, R, C, q.code, ws, bytes, stream));
-    const int64_t cols[2] = {q.N, q.N};
-    if (nb > 0) check(lib.gmlp_colsum_grouped(nb, summed, db, ws, q.M, cols, q.code, stream));
+    check(lib.gmlp_hidden_bwd(ptr(dh), ptr(x), ptr(Wg), ptr(Wu), g, u, dg, du, out_ptr(out[0]), out_ptr(out[3]), out_ptr(out[1]),
+                              out_ptr(out[4]), out_ptr(out[2]), q.M, q.K, q.N, q.code, q.act, (float)q.p, q.seed, q.offset, ws,
+                              bytes, stream_of(dh)));
     refuse_second_derivative(*this, grad, out);
     return out;
   }

@@ -81,6 +81,10 @@ _SIGNATURES = {
         _int,
         [_c_ptr] * 17 + [_i64, _i64, _i64, _int, _int, _f32, _u64, _u64, _c_ptr, ctypes.c_size_t, _c_ptr],
     ),
+    "gmlp_hidden_bwd": (
+        _int,
+        [_c_ptr] * 13 + [_i64, _i64, _i64, _int, _int, _f32, _u64, _u64, _c_ptr, ctypes.c_size_t, _c_ptr],
+    ),
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
