@@ -1,5 +1,8 @@
+import gc
 import sys
 from pathlib import Path
+
+import pytest
 
 ROOT = Path(__file__).resolve().parent.parent
 for p in (ROOT, ROOT / "triton-gated-mlp_amd"):
@@ -9,3 +12,12 @@ for p in (ROOT, ROOT / "triton-gated-mlp_amd"):
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an AMD GPU (run on the MI355X box)")
+
+
+@pytest.fixture(autouse=True)
+def _collected_heap(request):
+    """Tests that account for device memory start without garbage of earlier ones, which a collection in the
+    middle of them would free."""
+    if request.node.path.name == "test_zz_no_alloc.py":
+        gc.collect()
+    yield

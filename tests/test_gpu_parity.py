@@ -1036,13 +1036,13 @@ def test_whole_pass_entry_points_equal_the_separate_launches(M, K, N, dtype, bia
 # dX beside the weight gradients in one grid: 128x128 tiles for both (a single tile each, remainders in every
 # direction, few rows), 256x256 tiles beside a split and an unsplit dX, 192-row and 128-row tiles of dX, reduction lengths
 # that are not a multiple of the 64 of a reduction tile; last, shapes next to these that keep launches of their own
-# (split weight gradients, shared-out tiles).  Bias gradients take their place behind the tiles.
+# (shared-out tiles) or split the weight gradients.  Bias gradients take their place behind the tiles.
 @pytest.mark.parametrize(
     "M,K,N",
     [(1, 8, 8), (129, 136, 264), (33, 512, 1528), (512, 512, 1536), (1024, 1024, 2816), (1000, 1024, 2824), (3000, 1536, 4096),
      (2999, 1528, 4104), (384, 1984, 5440), (271, 2456, 6600), (6656, 1472, 1472), (3456, 384, 1536), (842, 5032, 13520)],
 )
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
     """gmlp_mlp_bwd may run dX, whichever weight gradients are wanted and the bias gradients as one grid: the same sums in
     the same order as the entry points of their own (held against the oracle elsewhere), hence equal bit for bit."""

@@ -139,17 +139,18 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // widths 40 to 14400, both classes, 1 to 16 splits): standard deviation of the estimates 6 %, what it picks
 // costs 1.2 % over the fastest on average.  What that is worth at M=2048, K=1024, N=2816: down projection
 // on 128x128 tiles (128 of them) unsplit 136 us, in 4 splits 74, 64x64 unsplit 90; dX 258 / 128 / 169.
+// us per reduction tile with 1, 2, 3 workgroups on a CU; us of an epilogue
+const double kF32R128[] = {1.568, 2.482}, kF32R64[] = {0.696, 1.015, 1.334}, kF32R64x2[] = {1.140, 1.663};
+const double kF32E128 = 1.414, kF32E64 = 0.168;
 GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes, int64_t max_splits,
                   double split_us) {
   GemmPlan best = {gmlp::TILE_F32_128, 1, 1e30};
   const int64_t cus = num_cu();
   auto consider = [&](int tile_class, int64_t tiles, int64_t splits) {
-    // us per reduction tile with 1, 2, 3 workgroups on a CU; us of an epilogue
-    static const double r128[] = {1.568, 2.482}, r64[] = {0.696, 1.015, 1.334}, r64x2[] = {1.140, 1.663};
     const bool big = tile_class == gmlp::TILE_F32_128;
-    const double* r = big ? r128 : sets == 2 ? r64x2 : r64;
+    const double* r = big ? kF32R128 : sets == 2 ? kF32R64x2 : kF32R64;
     const int64_t cap = big || sets == 2 ? 2 : 3, wgs = tiles * splits, k = cdiv(red_tiles, splits), rest = wgs % (cus * cap);
-    const double e = big ? 1.414 : 0.168;
+    const double e = big ? kF32E128 : kF32E64;
     double us = 5.3 + (double)(wgs / (cus * cap)) * ((double)k * r[cap - 1] + e);
     if (rest > 0) {
       const int64_t per = cdiv(rest, cus);
@@ -500,6 +501,41 @@ double makespan_us(int64_t slots, int64_t n0, double d0, int64_t n1, double d1) 
   };
   return std::max(late, std::min(end_from(early), end_from(late)));
 }
+// float32: the estimates of plan_f32, all on the same tiles.
+DxDwPlan make_plan_dx_dw_f32(int64_t M, int64_t K, int64_t N, int count, const int64_t* R, const int64_t* C, size_t workspace_bytes) {
+  DxDwPlan p;
+  const GemmPlan pw = plan_dw_group_f32(count, M, R, C);
+  const size_t dw_bytes = dw_group_split_bytes(count, pw.splits, R, C);
+  if (dw_bytes > workspace_bytes) return p;
+  if (pw.splits == 1) p.dw_class = pw.tile_class;
+  GemmPlan px = plan_gemm(GMLP_F32, DX, M, K, N, true);
+  if (px.splits > 1 && workspace_bytes < split_workspace_bytes(px.splits, M, K)) px = plan_gemm(GMLP_F32, DX, M, K, N, false);
+  const size_t dx_bytes = split_workspace_bytes(px.splits, M, K);
+  if (dx_bytes + dw_bytes > workspace_bytes) return p;
+  double best = px.us + pw.us;
+  const int64_t cus = num_cu(), kx = cdiv(2 * cdiv(N, 32), px.splits), kw = cdiv(cdiv(M, 32), pw.splits);
+  for (int64_t b : {128, 64}) {
+    const double* r = b == 128 ? kF32R128 : kF32R64;
+    const double e = b == 128 ? kF32E128 : kF32E64;
+    const int64_t nx = cdiv(M, b) * cdiv(K, b) * px.splits;
+    int64_t nw = 0;
+    for (int i = 0; i < count; ++i) nw += cdiv(R[i], b) * cdiv(C[i], b) * pw.splits;
+    const int64_t per = std::min<int64_t>(cdiv(nx + nw, cus), b == 128 ? 2 : 3);
+    const double dx = (double)kx * r[per - 1] + e, dw = (double)kw * r[per - 1] + e;
+    const bool dx_first = dx >= dw;
+    double us = 5.3 + (dx_first ? makespan_us(per * cus, nx, dx, nw, dw) : makespan_us(per * cus, nw, dw, nx, dx));
+    if (dx_bytes + dw_bytes > 0) us += kSplitF32 + 0.382e-6 * (double)(dx_bytes + dw_bytes);
+    if (us < best) {
+      best = us;
+      p.merged = true;
+      p.dx_first = dx_first;
+      p.x_class = b == 128 ? gmlp::TILE_F32_128 : gmlp::TILE_F32_64;
+      p.splits = px.splits;
+      p.dw_splits = pw.splits;
+    }
+  }
+  return p;
+}
 DxDwPlan make_plan_dx_dw(int dtype, int64_t M, int64_t K, int64_t N, int count, const int64_t* R, const int64_t* C,
                          size_t workspace_bytes) {
   DxDwPlan p;
@@ -564,7 +600,8 @@ DxDwPlan plan_dx_dw(int dtype, int64_t M, int64_t K, int64_t N, int count, const
   const int64_t key[6] = {M, K, N, ((int64_t)num_cu() * 4 + dtype) * 8 + count, wide, (int64_t)workspace_bytes};
   Entry& e = cache[(uint64_t)(M * 0x9E3779B1 + K * 0x85EBCA77 + N * 0xC2B2AE3D + key[3] * 0x27D4EB2F + wide) >> 7 & 31];
   if (!std::equal(key, key + 6, e.key)) {
-    e.plan = make_plan_dx_dw(dtype, M, K, N, count, R, C, workspace_bytes);
+    e.plan = dtype == GMLP_F32 ? make_plan_dx_dw_f32(M, K, N, count, R, C, workspace_bytes)
+                               : make_plan_dx_dw(dtype, M, K, N, count, R, C, workspace_bytes);
     std::copy(key, key + 6, e.key);
   }
   return e.plan;
@@ -1138,7 +1175,7 @@ int run_gradients(const char* fn, const void* dg, const void* du, const void* w_
                   void* workspace, size_t ws_bytes, void* stream) {
   using namespace gmlp;
   DxDwPlan plan;
-  if (count > 0 && dtype != GMLP_F32 && (dx || nsums > 0))
+  if (count > 0 && (dx || nsums > 0))
     plan = plan_dx_dw(dtype, M, K, N, count, R, C, workspace ? ws_bytes : 0);
   const bool dx_inside = dx && plan.merged;
   if (dx && !dx_inside)
@@ -1151,57 +1188,54 @@ int run_gradients(const char* fn, const void* dg, const void* du, const void* w_
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = by_dtype(dtype, [&](auto tag) -> hipError_t {
     typedef decltype(tag) T;
-    if constexpr (std::is_same<T, float>::value) {
-      return hipErrorInvalidValue;  // not reached
-    } else {
-      ReduceGroup<T> sum = {};
-      float* ws = (float*)workspace;
-      auto partial = [&](int splits, void* out, int64_t rows, int64_t cols) {  // where the partial sums of an output go
-        const typename EpiPartial<T>::Args ea = {ws, (size_t)rows * cols, 0, (int)cols};
-        sum.ws[sum.count] = ws;
-        sum.out[sum.count] = (T*)out;
-        sum.n[sum.count] = (size_t)rows * cols;
-        sum.splits[sum.count++] = splits;
-        ws += (size_t)splits * rows * cols;
-        return ea;
-      };
-      auto launch = [&](auto grp) -> hipError_t {
-        GemmArgs& ga = grp.gx;
-        ga.nxcd = num_xcd();
-        ga.A[0] = dg; ga.A[1] = du; ga.B[0] = w_gate; ga.B[1] = w_up;
-        ga.M = dx_inside ? (int)M : 0; ga.N = (int)K; ga.K = (int)N; ga.lda = (int)N; ga.ldb = (int)K;
-        ga.nseg = 2; ga.group_m = pick_group(M, K); ga.splits = plan.splits;
-        if constexpr (std::is_same<decltype(grp.ex), typename EpiPartial<T>::Args>::value) grp.ex = partial(plan.splits, dx, M, K);
-        else grp.ex = {(T*)dx, nullptr, (int)K};
-        grp.w.count = count;
-        for (int i = 0; i < count; ++i) {
-          GemmArgs& gw = grp.w.ga[i];
-          gw.nxcd = num_xcd();
-          gw.A[0] = gw.A[1] = lhs[i]; gw.B[0] = gw.B[1] = rhs[i];
-          gw.M = (int)R[i]; gw.N = (int)C[i]; gw.K = (int)M; gw.lda = (int)R[i]; gw.ldb = (int)C[i];
-          gw.nseg = 1; gw.group_m = pick_group(R[i], C[i]); gw.splits = plan.dw_splits;
-          if constexpr (std::is_same<decltype(grp.w), GemmGroup<typename EpiPartial<T>::Args>>::value)
-            grp.w.ea[i] = partial(plan.dw_splits, dws[i], R[i], C[i]);
-          else grp.w.ea[i] = {(T*)dws[i], nullptr, (int)C[i]};
-        }
-        grp.nsums = nsums;
-        grp.sum_rows = M;
-        for (int i = 0; i < nsums; ++i) {
-          grp.sums.a[i] = (const T*)sum_in[i];
-          grp.sums.out[i] = (T*)sum_out[i];
-          grp.sums.C[i] = sum_cols[i];
-        }
-        const int x_class = dx_inside ? plan.x_class : plan.dw_class;
-        if (hipError_t err = N % 64 != 0 ? launch_dx_dw_kt<T, true>(x_class, grp, plan.dx_first, s)
-                                         : launch_dx_dw_kt<T, false>(x_class, grp, plan.dx_first, s))
-          return err;
-        return sum.count > 0 ? launch_splitk_reduce_group<T>(sum, s) : hipSuccess;
-      };
-      const bool dx_split = dx_inside && plan.splits > 1;
-      if (dx_inside && plan.dw_splits > 1)
-        return dx_split ? launch(DxDwGroup<T, EpiPartial<T>, EpiPartial<T>>{}) : launch(DxDwGroup<T, EpiStore<T>, EpiPartial<T>>{});
-      return dx_split ? launch(DxDwGroup<T, EpiPartial<T>>{}) : launch(DxDwGroup<T, EpiStore<T>>{});
-    }
+    ReduceGroup<T> sum = {};
+    float* ws = (float*)workspace;
+    auto partial = [&](int splits, void* out, int64_t rows, int64_t cols) {  // where the partial sums of an output go
+      const typename EpiPartial<T>::Args ea = {ws, (size_t)rows * cols, 0, (int)cols};
+      sum.ws[sum.count] = ws;
+      sum.out[sum.count] = (T*)out;
+      sum.n[sum.count] = (size_t)rows * cols;
+      sum.splits[sum.count++] = splits;
+      ws += (size_t)splits * rows * cols;
+      return ea;
+    };
+    auto launch = [&](auto grp) -> hipError_t {
+      GemmArgs& ga = grp.gx;
+      ga.nxcd = num_xcd();
+      ga.A[0] = dg; ga.A[1] = du; ga.B[0] = w_gate; ga.B[1] = w_up;
+      ga.M = dx_inside ? (int)M : 0; ga.N = (int)K; ga.K = (int)N; ga.lda = (int)N; ga.ldb = (int)K;
+      ga.nseg = 2; ga.group_m = pick_group(M, K); ga.splits = plan.splits;
+      if constexpr (std::is_same<decltype(grp.ex), typename EpiPartial<T>::Args>::value) grp.ex = partial(plan.splits, dx, M, K);
+      else grp.ex = {(T*)dx, nullptr, (int)K};
+      grp.w.count = count;
+      for (int i = 0; i < count; ++i) {
+        GemmArgs& gw = grp.w.ga[i];
+        gw.nxcd = num_xcd();
+        gw.A[0] = gw.A[1] = lhs[i]; gw.B[0] = gw.B[1] = rhs[i];
+        gw.M = (int)R[i]; gw.N = (int)C[i]; gw.K = (int)M; gw.lda = (int)R[i]; gw.ldb = (int)C[i];
+        gw.nseg = 1; gw.group_m = pick_group(R[i], C[i]); gw.splits = plan.dw_splits;
+        if constexpr (std::is_same<decltype(grp.w), GemmGroup<typename EpiPartial<T>::Args>>::value)
+          grp.w.ea[i] = partial(plan.dw_splits, dws[i], R[i], C[i]);
+        else grp.w.ea[i] = {(T*)dws[i], nullptr, (int)C[i]};
+      }
+      grp.nsums = nsums;
+      grp.sum_rows = M;
+      for (int i = 0; i < nsums; ++i) {
+        grp.sums.a[i] = (const T*)sum_in[i];
+        grp.sums.out[i] = (T*)sum_out[i];
+        grp.sums.C[i] = sum_cols[i];
+      }
+      const int x_class = dx_inside ? plan.x_class : plan.dw_class;
+      hipError_t err;
+      if constexpr (std::is_same<T, float>::value) err = launch_dx_dw_kt<T, false>(x_class, grp, plan.dx_first, s);
+      else err = N % 64 != 0 ? launch_dx_dw_kt<T, true>(x_class, grp, plan.dx_first, s) : launch_dx_dw_kt<T, false>(x_class, grp, plan.dx_first, s);
+      if (err) return err;
+      return sum.count > 0 ? launch_splitk_reduce_group<T>(sum, s) : hipSuccess;
+    };
+    const bool dx_split = dx_inside && plan.splits > 1;
+    if (dx_inside && plan.dw_splits > 1)
+      return dx_split ? launch(DxDwGroup<T, EpiPartial<T>, EpiPartial<T>>{}) : launch(DxDwGroup<T, EpiStore<T>, EpiPartial<T>>{});
+    return dx_split ? launch(DxDwGroup<T, EpiPartial<T>>{}) : launch(DxDwGroup<T, EpiStore<T>>{});
   });
   return hip_result(fn, e);
 }

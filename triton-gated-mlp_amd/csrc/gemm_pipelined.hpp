@@ -988,22 +988,8 @@ hipError_t launch_dx_dw_pipelined(DxDwGroup<T, EpiX, EpiW>& grp, bool dx_first, 
   constexpr int LDS = CfgX::LDS_BYTES > CfgW::LDS_BYTES ? CfgX::LDS_BYTES : CfgW::LDS_BYTES;
   constexpr auto kern = gemm_dx_dw_kernel_pipelined<T, BMX, BNX, BMW, EpiX, EpiW, KT>;
   if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, LDS>, s)) return e;
-  int total = 0;
-  for (int g = 0; g < grp.w.count; ++g) {
-    grp.w.first[g] = total;
-    total += ((grp.w.ga[g].M + BMW - 1) / BMW) * ((grp.w.ga[g].N + BMW - 1) / BMW) * (EpiW::SPLIT ? grp.w.ga[g].splits : 1);
-  }
-  for (int g = grp.w.count; g <= GEMM_GROUP_MAX; ++g) grp.w.first[g] = total;
-  // (no rows: dX not wanted, or in a launch of its own)
-  grp.dx_wgs = ((grp.gx.M + BMX - 1) / BMX) * ((grp.gx.N + BNX - 1) / BNX) * (EpiX::SPLIT ? grp.gx.splits : 1);
-  grp.x0 = dx_first ? 0 : total;
-  total += grp.dx_wgs;
   static_assert(LDS >= COLSUM_LDS_BYTES, "the sums' workgroups use the same allocation");
-  for (int i = 0; i < grp.nsums; ++i) {
-    grp.sum_first[i] = total;
-    total += (int)((grp.sums.C[i] + COLSUM_COLS - 1) / COLSUM_COLS);
-  }
-  hipLaunchKernelGGL(kern, dim3(total), dim3(256), LDS, s, grp);
+  hipLaunchKernelGGL(kern, dim3(place_dx_dw<BMX, BNX, BMW>(grp, dx_first)), dim3(256), LDS, s, grp);
   return hipGetLastError();
 }
 

@@ -138,5 +138,24 @@ struct DxDwGroup {
   int64_t sum_rows;
   int x0, dx_wgs, nsums, sum_first[COLSUM_GROUP_MAX];
 };
+// Hands the workgroups out, dX on BMX x BNX tiles, the weight gradients on BMW x BMW ones; how many there are.
+template <int BMX, int BNX, int BMW, typename T, typename EpiX, typename EpiW>
+int place_dx_dw(DxDwGroup<T, EpiX, EpiW>& grp, bool dx_first) {
+  int total = 0;
+  for (int g = 0; g < grp.w.count; ++g) {
+    grp.w.first[g] = total;
+    total += ((grp.w.ga[g].M + BMW - 1) / BMW) * ((grp.w.ga[g].N + BMW - 1) / BMW) * (EpiW::SPLIT ? grp.w.ga[g].splits : 1);
+  }
+  for (int g = grp.w.count; g <= GEMM_GROUP_MAX; ++g) grp.w.first[g] = total;
+  // (no rows: dX not wanted, or in a launch of its own)
+  grp.dx_wgs = ((grp.gx.M + BMX - 1) / BMX) * ((grp.gx.N + BNX - 1) / BNX) * (EpiX::SPLIT ? grp.gx.splits : 1);
+  grp.x0 = dx_first ? 0 : total;
+  total += grp.dx_wgs;
+  for (int i = 0; i < grp.nsums; ++i) {
+    grp.sum_first[i] = total;
+    total += (int)((grp.sums.C[i] + COLSUM_COLS - 1) / COLSUM_COLS);
+  }
+  return total;
+}
 
 }  // namespace gmlp
