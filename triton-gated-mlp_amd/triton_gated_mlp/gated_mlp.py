@@ -150,8 +150,8 @@ class FusedGatedMLPFullFunction(Function):
 
 
 class FusedGatedMLP(_GatedMLPBase):
-    """Drop-in gated MLP running on hand-written gfx950 kernels (float16, bfloat16, or float32 at the
-    rate of the fp32 matrix instructions).  `hidden_act` is any key of ACT_FWD.
+    """Drop-in gated MLP running on hand-written gfx950 kernels (float16, bfloat16, or float32 with each
+    operand split into three bf16 parts).  `hidden_act` is any key of ACT_FWD.
 
     Dropout is active in training mode only.  The keep mask comes from a counter-based generator:
     set `dropout_seed` (int) for a fixed mask stream, otherwise each forward draws a seed from
