@@ -37,7 +37,7 @@ sys.path.insert(0, str(ROOT))
 import torch  # noqa: E402
 
 PEAK_MFMA_F16_TFLOPS = 2500.0  # MI355X dense fp16/bf16 MFMA
-PEAK_MFMA_F32_TFLOPS = PEAK_MFMA_F16_TFLOPS / 6  # float32 products as six bf16 ones
+PEAK_MFMA_F32_TFLOPS = PEAK_MFMA_F16_TFLOPS / 8  # float32 products as eight bf16 ones
 PEAK_HBM_GBPS = 8000.0  # MI355X HBM3E
 
 M, K, N = 8192, 4096, 14336

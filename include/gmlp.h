@@ -11,7 +11,8 @@
  *   - M = tokens (rows of x), K = hidden_size, N = intermediate_size.
  *     W_gate, W_up are [N,K]; W_down is [K,N]  (torch.nn.Linear [out,in] layout).
  *   - dtype: GMLP_F16 or GMLP_BF16 storage (the tuned kernels) or GMLP_F32 (each operand split
- *     into three bf16 parts, at least the accuracy of fp32 MFMA; not for gmlp_decode_fwd); accumulation and epilogue arithmetic are fp32.
+ *     into three bf16 parts, products exact to 2^-33; not for gmlp_decode_fwd); accumulation and epilogue arithmetic
+ *     are fp32.
  *   - Every call only ENQUEUES work on `stream` (a hipStream_t; NULL = default stream) and returns.
  *     The library never allocates or frees device memory and keeps no pointer past a call; the
  *     caller owns every buffer, including workspaces (sizes from gmlp_workspace_bytes).  The one

@@ -1304,6 +1304,50 @@ def test_column_sums_against_float64(M, dtype):
         assert torch.equal(got, ops_bwd.colsum(a))
 
 
+@pytest.mark.parametrize("M,K,N", [(1, 8, 8), (65, 40, 136), (1, 1544, 264), (1, 2056, 4104)])  # both tile classes, splits
+def test_fp32_products_of_single_terms_are_rounded_once(M, K, N):
+    """Sums of which one term alone is not zero, with significands that leave all three bf16 parts of both operands as
+    large as they get (1 + 2^-8 - 2^-17: parts 1, 2^-8, -2^-17) and random ones.  Bound: half a unit of the result, 2^-24,
+    for the last addition; those before it add up what is below 2^-7 of the product, rounded to 2^-24 of that
+    each, and the part that no product covers (third parts with each other) is below 2^-34: 2^-24 (1 + 2^-5)."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(23)
+
+    def full(*shape):
+        """Signs, exponents of 2^-6 to 2^6, 24 significant bits, every fourth one the worst."""
+        t = 1 + torch.rand(shape, generator=g)
+        t[torch.rand(shape, generator=g) < 0.25] = 1 + 2.0**-8 - 2.0**-17
+        return t * 2.0 ** torch.randint(-6, 7, shape, generator=g) * (1 - 2.0 * torch.randint(0, 2, shape, generator=g))
+
+    def lone(rows, red):
+        """One nonzero element to a row."""
+        t = torch.zeros(rows, red)
+        at = torch.randint(0, red, (rows, 1), generator=g)
+        return t.scatter_(1, at, full(rows, 1))
+
+    def check(name, got, ref):
+        worst = ((got.double() - ref).abs() / ref.abs().clamp_min(1e-300)).max().item() * 2.0**24
+        print(f"  {name}: largest error {worst:.3f} of half a unit", flush=True)
+        assert worst <= 1 + 2.0**-5, name
+
+    d = lambda *ts: [t.to(dev) for t in ts]
+    print(f"fp32 single terms: M={M} K={K} N={N}", flush=True)
+    x, h, wg, wu, wd = d(lone(M, K), lone(M, N), full(N, K), full(N, K), full(K, N))
+    hs = ops_fwd.gateup_fwd(x, wg, None, wu, None, save_activations=True)
+    check("G", hs.gate, x.double() @ wg.double().T)
+    check("U", hs.up, x.double() @ wu.double().T)
+    check("Y", ops_fwd.linear_fwd(h, wd), h.double() @ wd.double().T)
+    ones = torch.ones(M, N, device=dev)
+    check("dH", ops_bwd.dh_bwd(x, wd, ones, ones, act_fn="no_act")[1], x.double() @ wd.double())
+    check("dX", ops_bwd.dx_bwd(h, torch.zeros_like(h), wg, wu), h.double() @ wg.double())
+    lhs, rhs = d(lone(N, M).T.contiguous(), full(M, K))  # the weight gradients of one token are such sums
+    (dw,) = ops_bwd.dw_bwd_grouped([(lhs, rhs)])
+    check("dW", dw, lhs.double().T @ rhs.double())
+
+
 @pytest.mark.parametrize("M,K,N", [(72, 40, 136), (130, 1544, 264)])  # one 64-row tile and a bit; split reductions
 def test_fp32_extreme_operands_against_float64_products(M, K, N):
     """Operands that three bf16 parts of 2^16 x do not hold (infinities, NaNs, 2^111 and more), products

@@ -137,11 +137,12 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // less where they are few.  A split reduction pays a second launch and the partial sums' round trip
 // through the caches.  One least-squares fit to the launches of five GEMMs of 70 shapes (M 32 to 6000,
 // widths 40 to 14400, both classes, 1 to 16 splits): standard deviation of the estimates 6 %, what it picks
-// costs 1.2 % over the fastest on average.  What that is worth at M=2048, K=1024, N=2816: down projection
-// on 128x128 tiles (128 of them) unsplit 136 us, in 4 splits 74, 64x64 unsplit 90; dX 258 / 128 / 169.
+// costs 0.5 % over the fastest on average.  What that is worth at M=2048, K=1024, N=2816: down projection
+// on 128x128 tiles (128 of them) unsplit 180 us, in 4 splits 101, 64x64 unsplit 104; dX 330 / 164 / 198.
 // us per reduction tile with 1, 2, 3 workgroups on a CU; us of an epilogue
-const double kF32R128[] = {1.568, 2.482}, kF32R64[] = {0.696, 1.015, 1.334}, kF32R64x2[] = {1.140, 1.663};
-const double kF32E128 = 1.414, kF32E64 = 0.168;
+const double kF32R128[] = {2.008, 3.095}, kF32R64[] = {0.721, 1.167, 1.549}, kF32R64x2[] = {1.271, 1.930};
+const double kF32E128 = 2.790, kF32E64 = 0.925;
+const double kF32Launch = 4.05, kF32Traffic = 0.345e-6;  // us of a launch; of a byte of partial sums
 GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes, int64_t max_splits,
                   double split_us) {
   GemmPlan best = {gmlp::TILE_F32_128, 1, 1e30};
@@ -151,13 +152,13 @@ GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets
     const double* r = big ? kF32R128 : sets == 2 ? kF32R64x2 : kF32R64;
     const int64_t cap = big || sets == 2 ? 2 : 3, wgs = tiles * splits, k = cdiv(red_tiles, splits), rest = wgs % (cus * cap);
     const double e = big ? kF32E128 : kF32E64;
-    double us = 5.3 + (double)(wgs / (cus * cap)) * ((double)k * r[cap - 1] + e);
+    double us = kF32Launch + (double)(wgs / (cus * cap)) * ((double)k * r[cap - 1] + e);
     if (rest > 0) {
       const int64_t per = cdiv(rest, cus);
       const double f = (double)rest / (double)cus - (double)(per - 1);
-      us += (double)k * (r[per - 1] - 0.129 * (1.0 - f) * (r[per - 1] - (per > 1 ? r[per - 2] : 0.0))) + e;
+      us += (double)k * (r[per - 1] - 0.114 * (1.0 - f) * (r[per - 1] - (per > 1 ? r[per - 2] : 0.0))) + e;
     }
-    if (splits > 1) us += split_us + 0.382e-6 * (double)splits * out_bytes * sets;
+    if (splits > 1) us += split_us + kF32Traffic * (double)splits * out_bytes * sets;
     if (us < best.us) best = GemmPlan{tile_class, (int)splits, us};
   };
   for (int64_t s = 1; s <= std::max<int64_t>(1, std::min(max_splits, red_tiles / 4)); ++s) {
@@ -167,10 +168,10 @@ GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets
   }
   return best;
 }
-// What a split costs beside its traffic: 1.6 us on the GPU, and the rest is what the second launch costs the
+// What a split costs beside its traffic: 1.7 us on the GPU, and the rest is what the second launch costs the
 // host, which bounds passes this small.  A forward down projection pays that twice: nothing else in its
 // pass is split at such sizes (training step at M=K=N=512 89.4 us with one launch, 92.4 with two).
-const double kSplitF32 = 4.6, kSplitF32Linear = 8.6;
+const double kSplitF32 = 4.7, kSplitF32Linear = 8.7;
 GemmPlan plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int kind, int64_t max_splits) {
   const int sets = kind == GATEUP ? 2 : 1;
   return plan_f32(cdiv(rows, 128) * cdiv(cols, 128 / sets), cdiv(rows, 64) * cdiv(cols, 64), red_tiles, sets,
@@ -523,8 +524,8 @@ DxDwPlan make_plan_dx_dw_f32(int64_t M, int64_t K, int64_t N, int count, const i
     const int64_t per = std::min<int64_t>(cdiv(nx + nw, cus), b == 128 ? 2 : 3);
     const double dx = (double)kx * r[per - 1] + e, dw = (double)kw * r[per - 1] + e;
     const bool dx_first = dx >= dw;
-    double us = 5.3 + (dx_first ? makespan_us(per * cus, nx, dx, nw, dw) : makespan_us(per * cus, nw, dw, nx, dx));
-    if (dx_bytes + dw_bytes > 0) us += kSplitF32 + 0.382e-6 * (double)(dx_bytes + dw_bytes);
+    double us = kF32Launch + (dx_first ? makespan_us(per * cus, nx, dx, nw, dw) : makespan_us(per * cus, nw, dw, nx, dx));
+    if (dx_bytes + dw_bytes > 0) us += kSplitF32 + kF32Traffic * (double)(dx_bytes + dw_bytes);
     if (us < best) {
       best = us;
       p.merged = true;

@@ -1,28 +1,31 @@
 // float32 path: the GEMMs and fused epilogues for callers that keep the module in float32 (as the
 // reference's own tests do), on the bf16 matrix cores: every operand element is split into three bf16
-// numbers and a product taken as six (gemm_f32_split.hpp).  Six bf16 products cost 6/16 of the time of
-// the fp32 MFMA (v_mfma_f32_32x32x2_f32: 157 TFLOP/s; 2500 bf16), and a bf16 MFMA adds up 32
-// reduction elements where the fp32 one rounds after every two, so the result is also closer to the
-// exact one: relative error against float64 at M=2048, K=1024, N=2816 with fp32 MFMAs -> split: G
-// 5.7e-7 -> 4.9e-7, Y 9.5e-7 -> 8.1e-7, dX 1.35e-6 -> 1.15e-6, dW 8.1e-7 -> 6.9e-7 (lower at all of
-// the 10 shapes measured, M 32 to 6974; also with inputs scaled by 1e-6).
+// numbers and a product taken as eight (gemm_f32_split.hpp), which cost half of the time of the fp32
+// MFMA (v_mfma_f32_32x32x2_f32: 157 TFLOP/s; 2500 bf16).
 //
-// Bound: the matrix cores at the board's power limit.  M=4096, K=2048, N=5632 (us, TFLOP/s of the float32
-// product): gate/up 1381 -> 952 (199), down 712 -> 464 (204), dH 769 -> 555 (170), dX 1428 -> 911 (208),
-// weight gradients 2231 -> 1550 (183); 208 is 1245 of bf16.
+// Precision.  A product enters the sum to 2^-33 of itself.  A bf16 MFMA does not round its sums to nearest (a sum of
+// one term by eight MFMAs into one accumulator comes out up to 2.6 half units off, with six or with eight products), so
+// the seven products that are at most 2^-8 of the whole go to an accumulator of their own, tile by tile, which
+// joins the one of the first parts by an addition.  A sum of one term is then rounded once, as by fp32 MFMAs (largest
+// error 1.00 half units, root mean square 0.47, both), and longer ones come out closer, by fewer roundings:
+// relative error against float64 at M=2048, K=1024, N=2816, fp32 MFMAs -> one accumulator for six products -> this:
+// G 5.7e-7 -> 4.9e-7 -> 2.1e-7, Y 9.5e-7 -> 4.0e-7 -> 1.8e-7, dX 1.34e-6 -> 5.9e-7 -> 2.5e-7, dW 8.1e-7 -> 4.9e-7 ->
+// 2.1e-7 (lower than fp32 MFMAs at all of the 10 shapes measured, 1 to 6974 rows).
+//
+// Bound: the matrix cores at the board's power limit.  M=4096, K=2048, N=5632, fp32 MFMAs -> this (us, TFLOP/s of the
+// float32 product): gate/up 1431 -> 1236 (153), down 717 -> 603 (157), dH 770 -> 619 (153), dX 1439 -> 1165 (162),
+// weight gradients 2234 -> 1762 (161); 162 is 1297 of bf16.  (Six products in one accumulator: 1018, 493, 508, 950, 1397.)
 //
 // A tile of 128 x 128 outputs (or 64 x 64) by 32 reduction elements per workgroup of 4 wavefronts.  The
 // split is done once per workgroup on the way from global memory to LDS (13 VALU instructions per two
 // elements: two or three between two MFMAs), not on every fragment read.  128 x 128: one LDS stage (48 KiB) and all
 // of a tile's fragments in registers (96 VGPRs); the next tile is written while the MFMAs of the current
 // one run, and a CU holds two workgroups, one of which multiplies while the other waits at a barrier or
-// for LDS (128 x 128 x 32 per CU: 1.57 us with one workgroup, 1.24 each with two).  64 x 64 tiles fill the
+// for LDS (128 x 128 x 32 per CU: 2.01 us with one workgroup, 1.55 each with two).  64 x 64 tiles fill the
 // chip on small problems, where a launch is as long as its chain of reduction tiles: two LDS stages (one
 // barrier a tile) and three reduction tiles in flight in registers (down projection at M=64, K=256, N=1024:
 // 27.8 us with one in flight, 26.0 with three).  Reading the fragments of the next tile ahead as well costs
-// the registers of a third workgroup per CU and was 3 to 5 % slower.  Launches of a few reduction tiles are
-// up to 1 us longer than with fp32 MFMAs fed straight from global memory to LDS (32-cube: forward 9.1 ->
-// 9.5 us, backward 12.6 -> 13.4), everything from about 5e8 multiplications on shorter.
+// the registers of a third workgroup per CU and was 3 to 5 % slower.
 #include "gemm_f32_split.hpp"
 #include "launch.hpp"
 
@@ -31,9 +34,13 @@ namespace gmlp {
 // What the chunks beyond the end of a reduction are fetched from.
 static __device__ __align__(16) float f32_zeros[8];
 
-// Which plane of A and which of B the six products take, smallest first.
-constexpr int PROD_A[6] = {2, 0, 1, 1, 0, 0};
-constexpr int PROD_B[6] = {0, 2, 1, 0, 1, 0};
+// Which plane of A and which of B the eight products take, smallest first.
+constexpr int PRODUCTS = 8;
+constexpr int PROD_A[PRODUCTS] = {2, 1, 2, 0, 1, 1, 0, 0};
+constexpr int PROD_B[PRODUCTS] = {1, 2, 0, 2, 1, 0, 1, 0};
+
+// Workgroups on a CU, which the registers have to allow.
+constexpr int f32_per_cu(int bm, int nb) { return bm == 64 && nb == 1 ? 3 : 2; }
 
 template <int BM, int BN, bool A_KS, bool B_KS, int NB>
 struct F32Config {
@@ -177,20 +184,29 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::
     }
     if (NS == 1) __syncthreads();  // and every wavefront has its part of it in registers
     __builtin_amdgcn_sched_barrier(0);
+    // Four 16 x 16 outputs at a time, the small products of the tile in accumulators of their own.
+    constexpr int TOGETHER = 4, GROUPS = TM * G / TOGETHER;
+    static_assert(TM * G % TOGETHER == 0, "whole groups");
 #pragma unroll
-    for (int q = 0; q < 6; ++q) {
+    for (int f = 0; f < GROUPS; ++f) {
 #pragma unroll
       for (int c = 0; c < CH; ++c)
-        if (c * 6 / CH == q) store_chunk(p, c, nxt), load_chunk(p, c);
+        if (c * GROUPS / CH == f) store_chunk(p, c, nxt), load_chunk(p, c);
+      f32x4 small[TOGETHER];
 #pragma unroll
-      for (int g = 0; g < G; ++g)
+      for (int q = 0; q < PRODUCTS; ++q)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int e = 0; e < TOGETHER; ++e) {
+          const int g = (f * TOGETHER + e) / TM, i = (f * TOGETHER + e) % TM;
+          f32x4& sum = q + 1 < PRODUCTS ? small[e] : acc[g][i];
+          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
           // operands swapped: a lane ends up with 4 consecutive output columns of one row
-          acc[g][i] =
-              __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[PROD_B[q]][g], af[PROD_A[q]][i], acc[g][i], 0, 0, 0);
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[PROD_B[q]][g], af[PROD_A[q]][i], q == 0 ? zero : sum, 0, 0, 0);
+        }
 #pragma unroll
-      for (int r = 0; r < TM * G; ++r) {
+      for (int e = 0; e < TOGETHER; ++e) acc[(f * TOGETHER + e) / TM][(f * TOGETHER + e) % TM] += small[e];
+#pragma unroll
+      for (int r = 0; r < PRODUCTS * TOGETHER; ++r) {
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // MFMA
         __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);  // VALU
       }
@@ -265,12 +281,12 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::
 }
 
 template <int BM, int BN, bool A_KS, bool B_KS, int NB, typename Epi>
-__global__ void __launch_bounds__(256, 2) gemm_f32_kernel(GemmArgs ga, typename Epi::Args ea) {
+__global__ void __launch_bounds__(256, f32_per_cu(BM, NB)) gemm_f32_kernel(GemmArgs ga, typename Epi::Args ea) {
   gemm_f32_body<BM, BN, A_KS, B_KS, NB, Epi>(ga, ea, blockIdx.x, gridDim.x);
 }
 
 template <int BM, int BN, typename Epi>
-__global__ void __launch_bounds__(256, 2) gemm_f32_group_kernel(GemmGroup<typename Epi::Args> grp) {
+__global__ void __launch_bounds__(256, f32_per_cu(BM, 1)) gemm_f32_group_kernel(GemmGroup<typename Epi::Args> grp) {
   int g = 0;
 #pragma unroll
   for (int i = 1; i < GEMM_GROUP_MAX; ++i)
@@ -283,7 +299,7 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_group_kernel(GemmGroup<typena
 // types), all on square tiles of the same size.  Backward passes, before and after: 512x512x512 41 -> 36 us, 684x56x224
 // 24.5 -> 17.2 and with biases 30 -> 17.5, 1280x320x1216 95 -> 76 and 103 -> 76.
 template <int B, typename EpiX, typename EpiW>
-__global__ void __launch_bounds__(256, 2) gemm_f32_dx_dw_kernel(DxDwGroup<float, EpiX, EpiW> grp) {
+__global__ void __launch_bounds__(256, f32_per_cu(B, 1)) gemm_f32_dx_dw_kernel(DxDwGroup<float, EpiX, EpiW> grp) {
   int pid = (int)blockIdx.x;
   if (grp.nsums > 0 && pid >= grp.sum_first[0]) {
     extern __shared__ __align__(1024) char smem[];

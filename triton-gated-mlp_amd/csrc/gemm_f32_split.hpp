@@ -1,9 +1,10 @@
 // float32 GEMM on the bf16 matrix cores: C[M,N] = sum_s sum_k A_s[m,k] * B_s[n,k] with every float32
 // operand element, times 2^16, written as the sum of three bf16 numbers, 2^16 x = h + m + l, and the product
-// of two of them as the six products hh, hm, mh, hl, lh, mm, each exact in float32.  Three times 8
+// of two of them as the eight products hh, hm, mh, hl, lh, mm, ml, lm, each exact in float32.  Three times 8
 // significant bits hold the 24 of a float32, and the factor puts the smallest float32 (2^-149) at the
 // smallest bf16 (2^-133; the matrix cores take subnormal ones), so the sum is x exactly for every |x| below
-// 2^111.  What is left out of a product (ml, lm, ll) is below 2^-25 of it.
+// 2^111.  What is left out of a product, ll, is at most 2^-34 of it: |m| <= 2^-8 |x|, |l| <= 2^-17 |x|.  (ml and lm
+// together reach 2^-24, half a unit of the product: both operands 1 + 2^-8 - 2^-17.)
 #pragma once
 #include "gemm.hpp"
 #include "gemm_tiles.hpp"
