@@ -1348,7 +1348,11 @@ def test_fp32_products_of_single_terms_are_rounded_once(M, K, N):
     check("dW", dw, lhs.double().T @ rhs.double())
 
 
-@pytest.mark.parametrize("M,K,N", [(72, 40, 136), (130, 1544, 264)])  # one 64-row tile and a bit; split reductions
+@pytest.mark.parametrize(
+    "M,K,N",
+    [(72, 40, 136), (130, 1544, 264),         # one 64-row tile and a bit; split reductions
+     (1050, 1144, 1096), (1403, 352, 2816)],  # 128-row tiles, with and without splits
+)
 def test_fp32_extreme_operands_against_float64_products(M, K, N):
     """Operands that three bf16 parts of 2^16 x do not hold (infinities, NaNs, 2^111 and more), products
     that overflow on the way, and subnormal ones, in rows and columns of their own beside ordinary ones: NaNs
@@ -1408,6 +1412,43 @@ def test_fp32_extreme_operands_against_float64_products(M, K, N):
     lhs = extreme(rnd(N, M)).T.contiguous()  # reduction over the rows: extremes in columns
     e = exact(M, K)
     check("dW", ops_bwd.dw_bwd(d(lhs), d(e)), [(lhs.T, e)])
+
+
+def test_fp32_operands_that_are_not_finite_cost_a_few_launches_at_most():
+    """A single infinity makes a whole row or column of a product non-finite, a row of them all of a weight gradient: those
+    outputs are computed a second time.  On the fp32 matrix cores that makes it up to three times the usual time here;
+    element by element, as it was, 5 to 43 times.  Bound: twice what is measured."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    M, K, N = 2048, 1024, 2816
+    g = torch.Generator(device=dev).manual_seed(29)
+    rnd = lambda *shape: torch.empty(shape, device=dev).normal_(generator=g)
+    x, dy, h, G, U, wg, wu = rnd(M, K), rnd(M, K), rnd(M, N), rnd(M, N), rnd(M, N), rnd(N, K), rnd(N, K)
+    row, one, w = x.clone(), x.clone(), wg.clone()
+    row[5], one[5, 7], w[3, 9] = float("inf"), float("inf"), float("inf")
+
+    def us(run):
+        times = []
+        for _ in range(4):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(5):
+                run()
+            end.record()
+            torch.cuda.synchronize()
+            times.append(200 * start.elapsed_time(end))
+        return min(times)
+
+    grads = lambda t: ops_bwd.dw_bwd_grouped([(G, t), (U, t), (dy, h)])
+    gates = lambda t: ops_fwd.gateup_fwd(x, t, None, wu, None, save_activations=True)
+    for name, run, finite, extremes in (("weight gradients", grads, x, (row, one)), ("gate/up", gates, wg, (w, wg * 2.0**100))):
+        usual = us(lambda: run(finite))
+        for t in extremes:
+            slow = us(lambda: run(t))
+            print(f"{name}: {usual:.0f} us, with operands that are not finite or near it {slow:.0f}", flush=True)
+            assert slow < 6 * usual, name
 
 
 def test_random_modules_through_the_one_call_entries_no_worse_than_torch_16bit():

@@ -10,7 +10,7 @@
 // error 1.00 half units, root mean square 0.47, both), and longer ones come out closer, by fewer roundings:
 // relative error against float64 at M=2048, K=1024, N=2816, fp32 MFMAs -> one accumulator for six products -> this:
 // G 5.7e-7 -> 4.9e-7 -> 2.1e-7, Y 9.5e-7 -> 4.0e-7 -> 1.8e-7, dX 1.34e-6 -> 5.9e-7 -> 2.5e-7, dW 8.1e-7 -> 4.9e-7 ->
-// 2.1e-7 (lower than fp32 MFMAs at all of the 10 shapes measured, 1 to 6974 rows).
+// 2.1e-7 (10 shapes of 1 to 6974 rows: sums of one term the same as by fp32 MFMAs, of 32 and more 0.2 to 0.6 of the error).
 //
 // Bound: the matrix cores at the board's power limit.  M=4096, K=2048, N=5632, fp32 MFMAs -> this (us, TFLOP/s of the
 // float32 product): gate/up 1431 -> 1236 (153), down 717 -> 603 (157), dH 770 -> 619 (153), dX 1439 -> 1165 (162),
@@ -56,31 +56,54 @@ struct F32Config {
 };
 
 // What the split does not give: operands of magnitude 2^111 and more, infinities among them, leave a NaN
-// as their residual, and results of 2^96 and more overflow in the scaled accumulators.  An accumulator that is
-// not finite is therefore computed again in plain float32; overflows, infinities and NaNs then come out
-// as IEEE arithmetic gives them.
-// Element (m, n) of accumulator set b over reduction tiles [kt_first, kt_end), in float32.
-__device__ __forceinline__ float f32_dot(const GemmArgs& ga, bool a_ks, bool b_ks, int nb, int b, int m, int n, int kt_seg,
-                                         int kt_first, int kt_end) {
-  float sum = 0.f;
+// as their residual, and results of 2^96 and more overflow in the scaled accumulators.  Accumulators that are
+// not finite are therefore computed again with fp32 MFMAs; overflows, infinities and NaNs then come out
+// as IEEE arithmetic gives them.  A launch with few of them takes up to 1.7 times as long, one in which every output is
+// done again two to three times (gate/up of x scaled by 2^100 at M=4096, K=2048, N=5632 1240 -> 3570 us; weight gradients
+// with a row of infinities 1840 -> 4660, all on fp32 MFMAs 2220).  Before, each such output was one lane's dot product:
+// 49000 and 51000 us.
+// 16 rows from m and G times 16 columns (of G / TN operands) from n over reduction tiles [kt_first, kt_end), laid out as
+// the accumulators; operands straight from global memory, 32 reduction elements at a time, lane / 16 choosing four of each half.
+template <bool A_KS, bool B_KS, int G, int TN>
+__device__ __forceinline__ void f32_again(const GemmArgs& ga, f32x4 (&sum)[G], int m, int n, int kt_seg, int kt_first, int kt_end, int lane) {
+#pragma unroll
+  for (int g = 0; g < G; ++g) sum[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // (beyond the matrix: its last row or column, which is not stored)
+  auto four = [&](auto strided, const float* p, int ld, int row, int k, int end) __attribute__((always_inline)) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (decltype(strided)::value) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (k + j < end) v[j] = p[(size_t)(k + j) * ld + row];
+    } else if (k < end) {
+      v = *(const f32x4*)(p + (size_t)row * ld + k);
+    }
+    return v;
+  };
   for (int s = 0; s < ga.nseg; ++s) {
     const int k0 = max(kt_first - s * kt_seg, 0) * 32, k1 = min(min(kt_end - s * kt_seg, kt_seg) * 32, ga.K);
-    const float* pa = (const float*)ga.A[s] + (a_ks ? (size_t)m : (size_t)m * ga.lda);
-    const float* pb = (const float*)ga.B[nb == 2 ? b : s] + (b_ks ? (size_t)n : (size_t)n * ga.ldb);
-    const size_t sa = a_ks ? ga.lda : 1, sb = b_ks ? ga.ldb : 1;
-    int k = k0;
+    const float* pa = (const float*)ga.A[s];
 #pragma unroll 1
-    for (; k + 8 <= k1 && sum == sum; k += 8) {  // (a NaN stays one)
-      float va[8], vb[8];
+    for (int k = k0; k < k1; k += 32) {
+      f32x4 a[2], b[2][G];
+      const int r = lane & 15;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) va[j] = pa[(size_t)(k + j) * sa], vb[j] = pb[(size_t)(k + j) * sb];
+      for (int h = 0; h < 2; ++h) {
+        const int kl = k + 16 * h + 4 * (lane >> 4);
+        a[h] = four(std::integral_constant<bool, A_KS>{}, pa, ga.lda, min(m + r, ga.M - 1), kl, k1);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sum = fmaf(va[j], vb[j], sum);
+        for (int g = 0; g < G; ++g)
+          b[h][g] = four(std::integral_constant<bool, B_KS>{}, (const float*)ga.B[G > TN ? g / TN : s], ga.ldb,
+                         min(n + g % TN * 16 + r, ga.N - 1), kl, k1);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int g = 0; g < G; ++g) sum[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[h][g][j], a[h][j], sum[g], 0, 0, 0);
     }
-#pragma unroll 1
-    for (; k < k1 && sum == sum; ++k) sum = fmaf(pa[(size_t)k * sa], pb[(size_t)k * sb], sum);
   }
-  return sum;
 }
 
 template <int BM, int BN, bool A_KS, bool B_KS, int NB, typename Epi>
@@ -228,17 +251,25 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::
     tile(t + u, (u + 1) % PF);
   }
 
-  float not_finite = 0.f;
 #pragma unroll
-  for (int g = 0; g < G; ++g)
+  for (int i = 0; i < TM; ++i) {
+    float not_finite = 0.f;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         not_finite = fmaf(acc[g][i][r], 0.f, not_finite);
         acc[g][i][r] *= 1.0f / (SPLIT_SCALE * SPLIT_SCALE);
       }
-  const bool suspects = __builtin_amdgcn_ballot_w64(!(not_finite == 0.f)) != 0;
+    if (__builtin_amdgcn_ballot_w64(!(not_finite == 0.f)) == 0) continue;
+    f32x4 again[G];
+    f32_again<A_KS, B_KS, G, TN>(ga, again, m0 + wm * WTM + i * 16, n0 + wn * WTN, kt_seg, kt_first, kt_end, lane);
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (!(acc[g][i][r] * 0.f == 0.f)) acc[g][i][r] = again[g][r];
+  }
 
   __syncthreads();  // the slabs overwrite the operand tiles
   constexpr int ELD = Cfg::ELD, CPW = WTN / 4, ITEMS = 16 * CPW / 64;
@@ -260,15 +291,6 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::
     for (int g = 0; g < G; ++g)
       *(f32x4*)(slab + ((g / TN) * 16 + mrow) * ELD + (g % TN) * 16 + nsub) = acc[g][i];
     // (same-wavefront LDS writes and reads are ordered)
-    if (suspects) {
-#pragma unroll 1
-      for (int e = lane; e < NB * 16 * WTN; e += 64) {
-        const int b = e / (16 * WTN), row = e / WTN % 16, col = e % WTN;
-        float* v = slab + (b * 16 + row) * ELD + col;
-        if (!(*v * 0.f == 0.f) && mw + row < ga.M && nw + col < ga.N)
-          *v = f32_dot(ga, A_KS, B_KS, NB, b, mw + row, nw + col, kt_seg, kt_first, kt_end);
-      }
-    }
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int q = it * 64 + lane, row = q / CPW, col = q % CPW * 4, m = mw + row, n = nw + col;
