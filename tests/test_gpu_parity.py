@@ -1033,6 +1033,18 @@ def test_whole_pass_entry_points_equal_the_separate_launches(M, K, N, dtype, bia
             assert a is None or torch.equal(a, ref[n]), f"{n} differs for subset {want}"
 
 
+def _launched(run):
+    """Names of the kernels that run() launches, and its result."""
+    from torch.profiler import ProfilerActivity, profile
+
+    run()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as prof:
+        result = run()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events() if "gmlp" in e.name], result
+
+
 # dX beside the weight gradients in one grid: 128x128 tiles for both (a single tile each, remainders in every
 # direction, few rows), 256x256 tiles beside a split and an unsplit dX, 192-row and 128-row tiles of dX, reduction lengths
 # that are not a multiple of the 64 of a reduction tile; last, shapes next to these that keep launches of their own
@@ -1078,6 +1090,29 @@ def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
     for t, want in zip(leaves, (ops_bwd.dx_bwd(dg, du, wg, wu), dwu, dbu, dwg, dbg)):
         assert torch.equal(t.grad, want)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize(
+    "M,K,N,dtype,apart",  # rows on both sides of the line; few tiles that all start at once, many, and float32
+    [(8192, 200, 600, torch.bfloat16, False), (65536, 200, 600, torch.bfloat16, True), (16384, 40, 56, torch.float16, False),
+     (43686, 264, 296, torch.float16, True), (8192, 64, 128, torch.float32, False), (123241, 112, 408, torch.float32, True)],
+)
+def test_bias_gradients_of_long_batches_leave_the_gradients_grid(M, K, N, dtype, apart):
+    """A workgroup of the gradients' grid sums all rows of its columns: behind tiles that take less time, launches of their
+    own are faster.  Same sums either way, which path by the launched kernels (on a whole MI355X)."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+
+    dev = _dev()
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    rnd = lambda *shape: torch.empty(shape, device=dev).normal_(generator=g).mul_(0.1).to(dtype)
+    dy, x, wg, wu, wd, gate, up, hidden = (rnd(M, K), rnd(M, K), rnd(N, K), rnd(N, K), rnd(K, N), rnd(M, N), rnd(M, N), rnd(M, N))
+    names, got = _launched(lambda: ops_bwd.mlp_bwd(dy, x, wg, wu, wd, gate, up, hidden))
+    dg, du = ops_bwd.dh_bwd(dy, wd, gate, up)
+    for i, db in zip((2, 4, 6), ops_bwd.colsum_grouped([dg, du, dy])):
+        assert torch.equal(got[i], db)
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert any("dx_dw_kernel" in n for n in names), names
+        assert any("colsum" in n for n in names) == apart, names
 
 
 def test_random_shapes_every_operator_against_fp32_products():

@@ -485,6 +485,7 @@ struct DxDwPlan {
   int x_class = 0, splits = 1;           // ... its tiles
   int dw_splits = 1;                     // ... and of the weight gradients
   int dw_class = -1;                     // the weight gradients' tiles in one grid of their own, or -1: not one grid
+  double cover_us = 0;                   // from when the last tiles of the grid with dX start until it ends
 };
 // When `slots` that take the next workgroup as they get free are through with n0 workgroups of d0 us and then n1 of d1 us.
 double makespan_us(int64_t slots, int64_t n0, double d0, int64_t n1, double d1) {
@@ -533,6 +534,7 @@ DxDwPlan make_plan_dx_dw_f32(int64_t M, int64_t K, int64_t N, int count, const i
       p.x_class = b == 128 ? gmlp::TILE_F32_128 : gmlp::TILE_F32_64;
       p.splits = px.splits;
       p.dw_splits = pw.splits;
+      p.cover_us = nx + nw <= per * cus ? std::max(dx, dw) : std::min(dx, dw);
     }
   }
   return p;
@@ -579,6 +581,7 @@ DxDwPlan make_plan_dx_dw(int dtype, int64_t M, int64_t K, int64_t N, int count, 
       p.x_class = cx.tile_class;
       p.splits = px.splits;
       p.dw_splits = pw.splits;
+      p.cover_us = nx + nw <= slots ? std::max(dx, dw) : std::min(dx, dw);
     }
   };
   consider(kMedium, kMedium);
@@ -1165,10 +1168,25 @@ int gmlp_dropout_mask(uint8_t* mask, int64_t M, int64_t N, float dropout_p, uint
 // ---------------------------------------------------------------- whole passes in one call
 namespace {
 
+// Whether column sums should run at the end of the grid with dX.  A workgroup there sums all rows of 64 columns, 1.1 ns
+// a row and byte of an element, from about when the last tiles start.  Launches of their own, the other two terms,
+// stream the arrays at 4 TB/s but have a chain of loads too, half as long.  K=200, N=600, bf16, backward pass with three
+// bias gradients, in the grid / apart (us): M=4096 41 / 45, 8192 64 / 70, 16384 112 / 110, 32768 216 / 187, 65536 432 / 385;
+// K=256, N=512 16384 79 / 87, 32768 146 / 144; float32 32768 497 / 498, 65536 1046 / 879.  Over 1180 shapes of 1500 to
+// 140000 rows and 32 to 2048 inputs, bf16 and float32, this takes 1.005 times what the better form does (at worst
+// 1.21), in the grid throughout 1.021 (1.41), apart throughout 1.098.
+bool sums_beside_tiles(int64_t M, int nsums, const int64_t* cols, int dtype, double cover_us) {
+  const double size = dtype == GMLP_F32 ? 4.0 : 2.0, column = size * (double)M;  // bytes
+  double all = 0;
+  for (int i = 0; i < nsums; ++i) all += column * (double)cols[i];
+  return 1.1e-3 * column <= cover_us + 5.0 + std::max(all / 4e6, 0.6e-3 * column);
+}
+
 // The gradients of a pass behind dG and dU, its arguments checked: dX (if wanted), the weight gradients
 // lhs[i]^T . rhs[i] and the column sums.  The sums run as workgroups at the end of the grid that computes the
-// weight gradients, on CUs that its last round leaves free and without a launch (or two) of their own; unsplit weight
-// gradients in a single grid without dX take them along too.  Backward passes with three bias gradients over
+// weight gradients, on CUs that its last round leaves free and without a launch (or two) of their own, see
+// sums_beside_tiles; unsplit weight gradients in a single grid without dX take them along too (their tiles take
+// about ten times what a sum over the same rows does).  Backward passes with three bias gradients over
 // 46 shapes of 75 to 8192 rows: 0.73 of the time of separate launches (without biases 0.84), none above 1.02.
 int run_gradients(const char* fn, const void* dg, const void* du, const void* w_gate, const void* w_up, void* dx, int count,
                   const void* const* lhs, const void* const* rhs, void* const* dws, int64_t M, int64_t K, int64_t N, const int64_t* R,
@@ -1179,6 +1197,12 @@ int run_gradients(const char* fn, const void* dg, const void* du, const void* w_
   if (count > 0 && (dx || nsums > 0))
     plan = plan_dx_dw(dtype, M, K, N, count, R, C, workspace ? ws_bytes : 0);
   const bool dx_inside = dx && plan.merged;
+  if (dx_inside && nsums > 0 && !sums_beside_tiles(M, nsums, sum_cols, dtype, plan.cover_us)) {
+    if (int rc = run_gradients(fn, dg, du, w_gate, w_up, dx, count, lhs, rhs, dws, M, K, N, R, C, 0, nullptr, nullptr, nullptr, dtype,
+                               workspace, ws_bytes, stream))
+      return rc;
+    return gmlp_colsum_grouped(nsums, sum_in, sum_out, workspace, M, sum_cols, dtype, stream);
+  }
   if (dx && !dx_inside)
     if (int rc = gmlp_dx_bwd(dg, du, w_gate, w_up, dx, M, K, N, dtype, workspace, ws_bytes, stream)) return rc;
   if (!dx_inside && (nsums == 0 || plan.dw_class < 0)) {
