@@ -171,7 +171,7 @@ GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets
 // What a split costs beside its traffic: 1.7 us on the GPU, and the rest is what the second launch costs the
 // host, which bounds passes this small.  A forward down projection pays that twice: nothing else in its
 // pass is split at such sizes (training step at M=K=N=512 89.4 us with one launch, 92.4 with two).
-const double kSplitF32 = 4.7, kSplitF32Linear = 8.7;
+const double kSplitF32 = 4.9, kSplitF32Linear = 8.9;
 GemmPlan plan_f32(int64_t rows, int64_t cols, int64_t red_tiles, int kind, int64_t max_splits) {
   const int sets = kind == GATEUP ? 2 : 1;
   return plan_f32(cdiv(rows, 128) * cdiv(cols, 128 / sets), cdiv(rows, 64) * cdiv(cols, 64), red_tiles, sets,
