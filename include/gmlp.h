@@ -276,15 +276,25 @@ int gmlp_decode_stream_fwd(const void* x, const void* w_gate, const void* w_up, 
  * workspace: gmlp_mlp_workspace_bytes(GMLP_PASS_FWD or GMLP_PASS_BWD, M, K, N, dtype) bytes (may be
  * NULL or smaller for a pass without bias gradients: launches then use what it holds, with the same
  * results up to the order of fp32 additions; bias gradients need it and fail with GMLP_EINVAL
- * without).  GMLP_PASS_BWD answers for a pass that computes every gradient.  One or two of the weight
- * gradients by themselves may use more (fewer tiles, more splits); such a pass uses the largest of
- * gmlp_workspace_bytes of GMLP_OP_DH_BWD and GMLP_OP_DX_BWD, gmlp_dw_bwd_grouped_workspace_bytes of
- * its weight gradients in the order above, and the sum of GMLP_OP_COLSUM over its bias gradients.
- * Where that holds the partial sums of dx and of the weight gradients side by side (GMLP_OP_DX_BWD's bytes plus
- * those of the weight gradients always do) they can share launches: the same results, sooner.
+ * without).  GMLP_PASS_BWD answers for every launch of a pass that computes every gradient, one after the other.
+ * gmlp_grads_workspace_bytes answers for the gradients in `grads` (GMLP_GRAD_*, or-ed) of a GMLP_PASS_BWD or
+ * GMLP_PASS_HIDDEN_BWD (gmlp_hidden_bwd) and is the one to ask: where dx and the weight gradients can share a launch
+ * it holds the partial sums of both side by side, and one or two of the weight gradients by themselves may use more
+ * than all three (fewer tiles, more splits).
  */
-enum gmlp_pass { GMLP_PASS_FWD = 0, GMLP_PASS_BWD = 1 };
+enum gmlp_pass { GMLP_PASS_FWD = 0, GMLP_PASS_BWD = 1, GMLP_PASS_HIDDEN_BWD = 2 };
+enum gmlp_grad {
+  GMLP_GRAD_X = 1,
+  GMLP_GRAD_W_GATE = 2,
+  GMLP_GRAD_W_UP = 4,
+  GMLP_GRAD_W_DOWN = 8,
+  GMLP_GRAD_B_GATE = 16,
+  GMLP_GRAD_B_UP = 32,
+  GMLP_GRAD_B_DOWN = 64,
+  GMLP_GRAD_ALL = 127
+};
 size_t gmlp_mlp_workspace_bytes(int pass, int64_t M, int64_t K, int64_t N, int dtype);
+size_t gmlp_grads_workspace_bytes(int pass, int grads, int64_t M, int64_t K, int64_t N, int dtype);
 int gmlp_mlp_fwd(const void* x, const void* w_gate, const void* w_up, const void* w_down, const void* b_gate,
                  const void* b_up, const void* b_down, void* y, void* h, void* g_save, void* u_save, int64_t M,
                  int64_t K, int64_t N, int dtype, int act, float dropout_p, uint64_t seed, uint64_t offset,
@@ -299,7 +309,7 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
  * gmlp_hidden_bwd: the backward pass of the hidden states alone, from dh [M,N]: dG, dU (gmlp_gating_bwd), then dx, dw_gate,
  *   dw_up, db_gate, db_up as in gmlp_mlp_bwd (any of them may be NULL), the same values as the separate
  *   calls give.  Stands behind the operator's autograd backward (src/triton_gated_mlp/ops/bwd.py:466-602).
- * workspace: as for gmlp_mlp_bwd, without GMLP_OP_DH_BWD and the down projection's gradients.
+ * workspace: gmlp_grads_workspace_bytes(GMLP_PASS_HIDDEN_BWD, ...) bytes, as for gmlp_mlp_bwd.
  */
 int gmlp_hidden_bwd(const void* dh, const void* x, const void* w_gate, const void* w_up, const void* g, const void* u,
                     void* dg, void* du, void* dx, void* dw_gate, void* dw_up, void* db_gate, void* db_up, int64_t M,

@@ -156,6 +156,36 @@ def test_whole_pass_entry_points_validate_before_touching_the_device():
     assert lib.gmlp_mlp_workspace_bytes(7, 8, 8, 8, 0) == 0 and lib.gmlp_mlp_workspace_bytes(0, 0, 8, 8, 0) == 0
 
 
+@pytest.mark.parametrize("M,K,N,dtype", [(3942, 416, 1280, 0), (775, 96, 512, 1), (590, 352, 544, 2), (8192, 4096, 14336, 0)])
+def test_workspace_of_a_pass_holds_what_its_launches_share(M, K, N, dtype):
+    """Partial sums of dX and of the weight gradients side by side where one grid computes both (the first three: both
+    split), for any set of gradients."""
+    lib = _cabi.lib()
+    ask = lambda grads, which=_cabi.GMLP_PASS_BWD: lib.gmlp_grads_workspace_bytes(which, grads, M, K, N, dtype)
+    op = lambda name, *sizes: lib.gmlp_workspace_bytes(getattr(_cabi, "GMLP_OP_" + name), *sizes, dtype)
+
+    def grouped(problems):
+        array = lambda values: ctypes.cast((ctypes.c_int64 * len(values))(*values), ctypes.c_void_p)
+        R, C = zip(*problems)
+        return lib.gmlp_dw_bwd_grouped_workspace_bytes(len(problems), M, array(R), array(C), dtype)
+
+    both_split = M != 8192
+    for weights in range(1, 8):
+        problems = [p for i, p in enumerate(((N, K), (N, K), (K, N))) if weights >> i & 1]
+        dw, dx, dh = grouped(problems), op("DX_BWD", M, K, N), op("DH_BWD", M, K, N)
+        assert ask(weights << 1) == max(dw, dh if weights & 3 else 0)
+        assert ask(weights << 1 | 1) in (max(dw, dx, dh), max(dw + dx, dh))
+    assert dx > 0 if both_split else dx == 0
+    sums = 2 * op("COLSUM", M, 0, N) + op("COLSUM", M, 0, K)
+    assert ask(_cabi.GMLP_GRAD_ALL) == max(dw + dx if both_split else dw, dh, sums)
+    assert lib.gmlp_mlp_workspace_bytes(_cabi.GMLP_PASS_BWD, M, K, N, dtype) == max(dw, dx, dh, sums)
+    hidden = ask(_cabi.GMLP_GRAD_ALL, _cabi.GMLP_PASS_HIDDEN_BWD)
+    assert hidden == ask(_cabi.GMLP_GRAD_ALL & ~72, _cabi.GMLP_PASS_HIDDEN_BWD) >= max(grouped([(N, K), (N, K)]), dx)
+    assert ask(_cabi.GMLP_GRAD_B_UP, _cabi.GMLP_PASS_HIDDEN_BWD) == op("COLSUM", M, 0, N)
+    assert ask(0) == 0 and ask(127, _cabi.GMLP_PASS_FWD) == 0 and ask(127, 9) == 0
+    assert lib.gmlp_grads_workspace_bytes(_cabi.GMLP_PASS_BWD, 127, 0, K, N, dtype) == 0
+
+
 def test_activation_tables_of_the_reference_are_importable():
     """ACT2CLS / ACT2FN / ClassInstantier (src/triton_gated_mlp/gated_mlp.py:10-26): name -> module
     class, and a table whose lookup instantiates."""

@@ -1269,14 +1269,6 @@ size_t bias_workspace_bytes(int64_t M, int64_t K, int64_t N, bool gate, bool up,
   return (gate + up) * gmlp::colsum_workspace_bytes(M, N) + down * gmlp::colsum_workspace_bytes(M, K);
 }
 
-// Workspace of a backward pass: what its launches ask for, one after the other on one stream, so
-// one buffer of the largest request serves them all.
-size_t bwd_workspace_bytes(int64_t M, int64_t K, int64_t N, int dtype) {
-  const int64_t R[3] = {N, N, K}, C[3] = {K, K, N};
-  return std::max({gmlp_workspace_bytes(GMLP_OP_DH_BWD, M, K, N, dtype), gmlp_workspace_bytes(GMLP_OP_DX_BWD, M, K, N, dtype),
-                   gmlp_dw_bwd_grouped_workspace_bytes(3, M, R, C, dtype), bias_workspace_bytes(M, K, N, true, true, true)});
-}
-
 }  // namespace
 
 extern "C" {
@@ -1288,8 +1280,29 @@ size_t gmlp_mlp_workspace_bytes(int pass, int64_t M, int64_t K, int64_t N, int d
     const size_t b = gmlp_workspace_bytes(GMLP_OP_LINEAR_FWD, M, N, K, dtype);
     return a > b ? a : b;
   }
-  if (pass == GMLP_PASS_BWD) return bwd_workspace_bytes(M, K, N, dtype);
-  return 0;
+  if (pass != GMLP_PASS_BWD) return 0;
+  const int64_t R[3] = {N, N, K}, C[3] = {K, K, N};
+  return std::max({gmlp_workspace_bytes(GMLP_OP_DH_BWD, M, K, N, dtype), gmlp_workspace_bytes(GMLP_OP_DX_BWD, M, K, N, dtype),
+                   gmlp_dw_bwd_grouped_workspace_bytes(3, M, R, C, dtype), bias_workspace_bytes(M, K, N, true, true, true)});
+}
+
+// The launches of a pass follow each other on one stream, so one buffer of the largest request serves them all;
+// dX and the weight gradients in one grid have their partial sums side by side.
+size_t gmlp_grads_workspace_bytes(int pass, int grads, int64_t M, int64_t K, int64_t N, int dtype) {
+  if ((pass != GMLP_PASS_BWD && pass != GMLP_PASS_HIDDEN_BWD) || M < 1 || K < 1 || N < 1) return 0;
+  if (pass == GMLP_PASS_HIDDEN_BWD) grads &= ~(GMLP_GRAD_W_DOWN | GMLP_GRAD_B_DOWN);
+  const bool hidden = grads & ~(GMLP_GRAD_W_DOWN | GMLP_GRAD_B_DOWN);
+  int64_t R[3], C[3];
+  int n = 0;
+  for (int w : {GMLP_GRAD_W_GATE, GMLP_GRAD_W_UP})
+    if (grads & w) R[n] = N, C[n] = K, ++n;
+  if (grads & GMLP_GRAD_W_DOWN) R[n] = K, C[n] = N, ++n;
+  const size_t dh = hidden && pass == GMLP_PASS_BWD ? gmlp_workspace_bytes(GMLP_OP_DH_BWD, M, K, N, dtype) : 0;
+  const size_t dx = grads & GMLP_GRAD_X ? gmlp_workspace_bytes(GMLP_OP_DX_BWD, M, K, N, dtype) : 0;
+  const size_t dw = n > 0 ? gmlp_dw_bwd_grouped_workspace_bytes(n, M, R, C, dtype) : 0;
+  const bool shared = grads & GMLP_GRAD_X && n > 0 && plan_dx_dw(dtype, M, K, N, n, R, C, dx + dw).merged;
+  return std::max({dh, shared ? dx + dw : std::max(dx, dw),
+                   bias_workspace_bytes(M, K, N, grads & GMLP_GRAD_B_GATE, grads & GMLP_GRAD_B_UP, grads & GMLP_GRAD_B_DOWN)});
 }
 
 int gmlp_mlp_fwd(const void* x, const void* w_gate, const void* w_up, const void* w_down, const void* b_gate,
@@ -1347,7 +1360,7 @@ int gmlp_mlp_bwd(const void* dy, const void* x, const void* w_gate, const void* 
   const size_t ws_bytes = workspace != nullptr ? workspace_bytes : 0;
   const size_t sums = bias_workspace_bytes(M, K, N, db_gate, db_up, db_down);
   if (sums > ws_bytes)
-    return fail(GMLP_EINVAL, "%s: bias gradients need a workspace of at least %zu bytes (gmlp_mlp_workspace_bytes)",
+    return fail(GMLP_EINVAL, "%s: bias gradients need a workspace of at least %zu bytes (gmlp_grads_workspace_bytes)",
                 __func__, sums);
 
   const void* lhs[3]; const void* rhs[3]; void* dws[3]; int64_t R[3], C[3];

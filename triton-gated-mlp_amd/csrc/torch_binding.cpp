@@ -42,7 +42,7 @@ typedef std::optional<Tensor> OptTensor;
 #define GMLP_ENTRY_POINTS(X)                                                                     \
   X(gmlp_last_error) X(gmlp_workspace_bytes) X(gmlp_mlp_workspace_bytes) X(gmlp_mlp_fwd)         \
   X(gmlp_mlp_bwd) X(gmlp_gateup_fwd) X(gmlp_decode_fwd) X(gmlp_decode_stream_fwd) X(gmlp_hidden_bwd) \
-  X(gmlp_dw_bwd_grouped_workspace_bytes)
+  X(gmlp_grads_workspace_bytes)
 struct Library {
 #define GMLP_MEMBER(name) decltype(&::name) name = nullptr;
   GMLP_ENTRY_POINTS(GMLP_MEMBER)
@@ -260,6 +260,13 @@ Tensor mlp_infer(const Tensor& x_in, const Tensor& Wg_in, const OptTensor& bg_in
   return y;
 }
 
+// The outputs that are there, as gmlp_grads_workspace_bytes takes them.
+int wanted_grads(const ag::variable_list& out, std::initializer_list<int> grads) {
+  int wanted = 0, i = 0;
+  for (int grad : grads) wanted |= out[i++].defined() ? grad : 0;
+  return wanted;
+}
+
 // dY -> (dX, dW_gate, db_gate, dW_up, db_up, dW_down, db_down), in the order of the edges
 struct MlpBackward : public ag::Node {
   Problem q;
@@ -275,22 +282,6 @@ struct MlpBackward : public ag::Node {
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
     for (ag::SavedVariable* v : {&x_, &Wg_, &Wu_, &Wd_, &acts_, &bg_, &bu_}) v->reset_data();
-  }
-  // What the launches for the gradients asked for use, one after the other, dX and the weight gradients side by
-  // side: some of the weight gradients by themselves may take more than all three together (fewer tiles, more splits).
-  size_t workspace_of(const ag::variable_list& out) const {
-    const bool hidden = out[0].defined() || out[1].defined() || out[2].defined() || out[3].defined() || out[4].defined();
-    size_t bytes = hidden ? lib.gmlp_workspace_bytes(GMLP_OP_DH_BWD, q.M, q.K, q.N, q.code) : 0;
-    size_t grads = out[0].defined() ? lib.gmlp_workspace_bytes(GMLP_OP_DX_BWD, q.M, q.K, q.N, q.code) : 0;
-    int64_t R[3], C[3];
-    int n = 0;
-    for (int i = 1; i <= 5; i += 2)
-      if (out[i].defined()) R[n] = i < 5 ? q.N : q.K, C[n] = i < 5 ? q.K : q.N, ++n;
-    if (n > 0) grads += lib.gmlp_dw_bwd_grouped_workspace_bytes(n, q.M, R, C, q.code);
-    size_t sums = 0;
-    for (int i = 2; i <= 6; i += 2)
-      if (out[i].defined()) sums += lib.gmlp_workspace_bytes(GMLP_OP_COLSUM, q.M, 0, i < 6 ? q.N : q.K, q.code);
-    return std::max({bytes, grads, sums});
   }
   ag::variable_list apply(ag::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -329,7 +320,9 @@ struct MlpBackward : public ag::Node {
     const Activations a(q, kept, true);
     // dG, dU and the library's workspace share one scratch allocation that is dropped on return
     const size_t plane = ((size_t)(q.M * q.N) * dy.element_size() + 255) / 256 * 256;
-    const size_t bytes = workspace_of(out);
+    const int wanted = wanted_grads(out, {GMLP_GRAD_X, GMLP_GRAD_W_GATE, GMLP_GRAD_B_GATE, GMLP_GRAD_W_UP, GMLP_GRAD_B_UP,
+                                          GMLP_GRAD_W_DOWN, GMLP_GRAD_B_DOWN});
+    const size_t bytes = lib.gmlp_grads_workspace_bytes(GMLP_PASS_BWD, wanted, q.M, q.K, q.N, q.code);
     const Tensor arena = scratch(2 * plane + bytes, x);
     char* const base = (char*)out_ptr(arena);
     check(lib.gmlp_mlp_bwd(ptr(dy), ptr(x), ptr(Wg), ptr(Wu), ptr(Wd), a.g, a.u, a.h, base, base + plane, out_ptr(out[0]),
@@ -424,14 +417,10 @@ struct HiddenBackward : public ag::Node {
       out[i] = q.M == 0 ? at::zeros(sizes, dh.options()) : at::empty(sizes, dh.options());
     }
     if (q.M == 0) return out;
-    // dG, dU and the library's workspace (dX and the weight gradients side by side, see MlpBackward) share one
-    // scratch allocation
+    // dG, dU and the library's workspace share one scratch allocation
     const size_t plane = ((size_t)(q.M * q.N) * dh.element_size() + 255) / 256 * 256;
-    const int64_t R[2] = {q.N, q.N}, C[2] = {q.K, q.K};
-    const int nw = (int)out[1].defined() + (int)out[3].defined(), nb = (int)out[2].defined() + (int)out[4].defined();
-    size_t bytes = out[0].defined() ? lib.gmlp_workspace_bytes(GMLP_OP_DX_BWD, q.M, q.K, q.N, q.code) : 0;
-    if (nw > 0) bytes += lib.gmlp_dw_bwd_grouped_workspace_bytes(nw, q.M, R, C, q.code);
-    if (nb > 0) bytes = std::max(bytes, nb * lib.gmlp_workspace_bytes(GMLP_OP_COLSUM, q.M, 0, q.N, q.code));
+    const int wanted = wanted_grads(out, {GMLP_GRAD_X, GMLP_GRAD_W_UP, GMLP_GRAD_B_UP, GMLP_GRAD_W_GATE, GMLP_GRAD_B_GATE});
+    const size_t bytes = lib.gmlp_grads_workspace_bytes(GMLP_PASS_HIDDEN_BWD, wanted, q.M, q.K, q.N, q.code);
     const Tensor arena = scratch(2 * plane + bytes, x);
     char *const dg = (char*)out_ptr(arena), *const du = dg + plane, *const ws = bytes > 0 ? du + plane : nullptr;
     const char* g = (const char*)ptr(kept);

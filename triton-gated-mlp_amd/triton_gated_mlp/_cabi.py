@@ -21,7 +21,9 @@ GMLP_F16, GMLP_BF16, GMLP_F32 = 0, 1, 2
 GMLP_OP_DECODE_FWD, GMLP_OP_COLSUM, GMLP_OP_LINEAR_FWD, GMLP_OP_DX_BWD, GMLP_OP_GATEUP_FWD = 0, 1, 2, 3, 4
 GMLP_OP_DH_BWD, GMLP_OP_DW_BWD, GMLP_OP_DW_BWD_GROUPED = 5, 6, 7
 ABI_VERSION = 8
-GMLP_PASS_FWD, GMLP_PASS_BWD = 0, 1
+GMLP_PASS_FWD, GMLP_PASS_BWD, GMLP_PASS_HIDDEN_BWD = 0, 1, 2
+GMLP_GRAD_X, GMLP_GRAD_W_GATE, GMLP_GRAD_W_UP, GMLP_GRAD_W_DOWN = 1, 2, 4, 8
+GMLP_GRAD_B_GATE, GMLP_GRAD_B_UP, GMLP_GRAD_B_DOWN, GMLP_GRAD_ALL = 16, 32, 64, 127
 
 # hidden_act name -> GMLP_ACT_* code.  The names are those of the reference's ACT2CLS / ACT_FWD
 # tables (src/triton_gated_mlp/gated_mlp.py:17-37).
@@ -73,6 +75,7 @@ _SIGNATURES = {
     "gmlp_decode_stream_fwd": (_int, [_c_ptr] * 9 + [_i64, _i64, _i64, _int, _int, _c_ptr]),
     "gmlp_dropout_mask": (_int, [_c_ptr, _i64, _i64, _f32, _u64, _u64, _c_ptr]),
     "gmlp_mlp_workspace_bytes": (ctypes.c_size_t, [_int, _i64, _i64, _i64, _int]),
+    "gmlp_grads_workspace_bytes": (ctypes.c_size_t, [_int, _int, _i64, _i64, _i64, _int]),
     "gmlp_mlp_fwd": (
         _int,
         [_c_ptr] * 11 + [_i64, _i64, _i64, _int, _int, _f32, _u64, _u64, _c_ptr, ctypes.c_size_t, _c_ptr],

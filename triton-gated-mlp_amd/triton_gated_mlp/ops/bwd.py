@@ -244,28 +244,11 @@ def colsum_grouped(arrays):
 
 
 def _mlp_bwd_workspace_bytes(M: int, K: int, N: int, code: int, need) -> int:
-    """What mlp_bwd's launches for the gradients in `need` use, one after the other, dX and the weight gradients
-    side by side: some of the weight gradients by themselves may take more than all three together (fewer tiles,
-    more splits)."""
-    import ctypes
-
-    lib = _cabi.lib()
-    dx, dwg, dbg, dwu, dbu, dwd, dbd = need
-    sizes = [0]
-    if any(need[:5]):
-        sizes.append(lib.gmlp_workspace_bytes(_cabi.GMLP_OP_DH_BWD, M, K, N, code))
-    grads = lib.gmlp_workspace_bytes(_cabi.GMLP_OP_DX_BWD, M, K, N, code) if dx else 0
-    problems = [p for p, wanted in (((N, K), dwg), ((N, K), dwu), ((K, N), dwd)) if wanted]
-    if problems:
-        I64Arr = ctypes.c_int64 * len(problems)
-        R, C = (I64Arr(*dims) for dims in zip(*problems))
-        grads += lib.gmlp_dw_bwd_grouped_workspace_bytes(
-            len(problems), M, ctypes.cast(R, ctypes.c_void_p), ctypes.cast(C, ctypes.c_void_p), code
-        )
-    sizes.append(grads)
-    sums = [c for c, wanted in ((N, dbg), (N, dbu), (K, dbd)) if wanted]
-    sizes.append(sum(lib.gmlp_workspace_bytes(_cabi.GMLP_OP_COLSUM, M, 0, c, code) for c in sums))
-    return max(sizes)
+    """What mlp_bwd's launches for the gradients in `need` use."""
+    order = (_cabi.GMLP_GRAD_X, _cabi.GMLP_GRAD_W_GATE, _cabi.GMLP_GRAD_B_GATE, _cabi.GMLP_GRAD_W_UP, _cabi.GMLP_GRAD_B_UP,
+             _cabi.GMLP_GRAD_W_DOWN, _cabi.GMLP_GRAD_B_DOWN)
+    grads = sum(grad for grad, wanted in zip(order, need) if wanted)
+    return _cabi.lib().gmlp_grads_workspace_bytes(_cabi.GMLP_PASS_BWD, grads, M, K, N, code)
 
 
 def mlp_bwd(
