@@ -1045,19 +1045,71 @@ def _launched(run):
     return [e.name for e in prof.events() if "gmlp" in e.name], result
 
 
-# dX beside the weight gradients in one grid: 128x128 tiles for both (a single tile each, remainders in every
-# direction, few rows), 256x256 tiles beside a split and an unsplit dX, 192-row and 128-row tiles of dX, reduction lengths
-# that are not a multiple of the 64 of a reduction tile; last, shapes next to these that keep launches of their own
-# (shared-out tiles) or split the weight gradients.  Bias gradients take their place behind the tiles.
-@pytest.mark.parametrize(
-    "M,K,N",
-    [(1, 8, 8), (129, 136, 264), (33, 512, 1528), (512, 512, 1536), (1024, 1024, 2816), (1000, 1024, 2824), (3000, 1536, 4096),
-     (2999, 1528, 4104), (384, 1984, 5440), (271, 2456, 6600), (6656, 1472, 1472), (3456, 384, 1536), (842, 5032, 13520)],
-)
+# dX beside the weight gradients in one grid: rows of a dX tile and of a weight gradient's, whether dX and whether the
+# weight gradients are split, or None for a dX of its own (shared-out tiles, or one grid takes longer by
+# estimate); then the weight gradients' tile where they are a grid with the bias gradients when dX is not in it.  16-bit types,
+# then float32; on a whole MI355X.  Single tiles, remainders in every direction, few rows, many.  Lengths that are not a
+# multiple of the 64 of a reduction tile have instances of their own (N, the reduction of dX).
+_GRADIENT_GRIDS = [
+    # M, K, N, 16-bit, without dX, float32, without dX
+    (1, 8, 8, (128, 128, 0, 0), 128, (64, 64, 0, 0), 64),
+    (129, 136, 264, (128, 128, 0, 0), 128, (64, 64, 1, 0), 64),
+    (33, 512, 1528, (128, 128, 1, 0), 128, (64, 64, 1, 0), 64),
+    (512, 512, 1536, (128, 128, 1, 0), 128, (64, 64, 1, 0), 64),
+    (1024, 1024, 2816, (256, 256, 1, 0), 256, None, 64),
+    (1000, 1024, 2824, (128, 256, 1, 0), 256, None, 64),
+    (3000, 1536, 4096, (192, 256, 0, 0), None, None, None),
+    (2999, 1528, 4104, (192, 256, 0, 0), None, (128, 128, 1, 0), 128),
+    (384, 1984, 5440, (128, 256, 1, 0), 128, (128, 128, 1, 0), 128),
+    (271, 2456, 6600, (128, 256, 1, 0), 128, (128, 128, 1, 0), 128),
+    (6656, 1472, 1472, (192, 256, 0, 0), 128, (128, 128, 1, 1), None),
+    (3456, 384, 1536, (128, 128, 1, 1), None, (128, 128, 1, 1), None),
+    (842, 5032, 13520, None, 256, (128, 128, 1, 0), 128),
+    (884, 3376, 448, (256, 256, 0, 0), 128, None, 64),
+    (896, 3496, 392, (256, 256, 0, 0), 128, (64, 64, 0, 0), 64),
+    (1022, 136, 6768, (256, 256, 1, 0), 128, None, 64),
+    (387, 3968, 576, (128, 256, 0, 0), 128, (64, 64, 0, 0), 128),
+    (513, 2240, 856, (128, 256, 0, 0), 128, (64, 64, 1, 0), 128),
+    (710, 72, 488, (128, 128, 1, 1), None, (64, 64, 1, 1), None),
+    (2381, 240, 128, (128, 128, 0, 1), None, (64, 64, 0, 1), None),
+    (1281, 136, 72, (128, 128, 0, 1), None, (64, 64, 0, 1), None),
+    (565, 48, 64, (128, 128, 0, 0), 128, (64, 64, 0, 1), None),
+    (1632, 720, 72, (128, 128, 0, 1), None, (128, 128, 0, 1), None),
+    (442, 3080, 136, (128, 128, 0, 0), 128, (128, 128, 0, 0), 64),
+    (590, 352, 544, (128, 128, 1, 0), 128, (64, 64, 1, 0), 64),
+    (2902, 2816, 3584, (256, 256, 0, 0), 256, None, 128),
+]
+
+
+def _gradient_grid(names):
+    """(dX rows, weight gradient rows, dX split, weight gradients split) of the grid among launched kernels, or None."""
+    import re
+
+    # (names come mangled, where a repeated type is a back reference, or, float32's, demangled)
+    found = [re.search(r"dx_dw_kernel(.*?)DxDwGroup", n) for n in names if "dx_dw_kernel" in n]
+    assert len(found) <= 1 and all(found), names
+    if not found:
+        return None
+    tiles = [int(t) for t in re.findall(r"(?:Li|<|, )(\d+)(?=E|,)", found[0][1])]
+    stored = re.findall("EpiStore|EpiPartial", found[0][1])
+    return tiles[0], tiles[-1], int(stored[0] == "EpiPartial"), int(stored[-1] == "EpiPartial")
+
+
+def test_gradient_grid_cases_cover_every_instance():
+    both = [(False, False), (True, False), (False, True), (True, True)]
+    large = [(t, 256, x, False) for t in (128, 192, 256) for x in (False, True) if not (t == 192 and x)]
+    half = large + [(128, 128, *splits) for splits in both]
+    assert {(grid, N % 64 != 0) for _, _, N, grid, *_ in _GRADIENT_GRIDS if grid} == {(g, t) for g in half for t in (False, True)}
+    assert {grid for *_, grid, _ in _GRADIENT_GRIDS if grid} == {(t, t, *splits) for t in (64, 128) for splits in both}
+    assert {(w, full) for _, _, _, _, w, _, full in _GRADIENT_GRIDS} >= {(128, 64), (256, 128), (None, None)}
+
+
+@pytest.mark.parametrize("M,K,N,half,half_w,full,full_w", _GRADIENT_GRIDS, ids=lambda v: str(v) if isinstance(v, int) else "")
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
+def test_input_and_weight_gradients_in_one_grid(M, K, N, half, half_w, full, full_w, dtype):
     """gmlp_mlp_bwd may run dX, whichever weight gradients are wanted and the bias gradients as one grid: the same sums in
-    the same order as the entry points of their own (held against the oracle elsewhere), hence equal bit for bit."""
+    the same order as the entry points of their own (held against the oracle elsewhere), hence equal bit for bit.  Which
+    grid ran, with every gradient and without dX, by the launched kernels' names."""
     from triton_gated_mlp.ops import bwd as ops_bwd
     from triton_gated_mlp.ops import fwd as ops_fwd
 
@@ -1072,7 +1124,14 @@ def test_input_and_weight_gradients_in_one_grid(M, K, N, dtype):
         dws = iter(ops_bwd.dw_bwd_grouped([p for p, w in zip(pairs, wanted) if w]))
         dbs = iter(ops_bwd.colsum_grouped([p[0] for p, w in zip(pairs, wanted) if w]) if biases else ())
         need = (bool(want_dx), *(bool(w and (i == 0 or biases)) for w in wanted for i in (0, 1)))
-        got = ops_bwd.mlp_bwd(dy, x, wg, wu, wd, gate, up, hidden, need)
+        if all(wanted) and biases and torch.cuda.get_device_properties(dy.device).multi_processor_count == 256:
+            names, got = _launched(lambda: ops_bwd.mlp_bwd(dy, x, wg, wu, wd, gate, up, hidden, need))
+            alone = full_w if dtype == torch.float32 else half_w
+            grid = (full if dtype == torch.float32 else half) if want_dx else None
+            expected = grid or (alone and (alone, alone, 0, 0))  # (dX by itself: the bias gradients join the weights')
+            assert _gradient_grid(names) == expected, names
+        else:
+            got = ops_bwd.mlp_bwd(dy, x, wg, wu, wd, gate, up, hidden, need)
         assert torch.equal(got[0], dx) if want_dx else got[0] is None, f"dX differs beside {wanted}"
         for w, a, b in zip(wanted, got[1::2], got[2::2]):
             assert torch.equal(a, next(dws)) if w else a is None, f"a weight gradient differs for {wanted}"
