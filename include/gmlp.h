@@ -33,6 +33,7 @@
 extern "C" {
 #endif
 
+/* Changes with anything that an existing caller relies on; entry points that are added leave it. */
 #define GMLP_ABI_VERSION 8
 
 enum gmlp_dtype { GMLP_F16 = 0, GMLP_BF16 = 1, GMLP_F32 = 2 };

@@ -1151,6 +1151,60 @@ def test_input_and_weight_gradients_in_one_grid(M, K, N, half, half_w, full, ful
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("M,K,N,dtype", [(710, 72, 488, torch.float16), (33, 512, 1528, torch.bfloat16), (590, 352, 544, torch.float32)])
+def test_hidden_backward_entry_with_any_outputs_and_workspace(M, K, N, dtype):
+    """gmlp_hidden_bwd for every set of gradients with all of its workspace, part of it and (without bias gradients)
+    none: the values of the separate calls with the same workspace, nothing written beyond it."""
+    import ctypes
+
+    from triton_gated_mlp import _cabi
+
+    dev, lib, code = _dev(), _cabi.lib(), _cabi.dtype_code(dtype)
+    g = torch.Generator(device=dev).manual_seed(31)
+    rnd = lambda *shape: torch.empty(shape, device=dev).normal_(generator=g).to(dtype)
+    dh, x, wg, wu, gate, up = rnd(M, N), rnd(M, K), rnd(N, K), rnd(N, K), rnd(M, N), rnd(M, N)
+    dg, du, dg_ref, du_ref = (torch.empty_like(dh) for _ in range(4))
+    stream, p, act = _cabi.stream_ptr(dev), _cabi.ptr, _cabi.act_code("gelu")
+    flags = (_cabi.GMLP_GRAD_X, _cabi.GMLP_GRAD_W_GATE, _cabi.GMLP_GRAD_W_UP, _cabi.GMLP_GRAD_B_GATE, _cabi.GMLP_GRAD_B_UP)
+    sizes = ((M, K), (N, K), (N, K), (N,), (N,))
+    new = lambda size: torch.full(size, float("nan"), device=dev, dtype=dtype)
+    _cabi.check(lib.gmlp_gating_bwd(p(dh), p(gate), p(up), p(dg_ref), p(du_ref), M, N, code, act, 0.1, 5, 7, stream))
+
+    def apart(want, ws, nbytes):
+        """The same by the entry points of their own."""
+        outs = [new(size) if w else None for size, w in zip(sizes, want)]
+        if want[0]:
+            _cabi.check(lib.gmlp_dx_bwd(p(dg_ref), p(du_ref), p(wg), p(wu), p(outs[0]), M, K, N, code, ws, nbytes, stream))
+        chosen = [(d, o) for d, o in ((dg_ref, outs[1]), (du_ref, outs[2])) if o is not None]
+        if chosen:
+            array = lambda kind, values: ctypes.cast((kind * len(values))(*values), ctypes.c_void_p)
+            lhs, rhs, dws = (array(ctypes.c_void_p, v) for v in zip(*[(p(d), p(x), p(o)) for d, o in chosen]))
+            R, C = array(ctypes.c_int64, [N] * len(chosen)), array(ctypes.c_int64, [K] * len(chosen))
+            _cabi.check(lib.gmlp_dw_bwd_grouped(len(chosen), lhs, rhs, dws, M, R, C, code, ws, nbytes, stream))
+        for d, o in ((dg_ref, outs[3]), (du_ref, outs[4])):
+            if o is not None:
+                _cabi.check(lib.gmlp_colsum(p(d), p(o), ws, M, N, code, stream))
+        return outs
+
+    for subset in range(32):
+        want = [subset >> i & 1 for i in range(5)]
+        grads = sum(f for f, w in zip(flags, want) if w)
+        need = lib.gmlp_grads_workspace_bytes(_cabi.GMLP_PASS_HIDDEN_BWD, grads, M, K, N, code)
+        least = (want[3] + want[4]) * lib.gmlp_workspace_bytes(_cabi.GMLP_OP_COLSUM, M, 0, N, code)
+        for nbytes in sorted({need, max(need // 2 // 16 * 16, least), least}):
+            buffer = torch.full((need + 4096,), 0xA5, device=dev, dtype=torch.uint8)
+            scratch = torch.empty(need + 16, device=dev, dtype=torch.uint8)
+            outs = [new(size) if w else None for size, w in zip(sizes, want)]
+            _cabi.check(lib.gmlp_hidden_bwd(
+                p(dh), p(x) if want[1] or want[2] else None, *((p(wg), p(wu)) if want[0] else (None, None)), p(gate), p(up), p(dg), p(du),
+                *(p(o) for o in outs), M, K, N, code, act, 0.1, 5, 7, p(buffer) if nbytes else None, nbytes, stream))
+            ref = apart(want, p(scratch) if nbytes else None, nbytes)
+            assert torch.equal(dg, dg_ref) and torch.equal(du, du_ref)
+            for i, (a, b) in enumerate(zip(outs, ref)):
+                assert a is None or torch.equal(a, b), (want, nbytes, i)
+            assert (buffer[nbytes:] == 0xA5).all(), (want, nbytes)
+
+
 @pytest.mark.parametrize(
     "M,K,N,dtype,apart",  # rows on both sides of the line; few tiles that all start at once, many, and float32
     [(8192, 200, 600, torch.bfloat16, False), (65536, 200, 600, torch.bfloat16, True), (16384, 40, 56, torch.float16, False),

@@ -156,6 +156,39 @@ def test_whole_pass_entry_points_validate_before_touching_the_device():
     assert lib.gmlp_mlp_workspace_bytes(7, 8, 8, 8, 0) == 0 and lib.gmlp_mlp_workspace_bytes(0, 0, 8, 8, 0) == 0
 
 
+def test_hidden_backward_entry_validates_before_touching_the_device():
+    lib = _cabi.lib()
+    _, a = _buf()
+    err = lambda: lib.gmlp_last_error().decode()
+
+    def bwd(dh=a, x=a, wg=a, wu=a, g=a, u=a, dg=a, du=a, dx=a, dwg=a, dwu=a, dbg=None, dbu=None, M=8, K=8, N=8, dt=0, act=0,
+            p=0.0, ws=None, nws=0):
+        return lib.gmlp_hidden_bwd(dh, x, wg, wu, g, u, dg, du, dx, dwg, dwu, dbg, dbu, M, K, N, dt, act, p, 0, 0, ws, nws, None)
+
+    for name in ("dh", "g", "u", "dg", "du"):  # always needed
+        assert bwd(**{name: None}) == -1 and f"'{name}'" in err()
+    # what a requested output needs
+    assert bwd(wg=None) == -1 and "'w_gate'" in err()
+    assert bwd(wu=None) == -1 and "'w_up'" in err()
+    assert bwd(x=None) == -1 and "'x'" in err()
+    assert bwd(x=None, dwg=None) == -1 and "'x'" in err()
+    assert bwd(dbg=a) == -1 and bwd(dbu=a) == -1 and "workspace" in err()
+    assert bwd(dbg=a, dbu=a, ws=a, nws=2 * 64 * 8 * 4 - 1) == -1 and str(2 * 64 * 8 * 4) in err()
+    assert bwd(dt=3) == -1 and bwd(act=7) == -1 and bwd(p=1.0) == -1 and bwd(p=float("nan")) == -1
+    assert bwd(N=20) == -2 and bwd(K=12) == -2 and bwd(M=0) == -2
+    for name in ("dh", "x", "wg", "wu", "g", "u", "dg", "du", "dx", "dwg", "dwu"):
+        assert bwd(**{name: a + 8}) == -3, name
+    assert bwd(dbu=a + 2, ws=a, nws=1 << 20) == -3 and bwd(ws=a + 4, nws=64) == -3 and "workspace" in err()
+
+
+def test_library_without_an_export_is_refused_by_name(monkeypatch):
+    """Added exports leave the ABI version: an older library is told apart by what it lacks."""
+    monkeypatch.setitem(_cabi._SIGNATURES, "gmlp_of_a_later_version", (ctypes.c_int, []))
+    monkeypatch.setattr(_cabi, "_lib", None)
+    with pytest.raises(RuntimeError, match="gmlp_of_a_later_version.*build it again"):
+        _cabi.lib()
+
+
 @pytest.mark.parametrize("M,K,N,dtype", [(3942, 416, 1280, 0), (775, 96, 512, 1), (590, 352, 544, 2), (8192, 4096, 14336, 0)])
 def test_workspace_of_a_pass_holds_what_its_launches_share(M, K, N, dtype):
     """Partial sums of dX and of the weight gradients side by side where one grid computes both (the first three: both

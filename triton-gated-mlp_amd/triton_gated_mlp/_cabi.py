@@ -115,7 +115,9 @@ def lib() -> ctypes.CDLL:
             )
         handle = ctypes.CDLL(str(path))
         for name, (restype, argtypes) in _SIGNATURES.items():
-            fn = getattr(handle, name)
+            fn = getattr(handle, name, None)
+            if fn is None:
+                raise RuntimeError(f"libgmlp.so at {path} lacks {name}: build it again with `make -C {path.parent.parent}`")
             fn.restype = restype
             fn.argtypes = argtypes
         got = handle.gmlp_abi_version()
