@@ -1562,6 +1562,35 @@ def test_fp32_extreme_operands_against_float64_products(M, K, N):
     check("dW", ops_bwd.dw_bwd(d(lhs), d(e)), [(lhs.T, e)])
 
 
+@pytest.mark.parametrize(
+    "M,K,N,halves",  # out [M, K], reduction N
+    [(1, 8, 256, True), (1, 8, 248, True), (64, 72, 264, True), (33, 1024, 2816, True), (65, 136, 272, True),  # 8, 9 and 88 tiles
+     (1, 16384, 256, True), (64, 8, 224, False), (1, 16392, 256, False)],  # a workgroup on every CU, 7 tiles, one more tile
+)
+def test_fp32_down_projections_in_two_halves(M, K, N, halves):
+    """Down projections of few rows: both halves of the reduction in one workgroup, odd numbers of reduction tiles and
+    ragged last ones included, without a workspace; elementwise within the bound of a float32 sum, and the kernel by name
+    (on a whole MI355X).  An infinity in either half comes out as such."""
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    g = torch.Generator(device=dev).manual_seed(37)
+    rnd = lambda *shape: torch.empty(shape, device=dev).normal_(generator=g)
+    h, w, b = rnd(M, N), rnd(K, N), rnd(K)
+    names, out = _launched(lambda: ops_fwd.linear_fwd(h, w, b))
+    ref, terms = h.double() @ w.double().T + b.double(), h.double().abs() @ w.double().abs().T + b.double().abs()
+    worst = ((out.double() - ref).abs() / ((N + 3) * 2.0**-24 * terms)).max().item()
+    print(f"M={M} K={K} N={N}: largest error {worst:.3f} of its bound", flush=True)
+    assert worst <= 1.0
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert any("halves" in n for n in names) == halves, names
+    for k in (0, N - 1):
+        t = h.clone()
+        t[0, k] = float("inf")
+        got = ops_fwd.linear_fwd(t, w, b)
+        assert torch.equal(got[0], w[:, k].sign() * float("inf")) and torch.equal(got[1:], out[1:])
+
+
 def test_fp32_operands_that_are_not_finite_cost_a_few_launches_at_most():
     """A single infinity makes a whole row or column of a product non-finite, a row of them all of a weight gradient: those
     outputs are computed a second time.  On the fp32 matrix cores that makes it up to three times the usual time here;

@@ -319,7 +319,13 @@ int64_t whole_rounds(int kind, int64_t rows, int64_t cols) {
 GemmPlan make_plan(int dtype, int kind, int64_t rows, int64_t cols, int64_t red, bool may_split) {
   if (dtype == GMLP_F32) {
     // (a down projection of at most 64 rows asks for no workspace in float32: its callers rely on that)
-    return plan_f32(rows, cols, (kind == DX ? 2 : 1) * cdiv(red, 32), kind, may_split && (kind != LINEAR || rows > 64) ? kMaxSplits : 1);
+    const int64_t tiles = (kind == DX ? 2 : 1) * cdiv(red, 32);
+    GemmPlan p = plan_f32(rows, cols, tiles, kind, may_split && (kind != LINEAR || rows > 64) ? kMaxSplits : 1);
+    // a chain of reduction tiles on at most one workgroup per CU: both halves of it at once (a tile takes 0.72 us with one
+    // chain on a CU, 0.58 with two; below 8 tiles that is about what adding the halves costs)
+    if (kind == LINEAR && p.tile_class == gmlp::TILE_F32_64 && p.splits == 1 && tiles >= 8 && cdiv(rows, 64) * cdiv(cols, 64) <= num_cu())
+      p.tile_class = gmlp::TILE_F32_HALVES;
+    return p;
   }
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
   // the buffer base sits up to 4 KB below the operand (shared-M0 loads)

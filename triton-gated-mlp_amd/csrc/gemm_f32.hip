@@ -23,7 +23,7 @@
 // one run, and a CU holds two workgroups, one of which multiplies while the other waits at a barrier or
 // for LDS (128 x 128 x 32 per CU: 2.01 us with one workgroup, 1.55 each with two).  64 x 64 tiles fill the
 // chip on small problems, where a launch is as long as its chain of reduction tiles: two LDS stages (one
-// barrier a tile) and three reduction tiles in flight in registers (down projection at M=64, K=256, N=1024:
+// barrier a tile) and three reduction tiles in flight in registers (down projection at M=64, K=256, N=1024, one chain:
 // 27.8 us with one in flight, 26.0 with three).  Reading the fragments of the next tile ahead as well costs
 // the registers of a third workgroup per CU and was 3 to 5 % slower.
 #include "gemm_f32_split.hpp"
@@ -106,15 +106,18 @@ __device__ __forceinline__ void f32_again(const GemmArgs& ga, f32x4 (&sum)[G], i
   }
 }
 
-template <int BM, int BN, bool A_KS, bool B_KS, int NB, typename Epi>
+// HALVES = 2: a workgroup of twice the wavefronts, whose second half reduces the second half of the range.
+template <int BM, int BN, bool A_KS, bool B_KS, int NB, typename Epi, int HALVES = 1>
 __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::Args ea, int pid, int nwg) {
   typedef F32Config<BM, BN, A_KS, B_KS, NB> Cfg;
   typedef typename Cfg::AT AT;
   typedef typename Cfg::BT BT;
   constexpr int BK = Cfg::BK, TM = Cfg::TM, TN = Cfg::TN, G = Cfg::G, WTM = Cfg::WTM, WTN = Cfg::WTN;
-  extern __shared__ __align__(1024) char smem[];
+  extern __shared__ __align__(1024) char smem_raw[];
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int half = HALVES == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  char* const smem = smem_raw + half * Cfg::LDS_BYTES;
+  const int tid = threadIdx.x - half * 256, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WGN, wn = wave % Cfg::WGN;
   const int tiles_m = (ga.M + BM - 1) / BM, tiles_n = (ga.N + BN - 1) / BN, ntiles = tiles_m * tiles_n;
@@ -132,6 +135,12 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::
     kt_first = min(split * per, kt_all);
     kt_end = min(kt_first + per, kt_all);
   }
+  if constexpr (HALVES == 2) {  // (as many tiles each, for the barriers; one past the end reads zeros)
+    static_assert(!Epi::SPLIT && NB == 1, "built for the down projection");
+    const int per = (kt_all + 1) / 2;
+    kt_first = half * per;
+    kt_end = kt_first + per;
+  }
 
   f32x4 acc[G][TM];
 #pragma unroll
@@ -143,7 +152,7 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::
   BT bt[NB];
   constexpr int NS = Cfg::NS, PF = Cfg::PF;
   f32x4 araw[PF][AT::CHUNKS][2], braw[PF][NB][BT::CHUNKS][2];
-  int seg = kt_first >= kt_seg ? 1 : 0, kleft = 0;
+  int seg = HALVES == 1 && kt_first >= kt_seg ? 1 : 0, kleft = 0;
   auto start = [&](int kk) __attribute__((always_inline)) {
     at.start((const float*)ga.A[seg], ga.lda, m0, kk * BK, ga.M, tid);
 #pragma unroll
@@ -272,6 +281,18 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::
   }
 
   __syncthreads();  // the slabs overwrite the operand tiles
+  if constexpr (HALVES == 2) {  // the second half's sums change hands through its part of LDS
+    f32x4* const other = (f32x4*)(smem_raw + Cfg::LDS_BYTES) + tid;
+    static_assert(G * TM * 256 * 16 <= Cfg::LDS_BYTES, "accumulators fit");
+    if (half == 1) {
+#pragma unroll
+      for (int q = 0; q < G * TM; ++q) other[q * 256] = acc[q / TM][q % TM];
+    }
+    __syncthreads();
+    if (half == 1) return;
+#pragma unroll
+    for (int q = 0; q < G * TM; ++q) acc[q / TM][q % TM] += other[q * 256];
+  }
   constexpr int ELD = Cfg::ELD, CPW = WTN / 4, ITEMS = 16 * CPW / 64;
   static_assert(16 * CPW % 64 == 0, "slab items divide over the lanes");
   float* slab = (float*)smem + wave * NB * 16 * ELD;
@@ -305,6 +326,15 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& ga, typename Epi::
 template <int BM, int BN, bool A_KS, bool B_KS, int NB, typename Epi>
 __global__ void __launch_bounds__(256, f32_per_cu(BM, NB)) gemm_f32_kernel(GemmArgs ga, typename Epi::Args ea) {
   gemm_f32_body<BM, BN, A_KS, B_KS, NB, Epi>(ga, ea, blockIdx.x, gridDim.x);
+}
+
+// Both halves of the reduction by one workgroup, for down projections of at most one workgroup per CU that leave no partial
+// sums in memory: the launch is as long as its chain of reduction tiles, and a CU has room for two chains.  fp32 MFMAs ->
+// six products, one chain -> eight, two chains (us): M=1 to 64, K=1024, N=2816 56 -> 66 -> 50, M=64, K=256, N=1024
+// 22 -> 26 -> 21, M=8, K=4096, N=11008 209 -> 247 -> 180.  (Gate/up, two accumulator sets: 13.6 -> 12.7 at 8 reduction tiles,
+// nothing at M=8, K=4096, N=11008, so it has no such kernel.)
+__global__ void __launch_bounds__(512, 2) gemm_f32_halves_kernel(GemmArgs ga, EpiStore<float>::Args ea) {
+  gemm_f32_body<64, 64, false, false, 1, EpiStore<float>, 2>(ga, ea, blockIdx.x, gridDim.x);
 }
 
 template <int BM, int BN, typename Epi>
@@ -367,7 +397,12 @@ hipError_t launch_gateup_kt<float, false>(int tc, const GemmArgs& ga, const EpiG
 }
 template <>
 hipError_t launch_linear_kt<float, false>(int tc, const GemmArgs& ga, const EpiStore<float>::Args& ea, hipStream_t s) {
-  return launch_f32<false, false, 1, EpiStore<float>>(tc, ga, ea, s);
+  if (tc != TILE_F32_HALVES) return launch_f32<false, false, 1, EpiStore<float>>(tc, ga, ea, s);
+  constexpr auto kern = gemm_f32_halves_kernel;
+  constexpr int LDS = 2 * F32Config<64, 64, false, false, 1>::LDS_BYTES;
+  if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, LDS>, s)) return e;
+  hipLaunchKernelGGL(kern, dim3(((ga.M + 63) / 64) * ((ga.N + 63) / 64)), dim3(512), LDS, s, ga, ea);
+  return hipGetLastError();
 }
 template <>
 hipError_t launch_dh_kt<float, false>(int tc, const GemmArgs& ga, const EpiDh<float>::Args& ea, hipStream_t s) {

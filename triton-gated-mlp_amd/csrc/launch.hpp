@@ -20,9 +20,9 @@ namespace gmlp {
 //   MEDIUM       128x128, predicated register-staged kernel, 64-bit addresses: operands too large for
 //                the pipelined kernels' 32-bit byte offsets
 //   F32_*        the float32 kernel's tiles (gemm_f32.hip): 128 x 128 or 64 x 64; with two accumulator
-//                sets 128 x 64 or 64 x 64
+//                sets 128 x 64 or 64 x 64; HALVES: 64 x 64, one workgroup for both halves of a down projection's reduction
 enum TileClass { TILE_LARGE = 0, TILE_MEDIUM = 1, TILE_MEDIUM_FULL = 2, TILE_F32_128 = 3, TILE_F32_64 = 4, TILE_WIDE = 5,
-                 TILE_TALL = 6 };
+                 TILE_TALL = 6, TILE_F32_HALVES = 7 };
 
 // kinds of GEMM the gated MLP needs; each is instantiated per dtype and tile class, and for reduction
 // lengths that are (KT = false) or are not a multiple of 64, the width of a reduction tile.
