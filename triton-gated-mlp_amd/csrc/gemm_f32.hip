@@ -1,7 +1,7 @@
 // float32 path: the GEMMs and fused epilogues for callers that keep the module in float32 (as the
 // reference's own tests do), on the bf16 matrix cores: every operand element is split into three bf16
-// numbers and a product taken as eight (gemm_f32_split.hpp), which cost half of the time of the fp32
-// MFMA (v_mfma_f32_32x32x2_f32: 157 TFLOP/s; 2500 bf16).
+// numbers and a product taken as eight (gemm_f32_split.hpp), which at the matrix cores' nominal rates cost half of the
+// time of the fp32 MFMA (v_mfma_f32_32x32x2_f32: 157 TFLOP/s; 2500 bf16).
 //
 // Precision.  A product enters the sum to 2^-33 of itself.  A bf16 MFMA does not round its sums to nearest (a sum of
 // one term by eight MFMAs into one accumulator comes out up to 2.6 half units off, with six or with eight products), so
@@ -348,8 +348,8 @@ __global__ void __launch_bounds__(256, f32_per_cu(BM, 1)) gemm_f32_group_kernel(
 }
 
 // The input gradient, the weight gradients and the bias gradients as one grid (see gemm_pipelined.hpp's of 16-bit
-// types), all on square tiles of the same size.  Backward passes, before and after: 512x512x512 41 -> 36 us, 684x56x224
-// 24.5 -> 17.2 and with biases 30 -> 17.5, 1280x320x1216 95 -> 76 and 103 -> 76.
+// types), all on square tiles of the same size.  Backward passes, launches of their own -> one grid: 512x512x512 42 -> 34 us,
+// 684x56x224 27 -> 20 and with biases 33 -> 20, 1280x320x1216 88 -> 73 and 92 -> 72.
 template <int B, typename EpiX, typename EpiW>
 __global__ void __launch_bounds__(256, f32_per_cu(B, 1)) gemm_f32_dx_dw_kernel(DxDwGroup<float, EpiX, EpiW> grp) {
   int pid = (int)blockIdx.x;
