@@ -2030,10 +2030,15 @@ def test_decode_with_two_token_tiles(dtype):
                            torch.zeros(512, 1024, dtype=dtype, device=dev), None)
 
 
-@pytest.mark.parametrize("M,K,N,streams", [(8, 2048, 4096, True), (24, 3584, 4096, True), (64, 1024, 4096, False)])
-def test_inference_forward_under_hip_graph_replay(M, K, N, streams):
+@pytest.mark.parametrize(
+    "M,K,N,streams,dtype",
+    [(8, 2048, 4096, True, torch.float16), (24, 3584, 4096, True, torch.float16), (64, 1024, 4096, False, torch.float16),
+     (33, 1024, 2816, False, torch.float32)],
+)
+def test_inference_forward_under_hip_graph_replay(M, K, N, streams, dtype):
     """Serving loops replay a captured forward: the skinny-M streaming path (one and two token
-    tiles) and the general path with split reductions are captured once and replayed with new
+    tiles) and the general path (split reductions; float32, whose down projection here is reduced in
+    two halves by one workgroup) are captured once and replayed with new
     inputs written into the captured input buffer; every replay must equal the eager result for
     that input, with eager work and synchronisations in between."""
     from triton_gated_mlp import FusedGatedMLP
@@ -2041,10 +2046,10 @@ def test_inference_forward_under_hip_graph_replay(M, K, N, streams):
 
     dev = _dev()
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    assert ops_fwd.decode_preferred(M, K, N, torch.float16, cus) == streams
-    mlp = FusedGatedMLP(K, N, bias=True).to(dev).to(torch.float16).eval()
+    assert ops_fwd.decode_preferred(M, K, N, dtype, cus) == streams
+    mlp = FusedGatedMLP(K, N, bias=True).to(dev).to(dtype).eval()
     g = torch.Generator().manual_seed(41)
-    inputs = [torch.randn(M, K, generator=g).half().to(dev) for _ in range(3)]
+    inputs = [torch.randn(M, K, generator=g).to(dtype).to(dev) for _ in range(3)]
     with torch.no_grad():
         eager = [mlp(v).clone() for v in inputs]
         x = inputs[0].clone()
