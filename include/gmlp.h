@@ -279,9 +279,9 @@ int gmlp_decode_stream_fwd(const void* x, const void* w_gate, const void* w_up, 
  * results up to the order of fp32 additions; bias gradients need it and fail with GMLP_EINVAL
  * without).  GMLP_PASS_BWD answers for every launch of a pass that computes every gradient, one after the other.
  * gmlp_grads_workspace_bytes answers for the gradients in `grads` (GMLP_GRAD_*, or-ed) of a GMLP_PASS_BWD or
- * GMLP_PASS_HIDDEN_BWD (gmlp_hidden_bwd) and is the one to ask: where dx and the weight gradients can share a launch
- * it holds the partial sums of both side by side, and one or two of the weight gradients by themselves may use more
- * than all three (fewer tiles, more splits).
+ * GMLP_PASS_HIDDEN_BWD (gmlp_hidden_bwd) and is the one to ask: it holds the partial sums of dx and of the weight
+ * gradients side by side, so that they can share launches, and one or two of the weight gradients by themselves may use
+ * more than all three (fewer tiles, more splits).
  */
 enum gmlp_pass { GMLP_PASS_FWD = 0, GMLP_PASS_BWD = 1, GMLP_PASS_HIDDEN_BWD = 2 };
 enum gmlp_grad {

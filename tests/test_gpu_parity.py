@@ -1056,8 +1056,8 @@ _GRADIENT_GRIDS = [
     (129, 136, 264, (128, 128, 0, 0), 128, (64, 64, 1, 0), 64),
     (33, 512, 1528, (128, 128, 1, 0), 128, (64, 64, 1, 0), 64),
     (512, 512, 1536, (128, 128, 1, 0), 128, (64, 64, 1, 0), 64),
-    (1024, 1024, 2816, (256, 256, 1, 0), 256, None, 64),
-    (1000, 1024, 2824, (128, 256, 1, 0), 256, None, 64),
+    (1024, 1024, 2816, (256, 256, 1, 0), 256, None, 128),
+    (1000, 1024, 2824, (128, 256, 1, 0), 256, None, 128),
     (3000, 1536, 4096, (192, 256, 0, 0), None, None, None),
     (2999, 1528, 4104, (192, 256, 0, 0), None, (128, 128, 1, 0), 128),
     (384, 1984, 5440, (128, 256, 1, 0), 128, (128, 128, 1, 0), 128),
@@ -1066,10 +1066,10 @@ _GRADIENT_GRIDS = [
     (3456, 384, 1536, (128, 128, 1, 1), None, (128, 128, 1, 1), None),
     (842, 5032, 13520, None, 256, (128, 128, 1, 0), 128),
     (884, 3376, 448, (256, 256, 0, 0), 128, None, 64),
-    (896, 3496, 392, (256, 256, 0, 0), 128, (64, 64, 0, 0), 64),
+    (896, 3496, 392, (256, 256, 0, 0), 128, None, 64),
     (1022, 136, 6768, (256, 256, 1, 0), 128, None, 64),
-    (387, 3968, 576, (128, 256, 0, 0), 128, (64, 64, 0, 0), 128),
-    (513, 2240, 856, (128, 256, 0, 0), 128, (64, 64, 1, 0), 128),
+    (387, 3968, 576, (128, 256, 0, 0), 128, (128, 128, 1, 0), 128),
+    (513, 2240, 856, (128, 256, 0, 0), 128, (128, 128, 1, 0), 128),
     (710, 72, 488, (128, 128, 1, 1), None, (64, 64, 1, 1), None),
     (2381, 240, 128, (128, 128, 0, 1), None, (64, 64, 0, 1), None),
     (1281, 136, 72, (128, 128, 0, 1), None, (64, 64, 0, 1), None),

@@ -137,11 +137,11 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // less where they are few.  A split reduction pays a second launch and the partial sums' round trip
 // through the caches.  One least-squares fit to the launches of five GEMMs of 70 shapes (M 32 to 6000,
 // widths 40 to 14400, both classes, 1 to 16 splits): standard deviation of the estimates 6 %, what it picks
-// costs 0.5 % over the fastest on average.  What that is worth at M=2048, K=1024, N=2816: down projection
+// costs 0.4 % over the fastest on average.  What that is worth at M=2048, K=1024, N=2816: down projection
 // on 128x128 tiles (128 of them) unsplit 180 us, in 4 splits 101, 64x64 unsplit 104; dX 330 / 164 / 198.
 // us per reduction tile with 1, 2, 3 workgroups on a CU; us of an epilogue
-const double kF32R128[] = {2.008, 3.095}, kF32R64[] = {0.721, 1.167, 1.549}, kF32R64x2[] = {1.271, 1.930};
-const double kF32E128 = 2.790, kF32E64 = 0.925;
+const double kF32R128[] = {1.802, 2.885}, kF32R64[] = {0.721, 1.167, 1.549}, kF32R64x2[] = {1.271, 1.930};
+const double kF32E128 = 2.597, kF32E64 = 0.925;
 const double kF32Launch = 4.05, kF32Traffic = 0.345e-6;  // us of a launch; of a byte of partial sums
 GemmPlan plan_f32(int64_t tiles128, int64_t tiles64, int64_t red_tiles, int sets, double out_bytes, int64_t max_splits,
                   double split_us) {
@@ -1293,7 +1293,8 @@ size_t gmlp_mlp_workspace_bytes(int pass, int64_t M, int64_t K, int64_t N, int d
 }
 
 // The launches of a pass follow each other on one stream, so one buffer of the largest request serves them all;
-// dX and the weight gradients in one grid have their partial sums side by side.
+// dX and the weight gradients, which may share a grid, have their partial sums side by side.  (Whether they do is not asked
+// here: the plan goes by the workspace, and a pass would have it made for two sizes each time.)
 size_t gmlp_grads_workspace_bytes(int pass, int grads, int64_t M, int64_t K, int64_t N, int dtype) {
   if ((pass != GMLP_PASS_BWD && pass != GMLP_PASS_HIDDEN_BWD) || M < 1 || K < 1 || N < 1) return 0;
   if (pass == GMLP_PASS_HIDDEN_BWD) grads &= ~(GMLP_GRAD_W_DOWN | GMLP_GRAD_B_DOWN);
@@ -1306,8 +1307,7 @@ size_t gmlp_grads_workspace_bytes(int pass, int grads, int64_t M, int64_t K, int
   const size_t dh = hidden && pass == GMLP_PASS_BWD ? gmlp_workspace_bytes(GMLP_OP_DH_BWD, M, K, N, dtype) : 0;
   const size_t dx = grads & GMLP_GRAD_X ? gmlp_workspace_bytes(GMLP_OP_DX_BWD, M, K, N, dtype) : 0;
   const size_t dw = n > 0 ? gmlp_dw_bwd_grouped_workspace_bytes(n, M, R, C, dtype) : 0;
-  const bool shared = grads & GMLP_GRAD_X && n > 0 && plan_dx_dw(dtype, M, K, N, n, R, C, dx + dw).merged;
-  return std::max({dh, shared ? dx + dw : std::max(dx, dw),
+  return std::max({dh, dx + dw,
                    bias_workspace_bytes(M, K, N, grads & GMLP_GRAD_B_GATE, grads & GMLP_GRAD_B_UP, grads & GMLP_GRAD_B_DOWN)});
 }
 
