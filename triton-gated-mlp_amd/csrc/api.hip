@@ -138,7 +138,7 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // through the caches.  One least-squares fit to the launches of five GEMMs of 70 shapes (M 32 to 6000,
 // widths 40 to 14400, both classes, 1 to 16 splits): standard deviation of the estimates 6 %, what it picks
 // costs 0.4 % over the fastest on average.  What that is worth at M=2048, K=1024, N=2816: down projection
-// on 128x128 tiles (128 of them) unsplit 180 us, in 4 splits 101, 64x64 unsplit 104; dX 330 / 164 / 198.
+// on 128x128 tiles (128 of them) unsplit 161 us, in 4 splits 94, 64x64 unsplit 105; dX 302 / 162 / 199.
 // us per reduction tile with 1, 2, 3 workgroups on a CU; us of an epilogue
 const double kF32R128[] = {1.802, 2.885}, kF32R64[] = {0.721, 1.167, 1.549}, kF32R64x2[] = {1.271, 1.930};
 const double kF32E128 = 2.597, kF32E64 = 0.925;

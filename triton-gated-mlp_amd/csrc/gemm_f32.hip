@@ -3,9 +3,8 @@
 // numbers and a product taken as eight (gemm_f32_split.hpp), which at the matrix cores' nominal rates cost half of the
 // time of the fp32 MFMA (v_mfma_f32_32x32x2_f32: 157 TFLOP/s; 2500 bf16).
 //
-// Precision.  A product enters the sum to 2^-33 of itself.  A bf16 MFMA does not round its sums to nearest (a sum of
-// one term by eight MFMAs into one accumulator comes out up to 2.6 half units off, with six or with eight products), so
-// the seven products that are at most 2^-8 of the whole go to an accumulator of their own, tile by tile, which
+// Precision.  A product enters the sum to 2^-33 of itself.  A bf16 MFMA does not round its sums to nearest (with one
+// accumulator a sum of one term comes out up to 2.6 half units off by six products, 1.9 by eight), so the seven products that are at most 2^-8 of the whole go to an accumulator of their own, tile by tile, which
 // joins the one of the first parts by an addition.  A sum of one term is then rounded once, as by fp32 MFMAs (largest
 // error 1.00 half units, root mean square 0.47, both), and longer ones come out closer, by fewer roundings:
 // relative error against float64 at M=2048, K=1024, N=2816, fp32 MFMAs -> one accumulator for six products -> this:
@@ -13,15 +12,15 @@
 // 2.1e-7 (10 shapes of 1 to 6974 rows: sums of one term the same as by fp32 MFMAs, of 32 and more 0.2 to 0.6 of the error).
 //
 // Bound: the matrix cores at the board's power limit.  M=4096, K=2048, N=5632, fp32 MFMAs -> this (us, TFLOP/s of the
-// float32 product): gate/up 1431 -> 1236 (153), down 717 -> 603 (157), dH 770 -> 619 (153), dX 1439 -> 1165 (162),
-// weight gradients 2234 -> 1762 (161); 162 is 1297 of bf16.  (Six products in one accumulator: 1018, 493, 508, 950, 1397.)
+// float32 product): gate/up 1424 -> 1182 (160), down 721 -> 582 (162), dH 772 -> 611 (155), dX 1441 -> 1148 (165),
+// weight gradients 2245 -> 1699 (167); 167 is 1334 of bf16.  (Six products in one accumulator: 1027, 498, 516, 960, 1419.)
 //
 // A tile of 128 x 128 outputs (or 64 x 64) by 32 reduction elements per workgroup of 4 wavefronts.  The
 // split is done once per workgroup on the way from global memory to LDS (13 VALU instructions per two
 // elements: two or three between two MFMAs), not on every fragment read.  128 x 128: one LDS stage (48 KiB) and all
 // of a tile's fragments in registers (96 VGPRs); the next tile is written while the MFMAs of the current
 // one run, and a CU holds two workgroups, one of which multiplies while the other waits at a barrier or
-// for LDS (128 x 128 x 32 per CU: 2.01 us with one workgroup, 1.55 each with two).  64 x 64 tiles fill the
+// for LDS (128 x 128 x 32 per CU: 1.80 us with one workgroup, 1.44 each with two).  64 x 64 tiles fill the
 // chip on small problems, where a launch is as long as its chain of reduction tiles: two LDS stages (one
 // barrier a tile) and three reduction tiles in flight in registers (down projection at M=64, K=256, N=1024, one chain:
 // 27.8 us with one in flight, 26.0 with three).  Reading the fragments of the next tile ahead as well costs
@@ -59,8 +58,8 @@ struct F32Config {
 // as their residual, and results of 2^96 and more overflow in the scaled accumulators.  Accumulators that are
 // not finite are therefore computed again with fp32 MFMAs; overflows, infinities and NaNs then come out
 // as IEEE arithmetic gives them.  A launch with few of them takes up to 1.7 times as long, one in which every output is
-// done again two to three times (gate/up of x scaled by 2^100 at M=4096, K=2048, N=5632 1240 -> 3570 us; weight gradients
-// with a row of infinities 1840 -> 4660, all on fp32 MFMAs 2220).  Before, each such output was one lane's dot product:
+// done again two to three times (gate/up of x scaled by 2^100 at M=4096, K=2048, N=5632 1180 -> 3800 us; weight gradients
+// with a row of infinities 1700 -> 4420, all on fp32 MFMAs 2220).  Before, each such output was one lane's dot product:
 // 49000 and 51000 us.
 // 16 rows from m and G times 16 columns (of G / TN operands) from n over reduction tiles [kt_first, kt_end), laid out as
 // the accumulators; operands straight from global memory, 32 reduction elements at a time, lane / 16 choosing four of each half.
@@ -351,7 +350,7 @@ __global__ void __launch_bounds__(256, f32_per_cu(BM, 1)) gemm_f32_group_kernel(
 
 // The input gradient, the weight gradients and the bias gradients as one grid (see gemm_pipelined.hpp's of 16-bit
 // types), all on square tiles of the same size.  Backward passes, launches of their own -> one grid: 512x512x512 42 -> 34 us,
-// 684x56x224 27 -> 20 and with biases 33 -> 20, 1280x320x1216 88 -> 73 and 92 -> 72.
+// 684x56x224 27 -> 20 and with biases 32 -> 20, 1280x320x1216 88 -> 79 and 92 -> 77.
 template <int B, typename EpiX, typename EpiW>
 __global__ void __launch_bounds__(256, f32_per_cu(B, 1)) gemm_f32_dx_dw_kernel(DxDwGroup<float, EpiX, EpiW> grp) {
   int pid = (int)blockIdx.x;
