@@ -511,3 +511,35 @@ def test_m0_checker_flags_compiler_generated_m0_uses(tmp_path):
         assert mod.check(str(f), minimum=0) == 0
     f.write_text(good)
     assert mod.check(str(f), minimum=2) == 1
+
+
+def test_wait_states_around_inline_assembly_products_are_checked(tmp_path):
+    """csrc/check_mfma.py (run on every GEMM unit by the build): an inline-assembly MFMA's result is left alone
+    by everything but in-place products for some wait states, along every path behind it, and its operands
+    are not written right before it."""
+    import importlib.util
+
+    spec = importlib.util.spec_from_file_location("check_mfma", ROOT / "triton-gated-mlp_amd" / "csrc" / "check_mfma.py")
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    product = "\t;;#ASMSTART\n\tv_mfma_f32_16x16x32_f16 a[0:3], v[0:3], v[4:7], a[0:3]\n\t;;#ASMEND\n"
+    settle = "\ts_nop 15\n\ts_nop 3\n"
+    read = "\tv_accvgpr_read_b32 v9, a2\n"
+    kernel = "_Z4kern:\n"
+    for text, violations in (
+        (kernel + product + settle + read, 0),
+        (kernel + product + product + settle + read, 0),                       # in place: ordered by the hardware
+        (kernel + product + read, 1),
+        (kernel + product + "\ts_nop 15\n" + read, 1),                         # too few
+        (kernel + product + "\tv_accvgpr_read_b32 v9, a4\n", 0),               # another register
+        (kernel + product + "\tv_mfma_f32_16x16x32_f16 a[8:11], v[0:3], v[4:7], a[0:3]\n", 1),
+        (kernel + ".LBB0_1:\n" + read + product + "\ts_cbranch_scc1 .LBB0_1\n" + settle, 1),  # round the loop
+        (kernel + product + "\ts_branch .LBB0_2\n" + read + ".LBB0_2:\n" + settle, 0),
+        (kernel + "\tv_mov_b32_e32 v5, v8\n" + product + settle, 1),
+        (kernel + "\tv_mov_b32_e32 v5, v8\n\ts_nop 3\n" + product + settle, 0),
+    ):
+        f = tmp_path / "k.s"
+        f.write_text(text + "\ts_endpgm\n")
+        assert mod.check(str(f)) == violations, text
+    f.write_text(kernel + "\tv_mfma_f32_16x16x32_f16 a[0:3], v[0:3], v[4:7], a[0:3]\n\ts_endpgm\n")
+    assert mod.check(str(f)) == 1  # nothing recognised: nothing verified

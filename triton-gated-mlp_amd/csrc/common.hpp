@@ -21,6 +21,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // per lane: column l % 16, rows 4*(l/16) .. +3).  An operand fragment of v_mfma_f32_32x32x16_{f16,bf16} is 8 consecutive
 // reduction elements per lane: lane l carries row (l % 32), reduction slots 8*(l / 32) .. +7.
 // The 16 accumulator floats of lane l sit at column (l % 32), rows 8*(i/4) + 4*(l/32) + (i%4).
+// mfma16_inplace is mfma16 with the accumulator read and written in the same registers: left to choose, the
+// register allocator gives the result other registers than the summand where accumulators go round a loop,
+// and pays with copies (12 to 72 in an iteration of loops of 32 to 128 products).  The compiler does not put
+// wait states around inline assembly: mfma_settle() goes behind the last one, and csrc/check_mfma.py
+// holds the build to it.
 template <typename T>
 struct Traits;
 
@@ -33,6 +38,9 @@ struct Traits<f16> {
   }
   static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ void mfma16_inplace(vec8 a, vec8 b, f32x4& c) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
   }
   static __device__ __forceinline__ float to_f32(f16 v) { return (float)v; }
   static __device__ __forceinline__ f16 from_f32(float v) { return (f16)v; }
@@ -48,9 +56,18 @@ struct Traits<bf16> {
   static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ void mfma16_inplace(vec8 a, vec8 b, f32x4& c) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  }
   static __device__ __forceinline__ float to_f32(bf16 v) { return (float)v; }
   static __device__ __forceinline__ bf16 from_f32(float v) { return (bf16)v; }
 };
+
+// Until the results of mfma16_inplace may be read by anything else (7 wait states for the 16x16x32 shape).
+__device__ __forceinline__ void mfma_settle() {
+  asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
 
 template <>
 struct Traits<float> {
