@@ -1357,6 +1357,44 @@ def test_wide_tiles_and_split_gradients_against_fp32_products(M, K, N):
     assert all(torch.equal(a, b) for a, b in zip(got, run()))
 
 
+@pytest.mark.parametrize("act", ["silu", "gelu"])  # epilogue in the accumulators' layout and behind the transpose
+@pytest.mark.parametrize(
+    "M,K,N",
+    [
+        (200, 3080, 14344),  # gate/up on 128x256 tiles, reduction tails, a row tile of 72, ragged columns
+        (200, 3072, 28200),  # dH on 128x256 tiles
+        (893, 712, 5112),    # gate/up on 192x256 tiles (three loads of A a wavefront), reduction tails
+        (1289, 464, 6344),   # dH on them, three ring entries of A
+        (391, 64, 136),      # one reduction tile: the loop in place does not run
+    ],
+)
+def test_gate_up_and_dh_tiles_of_eight_wavefronts_against_fp32_products(M, K, N, act):
+    """Every output of the two GEMMs with long epilogues, biases and dropout on; twice, bit-identical."""
+    from triton_gated_mlp.ops import bwd as ops_bwd
+    from triton_gated_mlp.ops import fwd as ops_fwd
+
+    dev = _dev()
+    print(f"eight wavefronts: M={M} K={K} N={N} {act}", flush=True)
+    g = torch.Generator().manual_seed(21)
+    rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g)).bfloat16().to(dev)
+    f = lambda t: t.float()
+    x, dy, G, U = rnd(M, K), rnd(M, K), rnd(M, N), rnd(M, N)
+    wg, wu, wd, bg, bu = rnd(N, K, s=0.03), rnd(N, K, s=0.03), rnd(K, N, s=0.03), rnd(N, s=0.1), rnd(N, s=0.1)
+
+    def run():
+        hs = ops_fwd.gateup_fwd(x, wg, bg, wu, bu, dropout_p=0.1, seed=5, save_activations=True, act_fn=act)
+        return [hs.hidden, hs.gate, hs.up, *ops_bwd.dh_bwd(dy, wd, G, U, dropout_p=0.1, seed=5, act_fn=act)]
+
+    got = run()
+    keep = torch.from_numpy(philox.keep_mask(M, N, 0.1, 5, 0)).to(dev)
+    gate, up = f(x) @ f(wg).T + f(bg), f(x) @ f(wu).T + f(bu)
+    hb = oracle.hidden_backward(f(dy) @ f(wd), f(G), f(U), keep, 0.1, act)
+    refs = [oracle.ACTS[act][0](gate) * up * keep.float() / 0.9, gate, up, hb["dG"], hb["dU"]]
+    for name, a, b in zip(("H", "G", "U", "dG", "dU"), got, refs):
+        _close(name, a, b)
+    assert all(torch.equal(a, b) for a, b in zip(got, run()))
+
+
 def test_second_stages_against_float64():
     """Sums of 2 to 16 partial results (every remainder of the groups that are in flight together) and
     column sums at the edges of their row ranges and of a workgroup's 256 columns.  fp16 results of

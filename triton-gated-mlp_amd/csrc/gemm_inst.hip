@@ -19,20 +19,25 @@ constexpr bool KT = GMLP_KT;
   launch_gemm_pipelined<DT, 256, BN_L, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M) \
   launch_gemm_pipelined<DT, 128, BN_M, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
-#define GMLP_TALL(AKS, BKS, NB, EPI, BN_T) \
-  launch_gemm_pipelined<DT, 192, BN_T, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
-#define GMLP_WIDE(AKS, BKS, NB, EPI, BN_W) \
-  launch_gemm_pipelined<DT, 128, BN_W, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
+// (WN: wavefronts side by side, 2 or 4.  A tile's epilogue is a chain of loads, conversions and stores per
+// wavefront: eight wavefronts halve it where it is long, at a third more LDS reads in the loop.  us, four -> eight:
+// gate/up with G and U kept TALL M=1357, K=1160, N=3096 gelu 37.3 -> 34.3, M=2048, K=2048, N=5632 gelu 90 -> 84,
+// silu 87 -> 85, WIDE M=1024, K=2048, N=5632 53.4 -> 49.7; dH WIDE 65.7 -> 62.3.  Plain stores and partial sums:
+// no difference; dH TALL has no registers for it.)
+#define GMLP_TALL(AKS, BKS, NB, EPI, BN_T, WN) \
+  launch_gemm_pipelined<DT, 192, BN_T, 16, 2, WN, AKS, BKS, NB, EPI<DT>, KT>
+#define GMLP_WIDE(AKS, BKS, NB, EPI, BN_W, WN) \
+  launch_gemm_pipelined<DT, 128, BN_W, 16, 2, WN, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_LARGE_GROUP \
   launch_gemm_group_pipelined<DT, 256, 256, 16, 2, 2, true, true, 1, EpiStore<DT>>
 #define GMLP_MEDIUM_GROUP \
   launch_gemm_group_pipelined<DT, 128, 128, 16, 2, 2, true, true, 1, EpiStore<DT>>
 
-#define GMLP_DISPATCH(AKS, BKS, NB, EPI, BN_L, BN_M)                                             \
+#define GMLP_DISPATCH(AKS, BKS, NB, EPI, BN_L, BN_M, WN_W, WN_T)                                 \
   if (tile_class == TILE_LARGE) return GMLP_LARGE(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
   if constexpr (!(AKS)) {                                                                        \
-    if (tile_class == TILE_WIDE) return GMLP_WIDE(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
-    if (tile_class == TILE_TALL) return GMLP_TALL(AKS, BKS, NB, EPI, BN_L)(ga, ea, s);           \
+    if (tile_class == TILE_WIDE) return GMLP_WIDE(AKS, BKS, NB, EPI, BN_L, WN_W)(ga, ea, s);     \
+    if (tile_class == TILE_TALL) return GMLP_TALL(AKS, BKS, NB, EPI, BN_L, WN_T)(ga, ea, s);     \
   }                                                                                              \
   if (tile_class == TILE_MEDIUM_FULL) return GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M)(ga, ea, s);    \
   if constexpr (KT) return hipErrorInvalidValue; /* launch.hpp sends it to the other unit */       \
@@ -45,50 +50,50 @@ hipError_t launch_gateup_kt<DT, KT>(int tile_class, const GemmArgs& ga, const Ep
   // the usual case (SiLU, no keep-mask output) has kernels of its own, see EpiGateUpPacked
   if (EpiGateUpPacked<DT>::packed_eligible(ea)) {
     if (tile_class == TILE_LARGE) return GMLP_LARGE(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
-    if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
-    if (tile_class == TILE_TALL) return GMLP_TALL(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
+    if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 2, EpiGateUpPacked, 128, 4)(ga, ea, s);
+    if (tile_class == TILE_TALL) return GMLP_TALL(false, false, 2, EpiGateUpPacked, 128, 4)(ga, ea, s);
     if (tile_class == TILE_MEDIUM_FULL) return GMLP_MEDIUM(false, false, 2, EpiGateUpPacked, 64)(ga, ea, s);
   }
-  GMLP_DISPATCH(false, false, 2, EpiGateUp, 128, 64)
+  GMLP_DISPATCH(false, false, 2, EpiGateUp, 128, 64, 4, 4)
 }
 template <>
 hipError_t launch_gateup_split_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
-  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 2, EpiPartial, 128)(ga, ea, s);
+  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 2, EpiPartial, 128, 2)(ga, ea, s);
   return launch_gemm_pipelined<DT, 128, 64, 16, 2, 2, false, false, 2, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 1
 template <>
 hipError_t launch_linear_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiStore<DT>::Args& ea,
                              hipStream_t s) {
-  GMLP_DISPATCH(false, false, 1, EpiStore, 256, 128)
+  GMLP_DISPATCH(false, false, 1, EpiStore, 256, 128, 2, 2)
 }
 template <>
 hipError_t launch_linear_split_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
-  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 1, EpiPartial, 256)(ga, ea, s);
+  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 1, EpiPartial, 256, 2)(ga, ea, s);
   return launch_gemm_pipelined<DT, 128, 128, 16, 2, 2, false, false, 1, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 2
 template <>
 hipError_t launch_dh_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiDh<DT>::Args& ea,
                          hipStream_t s) {
-  GMLP_DISPATCH(false, true, 1, EpiDh, 256, 128)
+  GMLP_DISPATCH(false, true, 1, EpiDh, 256, 128, 4, 2)
 }
 #elif GMLP_KIND == 3
 template <>
 hipError_t launch_dx_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiStore<DT>::Args& ea,
                          hipStream_t s) {
-  GMLP_DISPATCH(false, true, 1, EpiStore, 256, 128)
+  GMLP_DISPATCH(false, true, 1, EpiStore, 256, 128, 2, 2)
 }
 template <>
 hipError_t launch_dx_split_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {
-  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, true, 1, EpiPartial, 256)(ga, ea, s);
+  if (tile_class == TILE_WIDE) return GMLP_WIDE(false, true, 1, EpiPartial, 256, 2)(ga, ea, s);
   return launch_gemm_pipelined<DT, 128, 128, 16, 2, 2, false, true, 1, EpiPartial<DT>, KT>(ga, ea, s);
 }
 #elif GMLP_KIND == 4
 template <>
 hipError_t launch_dw<DT>(int tile_class, const GemmArgs& ga, const EpiStore<DT>::Args& ea,
                          hipStream_t s) {
-  GMLP_DISPATCH(true, true, 1, EpiStore, 256, 128)
+  GMLP_DISPATCH(true, true, 1, EpiStore, 256, 128, 2, 2)
 }
 template <>
 hipError_t launch_dw_group<DT>(int tile_class, GemmGroup<EpiStore<DT>::Args>& grp, hipStream_t s) {

@@ -47,13 +47,15 @@ constexpr int LOAD_CYCLES = 64;
 constexpr int B_LOOKAHEAD = 3;
 
 // Kernels that get the three-entry A ring (see PipeConfig::A3): those with a reduction-contiguous A
-// operand other than dH, i.e. gate/up, the down projection and the input gradient.  The long
+// operand other than dH on 256-row tiles, i.e. gate/up, the down projection, the input gradient and dH.  The long
 // reductions over the intermediate size gain most (they stall on a full vector-memory queue
-// otherwise), gate/up gains from a cold start only.  dH's epilogue prefetch and the weight
-// gradients' two transposed operands leave no registers for it (spills when tried).
-template <typename T, typename Epi>
+// otherwise), gate/up gains from a cold start only.  dH's epilogue prefetch on 256-row tiles and the weight
+// gradients' two transposed operands leave no registers for it (spills when tried).  dH on 128x128 tiles (bf16, us,
+// two entries -> three): M=2048, N=5632, K=2048 66 -> 58, M=1024, N=2816, K=1024 17.1 -> 14.7; 192x256: 37.6 -> 36.4 at
+// M=1357, N=3096, K=1160.
+template <typename T, typename Epi, int BM>
 constexpr bool wants_ring_a3() {
-  return !std::is_same<Epi, EpiDh<T>>::value;
+  return !std::is_same<Epi, EpiDh<T>>::value || BM < 256;
 }
 
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB, bool RING_A3 = false>
@@ -85,7 +87,8 @@ struct PipeConfig {
   static constexpr int LDS_BYTES = MAIN_BYTES > NW * EPI_WAVE_BYTES ? MAIN_BYTES : NW * EPI_WAVE_BYTES;
   static_assert(G >= 2 && TM >= 2 && TM % 2 == 0, "rolling scheme needs >= 2 groups and an even TM");
   static_assert((KSTEPS * G) % 4 == 0, "B ring index must be static");
-  static_assert(TM <= G, "one A fetch per group must cover the next step");
+  static constexpr int APG = (TM + G - 1) / G;  // A fragments of the next step fetched per group
+  static_assert(APG < TM, "a group has slots for its A fetches");
   static_assert(KSTEPS % 2 == 0, "A banks alternate by step and every tile starts on bank 0");
   static_assert(NS == 2, "the retiring barrier waits for everything in flight");
 };
@@ -94,7 +97,7 @@ template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool 
           typename Epi, bool SK = false, bool KT = false>
 __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const typename Epi::Args& ea_in,
                                                     int pid, int nwg) {
-  typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi>()> Cfg;
+  typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi, BM>()> Cfg;
   typedef typename Cfg::ATile ATile;
   typedef typename Cfg::BTile BTile;
   typedef typename Traits<T>::vec8 vec8;
@@ -190,22 +193,24 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
 
   // KT: chunks of 8 reduction elements beyond K in the last reduction tile of a KC operand.  A lane
   // fetches chunk (lane % 8) ^ swz(row) of its row, and swz depends on the load's number only by
-  // its parity (8 rows per load), so two masks per lane say which of its loads to drop there:
+  // its parity in the whole tile (8 rows per load), so two masks per lane say which of its loads to drop there:
   // bit 31 puts an offset beyond the end of any operand (they are smaller than 2 GiB).
-  uint32_t oob[2] = {0u, 0u};
+  uint32_t oob_a[2] = {0u, 0u}, oob_b[2] = {0u, 0u};
   if constexpr (KT) {
     const int kvalid = ga.K - (kt_seg - 1) * BK;
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
-      oob[p] = ((lane & 7) ^ ((4 * p + (lane >> 4)) & 7)) * 8 >= kvalid ? 0x80000000u : 0u;
+    for (int p = 0; p < 2; ++p) {
+      const int pa = p ^ (ATile::PER_WAVE & wave & 1), pb = p ^ (BTile::PER_WAVE & wave & 1);
+      oob_a[p] = ((lane & 7) ^ ((4 * pa + (lane >> 4)) & 7)) * 8 >= kvalid ? 0x80000000u : 0u;
+      oob_b[p] = ((lane & 7) ^ ((4 * pb + (lane >> 4)) & 7)) * 8 >= kvalid ? 0x80000000u : 0u;
+    }
   }
-  static_assert(!KT || (ATile::PER_WAVE % 2 == 0 && BTile::PER_WAVE % 2 == 0), "chunk masks go by the load's parity");
   // Offset of load i of an operand: `soff` says whether the load state stands at the last
   // reduction tile of the operand's rows, whose first tile is at `org`.
-  auto kt_offset = [&](uint32_t off, int i, uint32_t soff, uint32_t org) __attribute__((always_inline)) {
+  auto kt_offset = [&](uint32_t off, uint32_t mask, uint32_t soff, uint32_t org) __attribute__((always_inline)) {
     if constexpr (KT) {
       const uint32_t at_tail = soff == org + (uint32_t)(kt_seg - 1) * (BK * 2) ? 0xFFFFFFFFu : 0u;
-      return off | (oob[i & 1] & at_tail);
+      return off | (mask & at_tail);
     } else {
       return off;
     }
@@ -289,12 +294,12 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
     if (x < ATile::PER_WAVE) {
       r = buffer_rsrc{(int)(uint32_t)ld_head_a, (int)(uint32_t)(ld_head_a >> 32), ra[0][2], ra[0][3]};
       soff = ld_soff_a;
-      voff = A_KS ? aoff[x] : kt_offset(aoff[x], x, soff, a_org);
+      voff = A_KS ? aoff[x] : kt_offset(aoff[x], oob_a[x & 1], soff, a_org);
     } else {
       int y = x - ATile::PER_WAVE, bsel = y / BTile::PER_WAVE, i = y % BTile::PER_WAVE;
       r = NB == 2 ? rb[bsel] : buffer_rsrc{(int)(uint32_t)ld_head_b, (int)(uint32_t)(ld_head_b >> 32), rb[0][2], rb[0][3]};
       soff = ld_soff_b;
-      voff = B_KS ? boff[i] : kt_offset(boff[i], i, soff, b_org);
+      voff = B_KS ? boff[i] : kt_offset(boff[i], oob_b[i & 1], soff, b_org);
     }
     switch (load_index(x) & 3) {
       case 0: load16_to_lds_at<0>(r, voff, soff); break;
@@ -352,11 +357,11 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
       const int bsel = z / BTile::PER_WAVE, i = z % BTile::PER_WAVE;
       r = NB == 2 ? rb[bsel] : buffer_rsrc{(int)(uint32_t)l3_head[1], (int)(uint32_t)(l3_head[1] >> 32), rb[0][2], rb[0][3]};
       soff = l3_soff[1];
-      voff = B_KS ? boff[i] : kt_offset(boff[i], i, soff, b_org);
+      voff = B_KS ? boff[i] : kt_offset(boff[i], oob_b[i & 1], soff, b_org);
     } else {
       r = buffer_rsrc{(int)(uint32_t)l3_head[0], (int)(uint32_t)(l3_head[0] >> 32), ra[0][2], ra[0][3]};
       soff = l3_soff[0];
-      voff = A_KS ? aoff[z - LDB] : kt_offset(aoff[z - LDB], z - LDB, soff, a_org);
+      voff = A_KS ? aoff[z - LDB] : kt_offset(aoff[z - LDB], oob_a[(z - LDB) & 1], soff, a_org);
     }
     switch (l3_index(z) & 3) {
       case 0: load16_to_lds_at<0>(r, voff, soff); break;
@@ -436,7 +441,8 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
           }
           // --- A fragments of the next step: one per group, or all of them after the handover
           if (!last) {
-            if (i == 1 && g < TM) fetch_a((ks + 1) & 1, g, kt, ks + 1);
+            const int h = g * Cfg::APG + (i - 1);
+            if (i >= 1 && i <= Cfg::APG && h < TM) fetch_a((ks + 1) & 1, h, kt, ks + 1);
           } else if (NEXT && handover) {
             constexpr int AH = (TM + LA - 1) / LA;  // A fragments per handover group
             const int h = (g - (G - LA)) * AH + (i - 1);
@@ -502,7 +508,8 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
             else if (NEXT) fetch_b3((g2 - G) % 4, g2 - G, b_nxt, 0);
           }
           if (!last) {
-            if (i == 1 && g < TM) fetch_a3((ks + 1) & 1, g, a_rd, ks + 1);
+            const int h = g * Cfg::APG + (i - 1);
+            if (i >= 1 && i <= Cfg::APG && h < TM) fetch_a3((ks + 1) & 1, h, a_rd, ks + 1);
           } else if (NEXT && handover) {
             constexpr int AH = (TM + LA - 1) / LA;
             const int h = (g - (G - LA)) * AH + (i - 1);
@@ -619,7 +626,10 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
       l3_issue(z);
     }
     l3_advance(0);
-    static_assert(HEAD_SLOTS % LSL3 != PH3 || HEAD_B % 4 != 0, "no handover slot leaves an M0 for the first load of a tile proper");
+    // (and the M0 that the last handover slot would have left for the next load: 128x256 tiles of eight wavefronts)
+    static_assert(HEAD_SLOTS % LSL3 != PH3 || HEAD_B < LDB, "that load is one of the B operand's");
+    if constexpr (HEAD_SLOTS % LSL3 == PH3)
+      if (l3_starts_group(HEAD_B)) l3_base(HEAD_B, B3 ? 2u * B_ENTRY : b1, 0u);
     wait_vmem<(B3 ? L3 : LDA) + HEAD_B>();
     __syncthreads();
 #pragma unroll
@@ -913,7 +923,7 @@ template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool 
           typename Epi, bool KT>
 hipError_t launch_streamk_tail(const GemmArgs& ga, const typename Epi::Args& ea, hipStream_t s) {
   if constexpr (!Epi::SPLIT && BM == 256) {
-    typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi>()> Cfg;
+    typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi, BM>()> Cfg;
     constexpr auto kern = gemm_kernel_pipelined<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, true, KT>;
     if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, Cfg::LDS_BYTES>, s)) return e;
     hipLaunchKernelGGL(kern, dim3(ga.sk_wgs), dim3(Cfg::NW * 64), Cfg::LDS_BYTES, s, ga, ea);
@@ -993,8 +1003,8 @@ __global__ void __launch_bounds__(256) gemm_dx_dw_kernel_pipelined(DxDwGroup<T, 
 
 template <typename T, int BMX, int BNX, int BMW, bool KT, typename EpiX, typename EpiW>
 hipError_t launch_dx_dw_pipelined(DxDwGroup<T, EpiX, EpiW>& grp, bool dx_first, hipStream_t s) {
-  typedef PipeConfig<T, BMX, BNX, 16, 2, 2, false, true, 1, wants_ring_a3<T, EpiX>()> CfgX;
-  typedef PipeConfig<T, BMW, BMW, 16, 2, 2, true, true, 1, wants_ring_a3<T, EpiW>()> CfgW;
+  typedef PipeConfig<T, BMX, BNX, 16, 2, 2, false, true, 1, wants_ring_a3<T, EpiX, BMX>()> CfgX;
+  typedef PipeConfig<T, BMW, BMW, 16, 2, 2, true, true, 1, wants_ring_a3<T, EpiW, BMW>()> CfgW;
   constexpr int LDS = CfgX::LDS_BYTES > CfgW::LDS_BYTES ? CfgX::LDS_BYTES : CfgW::LDS_BYTES;
   constexpr auto kern = gemm_dx_dw_kernel_pipelined<T, BMX, BNX, BMW, EpiX, EpiW, KT>;
   if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, LDS>, s)) return e;
@@ -1006,7 +1016,7 @@ hipError_t launch_dx_dw_pipelined(DxDwGroup<T, EpiX, EpiW>& grp, bool dx_first, 
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
           typename Epi, bool KT = false>
 hipError_t launch_gemm_pipelined(const GemmArgs& ga, const typename Epi::Args& ea, hipStream_t s) {
-  typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi>()> Cfg;
+  typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi, BM>()> Cfg;
   constexpr auto kern = gemm_kernel_pipelined<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi, false, KT>;
   if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, Cfg::LDS_BYTES>, s)) return e;
   const int splits = Epi::SPLIT ? ga.splits : 1;
@@ -1023,7 +1033,7 @@ hipError_t launch_gemm_pipelined(const GemmArgs& ga, const typename Epi::Args& e
 template <typename T, int BM, int BN, int MI, int WGM, int WGN, bool A_KS, bool B_KS, int NB,
           typename Epi>
 hipError_t launch_gemm_group_pipelined(GemmGroup<typename Epi::Args>& grp, hipStream_t s) {
-  typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi>()> Cfg;
+  typedef PipeConfig<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, wants_ring_a3<T, Epi, BM>()> Cfg;
   constexpr auto kern = gemm_group_kernel_pipelined<T, BM, BN, MI, WGM, WGN, A_KS, B_KS, NB, Epi>;
   if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, Cfg::LDS_BYTES>, s)) return e;
   int total = 0;

@@ -6,7 +6,8 @@
 
 namespace gmlp {
 
-// Tile classes (all four wavefronts per workgroup, 64-wide reduction tiles).
+// Tile classes (four wavefronts per workgroup, eight on WIDE and TALL tiles of gate/up and WIDE ones of dH; 64-wide
+// reduction tiles).
 //   LARGE        256x256 output tiles, wavefronts of 128x128, pipelined kernel
 //   WIDE         128x256 output tiles, wavefronts of 64x128, pipelined kernel (not the weight gradients):
 //                one workgroup per CU, three ring entries of both operands.  Half of LARGE's work per
