@@ -1357,26 +1357,40 @@ def test_wide_tiles_and_split_gradients_against_fp32_products(M, K, N):
     assert all(torch.equal(a, b) for a, b in zip(got, run()))
 
 
+# The GEMMs with long epilogues: output tile (gate/up: of each accumulator set) and wavefronts of gate/up with SiLU, with
+# another activation, and of dH; on a whole MI355X.
+_LONG_EPILOGUES = [
+    # M, K, N, gate/up SiLU, gate/up GELU, dH
+    (200, 3080, 14344, (128, 128, 8), (128, 128, 8), (128, 128, 4)),  # reduction tails, a row tile of 72, ragged columns
+    (200, 3072, 14344, (128, 128, 8), (128, 128, 8), (128, 128, 4)),
+    (1000, 3080, 8192, (256, 128, 4), (256, 128, 4), (128, 256, 8)),  # dH: a row tile of 104, reduction tails
+    (1000, 3072, 8192, (256, 128, 4), (256, 128, 4), (128, 256, 8)),
+    (893, 712, 5112, (192, 128, 8), (192, 128, 8), (128, 128, 4)),    # 12 reduction tiles; three loads of A a wavefront
+    (900, 960, 4104, (192, 128, 8), (192, 128, 8), (128, 128, 4)),    # 15
+    (900, 968, 4104, (192, 128, 4), (192, 128, 8), (128, 128, 4)),    # 16: SiLU's epilogue no longer outweighs the loop
+    (900, 1472, 4104, (192, 128, 4), (192, 128, 8), (128, 128, 4)),   # 23
+    (900, 1480, 4104, (192, 128, 4), (192, 128, 4), (128, 128, 4)),   # 24: nor does GELU's
+    (900, 1536, 4104, (192, 128, 4), (192, 128, 4), (128, 128, 4)),
+    (1289, 464, 6344, (128, 64, 4), (128, 64, 4), (192, 256, 4)),     # dH: three ring entries of A
+    (391, 64, 136, (128, 64, 4), (128, 64, 4), (128, 128, 4)),        # one reduction tile: the loop in place does not run
+]
+
+
+@pytest.mark.parametrize("M,K,N,silu,gelu,dh", _LONG_EPILOGUES, ids=lambda v: str(v) if isinstance(v, int) else "")
 @pytest.mark.parametrize("act", ["silu", "gelu"])  # epilogue in the accumulators' layout and behind the transpose
-@pytest.mark.parametrize(
-    "M,K,N",
-    [
-        (200, 3080, 14344),  # gate/up on 128x256 tiles, reduction tails, a row tile of 72, ragged columns
-        (200, 3072, 28200),  # dH on 128x256 tiles
-        (893, 712, 5112),    # gate/up on 192x256 tiles (three loads of A a wavefront), reduction tails
-        (1289, 464, 6344),   # dH on them, three ring entries of A
-        (391, 64, 136),      # one reduction tile: the loop in place does not run
-    ],
-)
-def test_gate_up_and_dh_tiles_of_eight_wavefronts_against_fp32_products(M, K, N, act):
-    """Every output of the two GEMMs with long epilogues, biases and dropout on; twice, bit-identical."""
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gate_up_and_dh_tiles_and_wavefronts_against_fp32_products(M, K, N, silu, gelu, dh, act, dtype):
+    """Every output of the two GEMMs with long epilogues, biases and dropout on; twice, bit-identical; with the launched
+    kernels' tiles and wavefronts."""
+    import re
+
     from triton_gated_mlp.ops import bwd as ops_bwd
     from triton_gated_mlp.ops import fwd as ops_fwd
 
     dev = _dev()
-    print(f"eight wavefronts: M={M} K={K} N={N} {act}", flush=True)
+    print(f"long epilogues: M={M} K={K} N={N} {act} {dtype}", flush=True)
     g = torch.Generator().manual_seed(21)
-    rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g)).bfloat16().to(dev)
+    rnd = lambda *shape, s=1.0: (s * torch.randn(*shape, generator=g)).to(dtype).to(dev)
     f = lambda t: t.float()
     x, dy, G, U = rnd(M, K), rnd(M, K), rnd(M, N), rnd(M, N)
     wg, wu, wd, bg, bu = rnd(N, K, s=0.03), rnd(N, K, s=0.03), rnd(K, N, s=0.03), rnd(N, s=0.1), rnd(N, s=0.1)
@@ -1385,7 +1399,13 @@ def test_gate_up_and_dh_tiles_of_eight_wavefronts_against_fp32_products(M, K, N,
         hs = ops_fwd.gateup_fwd(x, wg, bg, wu, bu, dropout_p=0.1, seed=5, save_activations=True, act_fn=act)
         return [hs.hidden, hs.gate, hs.up, *ops_bwd.dh_bwd(dy, wd, G, U, dropout_p=0.1, seed=5, act_fn=act)]
 
-    got = run()
+    names, got = _launched(run)
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        # tile rows, tile columns, (MFMA shape), wavefronts below and beside each other
+        numbers = r"gemm_kernel_pipelined.*?" + r"(?:Li|, )(\d+)E?" * 5
+        found = [tuple(map(int, m.groups())) for m in (re.search(numbers, n) for n in names) if m]
+        launched = [(rows, cols, down * beside) for rows, cols, _, down, beside in found]
+        assert launched == [silu if act == "silu" else gelu, dh], names
     keep = torch.from_numpy(philox.keep_mask(M, N, 0.1, 5, 0)).to(dev)
     gate, up = f(x) @ f(wg).T + f(bg), f(x) @ f(wu).T + f(bu)
     hb = oracle.hidden_backward(f(dy) @ f(wd), f(G), f(U), keep, 0.1, act)

@@ -20,10 +20,8 @@ constexpr bool KT = GMLP_KT;
 #define GMLP_MEDIUM(AKS, BKS, NB, EPI, BN_M) \
   launch_gemm_pipelined<DT, 128, BN_M, 16, 2, 2, AKS, BKS, NB, EPI<DT>, KT>
 // (WN: wavefronts side by side, 2 or 4.  A tile's epilogue is a chain of loads, conversions and stores per
-// wavefront: eight wavefronts halve it where it is long, at a third more LDS reads in the loop.  us, four -> eight:
-// gate/up with G and U kept TALL M=1357, K=1160, N=3096 gelu 37.3 -> 34.3, M=2048, K=2048, N=5632 gelu 90 -> 84,
-// silu 87 -> 85, WIDE M=1024, K=2048, N=5632 53.4 -> 49.7; dH WIDE 65.7 -> 62.3.  Plain stores and partial sums:
-// no difference; dH TALL has no registers for it.)
+// wavefront: eight wavefronts halve it where it is long, at up to 43 % more LDS reads in the loop.  Plain stores and
+// partial sums: no difference; dH: WIDE 1 % at most, no registers for it on TALL.  Gate/up: gate_up_eight_wavefronts.)
 #define GMLP_TALL(AKS, BKS, NB, EPI, BN_T, WN) \
   launch_gemm_pipelined<DT, 192, BN_T, 16, 2, WN, AKS, BKS, NB, EPI<DT>, KT>
 #define GMLP_WIDE(AKS, BKS, NB, EPI, BN_W, WN) \
@@ -44,6 +42,19 @@ constexpr bool KT = GMLP_KT;
   else return launch_gemm<DT, 128, BN_M, 64, 2, 2, AKS, BKS, NB, true, EPI<DT>>(ga, ea, s);
 
 #if GMLP_KIND == 0
+// Gate/up on TALL tiles: the shorter epilogue of eight wavefronts against their slower loop, by the reduction's
+// length.  Time with four over eight by the number of 64-wide reduction tiles, weights from memory / from cache (geometric
+// means over 1396 launches of random shapes):
+//                          8..11        12..15       16..19       20..23       32..35       48..55       96 on
+//   SiLU (packed)      1.07 / 1.08  1.02 / 1.05  0.98 / 1.03  0.96 / 1.02  0.93 / 1.00  0.91 / 0.98  0.89 / 0.90
+//   other activations  1.13 / 1.14  1.07 / 1.10  1.02 / 1.08  1.00 / 1.06  0.95 / 1.03  0.93 / 1.00  0.91 / 0.90
+// The lines are where the ones from memory cross: a model's layers come by in turn, and its weights with them.  us, eight ->
+// four: M=3582, K=3200, N=11992 G and U kept 518 -> 482; M=1357, K=1160, N=3096 gelu stays on eight (37.3 with four, 34.3).
+// On WIDE tiles eight are never behind (1.03 at 20 tiles, 1.00 from 96 on).
+template <typename Epi>
+static bool gate_up_eight_wavefronts(const GemmArgs& ga) {
+  return ga.K <= 64 * (std::is_same<Epi, EpiGateUpPacked<DT>>::value ? 15 : 23);
+}
 template <>
 hipError_t launch_gateup_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiGateUp<DT>::Args& ea,
                              hipStream_t s) {
@@ -51,10 +62,14 @@ hipError_t launch_gateup_kt<DT, KT>(int tile_class, const GemmArgs& ga, const Ep
   if (EpiGateUpPacked<DT>::packed_eligible(ea)) {
     if (tile_class == TILE_LARGE) return GMLP_LARGE(false, false, 2, EpiGateUpPacked, 128)(ga, ea, s);
     if (tile_class == TILE_WIDE) return GMLP_WIDE(false, false, 2, EpiGateUpPacked, 128, 4)(ga, ea, s);
-    if (tile_class == TILE_TALL) return GMLP_TALL(false, false, 2, EpiGateUpPacked, 128, 4)(ga, ea, s);
+    if (tile_class == TILE_TALL)
+      return gate_up_eight_wavefronts<EpiGateUpPacked<DT>>(ga) ? GMLP_TALL(false, false, 2, EpiGateUpPacked, 128, 4)(ga, ea, s)
+                                                               : GMLP_TALL(false, false, 2, EpiGateUpPacked, 128, 2)(ga, ea, s);
     if (tile_class == TILE_MEDIUM_FULL) return GMLP_MEDIUM(false, false, 2, EpiGateUpPacked, 64)(ga, ea, s);
   }
-  GMLP_DISPATCH(false, false, 2, EpiGateUp, 128, 64, 4, 4)
+  if (tile_class == TILE_TALL && gate_up_eight_wavefronts<EpiGateUp<DT>>(ga))
+    return GMLP_TALL(false, false, 2, EpiGateUp, 128, 4)(ga, ea, s);
+  GMLP_DISPATCH(false, false, 2, EpiGateUp, 128, 64, 4, 2)
 }
 template <>
 hipError_t launch_gateup_split_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiPartial<DT>::Args& ea, hipStream_t s) {

@@ -6,16 +6,17 @@
 
 namespace gmlp {
 
-// Tile classes (four wavefronts per workgroup, eight on WIDE and TALL tiles of gate/up and WIDE ones of dH; 64-wide
-// reduction tiles).
+// Tile classes (four wavefronts per workgroup, eight of half the width where said; 64-wide reduction tiles).
 //   LARGE        256x256 output tiles, wavefronts of 128x128, pipelined kernel
-//   WIDE         128x256 output tiles, wavefronts of 64x128, pipelined kernel (not the weight gradients):
+//   WIDE         128x256 output tiles, wavefronts of 64x128 (gate/up without a split, dH: eight of 64x64), pipelined kernel
+//                (not the weight gradients):
 //                one workgroup per CU, three ring entries of both operands.  Half of LARGE's work per
 //                workgroup at 5/6 of its throughput: for grids that LARGE fills badly and for short
 //                batches, where it reads the weights once per 128 token rows from L2 and needs fewer
 //                splits than MEDIUM_FULL
-//   TALL         192x256 output tiles, wavefronts of 96x128, pipelined kernel (not the weight gradients, no
-//                split reductions): three quarters of LARGE's work, for grids that LARGE fills badly
+//   TALL         192x256 output tiles, wavefronts of 96x128 (gate/up with a short reduction: eight of 96x64), pipelined
+//                kernel (not the weight gradients, no split reductions): three quarters of LARGE's work, for grids that
+//                LARGE fills badly
 //   MEDIUM_FULL  128x128 output tiles, wavefronts of 64x64, pipelined kernel; two workgroups per CU,
 //                for problems with too few 256x256 tiles to fill the chip
 //   MEDIUM       128x128, predicated register-staged kernel, 64-bit addresses: operands too large for
