@@ -2045,26 +2045,27 @@ def test_decode_streaming_kernels_short_segments(M, K, N, gated, down):
 
 
 @pytest.mark.parametrize(
-    "M,K,N,down",  # down: token tiles, bytes of a row per stage, rows of a region, wavefronts (on a whole MI355X)
+    "M,K,N,down",  # down: token tiles, bytes of a row per stage, ring slots, row tails, rows of a region, wavefronts (on a whole MI355X)
     [
-        (1, 768, 1024, (1, 128, 8, 4)),     # 96 workgroups; four chunks a wavefront
-        (16, 2048, 1280, (1, 128, 8, 4)),   # 256 workgroups of 8 rows
-        (3, 1984, 776, (1, 512, 8, 3)),     # 248; one 16-byte piece in the last chunk, rows across 128-byte lines
-        (11, 1000, 4104, (1, 512, 8, 3)),   # H in fragment order
-        (17, 2040, 768, (2, 512, 8, 3)),    # 255; two token tiles, a chunk a wavefront
-        (32, 2048, 1032, (2, 512, 8, 3)),
-        (5, 2112, 4096, (1, 128, 16, 4)),   # 8.25 rows a share
-        (9, 3328, 2048, (1, 128, 16, 4)),   # 13
-        (2, 3392, 2048, (1, 128, 16, 3)),   # 13.25
+        (1, 768, 1024, (1, 128, 8, 0, 8, 4)),     # 96 workgroups; four chunks a wavefront
+        (16, 2048, 1280, (1, 128, 8, 0, 8, 4)),   # 256 workgroups of 8 rows
+        (1, 2048, 8192, (1, 512, 3, 0, 8, 3)),    # more weights than short segments take at this M; ten or eleven chunks
+        (11, 2040, 2048, (1, 512, 3, 0, 8, 3)),   # 255 workgroups, fewer chunks than slots; H in fragment order
+        (1, 776, 768, (1, 512, 3, 0, 8, 3)),      # one chunk a wavefront
+        (3, 1984, 776, (1, 512, 3, 1, 8, 3)),     # 248; one 16-byte piece in the last chunk, rows across 128-byte lines
+        (11, 1000, 4104, (1, 512, 3, 1, 8, 3)),
+        (17, 2040, 768, (2, 512, 3, 0, 8, 3)),    # two token tiles, a chunk a wavefront
+        (32, 2048, 1032, (2, 512, 3, 1, 8, 3)),
+        (5, 2112, 4096, (1, 128, 8, 0, 16, 4)),   # 8.25 rows a share
+        (9, 3328, 2048, (1, 128, 8, 0, 16, 4)),   # 13
+        (2, 3392, 2048, (1, 128, 8, 0, 16, 3)),   # 13.25
     ],
     ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v),
 )
 def test_decode_down_projection_of_small_shares(M, K, N, down):
     """Regions of 8 rows and four wavefronts, at the ends of the widths that take them, against float64
-    products; with the launched kernel's name."""
+    products; twice, bit-identical; with the launched kernel's name."""
     import re
-
-    from torch.profiler import ProfilerActivity, profile
 
     dev = _dev()
     dtype = torch.bfloat16 if M % 2 else torch.float16
@@ -2075,21 +2076,24 @@ def test_decode_down_projection_of_small_shares(M, K, N, down):
     rnd = lambda *shape, s=1.0: torch.empty(shape, device=dev).normal_(0.0, s, generator=g).to(dtype)
     x, wg, wu, wd, bd = rnd(M, K, s=0.5), rnd(N, K, s=0.02), rnd(N, K, s=0.02), rnd(K, N, s=0.02), rnd(K, s=0.1)
     wd[:, :8] *= 16
-    h = torch.full((16 if M <= 16 else 32, N), float("nan"), dtype=dtype, device=dev)
-    y = torch.full((M, K), float("nan"), dtype=dtype, device=dev)
-    torch.cuda.synchronize()
-    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as prof:
+
+    def run():
+        h = torch.full((16 if M <= 16 else 32, N), float("nan"), dtype=dtype, device=dev)
+        y = torch.full((M, K), float("nan"), dtype=dtype, device=dev)
         _cabi.check(_cabi.lib().gmlp_decode_stream_fwd(
             *(_cabi.ptr(t) for t in (x, wg, wu, wd, None, None, bd, h, y)), M, K, N, _cabi.dtype_code(dtype),
             _cabi.act_code("silu"), _cabi.stream_ptr(dev)))
-        torch.cuda.synchronize()
+        return y
+
+    names, y = _launched(run)
     hidden = torch.nn.functional.silu(x.double() @ wg.double().T) * (x.double() @ wu.double().T)
     _close("Y", y, hidden.to(dtype).double() @ wd.double().T + bd.double())
+    assert torch.equal(y, run())
     if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
-        numbers = r"(?:ELi|, )(\d+)" * 4 + r"(?:ELb|, )(?:0|1|false|true)" + r"(?:ELi|, )(\d+)" * 2
-        found = [m.groups() for m in (re.search(r"decode_stream_kernel.*?" + numbers, e.name) for e in prof.events()) if m]
-        _, tiles, segment, _, rows, waves = map(int, found[-1])
-        assert (tiles, segment, rows, waves) == down, found
+        numbers = r"(?:ELi|, )(\d+)" * 4 + r"(?:ELb|, )(0|1|false|true)" + r"(?:ELi|, )(\d+)" * 2
+        found = [m.groups() for m in (re.search(r"decode_stream_kernel.*?" + numbers, n) for n in names) if m]
+        _, tiles, segment, slots, tail, rows, waves = found[-1]
+        assert (*map(int, (tiles, segment, slots)), int(tail in ("1", "true")), int(rows), int(waves)) == down, found
 
 
 def test_decode_streaming_entry_refuses_what_its_kernels_do_not_take():

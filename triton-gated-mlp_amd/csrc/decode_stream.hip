@@ -136,6 +136,11 @@ hipError_t launch_decode_stream(const T* x, const T* wg, const T* wu, const T* w
   // M=1: K=1024, N=4096 7.8 -> 6.2, K=2048, N=5632 9.5 -> 7.8, K=2048, N=8192 12.0 -> 9.7; M=16 9.5 -> 8.8 and 12.2 ->
   // 10.6; M=24 11.4 -> 10.7 and 13.7 -> 12.9.  Four wavefronts also for whole regions that a share leaves partly
   // empty (M=1: K=2560, N=6912 11.2 -> 9.5, K=3072, N=8192 12.3 -> 10.8; from 14 rows of 16 on equal or 2 % slower).
+  // Long segments, one token tile: three slots.  A wavefront has a few stages only, and the ones past the end cost
+  // their instructions: whole forwards (launches in a graph, K = 768 to 2048, every kind of row) take 0.92 of the time with
+  // six slots up to N = 4096, 0.96 around 8192, 0.97 beyond 12288 (two slots: 0.90, 0.95, 0.99), and 0.92 of the time
+  // with regions of 16 rows throughout.  M=1, K=2048, N=8192: 16 rows 23.4, six slots 22.5, three 21.8.  Two token tiles: 8
+  // rows take 0.98 of 16.
   const bool half = K <= 8 * num_cu;
   const bool one = K <= 16 * num_cu, lines = ds_whole_lines(N), four = K > 48 * num_cu && lines;
   if (M <= 16) {
@@ -144,7 +149,7 @@ hipError_t launch_decode_stream(const T* x, const T* wg, const T* wu, const T* w
              : K <= 13 * num_cu ? launch_stream<T, false, 1, 1, 128, 8, 16, 4>(a2, num_cu, s)
              : one              ? launch_stream<T, false, 1, 1, 128, 8>(a2, num_cu, s)
                                 : launch_stream<T, false, 2, 1, 128, 8>(a2, num_cu, s);
-    if (half) return launch_stream<T, false, 1, 1, 512, 6, 8>(a2, num_cu, s);
+    if (half) return launch_stream<T, false, 1, 1, 512, 3, 8>(a2, num_cu, s);
     if (one) return launch_stream<T, false, 1, 1, 512, 4>(a2, num_cu, s);
     return lines ? launch_stream<T, false, 2, 1, 256, 4>(a2, num_cu, s) : launch_stream<T, false, 2, 1, 512, 3>(a2, num_cu, s);
   }
