@@ -515,8 +515,8 @@ def test_m0_checker_flags_compiler_generated_m0_uses(tmp_path):
 
 def test_wait_states_around_inline_assembly_products_are_checked(tmp_path):
     """csrc/check_mfma.py (run on every GEMM unit by the build): an inline-assembly MFMA's result is left alone
-    by everything but in-place products for some wait states, along every path behind it, and its operands
-    are not written right before it."""
+    by everything but in-place products for some wait states, along every path behind it, its operands are not
+    written right before it, and no pipelined kernel's loop goes without."""
     import importlib.util
 
     spec = importlib.util.spec_from_file_location("check_mfma", ROOT / "triton-gated-mlp_amd" / "csrc" / "check_mfma.py")
@@ -526,6 +526,8 @@ def test_wait_states_around_inline_assembly_products_are_checked(tmp_path):
     settle = "\ts_nop 15\n\ts_nop 3\n"
     read = "\tv_accvgpr_read_b32 v9, a2\n"
     kernel = "_Z4kern:\n"
+    issued = "\tv_mfma_f32_16x16x32_f16 "  # by the compiler
+    pipelined = "_ZN4gmlp21gemm_kernel_pipelinedIDF16_Li256ELi256ELi16ELi2ELi2ELb0ELb0ELi1ENS_8EpiStoreIDF16_EELb%dELb0EEEvT_:\n"
     for text, violations in (
         (kernel + product + settle + read, 0),
         (kernel + product + product + settle + read, 0),                       # in place: ordered by the hardware
@@ -537,6 +539,18 @@ def test_wait_states_around_inline_assembly_products_are_checked(tmp_path):
         (kernel + product + "\ts_branch .LBB0_2\n" + read + ".LBB0_2:\n" + settle, 0),
         (kernel + "\tv_mov_b32_e32 v5, v8\n" + product + settle, 1),
         (kernel + "\tv_mov_b32_e32 v5, v8\n\ts_nop 3\n" + product + settle, 0),
+        (kernel + "\tv_swap_b32 v8, v5\n" + product + settle, 1),                                     # writes both
+        (kernel + "\tv_permlane32_swap_b32_e32 v8, v5\n" + product + settle, 1),
+        (kernel + "\tv_add_u32_e32 v8, v5, v6\n" + product + settle, 0),
+        (kernel + issued + "v[4:7], v[8:11], v[12:15], 0\n" + product + settle, 1),                    # its result as an operand
+        (kernel + issued + "v[4:7], v[8:11], v[12:15], 0\n" + settle + product + settle, 0),
+        (kernel + issued + "a[2:5], v[8:11], v[12:15], a[2:5]\n" + product + settle, 1),               # overlaps the accumulator
+        (kernel + issued + "a[0:3], v[8:11], v[12:15], a[0:3]\n" + product + settle, 0),               # in place
+        (kernel + product + settle + issued + "v[4:7], v[8:11], v[12:15], 0\n" + issued + "v[8:11], v[4:7], v[12:15], 0\n", 0),
+        (pipelined % 0 + product + settle + issued + "a[0:3], v[0:3], v[4:7], a[0:3]\n", 0),
+        (pipelined % 0 + product + settle + 2 * (issued + "a[0:3], v[0:3], v[4:7], a[0:3]\n"), 1),     # one of the loop's
+        (kernel + product + settle + "\ts_endpgm\n" + pipelined % 0 + issued + "a[0:3], v[0:3], v[4:7], a[0:3]\n", 1),
+        (kernel + product + settle + "\ts_endpgm\n" + pipelined % 1 + issued + "a[0:3], v[0:3], v[4:7], a[0:3]\n", 0),
     ):
         f = tmp_path / "k.s"
         f.write_text(text + "\ts_endpgm\n")

@@ -6,14 +6,18 @@ operand (Traits::mfma16_inplace).  The compiler's hazard recogniser does not loo
 the wait states that a matrix instruction needs are not inserted for it:
   * its result may be touched by any other kind of instruction only some wait states later (7 for the
     16x16x32 shape; SETTLE are asked for here);
+  * the result of a matrix instruction that the compiler issued may be its operand no sooner either, other than as
+    the accumulator in the very same registers;
   * a vector register that an ordinary vector instruction wrote may be its operand only 2 wait states later
     (FEED are asked for).
 In the source the accumulators are zeroed long before the loop, operands come from LDS reads (which the
 compiler does wait for) and mfma_settle() stands behind the last product.  What remains are copies that the
 register allocator may insert anywhere.  This scan follows every path of SETTLE wait states behind each
-inline-assembly MFMA, and of FEED behind each vector instruction, and fails if it finds one too close.
+MFMA, and of FEED behind each vector instruction, and fails if it finds one too close.
 
-A file in which no kernel with such instructions is recognised fails too.
+A file in which no kernel with such instructions is recognised fails too, and so does a pipelined kernel whose loops do
+not have them all: the last reduction tile, which the compiler issues, repeats the loop's tile, so there are as many
+of one kind as of the other (none in the stream-K kernels, which leave all products to the compiler).
 
 usage: check_mfma.py file.s     (exit status 1 on a violation)
 """
@@ -82,6 +86,12 @@ def follow(code, labels, start, budget, visit):
             i += 1
 
 
+# instructions that write both of their operands
+SWAPS = re.compile(r"v_(swap_|permlane(16|32)_swap_)")
+PIPELINED = re.compile(r"gemm_(group_|dx_dw_)?kernel_pipelined")
+STREAM_K = re.compile(r"gemm_kernel_pipelined.*Lb1ELb[01]EEEv")
+
+
 def check(path):
     lines = open(path).read().split("\n")
     starts = [i for i, l in enumerate(lines) if re.match(r"^_Z\w+:", l)] + [len(lines)]
@@ -89,18 +99,24 @@ def check(path):
     for begin, end in zip(starts, starts[1:]):
         name = lines[begin].split(":")[0]
         code, labels = parse([(n + 1, lines[n]) for n in range(begin + 1, end)])
-        mine = [i for i, (text, asm, _) in enumerate(code) if asm and text.startswith("v_mfma")]
+        matrix = [i for i, (text, _, _) in enumerate(code) if text.startswith("v_mfma")]
+        mine = sum(code[i][1] for i in matrix)
+        if PIPELINED.search(name) and 2 * mine != (0 if STREAM_K.search(name) else len(matrix)):
+            print(f"{path}: {name}: {mine} of {len(matrix)} matrix instructions are inline assembly")
+            failures += 1
         if not mine:
             continue
         kernels += 1
-        products += len(mine)
+        products += mine
         found = set()
-        for i in mine:
-            text, _, line = code[i]
+        for i in matrix:
+            text, inline, line = code[i]
             dst = registers(operands(text)[0])
 
             def near(other, asm, at):
                 if other.startswith("v_mfma"):
+                    if not (inline or asm):
+                        return
                     ops = operands(other)
                     used = [registers(o) for o in ops[:4]]
                     # (in place on the same registers is what the hardware orders by itself)
@@ -108,15 +124,14 @@ def check(path):
                         return
                     if any(u & dst for u in used):
                         found.add((line, at, other))
-                elif registers(other) & dst:
+                elif inline and registers(other) & dst:
                     found.add((line, at, other))
 
             follow(code, labels, i + 1, SETTLE, near)
         for i, (text, asm, line) in enumerate(code):
             if not text.startswith("v_") or text.startswith(("v_mfma", "v_cmp", "v_readfirstlane")):
                 continue
-            ops = operands(text)
-            dst = registers(ops[0]) if ops else set()
+            dst = registers(",".join(operands(text)[: 2 if SWAPS.match(text) else 1]))
             if not dst:
                 continue
 
