@@ -1,18 +1,407 @@
-// Skinny-M (M <= 32) forward in two launches, gate/up and down, on the streaming body of decode_stream.hpp.
+// Skinny-M (M <= 32) weight-streaming kernels, HBM-bound: every weight byte is fetched once, in
+// row segments of 128, 256 or 512 bytes moved global -> LDS without passing through registers.
+//
+// One persistent workgroup of three or four wavefronts per CU.  The workgroup takes blocks of weight rows
+// that share one set of token operands: 16 to 80 rows of W_gate and as many of W_up (GATED), or 8, 16,
+// 32 or 64 consecutive rows of W_down.  Whole blocks go round-robin over the workgroups, the rows that
+// do not fill a last round are shared out evenly as one partly empty block each.  Its wavefronts split
+// the reduction range in near-equal runs of chunks (64 to 256 elements) and combine their partial
+// sums through LDS at the end of each block (fixed order, so the result is deterministic).  Each
+// wavefront runs a private ring of 2 to 8 LDS slots; a slot holds one stage = one chunk of the
+// block's weight rows.  The matching token-row operands (x or H, L2-resident)
+// are fetched straight into registers, as many stages ahead: one 16-token tile for M <= 16, two
+// beyond (MT; the weight fragment read from LDS then feeds two MFMAs).  The stream of stages runs on
+// across block boundaries, so the ring never drains; the loads of stages past the end go nowhere (an offset beyond the
+// descriptor reads as zero and moves no data), which keeps the in-flight count constant.  (Fetching the last stage
+// again instead: whole forward M=24, K=4096, N=11008 55.8 us for 53.4, M=16, K=8192, N=28672 214.0 for 211.6.)
 //
 // Which block (chosen in launch_decode_stream; kernel times, us, fp16): the height decides what a block
 // costs in token operands and how well it fits a CU's share of the rows; the row segment of a stage (SEGB)
 // how evenly the chunks divide over the wavefronts (16 chunks of 256 elements at K = 4096: 6, 5 and 5; 64 of
 // 64: 22, 21 and 21), how soon the first MFMA can start, and how finely the ring's slots take up what the
 // loads in flight leave.  512- -> 128-byte segments, W_gate / W_up, 16 rows a block: K=2048, N=8192 M=8
-// 17.4 -> 14.6, M=16 19.1 -> 15.4; K=1024, N=4096 9.3 -> 7.1, 10.1 -> 7.6.  Bytes in flight do not decide at
-// 96 KiB per CU: four, six and eight wavefronts with 128 to 144 KiB were no faster on any of eleven
-// widths.
-#include "decode_stream.hpp"
+// 17.4 -> 14.6, M=16 19.1 -> 15.4; K=1024, N=4096 9.3 -> 7.1, 10.1 -> 7.6.  Bytes in flight do not decide once full
+// slots hold 96 KiB per CU: four, six and eight wavefronts with 128 to 144 KiB were no faster on any of eleven
+// widths.  Where a CU's share leaves slots partly empty they do: four wavefronts then, see launch_decode_stream.
+//
+//   GATED:   H[m, r] = act(x.W_gate[r] + b_gate[r]) * (x.W_up[r] + b_up[r])      (r over N)
+//   !GATED:  Y[m, r] = H.W_down[r] + b_down[r]                                   (r over K)
+//
+// LDS layout of a slot: regions of 16 (or 8, RR) rows x SEGB bytes; the 16-byte chunk c of row r is stored at
+// position c ^ r (128-byte segments, two rows to all banks: c ^ (r / 2)), so the 16 lanes that read one
+// chunk index of 16 different rows for v_mfma_f32_16x16x32 hit 16 different bank groups.
+//
+// All vector-memory loads of the main loop are written as assembly and ordered by explicit
+// s_waitcnt vmcnt(N): the compiler does not see them, so it cannot serialise them either (the
+// build checks the generated assembly for uses of a load's destination ahead of its wait).
+#include "launch.hpp"
+#include "lds_dma.hpp"
 
 namespace gmlp {
 
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+template <typename T>
+struct Mfma16x;
+template <>
+struct Mfma16x<f16> {
+  static __device__ __forceinline__ f32x4v run(f16x8 a, f16x8 b, f32x4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Mfma16x<bf16> {
+  static __device__ __forceinline__ f32x4v run(bf16x8 a, bf16x8 b, f32x4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+
+constexpr int DS_MAX_LDS = 160 * 1024;
+constexpr int DS_MIN_RED = 768;               // a chunk for every wavefront (three of 256 elements, four of 64)
+constexpr uint32_t DS_NOWHERE = 0x80000000u;  // voffset beyond any operand (operands are < 2 GiB)
 constexpr int DS_WIDE_SEGMENT_MAX_M = 20;     // see ds_tall_gated, ds_short_segments
+constexpr int DS_H_TILED_MIN_M = 10;           // H goes out in fragment order above this many token rows
+
+struct StreamArgs {
+  const void* x;      // [M, ldx] token rows (x or H)
+  const void* w[2];   // [R, red] weight matrices
+  const void* bias[2];
+  void* out;          // [M, ldo]
+  int M, R, red, ldx, ldo;
+  int act;            // Act code (GATED only)
+  int tiled;          // H (GATED: out, otherwise: x) is in fragment order, see ds_h_tiled()
+};
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes per lane into registers; completion is tracked by the caller (wait_vmem_keep).
+__device__ __forceinline__ i32x4 load16_async(buffer_rsrc r, uint32_t voffset, uint32_t soffset) {
+  i32x4 v;
+  asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"
+               : "=v"(v)
+               : "v"(voffset), "s"(r), "s"(soffset)
+               : "memory");
+  return v;
+}
+// s_waitcnt vmcnt(N) that also "defines" the registers a stage's token operands arrive in, so no use
+// of them can be scheduled above the wait.  The other statements issue no instruction: volatile asm
+// statements keep their order, so they tie the other registers to the same point.
+template <int N, int NX>
+__device__ __forceinline__ void wait_vmem_keep(i32x4 (&x)[NX]) {
+  static_assert(NX % 2 == 0, "pairs");
+  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(x[0]), "+v"(x[1]) : "n"(N) : "memory");
+#pragma unroll
+  for (int i = 2; i < NX; i += 2) asm volatile("" : "+v"(x[i]), "+v"(x[i + 1]) : : "memory");
+}
+
+// A workgroup barrier that orders LDS accesses only: loads in flight stay in flight.
+__device__ __forceinline__ void ds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// HALVES: regions per matrix and stage.
+// MT:   tiles of 16 token slots (M <= 16 * MT).
+// SEGB: bytes of a weight row per stage, 512, 256 or 128.
+// DS_RD: ring slots per wavefront and stages in flight.
+// TAIL: the reduction length need not be a multiple of the chunk (only of 8): the 16-byte pieces of the
+//       last chunk that lie beyond the row's end are pushed out of the descriptors, weights and token
+//       operands, and read as zeros.  An instance of its own: the others have no such selects.
+// RR:   rows of a region: 16, or 8, which the MFMA's rows 8 to 15 read again, for shares of the rows (see share)
+//       of no more than 8: of a 16-row slot only half would hold weights.
+// NW:   wavefronts.
+// (wg and G, the workgroup's number and count, are members and not read where they are used: the compiler then spills
+// twice the scalars, and over 1247 shapes the forward takes 1.02 of the time, small ones up to 1.15.  The same body as one
+// function takes 1.00 of it, 1.01 to 1.02 with two token tiles.)
+template <typename T, bool GATED, int HALVES, int MT, int SEGB, int DS_RD, bool TAIL, int RR, int NW>
+struct StreamBody {
+  typedef typename Traits<T>::vec8 vec8;
+  static_assert(SEGB == 512 || SEGB == 256 || SEGB == 128, "row segment of a stage");
+  static constexpr int NREG = (GATED ? 2 : 1) * HALVES;  // regions per stage
+  static constexpr int REGION = RR * SEGB;               // bytes of a region
+  static constexpr int CH = SEGB / 2;                    // reduction elements per stage
+  static constexpr int KS = CH / 32;                     // MFMA steps per stage
+  static constexpr int CPR = SEGB / 16;                  // 16-byte chunks per row segment
+  static constexpr int LPR = REGION / 1024;  // load instructions per region (64 lanes x 16 bytes each)
+  // The token operands in flight live in VGPRs that the loads fill asynchronously.  Were there not
+  // enough of the 256 left beside them, the compiler would park them elsewhere right after the
+  // load instruction, before the data has arrived.
+  static_assert(DS_RD * KS * MT * 4 <= 192, "token operands in flight must leave room in the VGPRs");
+  // weight rows (per matrix) a block advances by
+  static constexpr int BLOCK_ROWS = RR * HALVES;
+  static constexpr int SLOT = NREG * REGION;
+  static constexpr int LPS = KS * MT + NREG * LPR;  // load instructions per stage (token operands + weights)
+  // A stage is complete when no more than the DS_RD - 1 younger stages are in flight.  vmcnt has 6
+  // bits: where that count exceeds 63 the wait also covers the first token-operand loads of the
+  // next stage (issued right behind the awaited weights, and loads return in order).
+  static constexpr int YOUNGER = (DS_RD - 1) * LPS < 63 ? (DS_RD - 1) * LPS : 63;
+  static_assert((DS_RD - 1) * LPS - YOUNGER <= KS * MT, "the wait may only reach into the next stage's token operands");
+  // Partial sums change hands through LDS in two alternating buffers, or, where LDS does not hold
+  // two, in one buffer with a second barrier behind its readers.
+  static constexpr int RING_BYTES = NW * DS_RD * SLOT;
+  static constexpr int PART_FLOATS = (NW - 1) * NREG * MT * 256;
+  static constexpr int PARITIES = RING_BYTES + 2 * PART_FLOATS * 4 <= DS_MAX_LDS ? 2 : 1;
+  static constexpr int LDS_BYTES = RING_BYTES + PARITIES * PART_FLOATS * 4;
+  static_assert(LDS_BYTES <= DS_MAX_LDS, "a workgroup has 160 KiB of LDS");
+
+  static __device__ __forceinline__ int swz(int r) { return SEGB == 128 ? r >> 1 : r; }
+
+  int lane, wave, wg, G;
+  uint32_t lds_base;
+  char* ring;
+  float* part;  // [parities][waves-1][NREG][MT][64][4]
+  int full, t_begin, t_end, my_blocks, c0, spb, total, rot;
+  int r16, kg;
+  uint32_t woff[LPR], xoff[MT];
+  int wrow[LPR];    // row of the region that load q of this lane fetches
+  int wchunk[LPR];  // TAIL: and its 16-byte piece of the row's segment
+  bool tiled_x;
+  uint32_t xq, pitch;
+  i32x4 xf[DS_RD][KS * MT];  // [stage in flight][MFMA step q][token tile]
+  f32x4v acc[NREG][MT];
+
+  // Blocks of BLOCK_ROWS weight rows go round-robin over the workgroups (block b, b + G, ...: at any
+  // time the chip streams one contiguous band of rows) for as many rounds as every workgroup gets a
+  // whole block.  The rows left over (the tail) are shared out evenly instead, in multiples of 4
+  // (what one lane stores), so that every CU streams the same number of bytes whatever R is: a
+  // workgroup's tail share [t_begin, t_end) is one last block with fewer valid rows, the loads of
+  // the others go nowhere and their results are not stored.
+  __device__ __forceinline__ void share(const StreamArgs& a, int wg_, int G_) {
+    wg = wg_;
+    G = G_;
+    full = a.R / BLOCK_ROWS / G;
+    const int tail0 = full * G * BLOCK_ROWS, tail_rows = a.R - tail0;
+    t_begin = tail0 + ((wg * tail_rows / G) & ~3);
+    t_end = wg + 1 == G ? a.R : tail0 + (((wg + 1) * tail_rows / G) & ~3);
+    my_blocks = full + (t_end - t_begin + BLOCK_ROWS - 1) / BLOCK_ROWS;
+  }
+  // first row and number of existing rows (BLOCK_ROWS or more: all) of this workgroup's j-th block
+  __device__ __forceinline__ void block_rows(int j, int& row0, int& valid) const {
+    if (j < full) {
+      row0 = (wg + j * G) * BLOCK_ROWS;
+      valid = BLOCK_ROWS;
+    } else {
+      row0 = t_begin + (j - full) * BLOCK_ROWS;
+      valid = t_end - row0;
+    }
+  }
+
+  // A wavefront's part in the share of workgroup wg_ of G_.
+  __device__ __forceinline__ void start(const StreamArgs& a, char* smem, int wave_, int wg_, int G_) {
+    lane = threadIdx.x & 63;
+    wave = wave_;
+    lds_base = (uint32_t)(uintptr_t)(lds_void*)smem + wave * (DS_RD * SLOT);
+    ring = smem + wave * (DS_RD * SLOT);
+    part = (float*)(smem + RING_BYTES);
+    share(a, wg_, G_);
+    const int chunks = TAIL ? (a.red + CH - 1) / CH : a.red / CH;
+    // wavefront w reduces chunks [c0, c0 + spb)
+    c0 = (chunks * wave) / NW;
+    spb = (chunks * (wave + 1)) / NW - c0;
+    total = my_blocks * spb;
+    // Workgroup b starts each block at chunk b % spb of its wavefronts' ranges and wraps around (a
+    // sum does not mind the order).  Without it every workgroup on the chip reads the same offset
+    // along its rows at the same time, and for a power-of-two row pitch (W_gate, W_up of the usual
+    // hidden sizes) those addresses crowd onto a few memory channels: 154 -> 142 us at K = 8192.
+    rot = wg % spb;
+
+    // Per-lane byte offsets: weights, LPR load instructions per region (1024 / SEGB rows each);
+    // token operands, the 16 bytes of token row 16 t + lane%16 this lane feeds to the MFMAs of tile t.
+    r16 = lane & 15;
+    kg = lane >> 4;
+#pragma unroll
+    for (int q = 0; q < LPR; ++q) {
+      int row = (64 / CPR) * q + lane / CPR, pos = lane % CPR;
+      wrow[q] = row;
+      wchunk[q] = pos ^ swz(row);
+      woff[q] = (uint32_t)(row * a.red + (pos ^ swz(row)) * 8) * 2u;
+    }
+    tiled_x = !GATED && a.tiled;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      if (tiled_x) {
+        // [red/8][16 MT token slots][8 elements]: the 8-element group kg of a fragment is 256 MT
+        // bytes after the previous one (for MT = 1 a fragment is one contiguous KiB)
+        xoff[t] = (uint32_t)(kg * (256 * MT) + t * 256 + r16 * 16);
+      } else {
+        int xr = 16 * t + r16 < a.M ? 16 * t + r16 : a.M - 1;  // rows past M repeat the last token row
+        xoff[t] = (uint32_t)(xr * a.ldx + kg * 8) * 2u;
+      }
+    }
+    xq = tiled_x ? 1024u * MT : 64u;  // from one MFMA's token operand to the next
+    pitch = (uint32_t)a.red * 2u;
+#pragma unroll
+    for (int g = 0; g < NREG; ++g)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[g][t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  }
+
+  // Exact sizes: an offset past the end reads as zero instead of touching memory.  (Put together from the kernel's
+  // arguments where they are used: carried along as members they came to lie in VGPRs.)
+  __device__ __forceinline__ buffer_rsrc token_rsrc(const StreamArgs& a) const {
+    return make_rsrc(a.x, !GATED && a.tiled ? (uint32_t)(16 * MT) * (uint32_t)a.red * 2u : (uint32_t)a.M * (uint32_t)a.ldx * 2u);
+  }
+  // of region g of a stage: GATED: matrix g / HALVES, rows RR (g % HALVES) on of the block; otherwise rows
+  // RR g on of the block of W_down
+  __device__ __forceinline__ buffer_rsrc weight_rsrc(const StreamArgs& a, int g) const {
+    return make_rsrc(a.w[GATED ? g / HALVES : 0], (uint32_t)a.R * (uint32_t)a.red * 2u);
+  }
+
+  // Stage i of this wavefront's stream: where in the block and along the reduction it is, and how many
+  // 16-byte pieces of its segment lie inside the row (0: no such stage).
+  __device__ __forceinline__ void stage(const StreamArgs& a, int i, int& row0, int& valid, uint32_t& koff, int& pieces) const {
+    const bool past = i >= total;
+    const int ii = past ? total - 1 : i;
+    const int j = ii / spb;
+    int c = ii - j * spb + rot;
+    c = c < spb ? c : c - spb;
+    block_rows(j, row0, valid);
+    koff = (uint32_t)((c0 + c) * CH) * 2u;
+    pieces = past ? 0 : TAIL ? (a.red - (c0 + c) * CH) / 8 : CPR;
+    valid = past ? 0 : valid;
+  }
+  // Its token operands into xf[u].
+  __device__ __forceinline__ void issue_tokens(const StreamArgs& a, int i, int u) {
+    int row0, valid, pieces;
+    uint32_t koff;
+    stage(a, i, row0, valid, koff, pieces);
+    // token operand of the stage's q-th MFMA step: 64 bytes further along each row of x, or the
+    // next fragment of H (a stage of CH elements x 16 MT token slots)
+    const uint32_t xstage = tiled_x ? koff * (16u * MT) : koff;
+#pragma unroll
+    for (int q = 0; q < KS; ++q)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        xf[u][q * MT + t] = load16_async(token_rsrc(a), (TAIL ? q * 4 + kg < pieces : pieces > 0) ? xoff[t] : DS_NOWHERE, xstage + q * xq);
+  }
+  // Its weights into ring slot u.
+  __device__ __forceinline__ void issue_weights(const StreamArgs& a, int i, int u) {
+    int row0, valid, pieces;
+    uint32_t koff;
+    stage(a, i, row0, valid, koff, pieces);
+    uint32_t slot = lds_base + (uint32_t)u * SLOT;
+    uint32_t woffs = (uint32_t)row0 * pitch + koff;
+#pragma unroll
+    for (int g = 0; g < NREG; ++g) {
+      const int first = GATED ? RR * (g % HALVES) : RR * g;  // region's first row within the block
+      const int valid_g = valid - first;
+#pragma unroll
+      for (int q = 0; q < LPR; ++q)
+        load16_to_lds<true>(weight_rsrc(a, g),
+                            wrow[q] < valid_g && (!TAIL || wchunk[q] < pieces) ? woff[q] : DS_NOWHERE,
+                            woffs + (uint32_t)first * pitch, slot + g * REGION + q * 1024);
+    }
+  }
+  __device__ __forceinline__ void issue_stage(const StreamArgs& a, int i, int u) {
+    issue_tokens(a, i, u);
+    issue_weights(a, i, u);
+  }
+
+  // Block blk's sums, this wavefront's (0) and those that the others left in LDS, and what comes of them.  A
+  // lane holds, per token tile t, token row 16 t + lane%16 and, per region, weight rows 4*(lane/16) + r of
+  // the region.
+  __device__ __forceinline__ void finish_block(const StreamArgs& a, int blk, const float* pp) {
+    int row0, valid;
+    block_rows(blk, row0, valid);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const int tok = 16 * t + r16;
+      if (!((GATED && a.tiled) || tok < a.M)) continue;
+      float v[NREG][4];
+#pragma unroll
+      for (int g = 0; g < NREG; ++g) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[g][r] = acc[g][t][r];
+#pragma unroll
+        for (int w = 0; w < NW - 1; ++w) {
+          f32x4v o = *(const f32x4v*)(pp + ((w * NREG + g) * MT + t) * 256 + lane * 4);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[g][r] += o[r];
+        }
+        // this lane's four rows of the region, as rows of the block
+        const int first = (GATED ? RR * (g % HALVES) : RR * g) + 4 * kg;
+        const T* bias = (const T*)a.bias[GATED ? g / HALVES : 0];
+        if (bias && 4 * kg < RR && first < valid) add_w<T, 4>(bias + row0 + first, v[g]);
+      }
+      if (GATED) {
+#pragma unroll
+        for (int hf = 0; hf < HALVES; ++hf) {
+          const int first = RR * hf + 4 * kg;
+          const int r0 = row0 + first;
+          float res[4];
+          act_fwd_w<4>(a.act, v[hf], res);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) res[r] *= v[HALVES + hf][r];
+          // Fragment order: H goes out the way the down projection's MFMAs take it in,
+          // [N/8][16 MT token slots][8 elements], so that a token-operand fragment there is
+          // 4 runs of 256 MT bytes (one contiguous KiB for MT = 1) instead of 16 row pieces
+          // of 64 bytes.  All slots are written (slots past M repeat the last token), so
+          // nothing uninitialised is multiplied.
+          if (4 * kg < RR && first < valid)
+            store_w<T, 4>(a.tiled ? (T*)a.out + ((size_t)(r0 >> 3) * (16 * MT) + tok) * 8 + (r0 & 7)
+                                  : (T*)a.out + (size_t)tok * a.ldo + r0,
+                          res);
+        }
+      } else {
+#pragma unroll
+        for (int g = 0; g < NREG; ++g)
+          if (4 * kg < RR && RR * g + 4 * kg < valid)
+            store_w<T, 4>((T*)a.out + (size_t)tok * a.ldo + row0 + RR * g + 4 * kg, v[g]);
+      }
+    }
+  }
+
+  // All stages, the first DS_RD of which are in flight.  Loads of stages past the end may be in flight behind it.
+  __device__ __forceinline__ void run(const StreamArgs& a) {
+    int in_block = 0, blk = 0;
+    for (int i0 = 0; i0 < total; i0 += DS_RD) {
+#pragma unroll
+      for (int u = 0; u < DS_RD; ++u) {
+        const int i = i0 + u;
+        if (i < total) {
+          wait_vmem_keep<YOUNGER, KS * MT>(xf[u]);
+          const char* slot = ring + u * SLOT;
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            int pos = ((ks * 4 + kg) ^ swz(RR == 16 ? r16 : r16 & (RR - 1))) << 4;
+#pragma unroll
+            for (int g = 0; g < NREG; ++g) {
+              vec8 wf = *(const vec8*)(slot + g * REGION + (RR == 16 ? r16 : r16 & (RR - 1)) * SEGB + pos);
+#pragma unroll
+              for (int t = 0; t < MT; ++t)
+                acc[g][t] = Mfma16x<T>::run(wf, __builtin_bit_cast(vec8, xf[u][ks * MT + t]), acc[g][t]);
+            }
+          }
+          // The MFMAs above consumed every LDS read of this slot, so it can be refilled.
+          issue_stage(a, i + DS_RD, u);
+
+          if (++in_block == spb) {
+            // Block finished: wavefronts 1.. hand their partial sums to wavefront 0.
+            in_block = 0;
+            float* pp = part + (PARITIES == 2 ? (blk & 1) * PART_FLOATS : 0);
+            if (wave > 0) {
+#pragma unroll
+              for (int g = 0; g < NREG; ++g)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                  *(f32x4v*)(pp + (((wave - 1) * NREG + g) * MT + t) * 256 + lane * 4) = acc[g][t];
+            }
+            ds_barrier();
+            if (wave == 0) finish_block(a, blk, pp);
+            // one buffer: nobody writes the next block's partial sums before wavefront 0 has read these
+            if (PARITIES == 1) ds_barrier();
+#pragma unroll
+            for (int g = 0; g < NREG; ++g)
+#pragma unroll
+              for (int t = 0; t < MT; ++t) acc[g][t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+            ++blk;
+          }
+        }
+      }
+    }
+  }
+};
 
 template <typename T, bool GATED, int HALVES, int MT, int SEGB, int DS_RD, bool TAIL, int RR, int NW>
 __global__ void __launch_bounds__(NW * 64) decode_stream_kernel(StreamArgs a) {
@@ -30,7 +419,10 @@ static hipError_t launch_stream_tail(const StreamArgs& a, int num_cu, hipStream_
   constexpr int LDS = StreamBody<T, GATED, HALVES, MT, SEGB, RD, TAIL, RR, NW>::LDS_BYTES;
   constexpr auto kern = decode_stream_kernel<T, GATED, HALVES, MT, SEGB, RD, TAIL, RR, NW>;
   if (hipError_t e = allow_dynamic_lds(lds_kernel_of<kern, LDS>, s)) return e;
-  hipLaunchKernelGGL(kern, dim3(ds_grid(a.R, num_cu)), dim3(NW * 64), LDS, s, a);
+  // one workgroup per CU, each with its share of the rows (a partly empty block when that is less
+  // than a block); fewer workgroups when a share would be under 8 rows
+  int grid = a.R / 8 < num_cu ? a.R / 8 : num_cu;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), LDS, s, a);
   return hipGetLastError();
 }
 template <typename T, bool GATED, int HALVES, int MT, int SEGB, int RD, int RR = 16, int NW = 3>
@@ -39,6 +431,11 @@ static hipError_t launch_stream(const StreamArgs& a, int num_cu, hipStream_t s) 
     if (a.red % (SEGB / 2) != 0) return launch_stream_tail<T, GATED, HALVES, MT, SEGB, RD, true, RR, NW>(a, num_cu, s);
   return launch_stream_tail<T, GATED, HALVES, MT, SEGB, RD, false, RR, NW>(a, num_cu, s);
 }
+
+// Layout of the intermediate H between the two kernels.  Row-major [M, N] costs the down projection
+// M pieces of 64 bytes per token-operand fragment, fragment order always one KiB (16 token slots):
+// cheaper from about half-full upwards.  Two token tiles always use fragment order.
+static int ds_h_tiled(int M) { return M > DS_H_TILED_MIN_M ? 1 : 0; }
 
 bool decode_stream_supported(int M, int K, int N) {
   return M >= 1 && M <= 32 && K % 8 == 0 && N % 8 == 0 && K >= DS_MIN_RED && N >= DS_MIN_RED &&
