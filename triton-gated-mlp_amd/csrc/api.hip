@@ -238,8 +238,11 @@ int64_t red_tiles_of(int kind, int64_t red) { return (kind == DX ? 2 : 1) * cdiv
 // tiles gain less once a CU has two: base + half up to f = 1/2, 1 at f = 1).  A split reduction adds a
 // second launch and the partial sums' round trip.  All constants are one least-squares fit to 3100
 // launches (five GEMMs of 89 random shapes, M 33 to 6000, widths 128 to 15000, every class and split;
-// standard deviation of the estimates 3 to 12 %); the class chosen costs 1.5 % over the fastest on
-// average.
+// standard deviation of the estimates 3 to 12 %); the class chosen cost 1.5 % over the fastest on
+// average.  The kernels are faster since (accumulators in place; eight wavefronts on WIDE): of 1929 launches of those, the
+// class chosen costs 2.2 % over the fastest for gate/up, 5.9 % for dH and 2.5 % for the down projection.  Constants
+// fitted to them cost 1.6, 4.8 and 3.0 %, and no whole pass of 22 moved by more than 1 %: these stay.  What they misjudge, for
+// one: gate/up at M=1024, K=2048, N=5632, 55 us estimated on LARGE and 63 on WIDE, takes 52 and 50.
 struct TileCost {
   int tile_class;
   int rows, col_div, per_cu;
@@ -249,7 +252,7 @@ struct TileCost {
 };
 const TileCost kLarge = {gmlp::TILE_LARGE, 256, 1, 1, 0.69, 0, {1.443, 1.477, 1.494}, {11.4, 6.1, 19.0, 6.8, 7.1, 12.0}};
 const TileCost kWide = {gmlp::TILE_WIDE, 128, 1, 1, 0.74, 0, {0.846, 0.940, 0.983}, {5.7, 2.7, 9.7, 3.3, 3.7, 2.0}};
-// (TALL: fitted the same way to 160 launches, four GEMMs of 40 shapes, standard deviation 7 %; it is the
+// (TALL, four wavefronts: fitted the same way to 160 launches, four GEMMs of 40 shapes, standard deviation 7 %; it is the
 // fastest unsplit class in 55 of them, by up to 27 %.  bf16, back to back, without and with the class:
 // gate/up with biases, G and U kept, at M=1357, K=1160, N=3096 44.1 -> 35.3 us (gelu 44.1 -> 37.5, silu
 // without G and U 37.6 -> 28.8), M=1346, K=2264, N=8120 111 -> 106, dH at M=2048, K=2048, N=5632 60 -> 54,

@@ -3,8 +3,8 @@
 // Same contract as gemm_kernel (gemm.hpp): C[M,N] = sum_s sum_k A_s[m,k] * B_s[n,k], operands
 // reduction-contiguous (KC) or reduction-strided (KS), NB accumulator sets, fused epilogue.
 // Reduction tiles of 64 elements travel global -> LDS without passing through registers
-// (gemm_tiles.hpp) into a two-slot ring (three slots for the A operand of the plain-store GEMMs with a
-// long reduction, see PipeConfig::A3); the epilogue transposes accumulators (or finished
+// (gemm_tiles.hpp) into a two-slot ring (three slots for reduction-contiguous A operands, dH's on 256-row tiles
+// aside, and for both operands of 128x256 tiles, see PipeConfig::A3); the epilogue transposes accumulators (or finished
 // results) through LDS so that every global access is a 16-byte, row-contiguous one.
 //
 // Ragged edges cost nothing in the main loop: operands are read through buffer descriptors of
@@ -22,7 +22,8 @@
 // Per 512/MI-wide reduction step a wavefront issues G groups of TM MFMAs: group g multiplies one
 // B fragment (accumulator set b, column block j; G = NB * TN) with the step's TM A fragments.
 // Operands roll through registers instead of being double-buffered a whole step at a time:
-//   * A fragments: two banks of TM; during step s, group g fetches A fragment g of step s+1;
+//   * A fragments: two banks of TM; during step s, group g fetches A fragment g of step s+1 (fragments 2g and 2g+1
+//     where there are more fragments than groups: 192-row tiles of eight wavefronts);
 //   * B fragments: a ring of 4; group g fetches the B fragment of group g+LA (LA = 3 by default).
 // That is 2*TM + 4 fragments in flight (72 VGPRs for the 16x16x32 shape instead of 128), which is
 // what lets v_mfma_f32_16x16x32 be used with a 128x128 register tile: it moves a fifth fewer
@@ -47,7 +48,7 @@ constexpr int LOAD_CYCLES = 64;
 constexpr int B_LOOKAHEAD = 3;
 
 // Kernels that get the three-entry A ring (see PipeConfig::A3): those with a reduction-contiguous A
-// operand other than dH on 256-row tiles, i.e. gate/up, the down projection, the input gradient and dH.  The long
+// operand, i.e. gate/up, the down projection, the input gradient, and dH on tiles of fewer than 256 rows.  The long
 // reductions over the intermediate size gain most (they stall on a full vector-memory queue
 // otherwise), gate/up gains from a cold start only.  dH's epilogue prefetch on 256-row tiles and the weight
 // gradients' two transposed operands leave no registers for it (spills when tried).  dH on 128x128 tiles (bf16, us,
@@ -404,12 +405,14 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
   // registers per reduction tile, dX's partial sums on 256-row ones 72, each copy waiting for a product): 128x256
   // tiles at M=2048, N=4096, K=4096 57.7 -> 54.6 us, 1500 -> 1316 clocks per reduction tile; training step at M=8192,
   // K=4096, N=14336 (fp16) 6617 -> 6465 us.  The last reduction tile is left to the compiler, which copies and
-  // converts the accumulators behind it.
+  // converts the accumulators behind it, and so are stream-K pieces (120 us of that step; the loop of the down
+  // projection's has no copies, that of dX's 40 to 128 products; in place not measured there).
   auto mma = [&](auto next_c, acc_t& c, const vec8& b, const vec8& a) __attribute__((always_inline)) {
     if constexpr (decltype(next_c)::value && !SK) Traits<T>::mfma16_inplace(b, a, c);
     else c = Traits<T>::mfma16(b, a, c);
   };
-  // One reduction tile.  NEXT: tile kt+1 exists.  The wavefront is alone on its SIMD: whatever
+  // One reduction tile.  NEXT: tile kt+1 exists.  The schedule is that of a wavefront alone on its SIMD, as it is on
+  // 192- and 256-row tiles of four wavefronts (otherwise two share it): whatever
   // issues between two MFMAs is hidden behind the matrix pipe, so every group is laid out as TM
   // slots of {one MFMA; at most a couple of LDS fetches or one global->LDS load} and the
   // scheduler is told to keep the slots.
@@ -439,7 +442,7 @@ __device__ __forceinline__ void gemm_pipelined_body(const GemmArgs& ga, const ty
             else if (!last) fetch_b(((ks + 1) * G + g2 - G) % 4, g2 - G, kt, ks + 1);
             else if (NEXT) fetch_b((g2 - G) % 4, g2 - G, kt + 1, 0);
           }
-          // --- A fragments of the next step: one per group, or all of them after the handover
+          // --- A fragments of the next step: APG per group, or all of them after the handover
           if (!last) {
             const int h = g * Cfg::APG + (i - 1);
             if (i >= 1 && i <= Cfg::APG && h < TM) fetch_a((ks + 1) & 1, h, kt, ks + 1);
