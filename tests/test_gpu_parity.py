@@ -1368,9 +1368,10 @@ _LONG_EPILOGUES = [
     (893, 712, 5112, (192, 128, 8), (192, 128, 8), (128, 128, 4)),    # 12 reduction tiles; three loads of A a wavefront
     (900, 960, 4104, (192, 128, 8), (192, 128, 8), (128, 128, 4)),    # 15
     (900, 968, 4104, (192, 128, 4), (192, 128, 8), (128, 128, 4)),    # 16: SiLU's epilogue no longer outweighs the loop
-    (900, 1472, 4104, (192, 128, 4), (192, 128, 8), (128, 128, 4)),   # 23
-    (900, 1480, 4104, (192, 128, 4), (192, 128, 4), (128, 128, 4)),   # 24: nor does GELU's
-    (900, 1536, 4104, (192, 128, 4), (192, 128, 4), (128, 128, 4)),
+    (900, 1536, 4104, (192, 128, 4), (192, 128, 8), (128, 128, 4)),   # 24
+    (900, 1984, 4104, (192, 128, 4), (192, 128, 8), (128, 128, 4)),   # 31
+    (900, 1992, 4104, (192, 128, 4), (192, 128, 4), (128, 128, 4)),   # 32: nor does GELU's
+    (900, 2048, 4104, (192, 128, 4), (192, 128, 4), (128, 128, 4)),
     (1289, 464, 6344, (128, 64, 4), (128, 64, 4), (192, 256, 4)),     # dH: three ring entries of A
     (391, 64, 136, (128, 64, 4), (128, 64, 4), (128, 128, 4)),        # one reduction tile: the loop in place does not run
 ]

@@ -45,15 +45,16 @@ constexpr bool KT = GMLP_KT;
 // Gate/up on TALL tiles: the shorter epilogue of eight wavefronts against their slower loop, by the reduction's
 // length.  Time with four over eight by the number of 64-wide reduction tiles, weights from memory / from cache (geometric
 // means over 1396 launches of random shapes):
-//                          8..11        12..15       16..19       20..23       32..35       48..55       96 on
-//   SiLU (packed)      1.07 / 1.08  1.02 / 1.05  0.98 / 1.03  0.96 / 1.02  0.93 / 1.00  0.91 / 0.98  0.89 / 0.90
-//   other activations  1.13 / 1.14  1.07 / 1.10  1.02 / 1.08  1.00 / 1.06  0.95 / 1.03  0.93 / 1.00  0.91 / 0.90
-// The lines are where the ones from memory cross: a model's layers come by in turn, and its weights with them.  us, eight ->
-// four: M=3582, K=3200, N=11992 G and U kept 518 -> 482; M=1357, K=1160, N=3096 gelu stays on eight (37.3 with four, 34.3).
-// On WIDE tiles eight are never behind (1.03 at 20 tiles, 1.00 from 96 on).
+//                          8..11        12..15       16..19       20..23       28..31       32..35       48..55       96 on
+//   SiLU (packed)      1.07 / 1.08  1.02 / 1.05  0.98 / 1.03  0.96 / 1.02  0.94 / 1.01  0.93 / 1.00  0.91 / 0.98  0.89 / 0.90
+//   other activations  1.13 / 1.14  1.07 / 1.10  1.02 / 1.08  1.00 / 1.06  0.97 / 1.04  0.95 / 1.03  0.93 / 1.00  0.91 / 0.90
+// The lines are about where what eight lose from memory (a model's layers come by in turn, and its weights with them) outweighs
+// what they gain from cache (one layer called over and over).  us, eight -> four: M=3582, K=3200, N=11992 G and U kept 518 ->
+// 482; M=1357, K=1160, N=3096 gelu stays on eight (37.3 with four, 34.3).  On WIDE tiles eight are never behind (1.03 at 20
+// tiles, 1.00 from 96 on).
 template <typename Epi>
 static bool gate_up_eight_wavefronts(const GemmArgs& ga) {
-  return ga.K <= 64 * (std::is_same<Epi, EpiGateUpPacked<DT>>::value ? 15 : 23);
+  return ga.K <= 64 * (std::is_same<Epi, EpiGateUpPacked<DT>>::value ? 15 : 31);
 }
 template <>
 hipError_t launch_gateup_kt<DT, KT>(int tile_class, const GemmArgs& ga, const EpiGateUp<DT>::Args& ea,
